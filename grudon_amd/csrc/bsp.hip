@@ -294,63 +294,98 @@ __global__ void __launch_bounds__(kBlock) k_bcast_recv(uint32_t nw, const uint64
 // traversal: push over the active list (degree-binned, LDS-staged tiles)
 // ------------------------------------------------------------------------
 
-// A block stages 256 active vertices in LDS.  Vertices with out-degree below
-// kHeavyDeg are processed together: the block scans their degrees and every thread
-// walks the concatenated edge range (coalesced col reads), locating its
-// source by binary search in the LDS prefix array.  Vertices with degree
-// >= kHeavyDeg are appended to the heavy list as chunks of kHeavyDeg arcs and
-// handled by k_push_heavy, one workgroup per chunk.
+// owner of position j among a tile's 256 offsets: the last t with s_off[t] <= j
+// (s_off[0] = 0; eight halvings, no branch)
+__device__ __forceinline__ uint32_t push_owner(const uint32_t *s_off, uint32_t j)
+{
+  uint32_t t = 0;
+#pragma unroll
+  for (uint32_t step = kBlock / 2; step > 0; step >>= 1)
+    if (s_off[t + step] <= j) t += step;
+  return t;
+}
+
+// A block stages `tile` active vertices in LDS (256, or 64 where the frontier
+// would not fill the chip with tiles of 256).  Vertices with out-degree below
+// kHeavyDeg are processed together: the block scans their degrees and every
+// thread walks the concatenated edge range (coalesced col reads), locating its
+// source by binary search in the LDS prefix array, four arcs in flight per
+// thread.  Vertices with degree >= kHeavyDeg are appended to the heavy list as
+// chunks of kHeavyChunk arcs (one counter atomic per tile) and handled by
+// k_push_heavy, one workgroup per chunk.
+//
+// The active list is in degree order, so the vertices just below the threshold
+// share tiles: the threshold bounds a tile's work.  With 4096 (and chunks of
+// 4096) the first tiles held a million arcs each and ran alone: CC by pushes
+// over RMAT-20 symmetrized (31 M arcs) 16.7 ms a solve, with 256 and chunks of
+// 1024 3.4 ms.
 template <class Op>
 __global__ void __launch_bounds__(kBlock) k_push(const uint32_t *__restrict__ AL, const uint32_t *__restrict__ nact,
                                                  const uint32_t *__restrict__ rp, const uint32_t *__restrict__ col,
                                                  const uint32_t *__restrict__ wt, const typename Op::V *__restrict__ mprop,
-                                                 typename Op::V *upd, uint64_t *dirty, uint2 *heavy, Counters *cnt)
+                                                 typename Op::V *upd, uint64_t *dirty, uint2 *heavy, Counters *cnt,
+                                                 uint32_t tile)
 {
   using V = typename Op::V;
-  __shared__ uint32_t s_off[kBlock + 1];
+  constexpr int kIlp = 4;
+  __shared__ uint32_t s_off[kBlock];
   __shared__ uint32_t s_beg[kBlock];
   __shared__ V s_val[kBlock];
+  __shared__ unsigned long long s_slot;
   const uint32_t k = *nact;
   uint64_t my_edges = 0;
-  for (uint32_t tile = blockIdx.x * kBlock; tile < k; tile += gridDim.x * kBlock) {
-    uint32_t i = tile + threadIdx.x;
-    uint32_t deg = 0, beg = 0;
+  for (uint32_t t0 = blockIdx.x * tile; t0 < k; t0 += gridDim.x * tile) {
+    const uint32_t i = t0 + threadIdx.x;
+    uint32_t deg = 0, beg = 0, p = 0, nch = 0;
     V v = op_identity<Op>();
-    if (i < k) {
-      uint32_t p = AL[i];
+    if (threadIdx.x < tile && i < k) {
+      p = AL[i];
       beg = rp[p];
       deg = rp[p + 1] - beg;
       v = mprop[p];
-      if (deg >= kHeavyDeg) {
-        const uint32_t nch = (deg + kHeavyDeg - 1) / kHeavyDeg;
-        unsigned long long slot = atomicAdd(&cnt->heavy, (unsigned long long)nch);
-        for (uint32_t c = 0; c < nch; c++) heavy[slot + c] = make_uint2(p, c * kHeavyDeg);
-        atomicAdd(&cnt->heavy_edges, (unsigned long long)deg);
-        deg = 0;
+      if (deg >= kHeavyDeg) nch = (deg + kHeavyChunk - 1) / kHeavyChunk;
+    }
+    if (__syncthreads_or(nch != 0)) {
+      uint32_t hch, hdeg;
+      const uint32_t at = block_excl_scan(nch, &hch);
+      (void)block_excl_scan(nch ? deg : 0u, &hdeg);
+      if (threadIdx.x == 0) {
+        s_slot = atomicAdd(&cnt->heavy, (unsigned long long)hch);
+        atomicAdd(&cnt->heavy_edges, (unsigned long long)hdeg);
       }
+      __syncthreads();
+      for (uint32_t c = 0; c < nch; c++) heavy[s_slot + at + c] = make_uint2(p, c * kHeavyChunk);
+      if (nch) deg = 0;
     }
     uint32_t total;
-    uint32_t ex = block_excl_scan(deg, &total);
+    const uint32_t ex = block_excl_scan(deg, &total);
     s_off[threadIdx.x] = ex;
     s_beg[threadIdx.x] = beg;
     s_val[threadIdx.x] = v;
-    if (threadIdx.x == 0) s_off[kBlock] = total;
     __syncthreads();
-    for (uint32_t j = threadIdx.x; j < total; j += kBlock) {
-      // owner t: last index with s_off[t] <= j
-      uint32_t lo = 0, hi = kBlock;
-      while (hi - lo > 1) {
-        uint32_t mid = (lo + hi) >> 1;
-        if (s_off[mid] <= j) lo = mid;
-        else hi = mid;
+    for (uint32_t j0 = threadIdx.x; j0 < total; j0 += kIlp * kBlock) {
+      uint32_t c[kIlp], w[kIlp];
+      V x[kIlp];
+#pragma unroll
+      for (int q = 0; q < kIlp; q++) {
+        const uint32_t j = j0 + q * kBlock;
+        const uint32_t t = push_owner(s_off, j);
+        const uint32_t e = j < total ? s_beg[t] + (j - s_off[t]) : s_beg[0];
+        c[q] = 0;
+        w[q] = 1u;
+        if (j < total) {
+          c[q] = col[e];
+          if (wt) w[q] = wt[e];
+        }
+        x[q] = s_val[t];
       }
-      uint32_t e = s_beg[lo] + (j - s_off[lo]);
-      relax<Op>(upd, dirty, col[e], Op::edge(s_val[lo], wt ? wt[e] : 1u));
+#pragma unroll
+      for (int q = 0; q < kIlp; q++) x[q] = Op::edge(x[q], w[q]);
+      relax_many<Op, kIlp>(upd, dirty, c, x, (total - j0 + kBlock - 1) / kBlock);
     }
     if (threadIdx.x == 0) my_edges += total;
     __syncthreads();
   }
-  my_edges = block_sum(my_edges);
   if (threadIdx.x == 0 && my_edges) atomicAdd(&cnt->edges, (unsigned long long)my_edges);
 }
 
@@ -361,13 +396,30 @@ __global__ void __launch_bounds__(kBlock) k_push_heavy(const uint2 *__restrict__
                                                        const typename Op::V *__restrict__ mprop, typename Op::V *upd,
                                                        uint64_t *dirty)
 {
+  using V = typename Op::V;
+  constexpr int kIlp = kHeavyChunk / kBlock;
   const uint32_t nch = (uint32_t)cnt->heavy;
   for (uint32_t h = blockIdx.x; h < nch; h += gridDim.x) {
-    const uint2 c = heavy[h];
-    const uint32_t end = rp[c.x + 1];
-    const uint32_t b = rp[c.x] + c.y, e = min(end, b + kHeavyDeg);
-    const typename Op::V v = mprop[c.x];
-    for (uint32_t x = b + threadIdx.x; x < e; x += kBlock) relax<Op>(upd, dirty, col[x], Op::edge(v, wt ? wt[x] : 1u));
+    const uint2 ch = heavy[h];
+    const uint32_t end = rp[ch.x + 1];
+    const uint32_t b = rp[ch.x] + ch.y, e = min(end, b + kHeavyChunk);
+    const V v = mprop[ch.x];
+    if (b + threadIdx.x >= e) continue;
+    uint32_t c[kIlp], w[kIlp];
+    V x[kIlp];
+#pragma unroll
+    for (int q = 0; q < kIlp; q++) {
+      const uint32_t at = b + threadIdx.x + q * kBlock;
+      c[q] = 0;
+      w[q] = 1u;
+      if (at < e) {
+        c[q] = col[at];
+        if (wt) w[q] = wt[at];
+      }
+    }
+#pragma unroll
+    for (int q = 0; q < kIlp; q++) x[q] = Op::edge(v, w[q]);
+    relax_many<Op, kIlp>(upd, dirty, c, x, (e - b - threadIdx.x + kBlock - 1) / kBlock);
   }
 }
 
@@ -695,8 +747,9 @@ grd_status state_alloc(grd_state *s)
   GRD_TRY(m.alloc_n(&s->wrankR, nwP));
   GRD_TRY(m.alloc_n(&s->totals, 64));
   GRD_TRY(m.alloc_n(&s->AL, S));
-  // heavy chunks: sum over heavy vertices of ceil(deg / kHeavyDeg) <= 2 m / kHeavyDeg
-  GRD_TRY(m.alloc_n(&s->heavy, 2 * (g->m / kHeavyDeg) + 64));
+  // heavy chunks: a vertex's last chunk may be short, and at most m / kHeavyDeg
+  // vertices are heavy
+  GRD_TRY(m.alloc_n(&s->heavy, g->m / kHeavyChunk + g->m / kHeavyDeg + 64));
   GRD_TRY(m.alloc(&s->partial, (uint64_t)std::max<uint32_t>(1, g->n_pblk) * 8));
   if (s->algo == GRD_PR_PULL) {
     GRD_TRY(m.alloc_n(&s->red, 2ull * prp_grid(g)));
@@ -940,13 +993,18 @@ static grd_status traverse_t(grd_state *s, int option)
     if (timed && s->skip_pending && s->prm.time_kernel != 2) GRD_TRY(pull_done_arcs(s));
     s->edges += g->m;  // every arc of the memory partitions, less those left out (counters)
   } else {
-    uint32_t want = (uint32_t)std::min<uint64_t>((s->last_frontier + kBlock - 1) / kBlock, (uint64_t)ctx->num_cus * 8);
-    uint32_t grid = std::max<uint32_t>(1, want);
+    // tiles of 64 active vertices until those fill every workgroup slot
+    const uint64_t slots = (uint64_t)ctx->num_cus * 8;
+    const uint32_t tile = s->last_frontier <= 64 * slots ? 64u : (uint32_t)kBlock;
+    const uint32_t grid = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((s->last_frontier + tile - 1) / tile, slots));
     if (timed) GRD_HIP(hipEventRecord(s->kev[0], st));
     hipLaunchKernelGGL((k_push<Op>), dim3(grid), dim3(kBlock), 0, st, s->AL, s->totals + 0, g->rp, g->col, wt,
-                       (const V *)s->mprop, (V *)s->mupd, s->Du, s->heavy, s->cnt);
-    hipLaunchKernelGGL((k_push_heavy<Op>), dim3(ctx->num_cus * 4), dim3(kBlock), 0, st, s->heavy, s->cnt, g->rp, g->col,
-                       wt, (const V *)s->mprop, (V *)s->mupd, s->Du);
+                       (const V *)s->mprop, (V *)s->mupd, s->Du, s->heavy, s->cnt, tile);
+    // a vertex's out-arcs all hang off its own proxy, so the frontier's largest
+    // out-degree tells whether any chunk was appended
+    if (s->last_maxdeg >= kHeavyDeg)
+      hipLaunchKernelGGL((k_push_heavy<Op>), dim3((uint32_t)slots), dim3(kBlock), 0, st, s->heavy, s->cnt, g->rp, g->col,
+                         wt, (const V *)s->mprop, (V *)s->mupd, s->Du);
     if (timed) {
       GRD_HIP(hipEventRecord(s->kev[1], st));
       s->kern_pending = 2;  // bytes from the edge counters after the iteration

@@ -111,7 +111,8 @@ struct TierTile {
 constexpr uint32_t kPullNnz = 2048;     // arcs per block (8 per thread)
 constexpr uint32_t kPullMaxRows = 1024;  // rows per block
 constexpr uint32_t kPullHot = 2048;      // PR pull: hottest sources of a partition kept in LDS
-constexpr uint32_t kHeavyDeg = 4096;     // push: out-degree handled by k_push_heavy, in chunks of this many arcs
+constexpr uint32_t kHeavyDeg = 256;      // push: out-degree handled by k_push_heavy,
+constexpr uint32_t kHeavyChunk = 1024;   // in chunks of this many arcs (a workgroup each)
 constexpr uint32_t kShipTile = 1024;     // edge shipping: wire positions per workgroup tile
 constexpr int kMaxParts = 64;            // largest C and M
 constexpr uint32_t kTierBitsMax = 15;    // tiled pull: largest tier, 2^15 sources (128 KB of LDS)

@@ -77,6 +77,39 @@ __device__ __forceinline__ void relax(typename Op::V *upd, uint64_t *dirty, uint
   }
 }
 
+// relax for the first cnt of N destinations of one thread: the current values
+// are all loaded before any is compared, and the atomics are all issued before
+// any dirty mark waits for one
+template <class Op, int N>
+__device__ __forceinline__ void relax_many(typename Op::V *upd, uint64_t *dirty, const uint32_t (&dst)[N],
+                                           const typename Op::V (&cand)[N], uint32_t cnt)
+{
+  bool on[N], mark[N];
+#pragma unroll
+  for (int q = 0; q < N; q++) on[q] = (uint32_t)q < cnt;
+  if constexpr (Op::kMin) {
+    uint32_t cur[N], old[N];
+#pragma unroll
+    for (int q = 0; q < N; q++) cur[q] = on[q] ? __atomic_load_n(upd + dst[q], __ATOMIC_RELAXED) : 0u;
+#pragma unroll
+    for (int q = 0; q < N; q++) {
+      on[q] = cand[q] < cur[q];
+      old[q] = on[q] ? atomicMin(upd + dst[q], cand[q]) : 0u;
+    }
+#pragma unroll
+    for (int q = 0; q < N; q++) mark[q] = on[q] && cand[q] < old[q];
+  } else {
+    float old[N];
+#pragma unroll
+    for (int q = 0; q < N; q++) old[q] = on[q] ? atomicAdd(upd + dst[q], cand[q]) : 1.0f;
+#pragma unroll
+    for (int q = 0; q < N; q++) mark[q] = on[q] && old[q] == 0.0f;
+  }
+#pragma unroll
+  for (int q = 0; q < N; q++)
+    if (mark[q]) set_bit(dirty, dst[q]);
+}
+
 // relax without the dirty mark; returns whether the destination must be
 // marked (same rules as relax)
 template <class Op, bool kAlwaysMark = false>
