@@ -913,14 +913,25 @@ static grd_status build_hotcold(grd_graph *g)
     total += bcost.back();
   }
   std::vector<TierTile> ranges;
-  const uint64_t nwg = 16ull * (uint64_t)std::max(1, ctx->num_cus);  // sixteen per CU, in turn: dynamic balance
+  // Up to sixteen ranges per CU, in turn, for dynamic balance; but staging the
+  // window costs a workgroup about 3 us, so a range is given at least
+  // kRangeCost of work (about 10 us), and never fewer blocks than it has waves.
+  // With sixteen per CU at every size the staging alone moved 0.5 GB: the hot
+  // pass of RMAT-18 took 53 us for 4 M arcs, a million vertices 73 us (pull
+  // PageRank 3.2 -> 2.5 ms a solve with this rule); 32 K to 512 K of work per
+  // range measured alike, and RMAT-24 / 25 are unchanged.
+  constexpr uint64_t kRangeCost = 65536;
+  const uint64_t cus = (uint64_t)std::max(1, ctx->num_cus);
+  const uint64_t nwg = cus * std::max<uint64_t>(1, std::min<uint64_t>(16, total / (kRangeCost * cus)));
   for (uint32_t mp = 0; mp < M; mp++) {
     const uint32_t b0 = pblk0[mp], b1 = pblk0[mp + 1];
     if (b0 == b1) continue;
     const uint32_t wbase = pb[mp], wlen = std::min<uint32_t>(win, pb[mp + 1] - pb[mp]);
     uint64_t cm = 0;
     for (uint32_t i = b0; i < b1; i++) cm += bcost[i];
-    const uint64_t k = std::max<uint64_t>(1, std::min<uint64_t>(b1 - b0, cm * nwg / std::max<uint64_t>(total, 1)));
+    // a range keeps at least every wave of its workgroup busy
+    const uint64_t most = (b1 - b0 + kTierBlock / kWave - 1) / (kTierBlock / kWave);
+    const uint64_t k = std::max<uint64_t>(1, std::min<uint64_t>(most, cm * nwg / std::max<uint64_t>(total, 1)));
     uint64_t acc = 0;
     uint32_t start = b0, j = 1;
     for (uint32_t i = b0; i < b1 && j < k; i++) {
