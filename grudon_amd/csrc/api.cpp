@@ -555,6 +555,7 @@ grd_status grd_state_create_typed(grd_graph *g, int algo, uint32_t value_bytes, 
   if ((algo == GRD_PR_PULL && pm != 0) || pm == 3) {
     try {
       st = build_tiers(g);
+      if (st == GRD_OK && g->tier_mode == 3) st = build_cold(g, algo, &s->cold);
     } catch (const std::bad_alloc &) {
       st = fail(GRD_ERR_OOM, "tiled pull: host allocation failed");
     }

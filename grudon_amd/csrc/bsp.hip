@@ -773,7 +773,7 @@ grd_status state_alloc(grd_state *s)
       // hot / cold: one 4-byte partial per row and per hot segment
       GRD_TRY(m.alloc(reinterpret_cast<void **>(&s->tpart), std::max<uint64_t>(g->n_pairs, 1) * 4));
       GRD_TRY(m.alloc(reinterpret_cast<void **>(&s->tseg), (uint64_t)std::max<uint32_t>(g->n_tblk, 1) * 4));
-      GRD_TRY(m.alloc_n(&s->cseg, std::max<uint32_t>(g->n_cblk, 1)));
+      GRD_TRY(m.alloc_n(&s->cseg, std::max<uint32_t>(s->cold->nblk, 1)));
     } else {
       GRD_TRY(m.alloc_n(&s->tpart, std::max<uint64_t>(g->n_pairs, 1)));
       GRD_TRY(m.alloc_n(&s->tseg, std::max<uint32_t>(g->n_tblk, 1)));
@@ -781,7 +781,7 @@ grd_status state_alloc(grd_state *s)
   }
   if (s->Rdone) {
     // one flag per row block of the pull this state runs
-    const uint32_t nblk = bsp_hot_cold(s) ? g->n_cblk : g->n_pblk;
+    const uint32_t nblk = bsp_hot_cold(s) ? s->cold->nblk : g->n_pblk;
     GRD_TRY(m.alloc_n(&s->bskip, std::max<uint32_t>(nblk, 1)));
     if (bsp_hot_cold(s)) GRD_TRY(m.alloc_n(&s->hskip, std::max<uint32_t>(g->n_tblk, 1)));
   }
@@ -984,7 +984,7 @@ static grd_status traverse_t(grd_state *s, int option)
       // byte in the hot / cold split when every weight fits), a value per
       // row, and the rows-done bitmap; the arcs and rows of the blocks left
       // out come off when the counters are read
-      const uint64_t wb = !cwt ? 0 : (bsp_hot_cold(s) && g->cow8) ? 1 : 4;
+      const uint64_t wb = !cwt ? 0 : (bsp_hot_cold(s) && g->w8_fits) ? 1 : 4;
       s->kern_pending_bytes = (8 + wb) * g->m + 8ull * g->P + (s->rdone_sent ? g->P / 8 : 0);
       s->skip_arc_bytes = 8 + wb;
     }

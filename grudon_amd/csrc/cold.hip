@@ -1,0 +1,457 @@
+// cold.hip -- the cold pass of the hot / cold pull: the arcs outside each
+// partition's LDS window, gathered in source order.
+//
+// The rows (one per memory proxy) are cut into blocks of at most N arcs
+// (cold_set).  The arcs of a block are kept sorted by source, each with the
+// 16-bit place its value has in the block's row order (cpos).  A workgroup
+// takes one block:
+//   1. stage: the threads walk the block's arcs in source order, gather the
+//      values and store each at its place in LDS, so that LDS holds the
+//      block's values in row order;
+//   2. reduce: groups of G lanes reduce the rows from LDS, each row's hot
+//      partial first.
+//
+// Why sorted: the pass is bound by the rate at which the L2 serves gather
+// requests (about 175 G/s on random 4-byte loads, whatever the bytes), and
+// neighbouring lanes that fall into one 128-byte line make one request.  Sources are numbered in
+// degree order, so the sources of 16384 cold arcs repeat the same lines often
+// (RMAT-25, M = 4: 0.66 lines per arc, 0.90 in blocks of 2048).  Pull PageRank
+// over RMAT-25: requests to the L2 307 M -> 230 M a pass, 1.93 -> 1.67 ms; what
+// is left is the L2's misses (84 M lines, 6.4 TB/s from the fabric): every XCD
+// draws the partition's 33 MB of values through its own 4 MB.  Loads that go
+// past the L1 measured the same, nontemporal ones 1.7 times slower.
+#include <rocprim/block/block_radix_sort.hpp>
+
+#include <algorithm>
+
+#include "grd_device.hpp"
+#include "grd_internal.hpp"
+#include "grd_ops.hpp"
+
+namespace grd {
+
+namespace {
+
+// arcs in flight per thread
+constexpr int kBatch = 8;
+
+// lanes per row of a block of nrows rows for a workgroup of T threads
+template <int T>
+__device__ __forceinline__ uint32_t cold_group(uint32_t nrows)
+{
+  uint32_t g = kWave;
+  while (g > 1 && g * nrows > (uint32_t)T) g >>= 1;
+  return g;
+}
+
+// The row sums of one round: groups of G lanes over [b, e) of the staged
+// values; the sum is valid in the group's first lane.  A row much longer than
+// its group is left to the whole wave (blocks mix rows of one arc with rows of
+// thousands; a lane alone takes about 30 ns per compensated add).  Called by
+// the whole wave.
+constexpr uint32_t kWideRow = 24;  // arcs per lane beyond which the wave takes the row
+template <class Pol>
+__device__ __forceinline__ typename Pol::Acc cold_row(const typename Pol::V *s_v, uint32_t b, uint32_t e, uint32_t G)
+{
+  const uint32_t lane = lane_id(), sub = lane % G;
+  const bool wide = G < (uint32_t)kWave && e - b > kWideRow * G;
+  auto a = Pol::zero();
+  if (!wide)
+    for (uint32_t x = b + sub; x < e; x += G) Pol::add(a, s_v[x]);
+  Pol::merge_lanes(a, (int)G);
+  uint64_t m = __ballot(wide && sub == 0);
+  while (m) {
+    const int src = __ffsll((unsigned long long)m) - 1;
+    m &= m - 1;
+    const uint32_t wb = __shfl(b, src, kWave), we = __shfl(e, src, kWave);
+    auto t = Pol::zero();
+    for (uint32_t x = wb + lane; x < we; x += kWave) Pol::add(t, s_v[x]);
+    Pol::merge_lanes(t, kWave);
+    if ((int)lane == src) a = t;
+  }
+  return a;
+}
+
+// one segment of a long row: every thread over its staged values in order, the
+// waves merged in wave order by the first thread, which gets the sum
+template <class Pol, int T>
+__device__ __forceinline__ typename Pol::Acc cold_segment(const typename Pol::V *s_v, uint32_t ne)
+{
+  using Acc = typename Pol::Acc;
+  __shared__ uint64_t s_w[T / kWave];
+  static_assert(sizeof(Acc) <= 8, "an accumulator fits its slot");
+  auto a = Pol::zero();
+  for (uint32_t x = threadIdx.x; x < ne; x += T) Pol::add(a, s_v[x]);
+  Pol::merge_lanes(a, kWave);
+  if (lane_id() == 0) *reinterpret_cast<Acc *>(&s_w[wave_in_block()]) = a;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    for (int j = 1; j < T / kWave; j++) Pol::merge(a, *reinterpret_cast<const Acc *>(&s_w[j]));
+  return a;
+}
+
+template <int T, int N>
+__global__ void __launch_bounds__(T, 8) k_prp_pull_cold(const PullBlock *__restrict__ blocks,
+                                                        const uint32_t *__restrict__ rptr,
+                                                        const uint32_t *__restrict__ col,
+                                                        const uint16_t *__restrict__ pos,
+                                                        const float *__restrict__ mprop, float *__restrict__ out,
+                                                        float2 *__restrict__ partial, const float *__restrict__ pre)
+{
+  __shared__ float s_v[N];
+  const PullBlock d = blocks[blockIdx.x];
+  const uint32_t ne = d.e1 - d.e0;
+  const uint32_t G = cold_group<T>(d.nrows), ngroups = T / G;
+  const uint32_t rounds = (d.nrows + ngroups - 1) / ngroups, r1 = d.r0 + d.nrows;
+  // the first round's rows are loaded with the columns
+  uint32_t r = d.r0 + threadIdx.x / G, b = 0, e = 0;
+  float hot = 0.0f;
+  auto row = [&]() {
+    b = e = 0;
+    if (r < r1) {
+      b = rptr[r] - d.e0;
+      e = rptr[r + 1] - d.e0;
+      hot = pre[r];
+    }
+  };
+  row();
+  for (uint32_t i0 = threadIdx.x; i0 < ne; i0 += kBatch * T) {
+    uint32_t c[kBatch], p[kBatch];
+    float v[kBatch];
+#pragma unroll
+    for (int k = 0; k < kBatch; k++) {
+      const uint32_t i = i0 + k * T;
+      c[k] = i < ne ? col[d.e0 + i] : col[d.e0 + i0];
+      p[k] = i < ne ? pos[d.e0 + i] : pos[d.e0 + i0];
+    }
+#pragma unroll
+    for (int k = 0; k < kBatch; k++) v[k] = mprop[c[k]];
+    // (a thread's arcs past the end repeat its first one)
+#pragma unroll
+    for (int k = 0; k < kBatch; k++) s_v[p[k]] = v[k];
+  }
+  __syncthreads();
+  if (d.nrows == 0) {
+    const Kahan t = cold_segment<HotPR, T>(s_v, ne);
+    if (threadIdx.x == 0) partial[blockIdx.x] = make_float2(t.s, t.c);
+    return;
+  }
+  for (uint32_t k = 0; k < rounds; k++) {  // the same rounds for every group: the shuffles stay in step
+    const uint32_t rn = r, bn = b, en = e;
+    const float hn = hot;
+    r += ngroups;
+    row();  // the next round's rows are in flight during this one's sums
+    const Kahan acc = cold_row<HotPR>(s_v, bn, en, G);
+    if (threadIdx.x % G == 0 && rn < r1) {
+      Kahan t;
+      t.s = hn;  // the row's hot partial comes first
+      t.merge(acc.s, acc.c);
+      out[rn] = t.value();
+    }
+  }
+}
+
+// CC / SSSP / reference PageRank.  flag (skip): 1 = the block is left out, 2 =
+// some of its rows are done.  bcnt: a row whose hot partial is already at or
+// below the bound takes no cold candidate below it (every cold candidate is at
+// least the bound), so it gathers nothing and its result is the hot partial.
+template <class Op, class W, int T, int N>
+__global__ void __launch_bounds__(T, 8) k_bsp_pull_cold(const PullBlock *__restrict__ blocks,
+                                                        const uint32_t *__restrict__ rptr,
+                                                        const uint32_t *__restrict__ col,
+                                                        const uint16_t *__restrict__ pos, const W *__restrict__ cw,
+                                                        const typename Op::V *__restrict__ mprop,
+                                                        typename Op::V *__restrict__ upd, uint64_t *__restrict__ dirty,
+                                                        typename Op::V *__restrict__ partial,
+                                                        const typename Op::V *__restrict__ pre,
+                                                        const uint8_t *__restrict__ skip,
+                                                        const uint64_t *__restrict__ done,
+                                                        const uint64_t *__restrict__ hasarc,
+                                                        const Counters *__restrict__ bcnt, uint32_t inc)
+{
+  using V = typename Op::V;
+  using Pol = HotBsp<Op>;
+  __shared__ V s_v[N];
+  __shared__ unsigned long long s_dirty[kColdRows / 64 + 2];
+  const PullBlock d = blocks[blockIdx.x];
+  const uint32_t flag = skip ? skip[blockIdx.x] : 0u;
+  if (flag == 1) return;
+  const uint32_t ne = d.e1 - d.e0;
+  const uint32_t bnd = bcnt ? pull_bound(bcnt, inc) : 0u;
+  if (d.nrows == 0 && bcnt && pre[d.r0] <= bnd) {  // a segment of a row that gathers nothing
+    if (threadIdx.x == 0) partial[blockIdx.x] = op_identity<Op>();
+    return;
+  }
+  const uint32_t G = cold_group<T>(d.nrows), ngroups = T / G, sub = threadIdx.x % G;
+  const uint32_t rounds = (d.nrows + ngroups - 1) / ngroups, r1 = d.r0 + d.nrows;
+  const uint32_t w0 = d.r0 >> 6;
+  for (uint32_t i = threadIdx.x; i < d.nrows / 64 + 2; i += T) s_dirty[i] = 0ull;
+  // a done row, or one without arcs, has nothing to apply (its hot partial may
+  // not have been written)
+  auto live_row = [&](uint32_t q) {
+    if (!done) return true;
+    const uint64_t bit = 1ull << (q & 63);
+    return !(done[q >> 6] & bit) && (hasarc[q >> 6] & bit);
+  };
+  const bool marked = d.nrows != 0 && (flag == 2 || bcnt);  // uniform over the block
+  if (marked) {
+    // every place of the block is marked first: the identity where the row
+    // gathers nothing, 0 where the arc's value is wanted
+    for (uint32_t k = 0; k < rounds; k++) {
+      const uint32_t q = d.r0 + k * ngroups + threadIdx.x / G;
+      if (q < r1) {
+        bool gat = live_row(q);
+        if (gat && bcnt) gat = pre[q] > bnd;
+        const uint32_t b = rptr[q] - d.e0, e = rptr[q + 1] - d.e0;
+        for (uint32_t x = b + sub; x < e; x += G) s_v[x] = gat ? V(0) : op_identity<Op>();
+      }
+    }
+    __syncthreads();
+  }
+  for (uint32_t i0 = threadIdx.x; i0 < ne; i0 += kBatch * T) {
+    uint32_t c[kBatch], p[kBatch], w[kBatch];
+    bool on[kBatch];
+#pragma unroll
+    for (int k = 0; k < kBatch; k++) {
+      const uint32_t i = i0 + k * T;
+      on[k] = i < ne;
+      c[k] = on[k] ? col[d.e0 + i] : 0u;
+      p[k] = on[k] ? pos[d.e0 + i] : 0u;
+      w[k] = 1u;
+      if constexpr (Pol::kWeighted)
+        if (on[k]) w[k] = (uint32_t)cw[d.e0 + i];
+    }
+    if (marked) {
+#pragma unroll
+      for (int k = 0; k < kBatch; k++) on[k] = on[k] && s_v[p[k]] == V(0);
+    }
+    V v[kBatch];
+#pragma unroll
+    for (int k = 0; k < kBatch; k++) v[k] = on[k] ? mprop[c[k]] : V(0);
+#pragma unroll
+    for (int k = 0; k < kBatch; k++)
+      if (on[k]) s_v[p[k]] = Op::edge(v[k], w[k]);
+  }
+  __syncthreads();
+  if (d.nrows == 0) {
+    const V t = cold_segment<Pol, T>(s_v, ne);
+    if (threadIdx.x == 0) partial[blockIdx.x] = t;
+    return;
+  }
+  uint32_t r = d.r0 + threadIdx.x / G, b = 0, e = 0;
+  bool live = false;
+  V hot = op_identity<Op>();
+  auto row = [&]() {
+    b = e = 0;
+    live = r < r1 && live_row(r);
+    if (live) {
+      b = rptr[r] - d.e0;
+      e = rptr[r + 1] - d.e0;
+      hot = pre[r];
+    }
+  };
+  row();
+  for (uint32_t k = 0; k < rounds; k++) {
+    const uint32_t rn = r, bn = b, en = e;
+    const bool ln = live;
+    const V hn = hot;
+    r += ngroups;
+    row();
+    const V acc = op_combine<Op>(hn, cold_row<Pol>(s_v, bn, en, G));  // the row's hot partial first
+    if (sub == 0 && ln && pull_apply<Op>(upd, rn, acc)) atomicOr(&s_dirty[(rn >> 6) - w0], 1ull << (rn & 63));
+  }
+  __syncthreads();
+  const uint32_t nw = ((r1 - 1) >> 6) - w0 + 1;
+  for (uint32_t i = threadIdx.x; i < nw; i += T)
+    if (s_dirty[i]) atomicOr((unsigned long long *)(dirty + w0 + i), s_dirty[i]);
+}
+
+// Flags of the cold blocks (k_blocks_done of pull.hip, with a wave per block:
+// a block spans up to kColdRows rows): 1 = every row with arcs is done, 2 =
+// some are; counts the arcs and rows left out.
+__global__ void __launch_bounds__(kBlock) k_cold_blocks_done(uint32_t nblk, const PullBlock *__restrict__ blocks,
+                                                             const uint64_t *__restrict__ done,
+                                                             const uint64_t *__restrict__ hasarc,
+                                                             uint8_t *__restrict__ bskip, Counters *cnt)
+{
+  unsigned long long arcs = 0, rows = 0;
+  const uint32_t lane = lane_id();
+  for (uint32_t b = blockIdx.x * kWavesPerBlock + wave_in_block(); b < nblk; b += gridDim.x * kWavesPerBlock) {
+    const PullBlock d = blocks[b];
+    const uint32_t r1 = d.r0 + max(d.nrows, 1u);
+    bool all = true, any = false;
+    for (uint32_t w = (d.r0 >> 6) + lane; w <= (r1 - 1) >> 6; w += kWave) {
+      const uint32_t lo = max(d.r0, w * 64) - w * 64, hi = min(r1 - w * 64, 64u);
+      const uint64_t mask = (hi - lo == 64) ? ~0ull : (((1ull << (hi - lo)) - 1ull) << lo);
+      const uint64_t dn = done[w], ha = hasarc[w];
+      all = all && ((dn | ~ha) & mask) == mask;
+      any = any || (dn & ha & mask) != 0;
+    }
+    all = __ballot(!all) == 0;
+    any = __ballot(any) != 0;
+    if (lane == 0) {
+      bskip[b] = all ? 1 : any ? 2 : 0;
+      if (all) {
+        arcs += d.e1 - d.e0;
+        rows += d.nrows;
+      }
+    }
+  }
+  arcs = block_sum(arcs);
+  rows = block_sum(rows);
+  if (threadIdx.x == 0) {
+    if (arcs) atomicAdd(&cnt->pull_skipped, arcs);
+    if (rows) atomicAdd(&cnt->pull_skipped_rows, rows);
+  }
+}
+
+// Sorts each block's arcs by source in place (once per graph): the columns
+// come in row order, leave in source order with their row-order places in pos,
+// the weights with them.  Sources below 2^bits; padding keys sort last.
+template <class W, int T, int N>
+__global__ void __launch_bounds__(T) k_cold_sort(const PullBlock *__restrict__ blocks, uint32_t *__restrict__ col,
+                                                 W *__restrict__ cw, uint16_t *__restrict__ pos, int bits)
+{
+  constexpr int kPer = N / T;
+  using Sort = rocprim::block_radix_sort<uint32_t, T, kPer, uint16_t>;
+  __shared__ typename Sort::storage_type s_sort;
+  const PullBlock d = blocks[blockIdx.x];
+  const uint32_t ne = d.e1 - d.e0;
+  uint32_t key[kPer];
+  uint16_t at[kPer];
+#pragma unroll
+  for (int k = 0; k < kPer; k++) {
+    const uint32_t i = threadIdx.x + k * T;
+    key[k] = i < ne ? col[d.e0 + i] : 1u << bits;
+    at[k] = (uint16_t)i;
+  }
+  Sort().sort_to_striped(key, at, s_sort, 0, bits + 1);
+  W w[kPer];
+  if (cw) {
+#pragma unroll
+    for (int k = 0; k < kPer; k++) w[k] = threadIdx.x + k * T < ne ? cw[d.e0 + at[k]] : W(0);
+  }
+  __syncthreads();  // every weight is read before one is written
+#pragma unroll
+  for (int k = 0; k < kPer; k++) {
+    const uint32_t i = threadIdx.x + k * T;
+    if (i < ne) {
+      col[d.e0 + i] = key[k];
+      pos[d.e0 + i] = at[k];
+      if (cw) cw[d.e0 + i] = w[k];
+    }
+  }
+}
+
+}  // namespace
+
+// Cold set 0 serves the sums (pull and reference PageRank), 1 the min-combines
+// (CC, SSSP).  While a partition's values fit an L2 (2^20 sources, 4 MB) small
+// blocks are best for both: more of them in flight.  Beyond, the sums take
+// 16384 arcs, two workgroups per CU (pull PageRank over RMAT-23: 9.2 ms a solve
+// against 10.2 with 2048, RMAT-24 20.7 / 23.0, RMAT-25 46.3 / 53.2, RMAT-26
+// 118 / 126; 32768 arcs leave one workgroup per CU, whose two steps then do
+// not overlap: 50.2).  The min-combines leave out blocks and rows that cannot
+// improve, which large blocks do worse: CC over RMAT-24 symmetrized 4.98 ms
+// with 4096 arcs, 5.06 with 2048, 5.38 with 16384.
+uint32_t cold_set(const grd_graph *g, int algo, uint32_t *nnz)
+{
+  uint32_t widest = 0;
+  for (int m = 0; m < g->M; m++) {
+    uint64_t own = 0;
+    for (int c = 0; c < g->C; c++) own += g->ocnt[(size_t)m * g->C + c];
+    widest = std::max<uint32_t>(widest, (uint32_t)own);
+  }
+  const bool sums = algo == GRD_PR || algo == GRD_PR_PULL, large = widest > (1u << 20);
+  *nnz = !large ? 2048 : sums ? 16384 : 4096;
+  return large && !sums ? 1 : 0;
+}
+
+#define COLD_SHAPES(nnz, F)            \
+  switch (nnz) {                       \
+  case 2048: F(256, 2048); break;      \
+  case 4096: F(256, 4096); break;      \
+  default: F(1024, 16384);             \
+  }
+
+grd_status cold_sort(grd_graph *g, const ColdSet &c)
+{
+  hipStream_t st = g->ctx->stream;
+  if (!c.nblk) return GRD_OK;
+  int bits = 1;
+  while (bits < 31 && (g->P >> bits)) bits++;
+#define F(T, N)                                                                                                     \
+  if (c.w8)                                                                                                         \
+    hipLaunchKernelGGL((k_cold_sort<uint8_t, T, N>), dim3(c.nblk), dim3(T), 0, st, c.blk, c.col, c.w8, c.pos, bits); \
+  else                                                                                                              \
+    hipLaunchKernelGGL((k_cold_sort<uint32_t, T, N>), dim3(c.nblk), dim3(T), 0, st, c.blk, c.col, c.w, c.pos, bits)
+  COLD_SHAPES(c.nnz, F)
+#undef F
+  GRD_HIP(hipGetLastError());
+  return GRD_OK;
+}
+
+grd_status prp_pull_cold(grd_state *s, float *out, const float *pre)
+{
+  grd_graph *g = s->g;
+  const ColdSet &c = *s->cold;
+  hipStream_t st = g->ctx->stream;
+  if (!c.nblk) return GRD_OK;
+#define F(T, N)                                                                                           \
+  hipLaunchKernelGGL((k_prp_pull_cold<T, N>), dim3(c.nblk), dim3(T), 0, st, c.blk, g->corp, c.col, c.pos, \
+                     (const float *)s->mprop, out, s->cseg, pre)
+  COLD_SHAPES(c.nnz, F)
+#undef F
+  GRD_HIP(hipGetLastError());
+  return GRD_OK;
+}
+
+template <class Op>
+grd_status bsp_pull_cold(grd_state *s, const uint8_t *skip, const Counters *bcnt)
+{
+  grd_graph *g = s->g;
+  const ColdSet &c = *s->cold;
+  using V = typename Op::V;
+  hipStream_t st = g->ctx->stream;
+  if (!c.nblk) return GRD_OK;
+  const uint64_t *done = skip ? (const uint64_t *)s->Rdone : nullptr, *ha = skip ? (const uint64_t *)g->rarc : nullptr;
+#define L(W, w, T, N)                                                                                             \
+  hipLaunchKernelGGL((k_bsp_pull_cold<Op, W, T, N>), dim3(c.nblk), dim3(T), 0, st, c.blk, g->corp, c.col, c.pos, \
+                     (const W *)w, (const V *)s->mprop, (V *)s->mupd, s->Du, (V *)s->cseg, (const V *)s->tpart,  \
+                     skip, done, ha, bcnt, s->bound_inc)
+  if constexpr (std::is_same<Op, OpWeighted>::value) {
+    if (c.w8) {
+#define F(T, N) L(uint8_t, c.w8, T, N)
+      COLD_SHAPES(c.nnz, F)
+#undef F
+      GRD_HIP(hipGetLastError());
+      return GRD_OK;
+    }
+  }
+#define F(T, N) L(uint32_t, c.w, T, N)
+  COLD_SHAPES(c.nnz, F)
+#undef F
+#undef L
+  GRD_HIP(hipGetLastError());
+  return GRD_OK;
+}
+template grd_status bsp_pull_cold<OpCC>(grd_state *, const uint8_t *, const Counters *);
+template grd_status bsp_pull_cold<OpHop>(grd_state *, const uint8_t *, const Counters *);
+template grd_status bsp_pull_cold<OpWeighted>(grd_state *, const uint8_t *, const Counters *);
+template grd_status bsp_pull_cold<OpPR>(grd_state *, const uint8_t *, const Counters *);
+
+grd_status cold_blocks_done(grd_state *s)
+{
+  grd_graph *g = s->g;
+  const ColdSet &c = *s->cold;
+  if (c.nblk)
+    hipLaunchKernelGGL(k_cold_blocks_done,
+                       dim3(std::min<uint32_t>((c.nblk + kWavesPerBlock - 1) / kWavesPerBlock,
+                                               (uint32_t)g->ctx->num_cus * 8)),
+                       dim3(kBlock), 0, g->ctx->stream, c.nblk, c.blk, (const uint64_t *)s->Rdone,
+                       (const uint64_t *)g->rarc, s->bskip, s->cnt);
+  GRD_HIP(hipGetLastError());
+  return GRD_OK;
+}
+
+}  // namespace grd

@@ -108,9 +108,23 @@ struct PullLong {
 struct TierTile {
   uint32_t b0, nb, wbase, wlen;
 };
+// the cold arcs of the hot / cold split cut into row blocks of at most nnz
+// arcs, each block's arcs in source order (cold.hip)
+struct ColdSet {
+  uint32_t nnz = 0;         // arcs per block (0: not built)
+  uint32_t *col = nullptr;  // [cold arcs] source proxies
+  uint16_t *pos = nullptr;  // [cold arcs] the arc's place in its block's row order
+  uint32_t *w = nullptr;    // [cold arcs] arc weights (weighted graphs), as col
+  uint8_t *w8 = nullptr;    // the same as bytes, in their place when every weight is below 256
+  PullBlock *blk = nullptr;
+  uint32_t nblk = 0;
+  PullLong *lng = nullptr;
+  uint32_t nlong = 0;
+};
 constexpr uint32_t kPullNnz = 2048;     // arcs per block (8 per thread)
 constexpr uint32_t kPullMaxRows = 1024;  // rows per block
 constexpr uint32_t kPullHot = 2048;      // PR pull: hottest sources of a partition kept in LDS
+constexpr uint32_t kColdRows = 8192;     // hot / cold pull: most rows per cold block
 constexpr uint32_t kHeavyDeg = 256;      // push: out-degree handled by k_push_heavy,
 constexpr uint32_t kHeavyChunk = 1024;   // in chunks of this many arcs (a workgroup each)
 constexpr uint32_t kShipTile = 1024;     // edge shipping: wire positions per workgroup tile
@@ -222,16 +236,10 @@ struct grd_graph {
   // partial per row)
   uint32_t *hrp = nullptr;          // [P+1] hot arcs of each row
   uint32_t *corp = nullptr;         // [P+1] cold arcs of each row
-  uint32_t *cocol = nullptr;        // [cold arcs] source proxies
   uint32_t *hw = nullptr;           // [hot arcs] arc weights (weighted graphs), as tcol
-  uint32_t *cow = nullptr;          // [cold arcs] arc weights (weighted graphs), as cocol
   uint8_t *hw8 = nullptr;           // the same as bytes, in their place when every weight is below 256
-  uint8_t *cow8 = nullptr;
-  grd::PullBlock *cblk = nullptr;   // row blocks over the cold arcs
-  uint32_t *cblk_hot = nullptr;     // per cold block: its LDS window base (P: none)
-  uint32_t n_cblk = 0;
-  grd::PullLong *clong = nullptr;
-  uint32_t n_clong = 0;
+  bool w8_fits = false;             // every weight is below 256 (hw8 / the cold sets' w8)
+  grd::ColdSet cold[2];             // the cold arcs as the sums / as the min-combines block them (cold_set)
   grd::DevMem tmem;
 };
 
@@ -285,6 +293,7 @@ struct grd_state {
   uint2 *heavy = nullptr;  // push: (proxy, first arc offset) of each heavy-vertex chunk
   void *partial = nullptr;  // pull: one 8-byte partial per row block (long-row segments)
   bool tiled = false;       // PR_PULL: the tiled pull runs (else the plain row-block pull)
+  const grd::ColdSet *cold = nullptr;  // hot / cold pull: the cold blocks this state pulls over
   // tiled pull: Kahan partial per pair, then per tier-block segment; the hot /
   // cold pull keeps one 4-byte partial per row and per hot segment in them
   float2 *tpart = nullptr;
@@ -353,15 +362,17 @@ void take_frontier_parts(grd_state *s);
 grd_status build_ship_tables(grd_graph *g);
 grd_status op_frontier_parts(grd_state *s);  // per-partition frontier counts into the counters (C > 1)
 grd_status op_ship(grd_state *s);            // edge shipping: memory send + compute apply
-// pull.hip: the row-block PageRank pull over any CSC cut into PullBlocks, and its
-// long-row fix-up; `pre` (or null) holds a Kahan partial per row merged first
-grd_status prp_pull_rows(hipStream_t st, const PullBlock *blocks, uint32_t nblk, const uint32_t *hot_base,
-                         const uint32_t *rptr, const uint32_t *col, const float *mprop, uint32_t P, float *out,
-                         float2 *partial, const float *pre);
+// pull.hip: the long-row fix-up of a PageRank pull; `pre` (or null) holds a partial per row merged first
 grd_status prp_pull_rows_fixup(hipStream_t st, const PullLong *longs, uint32_t nlong, const float2 *partial,
                                float *out, const float *pre);
+// cold.hip: the cold pass of the hot / cold split
+uint32_t cold_set(const grd_graph *g, int algo, uint32_t *nnz);  // which cold set an algorithm pulls over
+grd_status cold_sort(grd_graph *g, const ColdSet &c);  // the cold blocks' arcs into source order
+grd_status prp_pull_cold(grd_state *s, float *out, const float *pre);
+grd_status cold_blocks_done(grd_state *s);  // k_blocks_done's flags for the cold blocks
 // tiers.hip
 grd_status build_tiers(grd_graph *g);
+grd_status build_cold(grd_graph *g, int algo, const ColdSet **out);  // mode 3: the algorithm's cold set
 // does this state pull through the hot / cold split (the BSP pull, CC / SSSP /
 // reference PageRank, over a graph split by mode 3)?
 inline bool bsp_hot_cold(const grd_state *s) { return s->tiled && s->g->tier_mode == 3; }

@@ -2,7 +2,10 @@
 // rules (shared by the push, pull and exchange kernels).
 #pragma once
 
+#include <type_traits>
+
 #include "grd_device.hpp"
+#include "grd_internal.hpp"
 
 namespace grd {
 
@@ -153,6 +156,73 @@ __device__ __forceinline__ void mark_wave(uint64_t *bits, uint32_t i, bool pred)
   }
 }
 
+// How the pull's row passes accumulate (the hot pass of tiers.hip, the cold
+// pass of cold.hip).  Pull PageRank: FP32 Kahan per lane, lanes
+// merged by TwoSum, the compensated sum of each row rounded once to FP32.  The BSP pull (CC,
+// SSSP, reference PageRank): Op::edge of the source's broadcast value and the
+// arc weight, combined with the operator (min, or + in a fixed order).
+// The hot part of a row is a few arcs on average (2.7 at RMAT-26, M = 4), so
+// its compensated sum is kept as one FP32 value (the sum rounded once): the
+// per-row partial is 4 bytes written and read instead of 8.
+struct HotPR {
+  using V = float;
+  using Part = float;
+  using Acc = Kahan;
+  static constexpr bool kWeighted = false;
+  __device__ static Acc zero() { return Kahan{}; }
+  __device__ static V value(V v, uint32_t) { return v; }
+  __device__ static void add(Acc &a, V x) { a.add(x); }
+  __device__ static void merge_lanes(Acc &a, int width) { kahan_wave_merge(a, width); }
+  __device__ static void merge(Acc &a, const Acc &o) { a.merge(o.s, o.c); }
+  __device__ static void add_part(Acc &a, Part p) { a.merge(p, 0.0f); }
+  __device__ static Part part(const Acc &a) { return a.value(); }
+};
+template <class Op>
+struct HotBsp {
+  using V = typename Op::V;
+  using Part = V;
+  using Acc = V;
+  static constexpr bool kWeighted = std::is_same<Op, OpWeighted>::value;
+  __device__ static Acc zero() { return op_identity<Op>(); }
+  __device__ static V value(V v, uint32_t w) { return Op::edge(v, w); }
+  __device__ static void add(Acc &a, V x) { a = op_combine<Op>(a, x); }
+  __device__ static void merge_lanes(Acc &a, int width)
+  {
+    for (int o = width / 2; o > 0; o >>= 1) a = op_combine<Op>(a, __shfl_xor(a, o, kWave));
+  }
+  __device__ static void merge(Acc &a, const Acc &o) { a = op_combine<Op>(a, o); }
+  __device__ static void add_part(Acc &a, Part p) { a = op_combine<Op>(a, p); }
+  __device__ static Part part(const Acc &a) { return a; }
+};
+
+// apply the pulled value to the proxy's running update; true = dirty
+template <class Op>
+__device__ __forceinline__ bool pull_apply(typename Op::V *upd, uint32_t r, typename Op::V acc)
+{
+  if constexpr (Op::kMin) {
+    if (acc < upd[r]) {
+      upd[r] = acc;
+      return true;
+    }
+    return false;
+  } else {
+    // contributions of active sources are strictly positive (pr.cpp:80)
+    if (acc > 0.0f) {
+      upd[r] = upd[r] + acc;
+      return true;
+    }
+    return false;
+  }
+}
+
+// the smallest candidate a pull superstep can produce: the smallest value
+// broadcast plus the smallest Op::edge increment, saturating
+__device__ __forceinline__ uint32_t pull_bound(const Counters *cnt, uint32_t inc)
+{
+  const uint32_t f = cnt->fmin;
+  return f + inc < f ? 0xFFFFFFFFu : f + inc;
+}
+
 // pull launchers (pull.hip)
 template <class Op>
 grd_status bsp_pull_launch(grd_state *s, const uint32_t *cw);
@@ -163,5 +233,9 @@ grd_status pull_done_arcs(grd_state *s);
 // the hot pass of the hot / cold split for the BSP pull (tiers.hip)
 template <class Op>
 grd_status bsp_pull_hot(grd_state *s);
+// its cold pass (cold.hip); skip: a flag per cold block (k_cold_blocks_done),
+// bcnt: the superstep's bound (either may be null)
+template <class Op>
+grd_status bsp_pull_cold(grd_state *s, const uint8_t *skip, const Counters *bcnt);
 
 }  // namespace grd

@@ -47,8 +47,7 @@ __global__ void __launch_bounds__(kBlock) k_prp_pull_rb(const PullBlock *__restr
                                                         const uint32_t *__restrict__ crp,
                                                         const uint32_t *__restrict__ ccol,
                                                         const float *__restrict__ mprop, uint32_t P,
-                                                        float *__restrict__ out, float2 *__restrict__ partial,
-                                                        const float *__restrict__ pre)
+                                                        float *__restrict__ out, float2 *__restrict__ partial)
 {
   __shared__ float s_v[kPullNnz];
   __shared__ float s_hot[kPullHot];
@@ -142,16 +141,7 @@ __global__ void __launch_bounds__(kBlock) k_prp_pull_rb(const PullBlock *__restr
       for (uint32_t x = b + sub; x < e; x += G) acc.add(s_v[x]);
     }
     kahan_wave_merge(acc, G);
-    if (sub == 0 && rl < d.nrows) {
-      if (pre) {  // the row's partial from the hot pass comes first
-        Kahan t;
-        t.s = pre[r];
-        t.merge(acc.s, acc.c);
-        out[r] = t.value();
-      } else {
-        out[r] = acc.value();
-      }
-    }
+    if (sub == 0 && rl < d.nrows) out[r] = acc.value();
   }
 }
 
@@ -194,7 +184,7 @@ __global__ void __launch_bounds__(kBlock) k_prp_pull_fixup(const PullLong *__res
 __global__ void __launch_bounds__(kBlock) k_blocks_done(uint32_t nblk, const PullBlock *__restrict__ blocks,
                                                         const uint64_t *__restrict__ done,
                                                         const uint64_t *__restrict__ hasarc,
-                                                        uint8_t *__restrict__ bskip, Counters *cnt, int cold)
+                                                        uint8_t *__restrict__ bskip, Counters *cnt, int hot)
 {
   unsigned long long arcs = 0, rows = 0;
   for (uint32_t b = blockIdx.x * kBlock + threadIdx.x; b < nblk; b += gridDim.x * kBlock) {
@@ -222,17 +212,9 @@ __global__ void __launch_bounds__(kBlock) k_blocks_done(uint32_t nblk, const Pul
   arcs = block_sum(arcs);
   rows = block_sum(rows);
   if (threadIdx.x == 0) {
-    if (arcs) atomicAdd(cold ? &cnt->pull_skipped : &cnt->pull_skipped_hot, arcs);
-    if (rows && cold) atomicAdd(&cnt->pull_skipped_rows, rows);
+    if (arcs) atomicAdd(hot ? &cnt->pull_skipped_hot : &cnt->pull_skipped, arcs);
+    if (rows && !hot) atomicAdd(&cnt->pull_skipped_rows, rows);
   }
-}
-
-// the smallest candidate a pull superstep can produce: the smallest value
-// broadcast plus the smallest Op::edge increment, saturating
-__device__ __forceinline__ uint32_t pull_bound(const Counters *cnt, uint32_t inc)
-{
-  const uint32_t f = cnt->fmin;
-  return f + inc < f ? 0xFFFFFFFFu : f + inc;
 }
 
 // Measurement only (time_kernel): the arcs, in the row-block pull's CSC (rp:
@@ -265,41 +247,18 @@ __global__ void __launch_bounds__(kBlock) k_rows_with_arcs(uint32_t nwP, const u
   }
 }
 
-// apply the pulled value to the proxy's running update; true = dirty
 template <class Op>
-__device__ __forceinline__ bool pull_apply(typename Op::V *upd, uint32_t r, typename Op::V acc)
-{
-  if constexpr (Op::kMin) {
-    if (acc < upd[r]) {
-      upd[r] = acc;
-      return true;
-    }
-    return false;
-  } else {
-    // contributions of active sources are strictly positive (pr.cpp:80)
-    if (acc > 0.0f) {
-      upd[r] = upd[r] + acc;
-      return true;
-    }
-    return false;
-  }
-}
-
-// W: the arc weights' storage type (a byte when every weight fits)
-template <class Op, class W = uint32_t>
 __global__ void __launch_bounds__(kBlock) k_bsp_pull_rb(const PullBlock *__restrict__ blocks,
                                                         const uint32_t *__restrict__ hot_base,
                                                         const uint32_t *__restrict__ crp,
                                                         const uint32_t *__restrict__ ccol,
-                                                        const W *__restrict__ cw,
+                                                        const uint32_t *__restrict__ cw,
                                                         const typename Op::V *__restrict__ mprop, uint32_t P,
                                                         typename Op::V *__restrict__ upd, uint64_t *__restrict__ dirty,
                                                         typename Op::V *__restrict__ partial,
-                                                        const typename Op::V *__restrict__ pre,
                                                         const uint8_t *__restrict__ bskip,
                                                         const uint64_t *__restrict__ done,
-                                                        const uint64_t *__restrict__ hasarc,
-                                                        const Counters *__restrict__ bcnt, uint32_t inc)
+                                                        const uint64_t *__restrict__ hasarc)
 {
   using V = typename Op::V;
   __shared__ V s_v[kPullNnz];
@@ -310,11 +269,6 @@ __global__ void __launch_bounds__(kBlock) k_bsp_pull_rb(const PullBlock *__restr
   const PullBlock d = blocks[bid];
   const uint32_t flag = bskip ? bskip[bid] : 0u;  // k_blocks_done: 1 = left out, 2 = some rows done
   if (flag == 1) return;
-  // with bcnt (a CC / SSSP pull over the hot / cold split): a row whose hot
-  // partial is already at or below the bound takes no cold candidate below it
-  // (every cold candidate is at least the bound), so it gathers nothing and
-  // its result is the hot partial
-  const uint32_t bnd = bcnt ? pull_bound(bcnt, inc) : 0u;
   if (d.nrows == 0) {  // segment (<= kPullNnz arcs) of a long row
     // column ids (and weights), then the gathers (hot sources from LDS),
     // then each thread combines its arcs in order
@@ -325,11 +279,7 @@ __global__ void __launch_bounds__(kBlock) k_bsp_pull_rb(const PullBlock *__restr
     for (int k = 0; k < kPer; k++) {
       const uint32_t i = threadIdx.x + k * kBlock;
       src[k] = i < ne ? ccol[d.e0 + i] : 0u;
-      wt[k] = (cw && i < ne) ? (uint32_t)cw[d.e0 + i] : 1u;
-    }
-    if (bcnt && pre[d.r0] <= bnd) {  // uniform over the block
-      if (threadIdx.x == 0) partial[bid] = op_identity<Op>();
-      return;
+      wt[k] = (cw && i < ne) ? cw[d.e0 + i] : 1u;
     }
     const uint32_t hb = hot_base[bid];
     const uint32_t hn = min(kPullHot, P - hb);
@@ -364,21 +314,19 @@ __global__ void __launch_bounds__(kBlock) k_bsp_pull_rb(const PullBlock *__restr
     for (int k = 0; k < kPer; k++) {
       uint32_t i = threadIdx.x + k * kBlock;
       src[k] = i < ne ? ccol[d.e0 + i] : 0u;
-      wt[k] = (cw && i < ne) ? (uint32_t)cw[d.e0 + i] : 1u;
+      wt[k] = (cw && i < ne) ? cw[d.e0 + i] : 1u;
     }
-    const bool marked = flag == 2 || bcnt;  // uniform over the block
+    const bool marked = flag == 2;  // uniform over the block
     if (marked) {
       // each row's group marks the row's arcs to gather or not (every arc of
-      // the block belongs to one of its rows): not for a done row, nor for
-      // one whose hot partial already reached the bound
+      // the block belongs to one of its rows): not for a done row
       for (uint32_t k = 0; k < rounds; k++) {
         const uint32_t rl = k * ngroups + threadIdx.x / G, r = d.r0 + rl;
         bool gat = false;
         uint32_t b = 0, e = 0;
         if (rl < d.nrows) {
           const uint64_t bit = 1ull << (r & 63);
-          gat = !done || (!(done[r >> 6] & bit) && (hasarc[r >> 6] & bit));
-          if (gat && bcnt) gat = pre[r] > bnd;
+          gat = !(done[r >> 6] & bit) && (hasarc[r >> 6] & bit);
           b = crp[r] - d.e0;
           e = crp[r + 1] - d.e0;
         }
@@ -407,8 +355,6 @@ __global__ void __launch_bounds__(kBlock) k_bsp_pull_rb(const PullBlock *__restr
     uint32_t rl = k * ngroups + threadIdx.x / G;
     V acc = op_identity<Op>();
     uint32_t r = d.r0 + rl;
-    // a done row, or one without arcs, has nothing to apply (its hot partial
-    // may not have been written)
     bool live = rl < d.nrows;
     if (done && live) {
       const uint64_t bit = 1ull << (r & 63);
@@ -419,7 +365,6 @@ __global__ void __launch_bounds__(kBlock) k_bsp_pull_rb(const PullBlock *__restr
       for (uint32_t x = b + sub; x < e; x += G) acc = op_combine<Op>(acc, s_v[x]);
     }
     for (int o = G / 2; o > 0; o >>= 1) acc = op_combine<Op>(acc, __shfl_xor(acc, o, kWave));
-    if (pre && sub == 0 && live) acc = op_combine<Op>(pre[r], acc);  // the row's hot partial first
     if (sub == 0 && live && pull_apply<Op>(upd, r, acc))
       atomicOr(&s_dirty[(r >> 6) - w0], 1ull << (r & 63));
   }
@@ -459,8 +404,11 @@ grd_status prp_pull_launch(grd_state *s)
 {
   grd_graph *g = s->g;
   hipStream_t st = g->ctx->stream;
-  return prp_pull_rows(st, g->pblk, g->n_pblk, g->pblk_hot, g->crp, g->ccol, (const float *)s->mprop, g->P,
-                       (float *)s->valR, (float2 *)s->partial, nullptr);
+  if (g->n_pblk)
+    hipLaunchKernelGGL(k_prp_pull_rb, dim3(g->n_pblk), dim3(kBlock), 0, st, g->pblk, g->pblk_hot, g->crp, g->ccol,
+                       (const float *)s->mprop, g->P, (float *)s->valR, (float2 *)s->partial);
+  GRD_HIP(hipGetLastError());
+  return GRD_OK;
 }
 
 grd_status prp_pull_fixup(grd_state *s)
@@ -468,17 +416,6 @@ grd_status prp_pull_fixup(grd_state *s)
   grd_graph *g = s->g;
   return prp_pull_rows_fixup(g->ctx->stream, g->plong, g->n_plong, (const float2 *)s->partial, (float *)s->valR,
                              nullptr);
-}
-
-grd_status prp_pull_rows(hipStream_t st, const PullBlock *blocks, uint32_t nblk, const uint32_t *hot_base,
-                         const uint32_t *rptr, const uint32_t *col, const float *mprop, uint32_t P, float *out,
-                         float2 *partial, const float *pre)
-{
-  if (nblk)
-    hipLaunchKernelGGL(k_prp_pull_rb, dim3(nblk), dim3(kBlock), 0, st, blocks, hot_base, rptr, col, mprop, P, out,
-                       partial, pre);
-  GRD_HIP(hipGetLastError());
-  return GRD_OK;
 }
 
 grd_status prp_pull_rows_fixup(hipStream_t st, const PullLong *longs, uint32_t nlong, const float2 *partial,
@@ -518,16 +455,18 @@ static grd_status blocks_done(grd_state *s, bool cold, const uint8_t **flags)
                          dim3(kBlock), 0, st, nwP, g->crp, g->rarc);
   }
   const uint32_t cap = (uint32_t)g->ctx->num_cus * 8;
-  const uint32_t nblk = cold ? g->n_cblk : g->n_pblk;
-  if (nblk)
-    hipLaunchKernelGGL(k_blocks_done, dim3(std::min<uint32_t>((nblk + kBlock - 1) / kBlock, cap)), dim3(kBlock), 0, st,
-                       nblk, cold ? g->cblk : g->pblk, (const uint64_t *)s->Rdone, (const uint64_t *)g->rarc, s->bskip,
-                       s->cnt, 1);
+  if (cold) {
+    GRD_TRY(cold_blocks_done(s));
+  } else if (g->n_pblk) {
+    hipLaunchKernelGGL(k_blocks_done, dim3(std::min<uint32_t>((g->n_pblk + kBlock - 1) / kBlock, cap)), dim3(kBlock), 0,
+                       st, g->n_pblk, g->pblk, (const uint64_t *)s->Rdone, (const uint64_t *)g->rarc, s->bskip, s->cnt,
+                       0);
+  }
   // the hot pass's wave blocks (their rows are counted once, with the cold pass's)
   if (cold && g->n_tblk && s->hskip) {
     hipLaunchKernelGGL(k_blocks_done, dim3(std::min<uint32_t>((g->n_tblk + kBlock - 1) / kBlock, cap)), dim3(kBlock), 0,
                        st, g->n_tblk, g->tblk, (const uint64_t *)s->Rdone, (const uint64_t *)g->rarc, s->hskip,
-                       s->cnt, 0);
+                       s->cnt, 1);
     s->hskip_on = true;
   }
   GRD_HIP(hipGetLastError());
@@ -547,24 +486,13 @@ grd_status bsp_pull_launch(grd_state *s, const uint32_t *cw)
     // the hot partials against the bound (CC / SSSP)
     const Counters *bcnt = (Op::kMin && s->bound_sent) ? s->cnt : nullptr;
     GRD_TRY(bsp_pull_hot<Op>(s));
-    if (g->n_cblk && cw && g->cow8)
-      hipLaunchKernelGGL((k_bsp_pull_rb<Op, uint8_t>), dim3(g->n_cblk), dim3(kBlock), 0, g->ctx->stream, g->cblk,
-                         g->cblk_hot, g->corp, g->cocol, (const uint8_t *)g->cow8, (const V *)s->mprop, g->P,
-                         (V *)s->mupd, s->Du, (V *)s->cseg, (const V *)s->tpart, skip,
-                         skip ? (const uint64_t *)s->Rdone : nullptr, skip ? (const uint64_t *)g->rarc : nullptr,
-                         bcnt, s->bound_inc);
-    else if (g->n_cblk)
-      hipLaunchKernelGGL((k_bsp_pull_rb<Op, uint32_t>), dim3(g->n_cblk), dim3(kBlock), 0, g->ctx->stream, g->cblk,
-                         g->cblk_hot, g->corp, g->cocol, cw ? g->cow : nullptr, (const V *)s->mprop, g->P,
-                         (V *)s->mupd, s->Du, (V *)s->cseg, (const V *)s->tpart, skip,
-                         skip ? (const uint64_t *)s->Rdone : nullptr, skip ? (const uint64_t *)g->rarc : nullptr,
-                         bcnt, s->bound_inc);
+    GRD_TRY(bsp_pull_cold<Op>(s, skip, bcnt));
   } else {
     GRD_TRY(blocks_done<Op>(s, false, &skip));
-    hipLaunchKernelGGL((k_bsp_pull_rb<Op, uint32_t>), dim3(g->n_pblk), dim3(kBlock), 0, g->ctx->stream, g->pblk,
+    hipLaunchKernelGGL(k_bsp_pull_rb<Op>, dim3(g->n_pblk), dim3(kBlock), 0, g->ctx->stream, g->pblk,
                        g->pblk_hot, g->crp, g->ccol, cw, (const V *)s->mprop, g->P, (V *)s->mupd, s->Du,
-                       (V *)s->partial, (const V *)nullptr, skip, skip ? (const uint64_t *)s->Rdone : nullptr,
-                       skip ? (const uint64_t *)g->rarc : nullptr, (const Counters *)nullptr, 0u);
+                       (V *)s->partial, skip, skip ? (const uint64_t *)s->Rdone : nullptr,
+                       skip ? (const uint64_t *)g->rarc : nullptr);
   }
   GRD_HIP(hipGetLastError());
   return GRD_OK;
@@ -576,10 +504,10 @@ grd_status bsp_pull_fixup(grd_state *s)
   grd_graph *g = s->g;
   using V = typename Op::V;
   const bool hc = bsp_hot_cold(s);
-  const uint32_t nlong = hc ? g->n_clong : g->n_plong;
+  const uint32_t nlong = hc ? s->cold->nlong : g->n_plong;
   if (!nlong) return GRD_OK;
   hipLaunchKernelGGL(k_bsp_pull_fixup<Op>, dim3(fixup_grid(nlong)), dim3(kBlock), 0, g->ctx->stream,
-                     hc ? g->clong : g->plong, nlong, hc ? (const V *)s->cseg : (const V *)s->partial, (V *)s->mupd,
+                     hc ? s->cold->lng : g->plong, nlong, hc ? (const V *)s->cseg : (const V *)s->partial, (V *)s->mupd,
                      s->Du, hc ? (const V *)s->tpart : (const V *)nullptr,
                      (Op::kMin && s->rdone_sent) ? (const uint64_t *)s->Rdone : nullptr);
   GRD_HIP(hipGetLastError());

@@ -191,6 +191,12 @@ grd_status t_scan(DevMem &mem, hipStream_t st, const T *in, T *out, uint64_t n)
   return GRD_OK;
 }
 
+// workgroups of a wave-per-row pass
+inline uint32_t row_wave_grid(uint64_t P)
+{
+  return (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(65535, (P + kWavesPerBlock - 1) / kWavesPerBlock));
+}
+
 template <typename T>
 grd_status t_upload(DevMem &mem, hipStream_t st, T **dst, const std::vector<T> &v)
 {
@@ -520,30 +526,41 @@ __global__ void k_h_split(uint32_t P, const uint32_t *__restrict__ crp, const ui
   }
 }
 
-// a wave per row: its hot arcs as 16-bit window offsets, its cold arcs as
-// source proxies, and their weights as W (a byte when every weight fits)
+// a wave per row: its hot arcs as 16-bit window offsets, with their weights as
+// W (a byte when every weight fits)
 template <class W>
 __global__ void k_h_copy(uint32_t P, const uint32_t *__restrict__ crp, const uint32_t *__restrict__ ccol,
                          const uint32_t *__restrict__ cw, const uint32_t *__restrict__ hrp,
-                         const uint32_t *__restrict__ corp, const uint32_t *__restrict__ pb, uint32_t M,
-                         uint16_t *__restrict__ hcol, uint32_t *__restrict__ cocol, W *__restrict__ hw,
-                         W *__restrict__ cow)
+                         const uint32_t *__restrict__ pb, uint32_t M, uint16_t *__restrict__ hcol, W *__restrict__ hw)
 {
   const uint32_t lane = lane_id();
   const uint64_t stride = (uint64_t)gridDim.x * kWavesPerBlock;
   for (uint64_t r = (uint64_t)blockIdx.x * kWavesPerBlock + wave_in_block(); r < P; r += stride) {
-    const uint32_t base = pb[part_of(pb, M, (uint32_t)r)];
-    const uint32_t e0 = crp[r], n = crp[r + 1] - e0;
-    const uint32_t h0 = hrp[r], nh = hrp[r + 1] - h0, c0 = corp[r];
-    for (uint32_t i = lane; i < n; i += kWave) {
-      const uint32_t v = ccol[e0 + i];
-      if (i < nh) {
-        hcol[h0 + i] = (uint16_t)(v - base);
-        if (cw) hw[h0 + i] = (W)cw[e0 + i];
-      } else {
-        cocol[c0 + (i - nh)] = v;
-        if (cw) cow[c0 + (i - nh)] = (W)cw[e0 + i];
-      }
+    const uint32_t h0 = hrp[r], nh = hrp[r + 1] - h0;
+    if (!nh) continue;
+    const uint32_t base = pb[part_of(pb, M, (uint32_t)r)], e0 = crp[r];
+    for (uint32_t i = lane; i < nh; i += kWave) {
+      hcol[h0 + i] = (uint16_t)(ccol[e0 + i] - base);
+      if (cw) hw[h0 + i] = (W)cw[e0 + i];
+    }
+  }
+}
+
+// a wave per row: its cold arcs as source proxies, with their weights as W
+template <class W>
+__global__ void k_c_copy(uint32_t P, const uint32_t *__restrict__ crp, const uint32_t *__restrict__ ccol,
+                         const uint32_t *__restrict__ cw, const uint32_t *__restrict__ corp,
+                         uint32_t *__restrict__ cocol, W *__restrict__ cow)
+{
+  const uint32_t lane = lane_id();
+  const uint64_t stride = (uint64_t)gridDim.x * kWavesPerBlock;
+  for (uint64_t r = (uint64_t)blockIdx.x * kWavesPerBlock + wave_in_block(); r < P; r += stride) {
+    const uint32_t c0 = corp[r], nc = corp[r + 1] - c0;
+    if (!nc) continue;
+    const uint32_t e0 = crp[r + 1] - nc;  // the hot arcs come first
+    for (uint32_t i = lane; i < nc; i += kWave) {
+      cocol[c0 + i] = ccol[e0 + i];
+      if (cw) cow[c0 + i] = (W)cw[e0 + i];
     }
   }
 }
@@ -584,42 +601,6 @@ __device__ __forceinline__ uint32_t hot_group(uint32_t n)
   if (n > 64) return 1;
   return 64u >> (32 - __builtin_clz(n - 1));  // 64 >> ceil(log2 n)
 }
-
-// How the hot pass accumulates.  Pull PageRank: FP32 Kahan per lane, lanes
-// merged by TwoSum, the compensated sum of each row rounded once to FP32.  The BSP pull (CC,
-// SSSP, reference PageRank): Op::edge of the source's broadcast value and the
-// arc weight, combined with the operator (min, or + in a fixed order).
-// The hot part of a row is a few arcs on average (2.7 at RMAT-26, M = 4), so
-// its compensated sum is kept as one FP32 value (the sum rounded once): the
-// per-row partial is 4 bytes written and read instead of 8.
-struct HotPR {
-  using V = float;
-  using Part = float;
-  using Acc = Kahan;
-  static constexpr bool kWeighted = false;
-  __device__ static Acc zero() { return Kahan{}; }
-  __device__ static V value(V v, uint32_t) { return v; }
-  __device__ static void add(Acc &a, V x) { a.add(x); }
-  __device__ static void merge_lanes(Acc &a, int width) { kahan_wave_merge(a, width); }
-  __device__ static void add_part(Acc &a, Part p) { a.merge(p, 0.0f); }
-  __device__ static Part part(const Acc &a) { return a.value(); }
-};
-template <class Op>
-struct HotBsp {
-  using V = typename Op::V;
-  using Part = V;
-  using Acc = V;
-  static constexpr bool kWeighted = std::is_same<Op, OpWeighted>::value;
-  __device__ static Acc zero() { return op_identity<Op>(); }
-  __device__ static V value(V v, uint32_t w) { return Op::edge(v, w); }
-  __device__ static void add(Acc &a, V x) { a = op_combine<Op>(a, x); }
-  __device__ static void merge_lanes(Acc &a, int width)
-  {
-    for (int o = width / 2; o > 0; o >>= 1) a = op_combine<Op>(a, __shfl_xor(a, o, kWave));
-  }
-  __device__ static void add_part(Acc &a, Part p) { a = op_combine<Op>(a, p); }
-  __device__ static Part part(const Acc &a) { return a; }
-};
 
 // kSkip (CC / SSSP): skip[b] = 1 marks a wave block whose rows are all done
 // or without arcs (k_blocks_done; 2, some rows done, runs in full); it is
@@ -842,16 +823,13 @@ static grd_status build_hotcold(grd_graph *g)
   GRD_TRY(gm.alloc_n(&g->corp, (uint64_t)P + 1));
   GRD_TRY(t_scan(tmp, st, hlen, g->hrp, (uint64_t)P + 1));
   GRD_TRY(t_scan(tmp, st, clen, g->corp, (uint64_t)P + 1));
-  std::vector<uint32_t> hrp((size_t)P + 1), corp((size_t)P + 1);
+  std::vector<uint32_t> hrp((size_t)P + 1);
   GRD_HIP(hipMemcpyAsync(hrp.data(), g->hrp, ((size_t)P + 1) * 4, hipMemcpyDeviceToHost, st));
-  GRD_HIP(hipMemcpyAsync(corp.data(), g->corp, ((size_t)P + 1) * 4, hipMemcpyDeviceToHost, st));
   GRD_HIP(hipStreamSynchronize(st));
   // padded: a wave block without hot arcs still reads the column at its start
   GRD_TRY(gm.alloc_n(&g->tcol, (uint64_t)hrp[P] + kWave));
-  GRD_TRY(gm.alloc_n(&g->cocol, std::max<uint64_t>(corp[P], 1)));
   // arc weights follow their arcs (the BSP pull of weighted SSSP), one byte
   // each when every weight is below 256
-  bool w8 = false;
   if (g->cw) {
     uint32_t *d_wmax = nullptr, wmax = 0;
     GRD_TRY(tmp.alloc_n(&d_wmax, 1));
@@ -859,23 +837,18 @@ static grd_status build_hotcold(grd_graph *g)
     hipLaunchKernelGGL(k_w_max, dim3(tgrid(g->m)), dim3(kBlock), 0, st, g->m, g->cw, d_wmax);
     GRD_HIP(hipMemcpyAsync(&wmax, d_wmax, 4, hipMemcpyDeviceToHost, st));
     GRD_HIP(hipStreamSynchronize(st));
-    w8 = wmax < 256;
-    if (w8) {
-      GRD_TRY(gm.alloc_n(&g->hw8, (uint64_t)hrp[P] + kWave));
-      GRD_TRY(gm.alloc_n(&g->cow8, std::max<uint64_t>(corp[P], 1)));
-    } else {
-      GRD_TRY(gm.alloc_n(&g->hw, (uint64_t)hrp[P] + kWave));
-      GRD_TRY(gm.alloc_n(&g->cow, std::max<uint64_t>(corp[P], 1)));
-    }
+    g->w8_fits = wmax < 256;
+    if (g->w8_fits) GRD_TRY(gm.alloc_n(&g->hw8, (uint64_t)hrp[P] + kWave));
+    else GRD_TRY(gm.alloc_n(&g->hw, (uint64_t)hrp[P] + kWave));
   }
   if (P) {
-    const uint64_t nb = std::min<uint64_t>(65535, ((uint64_t)P + kWavesPerBlock - 1) / kWavesPerBlock);
-    if (w8)
-      hipLaunchKernelGGL(k_h_copy<uint8_t>, dim3((uint32_t)nb), dim3(kBlock), 0, st, P, g->crp, g->ccol, g->cw,
-                         g->hrp, g->corp, d_pb, M, g->tcol, g->cocol, g->hw8, g->cow8);
+    const uint32_t nb = row_wave_grid(P);
+    if (g->w8_fits)
+      hipLaunchKernelGGL(k_h_copy<uint8_t>, dim3(nb), dim3(kBlock), 0, st, P, g->crp, g->ccol, g->cw, g->hrp, d_pb, M,
+                         g->tcol, g->hw8);
     else
-      hipLaunchKernelGGL(k_h_copy<uint32_t>, dim3((uint32_t)nb), dim3(kBlock), 0, st, P, g->crp, g->ccol, g->cw,
-                         g->hrp, g->corp, d_pb, M, g->tcol, g->cocol, g->hw, g->cow);
+      hipLaunchKernelGGL(k_h_copy<uint32_t>, dim3(nb), dim3(kBlock), 0, st, P, g->crp, g->ccol, g->cw, g->hrp, d_pb, M,
+                         g->tcol, g->hw);
   }
   GRD_HIP(hipGetLastError());
   // hot: wave blocks per partition, then each partition's blocks split into
@@ -944,54 +917,78 @@ static grd_status build_hotcold(grd_graph *g)
     }
     if (start < b1) ranges.push_back(TierTile{start, b1 - start, wbase, wlen});
   }
-  // cold: the row-block pull's cut over the remaining arcs, without the
-  // kernel's small LDS window (a window base of P is empty): the next 2048
-  // sources after the hot window draw too few arcs to pay for staging them
-  std::vector<PullBlock> cblk;
-  std::vector<PullLong> clong;
-  std::vector<uint32_t> chot;
-  {
-    uint32_t r = 0;
-    auto window_after = [&](uint32_t) { return P; };
-    while (r < P) {
-      const uint32_t len = corp[r + 1] - corp[r];
-      if (len > kPullNnz) {
-        PullLong L{r, (uint32_t)cblk.size(), 0, 0};
-        for (uint32_t e = corp[r]; e < corp[r + 1]; e += kPullNnz) {
-          cblk.push_back(PullBlock{r, 0, e, std::min(corp[r + 1], e + kPullNnz)});
-          chot.push_back(window_after(r));
-          L.nseg++;
-        }
-        clong.push_back(L);
-        r++;
-        continue;
-      }
-      const uint32_t r0 = r, e0 = corp[r];
-      while (r < P && r - r0 < kPullMaxRows && corp[r + 1] - corp[r] <= kPullNnz && corp[r + 1] - e0 <= kPullNnz) r++;
-      cblk.push_back(PullBlock{r0, r - r0, e0, corp[r]});
-      chot.push_back(window_after(r0));
-    }
-  }
   // the hot kernel reads its descriptors through a buffer of at most 2^31 bytes
-  if (hblk.size() * sizeof(PullBlock) >= 0x7FFFFFFFull || cblk.size() >= 0x7FFFFFFFull)
+  if (hblk.size() * sizeof(PullBlock) >= 0x7FFFFFFFull)
     return fail(GRD_ERR_ARG, "hot / cold pull: too many row blocks");
   GRD_TRY(t_upload(gm, st, &g->tblk, hblk));
   GRD_TRY(t_upload(gm, st, &g->tlong, hlong));
   GRD_TRY(t_upload(gm, st, &g->ttile, ranges));
-  GRD_TRY(t_upload(gm, st, &g->cblk, cblk));
-  GRD_TRY(t_upload(gm, st, &g->cblk_hot, chot));
-  GRD_TRY(t_upload(gm, st, &g->clong, clong));
   GRD_HIP(hipStreamSynchronize(st));  // the host vectors and temporaries go out of scope
   g->n_tblk = (uint32_t)hblk.size();
   g->n_tlong = (uint32_t)hlong.size();
   g->n_ttile = (uint32_t)ranges.size();
-  g->n_cblk = (uint32_t)cblk.size();
-  g->n_clong = (uint32_t)clong.size();
   g->n_pairs = P;
   g->tier_mode = 3;
   g->tier_bits = tb;
   g->tile_arcs = 0;
   g->tiers_built = true;
+  return GRD_OK;
+}
+
+// mode 3: the cold arcs blocked for one algorithm, once per graph and set
+grd_status build_cold(grd_graph *g, int algo, const ColdSet **out)
+{
+  uint32_t N = 0;
+  ColdSet &c = g->cold[cold_set(g, algo, &N)];
+  *out = &c;
+  if (c.nnz) return GRD_OK;
+  hipStream_t st = g->ctx->stream;
+  const uint32_t P = g->P;
+  std::vector<uint32_t> corp((size_t)P + 1);
+  GRD_HIP(hipMemcpyAsync(corp.data(), g->corp, ((size_t)P + 1) * 4, hipMemcpyDeviceToHost, st));
+  GRD_HIP(hipStreamSynchronize(st));
+  std::vector<PullBlock> blk;
+  std::vector<PullLong> lng;
+  for (uint32_t r = 0; r < P;) {
+    if (corp[r + 1] - corp[r] > N) {
+      PullLong L{r, (uint32_t)blk.size(), 0, 0};
+      for (uint32_t e = corp[r]; e < corp[r + 1]; e += N) {
+        blk.push_back(PullBlock{r, 0, e, std::min(corp[r + 1], e + N)});
+        L.nseg++;
+      }
+      lng.push_back(L);
+      r++;
+      continue;
+    }
+    const uint32_t r0 = r, e0 = corp[r], rows = std::min(N, kColdRows);
+    while (r < P && r - r0 < rows && corp[r + 1] - corp[r] <= N && corp[r + 1] - e0 <= N) r++;
+    blk.push_back(PullBlock{r0, r - r0, e0, corp[r]});
+  }
+  if (blk.size() >= 0x7FFFFFFFull) return fail(GRD_ERR_ARG, "hot / cold pull: too many row blocks");
+  DevMem &gm = g->tmem;
+  ColdSet t;
+  const uint64_t arcs = std::max<uint64_t>(corp[P], 1);
+  GRD_TRY(gm.alloc_n(&t.col, arcs));
+  GRD_TRY(gm.alloc_n(&t.pos, arcs));
+  if (g->cw && g->w8_fits) GRD_TRY(gm.alloc_n(&t.w8, arcs));
+  else if (g->cw) GRD_TRY(gm.alloc_n(&t.w, arcs));
+  if (P) {
+    if (t.w8)
+      hipLaunchKernelGGL(k_c_copy<uint8_t>, dim3(row_wave_grid(P)), dim3(kBlock), 0, st, P, g->crp, g->ccol, g->cw,
+                         g->corp, t.col, t.w8);
+    else
+      hipLaunchKernelGGL(k_c_copy<uint32_t>, dim3(row_wave_grid(P)), dim3(kBlock), 0, st, P, g->crp, g->ccol, g->cw,
+                         g->corp, t.col, t.w);
+  }
+  GRD_HIP(hipGetLastError());
+  GRD_TRY(t_upload(gm, st, &t.blk, blk));
+  GRD_TRY(t_upload(gm, st, &t.lng, lng));
+  t.nblk = (uint32_t)blk.size();
+  t.nlong = (uint32_t)lng.size();
+  t.nnz = N;
+  GRD_TRY(cold_sort(g, t));
+  GRD_HIP(hipStreamSynchronize(st));  // the host vectors go out of scope
+  c = t;
   return GRD_OK;
 }
 
@@ -1185,9 +1182,8 @@ grd_status prp_pull_tiled(grd_state *s)
       hipLaunchKernelGGL(k_hot_fixup<HotPR>, dim3(wave_grid((g->n_tlong + 7) / 8)), dim3(kBlock), 0, st, g->tlong, g->n_tlong,
                          (const float *)hseg, hpart);
     GRD_HIP(hipGetLastError());
-    GRD_TRY(prp_pull_rows(st, g->cblk, g->n_cblk, g->cblk_hot, g->corp, g->cocol, (const float *)s->mprop, g->P, out,
-                          s->cseg, hpart));
-    return prp_pull_rows_fixup(st, g->clong, g->n_clong, s->cseg, out, hpart);
+    GRD_TRY(prp_pull_cold(s, out, hpart));
+    return prp_pull_rows_fixup(st, s->cold->lng, s->cold->nlong, s->cseg, out, hpart);
   }
   if (g->tier_mode == 1 && g->n_ttile)
     hipLaunchKernelGGL(k_prp_pull_tiled, dim3(g->n_ttile), dim3(kTierBlock), 0, st, g->ttile, g->tblk, g->trec,
