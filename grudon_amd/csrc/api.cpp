@@ -293,6 +293,7 @@ grd_status grd_destroy(grd_ctx *c)
   if (c->sel_w) (void)hipFree(c->sel_w);
   if (c->sel_out) (void)hipFree(c->sel_out);
   if (c->sel_out_host) (void)hipHostFree(c->sel_out_host);
+  workspace_release(c);
   (void)hipStreamDestroy(c->stream);
   delete c;
   return GRD_OK;
@@ -545,6 +546,7 @@ grd_status grd_state_create_typed(grd_graph *g, int algo, uint32_t value_bytes, 
   grd_state *s = new (std::nothrow) grd_state();
   if (!s) return fail(GRD_ERR_OOM, "grd_state_create: host allocation failed");
   s->g = g;
+  s->mem.ctx = s->ship_mem.ctx = s->snap_mem.ctx = g->ctx;
   s->algo = algo;
   s->vbytes = value_bytes;
   s->wide = value_bytes == 8;
@@ -567,7 +569,7 @@ grd_status grd_state_create_typed(grd_graph *g, int algo, uint32_t value_bytes, 
   if (st == GRD_OK && (hipEventCreate(&s->kev[0]) != hipSuccess || hipEventCreate(&s->kev[1]) != hipSuccess))
     st = fail(GRD_ERR_HIP, "grd_state_create: hipEventCreate failed");
   if (st != GRD_OK) {
-    if (s->hcnt) (void)hipHostFree(s->hcnt);
+    host_counters_give(g->ctx, s->hcnt);
     for (auto &e : s->kev)
       if (e) (void)hipEventDestroy(e);
     delete s;
@@ -581,7 +583,7 @@ grd_status grd_state_free(grd_state *s)
 {
   if (!s) return GRD_OK;
   (void)hipStreamSynchronize(s->g->ctx->stream);
-  if (s->hcnt) (void)hipHostFree(s->hcnt);
+  host_counters_give(s->g->ctx, s->hcnt);
   for (auto &e : s->kev)
     if (e) (void)hipEventDestroy(e);
   delete s;

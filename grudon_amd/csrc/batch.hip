@@ -536,7 +536,7 @@ grd_status grd_batch_create(grd_ctx *ctx, uint32_t count, const uint32_t *n, con
   GRD_HIP(hipSetDevice(ctx->device));
   try {
     grd_batch *b = new grd_batch();
-    b->ctx = ctx;
+    b->ctx = b->mem.ctx = b->blk_mem.ctx = b->st_mem.ctx = ctx;
     b->count = count;
     b->vbase.assign(count + 1, 0);
     for (uint32_t g = 0; g < count; g++) {
@@ -691,15 +691,13 @@ grd_status grd_batch_download(grd_batch *b, uint32_t i, int algo, void *out)
   if (algo != b->last_algo) return fail(GRD_ERR_STATE, "grd_batch_download: that algorithm has not run last");
   const uint64_t v0 = b->vbase[i], n = b->vbase[i + 1] - v0;
   if (algo == GRD_PR_PULL) {
-    GRD_HIP(hipMemcpy(out, b->r + v0, n * 4, hipMemcpyDeviceToHost));
-  } else if (algo == GRD_CC) {
-    // the last superstep of graph i wrote buffer iters % 2 (and changed nothing)
-    const uint32_t *src = b->lab[b->last_iters[i] & 1];
-    GRD_HIP(hipMemcpy(out, src + v0, n * 4, hipMemcpyDeviceToHost));
-  } else {
-    return fail(GRD_ERR_ARG, "grd_batch_download: algo must be GRD_PR_PULL or GRD_CC");
+    return copy_out(b->ctx, out, b->r + v0, n);
   }
-  return GRD_OK;
+  if (algo == GRD_CC) {
+    // the last superstep of graph i wrote buffer iters % 2 (and changed nothing)
+    return copy_out(b->ctx, out, b->lab[b->last_iters[i] & 1] + v0, n);
+  }
+  return fail(GRD_ERR_ARG, "grd_batch_download: algo must be GRD_PR_PULL or GRD_CC");
 }
 
 }  // extern "C"

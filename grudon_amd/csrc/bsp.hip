@@ -786,8 +786,7 @@ grd_status state_alloc(grd_state *s)
     if (bsp_hot_cold(s)) GRD_TRY(m.alloc_n(&s->hskip, std::max<uint32_t>(g->n_tblk, 1)));
   }
   GRD_TRY(m.alloc_n(&s->cnt, 1));
-  GRD_HIP(hipHostMalloc((void **)&s->hcnt, sizeof(Counters), hipHostMallocDefault));
-  memset(s->hcnt, 0, sizeof(Counters));
+  GRD_TRY(host_counters_take(g->ctx, &s->hcnt));
   // snapshot list: every array whose content carries state between iterations
   s->snap = {{s->prop, nullptr}, {s->upd, nullptr}, {s->F, nullptr},     {s->Dc, nullptr},
              {s->Pend, nullptr}, {s->mprop, nullptr}, {s->mupd, nullptr},
@@ -903,7 +902,7 @@ static grd_status graph_min_weight(grd_graph *g, uint32_t *out)
 {
   if (!g->wmin_known) {
     hipStream_t st = g->ctx->stream;
-    DevMem tmp;
+    DevMem tmp(g->ctx);
     uint32_t *d = nullptr;
     GRD_TRY(tmp.alloc_n(&d, 1));
     hipLaunchKernelGGL(k_fill_u32, dim3(1), dim3(kBlock), 0, st, d, 1, 0xFFFFFFFFu);
@@ -1139,26 +1138,16 @@ grd_status op_download(grd_state *s, void *out)
 {
   grd_graph *g = s->g;
   hipStream_t st = g->ctx->stream;
-  void *dout = nullptr;
-  GRD_HIP(hipMallocAsync(&dout, (uint64_t)g->n * 4, st));
+  DevMem tmp(g->ctx);
+  uint32_t *dout = nullptr;
+  GRD_TRY(tmp.alloc_n(&dout, g->n));
   const void *src = (s->algo == GRD_PR || s->algo == GRD_PR_PULL) ? (const void *)s->pr : s->prop;
   hipLaunchKernelGGL(k_gather_result<uint32_t>, dim3(std::min<uint32_t>(4096, g->S / kBlock + 1)), dim3(kBlock), 0, st,
-                     g->S, g->slot_gid, (const uint32_t *)src, (uint32_t *)dout);
+                     g->S, g->slot_gid, (const uint32_t *)src, dout);
   GRD_HIP(hipGetLastError());
-  GRD_HIP(hipMemcpyAsync(out, dout, (uint64_t)g->n * 4, hipMemcpyDeviceToHost, st));
-  GRD_HIP(hipFreeAsync(dout, st));
-  GRD_HIP(hipStreamSynchronize(st));
-  if (s->wide) {
-    // 8-byte properties: widen in place from the top, the unreached 2^32 - 1
-    // to 2^64 - 1 (numeric_limits<uint64_t>::max)
-    const uint32_t *in = (const uint32_t *)out;
-    uint64_t *o = (uint64_t *)out;
-    for (uint64_t i = g->n; i-- > 0;) {
-      const uint32_t x = in[i];
-      o[i] = x == 0xFFFFFFFFu ? ~0ull : (uint64_t)x;
-    }
-  }
-  return GRD_OK;
+  // 8-byte properties are widened on the way, the unreached 2^32 - 1 to 2^64 - 1
+  // (numeric_limits<uint64_t>::max)
+  return copy_out(g->ctx, out, dout, g->n, s->wide);
 }
 
 }  // namespace grd

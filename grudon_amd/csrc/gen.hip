@@ -109,7 +109,7 @@ static grd_status keys_to_csr(grd_ctx *ctx, uint64_t *d_keys, uint64_t cnt, uint
                               std::vector<uint32_t> &col)
 {
   hipStream_t st = ctx->stream;
-  DevMem mem;
+  DevMem mem(ctx);
   uint64_t *d_alt = nullptr;
   GRD_TRY(mem.alloc_n(&d_alt, std::max<uint64_t>(cnt, 1)));
   const int end_bit = std::max(1, bits_for(n * n - 1));
@@ -164,7 +164,7 @@ grd_status generate_rmat(grd_ctx *ctx, int scale, int ef, double a, double b, do
   const uint64_t E = (uint64_t)ef << scale;
   const uint64_t raw = sym ? 2 * E : E;
   if (raw >= 0xFFFFFFF0ull) return fail(GRD_ERR_ARG, "rmat: raw edge count beyond the u32 limit");
-  DevMem mem;
+  DevMem mem(ctx);
   uint64_t *keys = nullptr;
   GRD_TRY(mem.alloc_n(&keys, raw));
   const uint64_t tA = (uint64_t)(a * 4294967296.0);
@@ -183,7 +183,7 @@ grd_status generate_er(grd_ctx *ctx, uint32_t n, double deg, uint64_t seed, std:
   if (n < 2 || deg <= 0) return fail(GRD_ERR_ARG, "er: need n >= 2 and mean degree > 0");
   const uint64_t M = (uint64_t)((double)n * deg / 2.0);
   if (2 * M >= 0xFFFFFFF0ull) return fail(GRD_ERR_ARG, "er: edge count beyond the u32 limit");
-  DevMem mem;
+  DevMem mem(ctx);
   uint64_t *keys = nullptr;
   GRD_TRY(mem.alloc_n(&keys, std::max<uint64_t>(2 * M, 1)));
   uint32_t grid = (uint32_t)std::min<uint64_t>(65535, (M + kBlock - 1) / kBlock + 1);

@@ -30,6 +30,8 @@
 #include <cstdint>
 #include <array>
 #include <functional>
+#include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -57,10 +59,30 @@ constexpr uint32_t kNone = 0xFFFFFFFFu;
 
 inline uint64_t pad64(uint64_t x) { return (x + 63) & ~uint64_t(63); }
 
-// Device allocation list owned by a graph or a state.
+// Freed device blocks a context keeps for its next allocations (workspace.cpp):
+// at most kMaxHeld bytes, given back when the context goes or when an
+// allocation would fail.
+struct BlockCache {
+  static constexpr uint64_t kMaxHeld = 4ull << 30, kMaxBlock = 1ull << 30;
+  std::mutex mu;
+  std::multimap<uint64_t, void *> blocks;  // by size
+  uint64_t held = 0;
+  void *take(uint64_t want, uint64_t *got);
+  bool give(void *p, uint64_t size);
+  void trim();
+};
+
+// Device allocation list owned by a graph or a state, from its context's
+// cache.  A block's users are ordered on the context's stream; release() waits
+// for that stream before the blocks can be taken again.
 struct DevMem {
-  std::vector<void *> ptrs;
+  grd_ctx *ctx = nullptr;
+  std::vector<std::pair<void *, uint64_t>> ptrs;
   uint64_t bytes = 0;
+  DevMem() = default;
+  explicit DevMem(grd_ctx *c) : ctx(c) {}
+  DevMem(const DevMem &) = delete;
+  DevMem &operator=(const DevMem &) = delete;
   grd_status alloc(void **p, uint64_t nbytes);
   template <typename T>
   grd_status alloc_n(T **p, uint64_t n) { return alloc(reinterpret_cast<void **>(p), n * sizeof(T)); }
@@ -133,6 +155,7 @@ constexpr uint32_t kTierBitsMax = 15;    // tiled pull: largest tier, 2^15 sourc
 constexpr uint32_t kTierTileArcs = 65536;  // tiled pull: default arcs per tile
 constexpr uint32_t kSegBitsMax = 24;       // segmented pull: largest segment, 2^24 sources
 constexpr uint32_t kSegBits = 19;          // segmented pull: default segment, 2^19 sources (2 MB of values)
+constexpr int kStageSlots = 4;             // pinned staging slots of a context (workspace.cpp)
 constexpr uint32_t kHotWin = 32768;        // hot / cold pull: hottest sources of a partition in LDS (128 KB)
 
 }  // namespace grd
@@ -154,6 +177,12 @@ struct grd_ctx {
   float sel_margin = 0.0f;
   float *sel_out = nullptr;       // device: 4 logits + chosen option
   float *sel_out_host = nullptr;  // pinned
+  // kept between calls (workspace.cpp)
+  grd::BlockCache cache;
+  char *stage = nullptr;        // pinned, kStageSlots slots
+  char *stage_small = nullptr;  // pinned, for short transfers
+  hipEvent_t stage_ev[grd::kStageSlots] = {};
+  std::vector<void *> host_counters;  // pinned counter blocks of freed states
 };
 
 struct grd_graph {
@@ -325,6 +354,15 @@ struct grd_state {
 };
 
 namespace grd {
+// workspace.cpp
+void workspace_release(grd_ctx *ctx);
+grd_status host_counters_take(grd_ctx *ctx, Counters **out);
+void host_counters_give(grd_ctx *ctx, Counters *p);
+// n 4-byte values from the device to the caller's array, widened to 8 bytes on
+// the way with `wide`; ordered after the context's stream, done on return
+grd_status copy_out(grd_ctx *ctx, void *dst, const void *src, uint64_t n, bool wide = false);
+// bytes to the device, ordered on the context's stream; the source is taken on return
+grd_status copy_in(grd_ctx *ctx, void *dst, const void *src, uint64_t bytes);
 // layout.cpp
 grd_status check_row_ptr(uint32_t n, const uint32_t *rp);
 grd_status build_row_blocks(grd_graph *g, const std::vector<uint32_t> &crp);

@@ -59,28 +59,6 @@ void parallel_for(int nthreads, uint64_t n, uint64_t grain, const std::function<
   for (auto &x : th) x.join();
 }
 
-grd_status DevMem::alloc(void **p, uint64_t nbytes)
-{
-  *p = nullptr;
-  uint64_t b = nbytes ? nbytes : 64;
-  hipError_t e = hipMalloc(p, b);
-  if (e != hipSuccess) {
-    *p = nullptr;
-    (void)hipGetLastError();
-    return fail(GRD_ERR_OOM, "hipMalloc(" + std::to_string(b) + " bytes) failed: " + hipGetErrorString(e));
-  }
-  ptrs.push_back(*p);
-  bytes += b;
-  return GRD_OK;
-}
-
-void DevMem::release()
-{
-  for (void *p : ptrs) (void)hipFree(p);
-  ptrs.clear();
-  bytes = 0;
-}
-
 template <typename T>
 static grd_status upload(grd_graph *g, T **dst, const std::vector<T> &src)
 {
@@ -147,7 +125,7 @@ static grd_status build_impl(grd_ctx *ctx, uint32_t n, const uint32_t *rp, const
   const uint32_t NW = (n + 63) / 64;
 
   grd_graph *g = new grd_graph();
-  g->ctx = ctx;
+  g->ctx = g->mem.ctx = g->tmem.ctx = ctx;
   g->n = n;
   g->m = m;
   g->C = C;

@@ -346,12 +346,10 @@ int bits_of(uint64_t x)
   return b;
 }
 
-template <typename T>
-grd_status download(hipStream_t st, std::vector<T> &dst, const T *src, uint64_t n)
+grd_status download(grd_ctx *ctx, std::vector<uint32_t> &dst, const uint32_t *src, uint64_t n)
 {
   dst.resize(n);
-  if (n) GRD_HIP(hipMemcpyAsync(dst.data(), src, n * sizeof(T), hipMemcpyDeviceToHost, st));
-  return GRD_OK;
+  return copy_out(ctx, dst.data(), src, n);
 }
 
 template <typename T>
@@ -368,20 +366,20 @@ grd_status build_dev_impl(grd_ctx *ctx, uint32_t n, const uint32_t *h_rp, const 
   hipStream_t st = ctx->stream;
   const uint64_t m = h_rp[n];
   const uint32_t NW = (n + 63) / 64;
-  DevMem tmp;  // scratch of the build, freed on return
+  DevMem tmp(ctx);  // scratch of the build, freed on return
   // inputs
   uint32_t *rp = nullptr, *col = nullptr, *w = nullptr, *mirror = nullptr;
   GRD_TRY(tmp.alloc_n(&rp, (uint64_t)n + 1));
   GRD_TRY(tmp.alloc_n(&col, std::max<uint64_t>(m, 1)));
-  GRD_HIP(hipMemcpyAsync(rp, h_rp, ((uint64_t)n + 1) * 4, hipMemcpyHostToDevice, st));
-  if (m) GRD_HIP(hipMemcpyAsync(col, h_col, m * 4, hipMemcpyHostToDevice, st));
+  GRD_TRY(copy_in(ctx, rp, h_rp, ((uint64_t)n + 1) * 4));
+  GRD_TRY(copy_in(ctx, col, h_col, m * 4));
   if (h_w) {
     GRD_TRY(tmp.alloc_n(&w, std::max<uint64_t>(m, 1)));
-    if (m) GRD_HIP(hipMemcpyAsync(w, h_w, m * 4, hipMemcpyHostToDevice, st));
+    GRD_TRY(copy_in(ctx, w, h_w, m * 4));
   }
   if (mirror_in && M > 1) {
     GRD_TRY(tmp.alloc_n(&mirror, n));
-    GRD_HIP(hipMemcpyAsync(mirror, mirror_in, (uint64_t)n * 4, hipMemcpyHostToDevice, st));
+    GRD_TRY(copy_in(ctx, mirror, mirror_in, (uint64_t)n * 4));
   }
   // vertices
   uint32_t *deg = nullptr, *err = nullptr, *maxdeg = nullptr;
@@ -442,9 +440,8 @@ grd_status build_dev_impl(grd_ctx *ctx, uint32_t n, const uint32_t *h_rp, const 
   hipLaunchKernelGGL(k_cross_count, dim3(grid_for(nwords)), dim3(kBlock), 0, st, nwords, NW, crossw, (uint32_t)C,
                      (uint32_t)M, xcnt, wcount);
   GRD_TRY(exclusive_scan_u32(tmp, st, wcount, wpos, nwords + 1));
-  GRD_TRY(download(st, g->ccnt, ccnt, NP));
-  GRD_TRY(download(st, g->xcnt, xcnt, NP));
-  GRD_HIP(hipStreamSynchronize(st));
+  GRD_TRY(download(ctx, g->ccnt, ccnt, NP));
+  GRD_TRY(download(ctx, g->xcnt, xcnt, NP));
   // bases (host, as in layout.cpp)
   g->cbase.assign(NP, 0);
   uint64_t cur = 0;
@@ -574,11 +571,10 @@ grd_status build_dev_impl(grd_ctx *ctx, uint32_t n, const uint32_t *h_rp, const 
   GRD_HIP(hipGetLastError());
   // host copies
   std::vector<uint32_t> crp_h;
-  GRD_TRY(download(st, g->h_deg, deg, n));
-  GRD_TRY(download(st, g->h_gid_slot, gid_slot, n));
-  GRD_TRY(download(st, g->h_proxy_gid, proxy_gid, P));
-  GRD_TRY(download(st, crp_h, g->crp, (uint64_t)P + 1));
-  GRD_HIP(hipStreamSynchronize(st));
+  GRD_TRY(download(ctx, g->h_deg, deg, n));
+  GRD_TRY(download(ctx, g->h_gid_slot, gid_slot, n));
+  GRD_TRY(download(ctx, g->h_proxy_gid, proxy_gid, P));
+  GRD_TRY(download(ctx, crp_h, g->crp, (uint64_t)P + 1));
   return build_row_blocks(g, crp_h);
 }
 
@@ -593,7 +589,7 @@ grd_status build_graph_device(grd_ctx *ctx, uint32_t n, const uint32_t *rp, cons
   GRD_TRY(check_row_ptr(n, rp));  // the device passes index by row_ptr
   grd_graph *g = new (std::nothrow) grd_graph();
   if (!g) return fail(GRD_ERR_OOM, "graph: host allocation failed");
-  g->ctx = ctx;
+  g->ctx = g->mem.ctx = g->tmem.ctx = ctx;
   g->n = n;
   g->m = rp[n];
   g->C = C;

@@ -419,7 +419,7 @@ grd_status grd_selector_train(grd_ctx *ctx, const float *feat, const uint32_t *l
   init(oW1, kH * kIn, kIn);
   init(oW2, kH * kH, kH);
   init(oW3, kOut * kH, kH);
-  DevMem mem;
+  DevMem mem(ctx);
   float *dw, *dm1, *dm2, *dg, *dfeat, *dsw, *dloss;
   uint32_t *dlab, *didx;
   uint16_t *dwb;
@@ -481,7 +481,7 @@ grd_status grd_selector_infer(grd_ctx *ctx, const float *feat, uint64_t n, float
   if (!ctx || !feat || !logits || n == 0) return fail(GRD_ERR_ARG, "grd_selector_infer: bad argument");
   if (!ctx->sel_loaded) return fail(GRD_ERR_STATE, "grd_selector_infer: no weights loaded");
   GRD_HIP(hipSetDevice(ctx->device));
-  DevMem mem;
+  DevMem mem(ctx);
   float *df, *dl;
   GRD_TRY(mem.alloc_n(&df, n * kIn));
   GRD_TRY(mem.alloc_n(&dl, n * kOut));
@@ -523,7 +523,7 @@ grd_status grd_selector_grad(grd_ctx *ctx, const float *w, const float *feat, co
   for (uint64_t i = 0; i < n; i++)
     if (label[i] >= (uint32_t)kOut) return fail(GRD_ERR_ARG, "grd_selector_grad: label out of range");
   GRD_HIP(hipSetDevice(ctx->device));
-  DevMem mem;
+  DevMem mem(ctx);
   float *dw, *df, *dsw = nullptr, *dg, *dloss;
   uint32_t *dl;
   GRD_TRY(mem.alloc_n(&dw, kParams));

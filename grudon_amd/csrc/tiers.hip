@@ -809,7 +809,7 @@ static grd_status build_hotcold(grd_graph *g)
   std::vector<uint32_t> pb(M + 1);
   for (uint32_t k = 0; k < M; k++) pb[k] = g->obase[(size_t)k * C];
   pb[M] = P;
-  DevMem tmp;
+  DevMem tmp(ctx);
   uint32_t *d_pb = nullptr, *hlen = nullptr, *clen = nullptr;
   GRD_TRY(t_upload(tmp, st, &d_pb, pb));
   GRD_TRY(tmp.alloc_n(&hlen, (uint64_t)P + 1));
@@ -824,8 +824,7 @@ static grd_status build_hotcold(grd_graph *g)
   GRD_TRY(t_scan(tmp, st, hlen, g->hrp, (uint64_t)P + 1));
   GRD_TRY(t_scan(tmp, st, clen, g->corp, (uint64_t)P + 1));
   std::vector<uint32_t> hrp((size_t)P + 1);
-  GRD_HIP(hipMemcpyAsync(hrp.data(), g->hrp, ((size_t)P + 1) * 4, hipMemcpyDeviceToHost, st));
-  GRD_HIP(hipStreamSynchronize(st));
+  GRD_TRY(copy_out(ctx, hrp.data(), g->hrp, (uint64_t)P + 1));
   // padded: a wave block without hot arcs still reads the column at its start
   GRD_TRY(gm.alloc_n(&g->tcol, (uint64_t)hrp[P] + kWave));
   // arc weights follow their arcs (the BSP pull of weighted SSSP), one byte
@@ -945,8 +944,7 @@ grd_status build_cold(grd_graph *g, int algo, const ColdSet **out)
   hipStream_t st = g->ctx->stream;
   const uint32_t P = g->P;
   std::vector<uint32_t> corp((size_t)P + 1);
-  GRD_HIP(hipMemcpyAsync(corp.data(), g->corp, ((size_t)P + 1) * 4, hipMemcpyDeviceToHost, st));
-  GRD_HIP(hipStreamSynchronize(st));
+  GRD_TRY(copy_out(g->ctx, corp.data(), g->corp, (uint64_t)P + 1));
   std::vector<PullBlock> blk;
   std::vector<PullLong> lng;
   for (uint32_t r = 0; r < P;) {
@@ -1017,7 +1015,7 @@ grd_status build_tiers(grd_graph *g)
   uint32_t ntier_max = 1;
   for (uint32_t k = 0; k < M; k++) ntier_max = std::max<uint32_t>(ntier_max, ((pb[k + 1] - pb[k]) >> tb) + 1);
   if ((uint64_t)ntier_max * M >= (1ull << 31)) return fail(GRD_ERR_ARG, "tiled pull: too many tiers");
-  DevMem tmp;
+  DevMem tmp(ctx);
   uint32_t *d_pb = nullptr;
   GRD_TRY(t_upload(tmp, st, &d_pb, pb));
   // row of every arc: max-scan of the row heads
