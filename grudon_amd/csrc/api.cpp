@@ -186,7 +186,6 @@ static grd_status superstep(grd_state *s, int option, bool select_next = false)
   GRD_TRY(finish_kernel_timing(s, s->last_frontier));
   const Counters &c = *s->hcnt;
   const grd_graph *g = s->g;
-  if (c.ship_error) return fail(GRD_ERR_STATE, "edge shipping: the active list differs from the frontier");
   // reduce bytes (GraphAlgorithm.cpp:409-423): bitvector + dirty values
   // (sparse) or every translation-table entry (dense); a shipping superstep
   // has no reduce (its wire bytes were counted by op_ship)
@@ -546,7 +545,7 @@ grd_status grd_state_create_typed(grd_graph *g, int algo, uint32_t value_bytes, 
   grd_state *s = new (std::nothrow) grd_state();
   if (!s) return fail(GRD_ERR_OOM, "grd_state_create: host allocation failed");
   s->g = g;
-  s->mem.ctx = s->ship_mem.ctx = s->snap_mem.ctx = g->ctx;
+  s->mem.ctx = s->snap_mem.ctx = g->ctx;
   s->algo = algo;
   s->vbytes = value_bytes;
   s->wide = value_bytes == 8;
@@ -676,7 +675,6 @@ grd_status grd_update(grd_state *s, uint64_t *frontier_out)
   GRD_TRY(op_read_counters(s));
   GRD_TRY(finish_kernel_timing(s, s->last_frontier));
   const Counters &c = *s->hcnt;
-  if (c.ship_error) return fail(GRD_ERR_STATE, "edge shipping: the active list differs from the frontier");
   if (s->last_option != GRD_OPT_SHIP_EDGES) {
     uint64_t vals = (s->last_option & 2) ? (uint64_t)s->g->n + s->g->X : c.dirty;
     s->bytes += bitvector_bytes(s->g) + vals * s->vbytes;

@@ -7,7 +7,7 @@
 //
 // Reference loops replaced (src/GraphAlgorithm.cpp):
 //   k_bcast_send / k_bcast_recv   compute pack + memory unpack       :199-343
-//   k_push / k_push_heavy / (pull.hip)  gen_updates (pr/cc/sssp.cpp)  :348-356
+//   (push.hip) / (pull.hip)       gen_updates (pr/cc/sssp.cpp)  :348-356
 //   k_reduce_send / k_reduce_recv memory pack + compute aggregate     :377-581
 //   k_update                      update_frontier + apply_updates +
 //                                 termination popcount               :643-662
@@ -291,139 +291,6 @@ __global__ void __launch_bounds__(kBlock) k_bcast_recv(uint32_t nw, const uint64
 }
 
 // ------------------------------------------------------------------------
-// traversal: push over the active list (degree-binned, LDS-staged tiles)
-// ------------------------------------------------------------------------
-
-// owner of position j among a tile's 256 offsets: the last t with s_off[t] <= j
-// (s_off[0] = 0; eight halvings, no branch)
-__device__ __forceinline__ uint32_t push_owner(const uint32_t *s_off, uint32_t j)
-{
-  uint32_t t = 0;
-#pragma unroll
-  for (uint32_t step = kBlock / 2; step > 0; step >>= 1)
-    if (s_off[t + step] <= j) t += step;
-  return t;
-}
-
-// A block stages `tile` active vertices in LDS (256, or 64 where the frontier
-// would not fill the chip with tiles of 256).  Vertices with out-degree below
-// kHeavyDeg are processed together: the block scans their degrees and every
-// thread walks the concatenated edge range (coalesced col reads), locating its
-// source by binary search in the LDS prefix array, four arcs in flight per
-// thread.  Vertices with degree >= kHeavyDeg are appended to the heavy list as
-// chunks of kHeavyChunk arcs (one counter atomic per tile) and handled by
-// k_push_heavy, one workgroup per chunk.
-//
-// The active list is in degree order, so the vertices just below the threshold
-// share tiles: the threshold bounds a tile's work.  With 4096 (and chunks of
-// 4096) the first tiles held a million arcs each and ran alone: CC by pushes
-// over RMAT-20 symmetrized (31 M arcs) 16.7 ms a solve, with 256 and chunks of
-// 1024 3.4 ms.
-template <class Op>
-__global__ void __launch_bounds__(kBlock) k_push(const uint32_t *__restrict__ AL, const uint32_t *__restrict__ nact,
-                                                 const uint32_t *__restrict__ rp, const uint32_t *__restrict__ col,
-                                                 const uint32_t *__restrict__ wt, const typename Op::V *__restrict__ mprop,
-                                                 typename Op::V *upd, uint64_t *dirty, uint2 *heavy, Counters *cnt,
-                                                 uint32_t tile)
-{
-  using V = typename Op::V;
-  constexpr int kIlp = 4;
-  __shared__ uint32_t s_off[kBlock];
-  __shared__ uint32_t s_beg[kBlock];
-  __shared__ V s_val[kBlock];
-  __shared__ unsigned long long s_slot;
-  const uint32_t k = *nact;
-  uint64_t my_edges = 0;
-  for (uint32_t t0 = blockIdx.x * tile; t0 < k; t0 += gridDim.x * tile) {
-    const uint32_t i = t0 + threadIdx.x;
-    uint32_t deg = 0, beg = 0, p = 0, nch = 0;
-    V v = op_identity<Op>();
-    if (threadIdx.x < tile && i < k) {
-      p = AL[i];
-      beg = rp[p];
-      deg = rp[p + 1] - beg;
-      v = mprop[p];
-      if (deg >= kHeavyDeg) nch = (deg + kHeavyChunk - 1) / kHeavyChunk;
-    }
-    if (__syncthreads_or(nch != 0)) {
-      uint32_t hch, hdeg;
-      const uint32_t at = block_excl_scan(nch, &hch);
-      (void)block_excl_scan(nch ? deg : 0u, &hdeg);
-      if (threadIdx.x == 0) {
-        s_slot = atomicAdd(&cnt->heavy, (unsigned long long)hch);
-        atomicAdd(&cnt->heavy_edges, (unsigned long long)hdeg);
-      }
-      __syncthreads();
-      for (uint32_t c = 0; c < nch; c++) heavy[s_slot + at + c] = make_uint2(p, c * kHeavyChunk);
-      if (nch) deg = 0;
-    }
-    uint32_t total;
-    const uint32_t ex = block_excl_scan(deg, &total);
-    s_off[threadIdx.x] = ex;
-    s_beg[threadIdx.x] = beg;
-    s_val[threadIdx.x] = v;
-    __syncthreads();
-    for (uint32_t j0 = threadIdx.x; j0 < total; j0 += kIlp * kBlock) {
-      uint32_t c[kIlp], w[kIlp];
-      V x[kIlp];
-#pragma unroll
-      for (int q = 0; q < kIlp; q++) {
-        const uint32_t j = j0 + q * kBlock;
-        const uint32_t t = push_owner(s_off, j);
-        const uint32_t e = j < total ? s_beg[t] + (j - s_off[t]) : s_beg[0];
-        c[q] = 0;
-        w[q] = 1u;
-        if (j < total) {
-          c[q] = col[e];
-          if (wt) w[q] = wt[e];
-        }
-        x[q] = s_val[t];
-      }
-#pragma unroll
-      for (int q = 0; q < kIlp; q++) x[q] = Op::edge(x[q], w[q]);
-      relax_many<Op, kIlp>(upd, dirty, c, x, (total - j0 + kBlock - 1) / kBlock);
-    }
-    if (threadIdx.x == 0) my_edges += total;
-    __syncthreads();
-  }
-  if (threadIdx.x == 0 && my_edges) atomicAdd(&cnt->edges, (unsigned long long)my_edges);
-}
-
-template <class Op>
-__global__ void __launch_bounds__(kBlock) k_push_heavy(const uint2 *__restrict__ heavy, const Counters *cnt,
-                                                       const uint32_t *__restrict__ rp, const uint32_t *__restrict__ col,
-                                                       const uint32_t *__restrict__ wt,
-                                                       const typename Op::V *__restrict__ mprop, typename Op::V *upd,
-                                                       uint64_t *dirty)
-{
-  using V = typename Op::V;
-  constexpr int kIlp = kHeavyChunk / kBlock;
-  const uint32_t nch = (uint32_t)cnt->heavy;
-  for (uint32_t h = blockIdx.x; h < nch; h += gridDim.x) {
-    const uint2 ch = heavy[h];
-    const uint32_t end = rp[ch.x + 1];
-    const uint32_t b = rp[ch.x] + ch.y, e = min(end, b + kHeavyChunk);
-    const V v = mprop[ch.x];
-    if (b + threadIdx.x >= e) continue;
-    uint32_t c[kIlp], w[kIlp];
-    V x[kIlp];
-#pragma unroll
-    for (int q = 0; q < kIlp; q++) {
-      const uint32_t at = b + threadIdx.x + q * kBlock;
-      c[q] = 0;
-      w[q] = 1u;
-      if (at < e) {
-        c[q] = col[at];
-        if (wt) w[q] = wt[at];
-      }
-    }
-#pragma unroll
-    for (int q = 0; q < kIlp; q++) x[q] = Op::edge(v, w[q]);
-    relax_many<Op, kIlp>(upd, dirty, c, x, (e - b - threadIdx.x + kBlock - 1) / kBlock);
-  }
-}
-
-// ------------------------------------------------------------------------
 // reduce: memory -> compute (bitvector = dirty words of the pair)
 // ------------------------------------------------------------------------
 
@@ -679,7 +546,6 @@ __global__ void k_zero_counters(Counters *cnt)
     cnt->pull_skipped_rows = 0;
     cnt->pull_done_arcs = 0;
     cnt->frontier_uncovered = 0;
-    cnt->ship_error = 0;
   }
   for (uint32_t c = threadIdx.x; c < (uint32_t)kMaxParts; c += blockDim.x) cnt->fpart[c] = 0;
 }
@@ -967,10 +833,7 @@ template <class Op>
 static grd_status traverse_t(grd_state *s, int option)
 {
   grd_graph *g = s->g;
-  grd_ctx *ctx = g->ctx;
-  hipStream_t st = ctx->stream;
-  using V = typename Op::V;
-  const uint32_t *wt = std::is_same<Op, OpWeighted>::value ? g->w : nullptr;
+  hipStream_t st = g->ctx->stream;
   const uint32_t *cwt = std::is_same<Op, OpWeighted>::value ? g->cw : nullptr;
   const bool timed = s->prm.time_kernel != 0;
   if (option & 1) {
@@ -992,18 +855,8 @@ static grd_status traverse_t(grd_state *s, int option)
     if (timed && s->skip_pending && s->prm.time_kernel != 2) GRD_TRY(pull_done_arcs(s));
     s->edges += g->m;  // every arc of the memory partitions, less those left out (counters)
   } else {
-    // tiles of 64 active vertices until those fill every workgroup slot
-    const uint64_t slots = (uint64_t)ctx->num_cus * 8;
-    const uint32_t tile = s->last_frontier <= 64 * slots ? 64u : (uint32_t)kBlock;
-    const uint32_t grid = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((s->last_frontier + tile - 1) / tile, slots));
     if (timed) GRD_HIP(hipEventRecord(s->kev[0], st));
-    hipLaunchKernelGGL((k_push<Op>), dim3(grid), dim3(kBlock), 0, st, s->AL, s->totals + 0, g->rp, g->col, wt,
-                       (const V *)s->mprop, (V *)s->mupd, s->Du, s->heavy, s->cnt, tile);
-    // a vertex's out-arcs all hang off its own proxy, so the frontier's largest
-    // out-degree tells whether any chunk was appended
-    if (s->last_maxdeg >= kHeavyDeg)
-      hipLaunchKernelGGL((k_push_heavy<Op>), dim3((uint32_t)slots), dim3(kBlock), 0, st, s->heavy, s->cnt, g->rp, g->col,
-                         wt, (const V *)s->mprop, (V *)s->mupd, s->Du);
+    GRD_TRY(push_launch<Op>(s));
     if (timed) {
       GRD_HIP(hipEventRecord(s->kev[1], st));
       s->kern_pending = 2;  // bytes from the edge counters after the iteration

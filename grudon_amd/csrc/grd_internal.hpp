@@ -105,7 +105,6 @@ struct Counters {
   double dangling[2];                 // PR pull: FP64 dangling mass (ping-pong)
   unsigned long long heavy_edges;     // push: edges of heavy vertices (k_push_heavy)
   unsigned long long frontier_uncovered;  // frontier vertices with an out-neighbour of another master
-  unsigned long long ship_error;      // edge shipping: the active list disagreed with the sized wire
   unsigned int fmin;                  // CC / SSSP pull: smallest value broadcast this superstep
   unsigned int pad32;
   unsigned long long pull_skipped;    // CC / SSSP pull: arcs of the cold row blocks left out (not read)
@@ -149,7 +148,6 @@ constexpr uint32_t kPullHot = 2048;      // PR pull: hottest sources of a partit
 constexpr uint32_t kColdRows = 8192;     // hot / cold pull: most rows per cold block
 constexpr uint32_t kHeavyDeg = 256;      // push: out-degree handled by k_push_heavy,
 constexpr uint32_t kHeavyChunk = 1024;   // in chunks of this many arcs (a workgroup each)
-constexpr uint32_t kShipTile = 1024;     // edge shipping: wire positions per workgroup tile
 constexpr int kMaxParts = 64;            // largest C and M
 constexpr uint32_t kTierBitsMax = 15;    // tiled pull: largest tier, 2^15 sources (128 KB of LDS)
 constexpr uint32_t kTierTileArcs = 65536;  // tiled pull: default arcs per tile
@@ -329,14 +327,6 @@ struct grd_state {
   float2 *tseg = nullptr;
   float2 *cseg = nullptr;   // hot / cold pull: partial per cold row block (long-row segments)
   double *red = nullptr;    // PR pull update: (residual, dangling) per workgroup
-  // edge shipping wire (grown on demand): record lengths / offsets, the first
-  // record of every tile, the records (gids) and their edge weights
-  grd::DevMem ship_mem;
-  uint32_t *ship_off = nullptr, *ship_tile = nullptr, *ship_buf = nullptr;
-  void *ship_w = nullptr;  // the records' weights, ship_wbytes each
-  uint64_t ship_kcap = 0, ship_cap = 0;
-  void *ship_tmp = nullptr;  // rocPRIM scan storage (in ship_mem)
-  size_t ship_tmp_bytes = 0;
   // NDPEngine inputs for the next decision: frontier size per compute
   // partition and frontier vertices not covered
   uint64_t last_fpart[grd::kMaxParts] = {};

@@ -83,7 +83,7 @@ __device__ __forceinline__ void relax(typename Op::V *upd, uint64_t *dirty, uint
 // relax for the first cnt of N destinations of one thread: the current values
 // are all loaded before any is compared, and the atomics are all issued before
 // any dirty mark waits for one
-template <class Op, int N>
+template <class Op, int N, bool kAlwaysMark>
 __device__ __forceinline__ void relax_many(typename Op::V *upd, uint64_t *dirty, const uint32_t (&dst)[N],
                                            const typename Op::V (&cand)[N], uint32_t cnt)
 {
@@ -101,6 +101,12 @@ __device__ __forceinline__ void relax_many(typename Op::V *upd, uint64_t *dirty,
     }
 #pragma unroll
     for (int q = 0; q < N; q++) mark[q] = on[q] && cand[q] < old[q];
+  } else if constexpr (kAlwaysMark) {
+#pragma unroll
+    for (int q = 0; q < N; q++) {
+      if (on[q]) atomicAdd(upd + dst[q], cand[q]);
+      mark[q] = on[q];
+    }
   } else {
     float old[N];
 #pragma unroll
@@ -223,6 +229,12 @@ __device__ __forceinline__ uint32_t pull_bound(const Counters *cnt, uint32_t inc
   return f + inc < f ? 0xFFFFFFFFu : f + inc;
 }
 
+// push launchers (push.hip): the active list's arcs into the memory side's
+// updates, or (edge shipping) into the compute side's
+template <class Op>
+grd_status push_launch(grd_state *s);
+template <class Op>
+grd_status ship_launch(grd_state *s);
 // pull launchers (pull.hip)
 template <class Op>
 grd_status bsp_pull_launch(grd_state *s, const uint32_t *cw);

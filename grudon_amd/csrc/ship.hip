@@ -8,24 +8,16 @@
 // include/offload_engine/NDPEngine.hpp:10-51 with the coverage vector of
 // src/DistributedGraph.cpp:286-370.
 //
-// On one GPU the wire is one buffer of records in active-list order (the
-// active list is grouped by (compute, memory) pair, so each pair's records
-// are contiguous).  A record names the source and its out-neighbours by
-// compute slot, the receiver's local id: the sender translates each proxy
-// with one lookup of the proxy -> slot table (the table the offloaded reduce
-// uses too), where gids would cost proxy -> gid on the way out and gid ->
-// slot on the way in.  An entry is 4 bytes either way.
-//   k_ship_len    record length (1 + out-degree) of every active proxy
-//   (rocPRIM exclusive scan: record offsets)
-//   k_ship_tiles  the record holding the first position of every tile
-//   k_ship_send   memory side: writes the records
-//   k_ship_recv   compute side: aggregate() of the source value
-// Both wire passes are merge-path tiled: a tile of kShipTile positions stages
-// the offsets of its records in LDS and each thread finds the record of its
-// position by binary search there, so the work per thread is even whatever
-// the degree spread, and the wire is read and written with unit stride.
-#include <rocprim/device/device_scan.hpp>
-
+// On one GPU the memory side's send and the compute side's receive are one
+// pass: the push over the active list (push.hip, kShip), reading each
+// out-neighbour by compute slot, the receiver's local id, and aggregating the
+// source's property into it.  The reference applies addUpdate in its receive
+// whatever the algorithm (a TODO at :624); this applies the algorithm's own
+// aggregate, which is what makes the schedule give the same result as the
+// offloaded one.  With the records written to a buffer and read back (record
+// lengths, their scan, tile starts, a send and a receive kernel) a shipping
+// superstep took five more launches and 8 to 10 bytes more per arc (CC on a
+// thousand vertices 364 -> 314 us a solve, weighted SSSP on RMAT-22 5.2 -> 5.1 ms).
 #include <algorithm>
 #include <cstring>
 #include <type_traits>
@@ -97,71 +89,8 @@ __global__ void __launch_bounds__(kBlock) k_frontier_parts(uint32_t nw, const ui
 }
 
 // ------------------------------------------------------------------------
-// the wire
+// shipped columns and weights
 // ------------------------------------------------------------------------
-
-// Record lengths of the k active proxies the host sized the wire for, and
-// len[k] = 0 so that the exclusive scan ends with the wire size.  If the
-// device's active list holds another count, every length is zero and the
-// error flag is raised; the later passes then find a wire size that differs
-// from the host's and do nothing.
-__global__ void __launch_bounds__(kBlock) k_ship_len(const uint32_t *__restrict__ AL, const uint32_t *__restrict__ nact,
-                                                     uint32_t k, const uint32_t *__restrict__ rp,
-                                                     uint32_t *__restrict__ len, Counters *cnt)
-{
-  const bool ok = *nact == k;
-  if (!ok && blockIdx.x == 0 && threadIdx.x == 0) cnt->ship_error = 1;
-  for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i <= k; i += gridDim.x * kBlock) {
-    uint32_t L = 0;
-    if (ok && i < k) {
-      const uint32_t p = AL[i];
-      L = rp[p + 1] - rp[p] + 1;
-    }
-    len[i] = L;
-  }
-}
-
-// tile[t] = the record holding wire position t * kShipTile.  Every record has
-// at least one position (its header), so each tile start is written once.
-__global__ void __launch_bounds__(kBlock) k_ship_tiles(const uint32_t *__restrict__ off, uint32_t k, uint32_t total,
-                                                       uint32_t *__restrict__ tile, Counters *cnt)
-{
-  if (off[k] != total) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) cnt->ship_error = 1;
-    return;
-  }
-  for (uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < k; i += gridDim.x * kBlock) {
-    const uint32_t a = off[i], b = off[i + 1];
-    for (uint64_t t = (a + (uint64_t)kShipTile - 1) / kShipTile; t * kShipTile < b; t++) tile[t] = i;
-  }
-}
-
-// Records of tile t: [tile[t], last], at most kShipTile + 1 of them, since all
-// records after the first start inside the tile.  Stages their offsets in
-// LDS; returns the record count (0: skip the tile).
-__device__ __forceinline__ uint32_t ship_tile_records(const uint32_t *__restrict__ off,
-                                                      const uint32_t *__restrict__ tile, uint32_t k, uint32_t t,
-                                                      uint32_t ntiles, uint32_t *s_off, uint32_t *first)
-{
-  const uint32_t a = tile[t], b = (t + 1 < ntiles) ? tile[t + 1] : k - 1;
-  if (b < a || b >= k || b - a + 1 > kShipTile + 1) return 0;
-  const uint32_t nr = b - a + 1;
-  for (uint32_t i = threadIdx.x; i <= nr; i += kBlock) s_off[i] = off[a + i];
-  *first = a;
-  return nr;
-}
-
-// the record of wire position q among the staged records: last i with s_off[i] <= q
-__device__ __forceinline__ uint32_t ship_owner(const uint32_t *s_off, uint32_t nr, uint32_t q)
-{
-  uint32_t lo = 0, hi = nr;
-  while (hi - lo > 1) {
-    const uint32_t mid = (lo + hi) >> 1;
-    if (s_off[mid] <= q) lo = mid;
-    else hi = mid;
-  }
-  return lo;
-}
 
 __global__ void __launch_bounds__(kBlock) k_ship_wmax(uint64_t m, const uint32_t *__restrict__ w, uint32_t *__restrict__ out)
 {
@@ -182,91 +111,6 @@ __global__ void __launch_bounds__(kBlock) k_slot_col(uint64_t m, const uint32_t 
 {
   for (uint64_t e = (uint64_t)blockIdx.x * kBlock + threadIdx.x; e < m; e += (uint64_t)gridDim.x * kBlock)
     scol[e] = proxy_slot[col[e]];
-}
-
-// Memory side (GraphAlgorithm.cpp:426-474): position 0 of a record is the
-// source's slot, position r > 0 the slot of its r-th out-neighbour (with the
-// arc weight in wbuf for weighted SSSP; the header's weight slot is 0).
-// The out-neighbours' slots come from scol, the push CSR with every column
-// translated to its compute slot once (a streaming read per shipped arc, not
-// a gather from the proxy -> slot table).
-// W: the weights' storage, a byte when every weight of the graph fits.
-template <class W>
-__global__ void __launch_bounds__(kBlock) k_ship_send(const uint32_t *__restrict__ AL, const uint32_t *__restrict__ off,
-                                                      const uint32_t *__restrict__ tile, uint32_t k, uint32_t total,
-                                                      uint32_t ntiles, const uint32_t *__restrict__ rp,
-                                                      const uint32_t *__restrict__ scol, const W *__restrict__ wt,
-                                                      const uint32_t *__restrict__ proxy_slot,
-                                                      uint32_t *__restrict__ buf, W *__restrict__ wbuf)
-{
-  __shared__ uint32_t s_off[kShipTile + 2];
-  __shared__ uint32_t s_beg[kShipTile + 1];
-  __shared__ uint32_t s_src[kShipTile + 1];
-  if (off[k] != total) return;
-  for (uint32_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
-    uint32_t a = 0;
-    const uint32_t nr = ship_tile_records(off, tile, k, t, ntiles, s_off, &a);
-    for (uint32_t i = threadIdx.x; i < nr; i += kBlock) {
-      const uint32_t p = AL[a + i];
-      s_beg[i] = rp[p];
-      s_src[i] = proxy_slot[p];
-    }
-    __syncthreads();
-    const uint32_t q0 = t * kShipTile, q1 = min(total, q0 + kShipTile);
-    if (nr)
-      for (uint32_t q = q0 + threadIdx.x; q < q1; q += kBlock) {
-        const uint32_t i = ship_owner(s_off, nr, q);
-        const uint32_t r = q - s_off[i];
-        uint32_t x;
-        W wx = 0;
-        if (r == 0) {
-          x = s_src[i];
-        } else {
-          const uint32_t e = s_beg[i] + r - 1;
-          x = scol[e];
-          if (wbuf) wx = wt[e];
-        }
-        buf[q] = x;
-        if (wbuf) wbuf[q] = wx;
-      }
-    __syncthreads();
-  }
-}
-
-// Compute side (GraphAlgorithm.cpp:582-637): aggregate() of the source's
-// property along each listed arc (the entries are already local ids, what
-// getLocalNode returns there).  The reference
-// applies addUpdate here whatever the algorithm (a TODO at :624); this applies
-// the algorithm's own aggregate, which is what makes the schedule give the
-// same result as the offloaded one.
-template <class Op, class W>
-__global__ void __launch_bounds__(kBlock) k_ship_recv(const uint32_t *__restrict__ off,
-                                                      const uint32_t *__restrict__ tile, uint32_t k, uint32_t total,
-                                                      uint32_t ntiles, const uint32_t *__restrict__ buf,
-                                                      const W *__restrict__ wbuf,
-                                                      const typename Op::V *__restrict__ prop, typename Op::V *upd,
-                                                      uint64_t *Dc)
-{
-  using V = typename Op::V;
-  __shared__ uint32_t s_off[kShipTile + 2];
-  __shared__ V s_val[kShipTile + 1];
-  if (off[k] != total) return;
-  for (uint32_t t = blockIdx.x; t < ntiles; t += gridDim.x) {
-    uint32_t a = 0;
-    const uint32_t nr = ship_tile_records(off, tile, k, t, ntiles, s_off, &a);
-    (void)a;
-    __syncthreads();
-    for (uint32_t i = threadIdx.x; i < nr; i += kBlock) s_val[i] = prop[buf[s_off[i]]];
-    __syncthreads();
-    const uint32_t q0 = t * kShipTile, q1 = min(total, q0 + kShipTile);
-    if (nr)
-      for (uint32_t q = q0 + threadIdx.x; q < q1; q += kBlock) {
-        const uint32_t i = ship_owner(s_off, nr, q);
-        if (q == s_off[i]) continue;  // the record's header
-        relax<Op, true>(upd, Dc, buf[q], Op::edge(s_val[i], wbuf ? (uint32_t)wbuf[q] : 1u));
-      }
-    __syncthreads();
-  }
 }
 
 // ------------------------------------------------------------------------
@@ -320,41 +164,16 @@ grd_status op_frontier_parts(grd_state *s)
   return GRD_OK;
 }
 
-// wire buffers for k records over `total` positions; grown (never shrunk)
-// outside any launch in flight
-static grd_status ship_reserve(grd_state *s, uint64_t k, uint64_t total, bool weighted, uint32_t wbytes)
-{
-  if (k + 1 <= s->ship_kcap && total <= s->ship_cap && (!weighted || s->ship_w)) return GRD_OK;
-  hipStream_t st = s->g->ctx->stream;
-  GRD_HIP(hipStreamSynchronize(st));
-  s->ship_mem.release();
-  s->ship_off = s->ship_tile = s->ship_buf = nullptr;
-  s->ship_w = nullptr;
-  s->ship_tmp = nullptr;
-  s->ship_tmp_bytes = 0;
-  const uint64_t kc = std::max<uint64_t>(k + 1 + (k + 1) / 4, 1024), cap = std::max<uint64_t>(total + total / 4, 4096);
-  const uint64_t tc = (cap + kShipTile - 1) / kShipTile + 1;
-  // lengths and offsets share one allocation: [len | off]
-  GRD_TRY(s->ship_mem.alloc_n(&s->ship_off, 2 * kc));
-  GRD_TRY(s->ship_mem.alloc_n(&s->ship_tile, tc));
-  GRD_TRY(s->ship_mem.alloc_n(&s->ship_buf, cap));
-  if (weighted) GRD_TRY(s->ship_mem.alloc(&s->ship_w, cap * wbytes));
-  s->ship_kcap = kc;
-  s->ship_cap = cap;
-  return GRD_OK;
-}
-
 template <class Op>
 static grd_status ship_t(grd_state *s)
 {
-  using V = typename Op::V;
   grd_graph *g = s->g;
-  grd_ctx *ctx = g->ctx;
-  hipStream_t st = ctx->stream;
+  hipStream_t st = g->ctx->stream;
   const uint64_t k = s->last_frontier, E = s->last_frontier_edges;
   if (k == 0) return GRD_OK;
   const uint64_t total = k + E;
-  if (total > 0xFFFFFFFFull - kShipTile) return fail(GRD_ERR_ARG, "edge shipping: the wire would exceed 2^32 entries");
+  // the records' entries (a source each, and its out-neighbours) are counted in 32 bits
+  if (total > 0xFFFFFFFFull - 1024) return fail(GRD_ERR_ARG, "edge shipping: the wire would exceed 2^32 entries");
   const bool weighted = std::is_same<Op, OpWeighted>::value;
   if (weighted && !g->ship_wbytes) {
     // the weights travel as bytes when every one of them is below 256
@@ -371,23 +190,6 @@ static grd_status ship_t(grd_state *s)
     }
     g->ship_wbytes = wmax < 256 ? 1 : 4;
   }
-  const uint32_t wbytes = weighted ? (uint32_t)g->ship_wbytes : 4u;
-  GRD_TRY(ship_reserve(s, k, total, weighted, wbytes));
-  uint32_t *len = s->ship_off + s->ship_kcap, *off = s->ship_off;
-  const uint32_t ntiles = (uint32_t)((total + kShipTile - 1) / kShipTile);
-  hipLaunchKernelGGL(k_ship_len, dim3(grid_for(k + 1)), dim3(kBlock), 0, st, s->AL, s->totals + 0, (uint32_t)k, g->rp,
-                     len, s->cnt);
-  size_t tb = 0;
-  GRD_HIP(rocprim::exclusive_scan(nullptr, tb, len, off, 0u, (size_t)k + 1, rocprim::plus<uint32_t>(), st));
-  if (tb > s->ship_tmp_bytes) {  // scan storage of the wire's own allocation
-    GRD_HIP(hipStreamSynchronize(st));
-    GRD_TRY(s->ship_mem.alloc(&s->ship_tmp, tb));
-    s->ship_tmp_bytes = tb;
-  }
-  GRD_HIP(rocprim::exclusive_scan(s->ship_tmp, tb, len, off, 0u, (size_t)k + 1, rocprim::plus<uint32_t>(), st));
-  hipLaunchKernelGGL(k_ship_tiles, dim3(grid_for(k)), dim3(kBlock), 0, st, off, (uint32_t)k, (uint32_t)total,
-                     s->ship_tile, s->cnt);
-  const uint32_t grid = std::max<uint32_t>(1, std::min<uint32_t>(ntiles, (uint32_t)ctx->num_cus * 8));
   if (!g->scol) {  // the push CSR's columns as compute slots, once per graph
     GRD_TRY(g->mem.alloc_n(&g->scol, std::max<uint64_t>(g->m, 1)));
     hipLaunchKernelGGL(k_slot_col, dim3(grid_for(g->m, 1u << 16)), dim3(kBlock), 0, st, g->m, g->col, g->proxy_slot,
@@ -396,32 +198,11 @@ static grd_status ship_t(grd_state *s)
   }
   const bool timed = s->prm.time_kernel != 0;
   if (timed) GRD_HIP(hipEventRecord(s->kev[0], st));
-  if (weighted && wbytes == 1) {
-    hipLaunchKernelGGL(k_ship_send<uint8_t>, dim3(grid), dim3(kBlock), 0, st, s->AL, off, s->ship_tile, (uint32_t)k,
-                       (uint32_t)total, ntiles, g->rp, g->scol, (const uint8_t *)g->w8, g->proxy_slot, s->ship_buf,
-                       (uint8_t *)s->ship_w);
-    hipLaunchKernelGGL((k_ship_recv<Op, uint8_t>), dim3(grid), dim3(kBlock), 0, st, off, s->ship_tile, (uint32_t)k,
-                       (uint32_t)total, ntiles, s->ship_buf, (const uint8_t *)s->ship_w, (const V *)s->prop,
-                       (V *)s->upd, s->Dc);
-  } else {
-    hipLaunchKernelGGL(k_ship_send<uint32_t>, dim3(grid), dim3(kBlock), 0, st, s->AL, off, s->ship_tile, (uint32_t)k,
-                       (uint32_t)total, ntiles, g->rp, g->scol, weighted ? (const uint32_t *)g->w : nullptr,
-                       g->proxy_slot, s->ship_buf, weighted ? (uint32_t *)s->ship_w : nullptr);
-    hipLaunchKernelGGL((k_ship_recv<Op, uint32_t>), dim3(grid), dim3(kBlock), 0, st, off, s->ship_tile, (uint32_t)k,
-                       (uint32_t)total, ntiles, s->ship_buf, weighted ? (const uint32_t *)s->ship_w : nullptr,
-                       (const V *)s->prop, (V *)s->upd, s->Dc);
-  }
-  GRD_HIP(hipGetLastError());
+  GRD_TRY(ship_launch<Op>(s));
   if (timed) {
-    // per arc: its slot (the slot column), wire write + read, the atomic
-    // read-modify-write (+ weight read, write, read, at its stored width);
-    // per record: active list, row bounds, offsets (twice), slot lookup,
-    // header write + read, property
     GRD_HIP(hipEventRecord(s->kev[1], st));
-    s->kern_pending = 1;
-    s->kern_pending_bytes = (20 + (weighted ? 3ull * wbytes : 0ull)) * E + 36 * k;
+    s->kern_pending = 2;  // bytes from the edge counters after the iteration
   }
-  s->edges += E;
   // wire bytes (MPI.hpp:44 counts count * sizeof(GNode) per send): one id
   // per record header and per arc, plus the weights of a weighted SSSP
   s->bytes += 4 * total + (weighted ? 4 * E : 0);
