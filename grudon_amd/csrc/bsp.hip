@@ -6,9 +6,9 @@
 // bitvector protocol works on 64-bit words, one wave per word (lane = bit).
 //
 // Reference loops replaced (src/GraphAlgorithm.cpp):
-//   k_bcast_send / k_bcast_recv   compute pack + memory unpack       :199-343
+//   k_bcast                       compute pack + memory unpack       :199-343
 //   (push.hip) / (pull.hip)       gen_updates (pr/cc/sssp.cpp)  :348-356
-//   k_reduce_send / k_reduce_recv memory pack + compute aggregate     :377-581
+//   k_reduce                      memory pack + compute aggregate    :377-581
 //   k_update                      update_frontier + apply_updates +
 //                                 termination popcount               :643-662
 //   k_popc_blocks/k_scan_blocks/k_word_rank  DynamicBitSet::getOffsets ranks
@@ -84,9 +84,44 @@ __global__ void __launch_bounds__(kBlock) k_word_rank(const uint64_t *__restrict
   }
 }
 
+// Short bitmaps in one launch: a workgroup of 1024, kRankPer consecutive words
+// per thread.  (Three launches of 2.5 us each for 4096 words; one of 3.)
+constexpr uint32_t kRankPer = 8;
+__global__ void __launch_bounds__(1024) k_word_rank_one(const uint64_t *__restrict__ w, uint32_t nw,
+                                                        uint32_t *__restrict__ wrank, uint32_t *total)
+{
+  __shared__ uint32_t s_w[16];
+  const uint32_t base = threadIdx.x * kRankPer;
+  uint32_t c[kRankPer], sum = 0;
+#pragma unroll
+  for (uint32_t i = 0; i < kRankPer; i++) c[i] = base + i < nw ? (uint32_t)__popcll(w[base + i]) : 0u;
+#pragma unroll
+  for (uint32_t i = 0; i < kRankPer; i++) sum += c[i];
+  const uint32_t inc = wave_incl_scan(sum);
+  if (lane_id() == kWave - 1) s_w[wave_in_block()] = inc;
+  __syncthreads();
+  uint32_t ex = inc - sum, tot = 0;
+#pragma unroll
+  for (int i = 0; i < 16; i++) {
+    if (i < wave_in_block()) ex += s_w[i];
+    tot += s_w[i];
+  }
+#pragma unroll
+  for (uint32_t i = 0; i < kRankPer; i++) {
+    if (base + i < nw) wrank[base + i] = ex;
+    ex += c[i];
+  }
+  if (threadIdx.x == 0) *total = tot;
+}
+
 static grd_status word_ranks(hipStream_t st, const uint64_t *w, uint32_t nw, uint32_t *blk, uint32_t *wrank,
                              uint32_t *total)
 {
+  if (nw <= 1024 * kRankPer) {
+    hipLaunchKernelGGL(k_word_rank_one, dim3(1), dim3(1024), 0, st, w, nw, wrank, total);
+    GRD_HIP(hipGetLastError());
+    return GRD_OK;
+  }
   uint32_t nb = (nw + kWordsPerScanBlock - 1) / kWordsPerScanBlock;
   if (nb == 0) nb = 1;
   hipLaunchKernelGGL(k_popc_blocks, dim3(nb), dim3(kBlock), 0, st, w, nw, blk);
@@ -147,17 +182,33 @@ __global__ void __launch_bounds__(kBlock) k_fill_u32(uint32_t *p, uint64_t n, ui
 {
   for (uint64_t i = blockIdx.x * (uint64_t)kBlock + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kBlock) p[i] = v;
 }
-__global__ void __launch_bounds__(kBlock) k_fill_u64(uint64_t *p, uint64_t n, uint64_t v)
-{
-  for (uint64_t i = blockIdx.x * (uint64_t)kBlock + threadIdx.x; i < n; i += (uint64_t)gridDim.x * kBlock) p[i] = v;
-}
+// the arrays a state starts from
+struct InitArrays {
+  uint64_t *F, *Dc, *Pend, *bvB;      // [S/64]
+  uint64_t *Du, *bvR;                 // [P/64]
+  uint32_t *valB;                     // [S]
+  uint32_t *mprop, *mupd, *valR;      // [P]
+};
 
-// compute-side init: pr.cpp:25-50, cc.cpp:24-36, sssp.cpp:22-46
-__global__ void __launch_bounds__(kBlock) k_init_compute(int algo, uint32_t nw, const uint32_t *__restrict__ slot_gid,
-                                                         const uint32_t *__restrict__ deg, void *prop_, void *upd_,
-                                                         float *pr, uint64_t *F, uint32_t source_slot)
+// compute-side init (pr.cpp:25-50, cc.cpp:24-36, sssp.cpp:22-46), and the
+// bitmaps, wires and memory-side values cleared, in one launch; a wave per
+// 64-vertex word
+__global__ void __launch_bounds__(kBlock) k_init_state(int algo, uint32_t nw, uint32_t nwP,
+                                                       const uint32_t *__restrict__ slot_gid,
+                                                       const uint32_t *__restrict__ deg, void *prop_, void *upd_,
+                                                       float *pr, InitArrays A, uint32_t neutral, uint32_t source_slot)
 {
   const int wpb = kWavesPerBlock;
+  for (uint32_t w = blockIdx.x * wpb + wave_in_block(); w < nwP; w += gridDim.x * wpb) {
+    const uint32_t p = w * 64 + lane_id();
+    A.mprop[p] = neutral;
+    A.mupd[p] = neutral;
+    A.valR[p] = neutral;
+    if (lane_id() == 0) {
+      A.Du[w] = 0;
+      A.bvR[w] = 0;
+    }
+  }
   for (uint32_t w = blockIdx.x * wpb + wave_in_block(); w < nw; w += gridDim.x * wpb) {
     uint32_t s = w * 64 + lane_id();
     uint32_t gid = slot_gid[s];
@@ -188,8 +239,14 @@ __global__ void __launch_bounds__(kBlock) k_init_compute(int algo, uint32_t nw, 
         f = src;
       }
     }
+    A.valB[s] = neutral;
     uint64_t fm = __ballot(f);
-    if (lane_id() == 0) F[w] = fm;
+    if (lane_id() == 0) {
+      A.F[w] = fm;
+      A.Dc[w] = 0;
+      A.Pend[w] = 0;
+      A.bvB[w] = 0;
+    }
   }
 }
 
@@ -197,36 +254,61 @@ __global__ void __launch_bounds__(kBlock) k_init_compute(int algo, uint32_t nw, 
 // broadcast: compute -> memory (bitvector = frontier words of the pair)
 // ------------------------------------------------------------------------
 
-// With fmin (a CC / SSSP pull), also the smallest value sent: the grid then
-// loops over the groups (loop_grid), so that one atomic per workgroup
-// carries it.
+// Send and receive in one pass.  A wave packs its group's words into the
+// pairs' bitvectors and values (the wire) and puts the same values into the
+// own proxies: the slot words of a pair map one to one onto its proxy words
+// (word_dst), so the receiver needs nothing that the sender does not hold.
+// For a push the active proxies get their value and the active list; for a
+// pull (want_list == 0) every own proxy is written, inactive ones with the
+// combine identity, so that the pull gathers one value per arc and needs no
+// activity test.  With fmin (a CC / SSSP pull), also the smallest value sent:
+// the grid then loops over the groups (loop_grid), so that one atomic per
+// workgroup carries it.  Every load of a group is issued before its first
+// store.  (With k_reduce, k_update, k_init_state and the one-launch ranks: CC on a thousand
+// vertices 314 -> 218 us a solve, hop SSSP by pushes on twenty thousand 727 -> 513,
+// delta-push PageRank on RMAT-18 85 -> 71 us a superstep.)
 template <typename V>
-__global__ void __launch_bounds__(kBlock) k_bcast_send(uint32_t nw, const uint64_t *__restrict__ F,
-                                                       const V *__restrict__ prop, const uint32_t *__restrict__ wrank,
-                                                       int dense, uint64_t *__restrict__ bv, V *__restrict__ val,
-                                                       unsigned int *fmin)
+__global__ void __launch_bounds__(kBlock) k_bcast(uint32_t nw, const uint64_t *__restrict__ F,
+                                                  const V *__restrict__ prop, const uint32_t *__restrict__ wrank,
+                                                  const uint32_t *__restrict__ word_dst, int dense, int want_list,
+                                                  V ident, uint64_t *__restrict__ bv, V *__restrict__ val,
+                                                  V *__restrict__ mprop, uint32_t *__restrict__ AL, unsigned int *fmin)
 {
   static_assert(sizeof(V) == 4, "4-byte values on the wire");
   const int l = lane_id();
+  const bool ranks = !dense || want_list;
   uint32_t lo = 0xFFFFFFFFu;
   for (uint32_t base = group_base(); base < nw; base += gridDim.x * kWavesPerBlock * kGroupWords) {
     const bool ok = l < (int)kGroupWords && base + l < nw;
     const uint64_t mine = ok ? F[base + l] : 0ull;
+    const uint32_t pwl = ok ? word_dst[base + l] : 0xFFFFFFFFu;
+    const uint32_t rkl = ok && ranks ? wrank[base + l] : 0u;
     if (ok) bv[base + l] = mine;
-    uint64_t todo = dense ? __ballot(ok) : __ballot(mine != 0);
-    while (todo) {
-      const int j = __ffsll((unsigned long long)todo) - 1;
-      todo &= todo - 1;
-      const uint64_t word = shfl_u64(mine, j);
-      const uint32_t w = base + j, s = w * 64 + l;
-      const bool on = (word >> l) & 1ull;
-      if (dense || on) {
-        const V x = prop[s];
-        if (dense) val[s] = x;
-        else val[wrank[w] + (uint32_t)__popcll(word & lanemask_lt())] = x;
-        const uint32_t u = __builtin_bit_cast(uint32_t, x);
-        if (on && u < lo) lo = u;
+    // a sparse push walks only the words that hold a frontier vertex
+    if (!dense && want_list && __ballot(mine != 0) == 0) continue;
+    V x[kGroupWords];
+    uint64_t word[kGroupWords];
+#pragma unroll
+    for (int j = 0; j < (int)kGroupWords; j++) {
+      word[j] = shfl_u64(mine, j);
+      x[j] = ident;
+      if (base + j < nw && (dense || ((word[j] >> l) & 1ull))) x[j] = prop[(base + j) * 64 + l];
+    }
+#pragma unroll
+    for (int j = 0; j < (int)kGroupWords; j++) {
+      const uint32_t w = base + j, pw = __shfl(pwl, j, kWave), rank = __shfl(rkl, j, kWave);
+      if (w >= nw) break;  // uniform over the wave
+      const bool on = (word[j] >> l) & 1ull;
+      const uint32_t r = rank + (uint32_t)__popcll(word[j] & lanemask_lt());
+      if (dense) val[w * 64 + l] = x[j];
+      else if (on) val[r] = x[j];
+      if (on) {
+        const uint32_t u = __builtin_bit_cast(uint32_t, x[j]);
+        lo = u < lo ? u : lo;
       }
+      if (pw == 0xFFFFFFFFu) continue;
+      if (on || !want_list) mprop[pw * 64 + l] = on ? x[j] : ident;
+      if (on && want_list) AL[r] = pw * 64 + l;
     }
   }
   if (fmin) {  // uniform: a kernel argument
@@ -256,201 +338,205 @@ __global__ void __launch_bounds__(kBlock) k_rows_done(uint32_t nwP, const uint32
   }
 }
 
-// Receive of the broadcast.  For a push the active proxies get their value
-// and the active list; for a pull (want_list == 0) every own proxy is written,
-// inactive ones with the combine identity, so that the pull gathers one value
-// per arc and needs no activity test.
-template <typename V>
-__global__ void __launch_bounds__(kBlock) k_bcast_recv(uint32_t nw, const uint64_t *__restrict__ bv,
-                                                       const V *__restrict__ val, const uint32_t *__restrict__ wrank,
-                                                       const uint32_t *__restrict__ word_dst, int dense, int want_list,
-                                                       V ident, V *__restrict__ mprop, uint32_t *__restrict__ AL)
-{
-  const uint32_t base = group_base();
-  const int l = lane_id();
-  const bool ok = l < (int)kGroupWords && base + l < nw;
-  const uint32_t pwl = ok ? word_dst[base + l] : 0xFFFFFFFFu;
-  const uint64_t mine = (pwl != 0xFFFFFFFFu) ? bv[base + l] : 0ull;
-  uint64_t todo = want_list ? __ballot(mine != 0) : __ballot(pwl != 0xFFFFFFFFu);
-  while (todo) {
-    const int j = __ffsll((unsigned long long)todo) - 1;
-    todo &= todo - 1;
-    const uint64_t word = shfl_u64(mine, j);
-    const uint32_t pw = __shfl(pwl, j, kWave);
-    const uint32_t w = base + j;
-    const uint32_t p = pw * 64 + l;
-    if ((word >> l) & 1ull) {
-      uint32_t r = (dense && !want_list) ? 0u : wrank[w] + (uint32_t)__popcll(word & lanemask_lt());
-      V x = dense ? val[w * 64 + l] : val[r];
-      mprop[p] = x;
-      if (want_list) AL[r] = p;
-    } else if (!want_list) {
-      mprop[p] = ident;
-    }
-  }
-}
-
 // ------------------------------------------------------------------------
 // reduce: memory -> compute (bitvector = dirty words of the pair)
 // ------------------------------------------------------------------------
 
-template <typename V>
-__global__ void __launch_bounds__(kBlock) k_reduce_send(uint32_t nw, uint64_t *__restrict__ Du, V *__restrict__ mupd,
-                                                        const uint32_t *__restrict__ wrank, int dense, int clear_vals,
-                                                        uint64_t *__restrict__ bv, V *__restrict__ val, Counters *cnt)
+// Send and receive in one pass: a wave packs its group's dirty words and values
+// into the pairs' messages (the wire) and aggregates the same values into the
+// compute side, all loads of the group (values, slots, and for min-combines the
+// current values) before the first store, all atomics before the first mark.
+// A capped grid loops over the groups (one counter atomic per workgroup).
+template <class Op>
+__global__ void __launch_bounds__(kBlock) k_reduce(uint32_t nw, uint64_t *__restrict__ Du,
+                                                   typename Op::V *__restrict__ mupd,
+                                                   const uint32_t *__restrict__ wrank,
+                                                   const uint32_t *__restrict__ proxy_slot, int dense,
+                                                   uint64_t *__restrict__ bv, typename Op::V *__restrict__ val,
+                                                   typename Op::V *upd, uint64_t *Dc, Counters *cnt)
 {
+  using V = typename Op::V;
   const int l = lane_id();
   uint32_t ndirty = 0;
-  // capped grid, wave-uniform loop over the word groups (fewer counter atomics)
   for (uint32_t base = group_base(); base < nw; base += gridDim.x * kWavesPerBlock * kGroupWords) {
     const bool ok = l < (int)kGroupWords && base + l < nw;
     const uint64_t mine = ok ? Du[base + l] : 0ull;
+    const uint32_t rkl = (ok && !dense) ? wrank[base + l] : 0u;
     if (ok) {
       bv[base + l] = mine;
       if (mine) Du[base + l] = 0;
     }
     ndirty += (uint32_t)__popcll(mine);
-    uint64_t todo = dense ? __ballot(ok) : __ballot(mine != 0);
-    while (todo) {
-      const int j = __ffsll((unsigned long long)todo) - 1;
-      todo &= todo - 1;
-      const uint64_t word = shfl_u64(mine, j);
-      const uint32_t w = base + j, p = w * 64 + l;
-      const bool bit = (word >> l) & 1ull;
-      if (dense) val[p] = mupd[p];
-      else if (bit) val[wrank[w] + (uint32_t)__popcll(word & lanemask_lt())] = mupd[p];
-      if (clear_vals && bit) mupd[p] = V(0);  // PropertyList::clear (DistributedGraph.hpp:140-166)
+    if (!dense && __ballot(mine != 0) == 0) continue;
+    uint64_t word[kGroupWords];
+    uint32_t s[kGroupWords];
+    V x[kGroupWords];
+#pragma unroll
+    for (int j = 0; j < (int)kGroupWords; j++) {
+      word[j] = shfl_u64(mine, j);
+      const uint32_t p = (base + j) * 64 + l;
+      const bool on = (word[j] >> l) & 1ull;
+      s[j] = 0xFFFFFFFFu;
+      x[j] = V{};
+      if (base + j < nw && (dense || on)) x[j] = mupd[p];
+      if (on) s[j] = proxy_slot[p];
+    }
+    V cur[kGroupWords];
+    if constexpr (Op::kMin) {
+#pragma unroll
+      for (int j = 0; j < (int)kGroupWords; j++)
+        cur[j] = s[j] != 0xFFFFFFFFu ? __atomic_load_n(upd + s[j], __ATOMIC_RELAXED) : V{};
+    }
+#pragma unroll
+    for (int j = 0; j < (int)kGroupWords; j++) {
+      const uint32_t w = base + j, p = w * 64 + l, rank = __shfl(rkl, j, kWave);
+      if (w >= nw) break;  // uniform over the wave
+      const bool on = (word[j] >> l) & 1ull;
+      if (dense) val[p] = x[j];
+      else if (on) val[rank + (uint32_t)__popcll(word[j] & lanemask_lt())] = x[j];
+      // PropertyList::clear (DistributedGraph.hpp:140-166); the min-combines keep theirs
+      if (!Op::kMin && on) mupd[p] = V(0);
+    }
+    // aggregate(): minUpdate / addUpdate, then the dirty marks of the wave
+    bool mark[kGroupWords];
+#pragma unroll
+    for (int j = 0; j < (int)kGroupWords; j++) {
+      mark[j] = false;
+      if (s[j] != 0xFFFFFFFFu) {
+        if constexpr (Op::kMin) {
+          mark[j] = x[j] < cur[j];
+          if (mark[j]) cur[j] = atomicMin(upd + s[j], x[j]);
+        } else {
+          atomicAdd(upd + s[j], x[j]);
+          mark[j] = true;
+        }
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < (int)kGroupWords; j++) {
+      if (word[j] == 0) continue;  // uniform over the wave
+      if constexpr (Op::kMin) mark[j] = mark[j] && x[j] < cur[j];
+      mark_wave(Dc, s[j], mark[j]);
     }
   }
   uint32_t t = block_sum(ndirty);
   if (threadIdx.x == 0 && t) atomicAdd(&cnt->dirty, (unsigned long long)t);
 }
 
-template <class Op>
-__global__ void __launch_bounds__(kBlock) k_reduce_recv(uint32_t nw, const uint64_t *__restrict__ bv,
-                                                        const typename Op::V *__restrict__ val,
-                                                        const uint32_t *__restrict__ wrank,
-                                                        const uint32_t *__restrict__ proxy_slot, int dense,
-                                                        typename Op::V *upd, uint64_t *Dc)
-{
-  using V = typename Op::V;
-  const uint32_t base = group_base();
-  const int l = lane_id();
-  const bool ok = l < (int)kGroupWords && base + l < nw;
-  const uint64_t mine = ok ? bv[base + l] : 0ull;
-  const uint32_t myrank = (ok && !dense) ? wrank[base + l] : 0u;
-  if (__ballot(mine != 0) == 0) return;
-  // the group's words in every lane, then every load of the group (values,
-  // slots, and for min-combines the current values) issued before any is
-  // waited for; the relaxations and marks then follow word by word
-  uint64_t word[kGroupWords];
-  uint32_t s[kGroupWords];
-  V x[kGroupWords];
-#pragma unroll
-  for (int j = 0; j < (int)kGroupWords; j++) {
-    word[j] = shfl_u64(mine, j);
-    const uint32_t rank = __shfl(myrank, j, kWave);
-    s[j] = 0xFFFFFFFFu;
-    x[j] = V{};
-    if ((word[j] >> l) & 1ull) {
-      const uint32_t p = (base + j) * 64 + l;
-      x[j] = dense ? val[p] : val[rank + (uint32_t)__popcll(word[j] & lanemask_lt())];
-      s[j] = proxy_slot[p];
-    }
-  }
-  V cur[kGroupWords];
-  if constexpr (Op::kMin) {
-#pragma unroll
-    for (int j = 0; j < (int)kGroupWords; j++)
-      cur[j] = s[j] != 0xFFFFFFFFu ? __atomic_load_n(upd + s[j], __ATOMIC_RELAXED) : V{};
-  }
-#pragma unroll
-  for (int j = 0; j < (int)kGroupWords; j++) {
-    if (word[j] == 0) continue;  // uniform over the wave
-    // aggregate(): minUpdate / addUpdate, then the dirty marks of the wave
-    bool mark = false;
-    if (s[j] != 0xFFFFFFFFu) {
-      if constexpr (Op::kMin) mark = x[j] < cur[j] && x[j] < atomicMin(upd + s[j], x[j]);
-      else mark = relax_nomark<Op, true>(upd, s[j], x[j]);
-    }
-    mark_wave(Dc, s[j], mark);
-  }
-}
-
 // ------------------------------------------------------------------------
 // update: update_frontier + apply_updates + frontier popcount
 // ------------------------------------------------------------------------
 
+// a workgroup's counters: sums of a, b, c and the largest m over its threads,
+// in thread 0 (one barrier)
+__device__ __forceinline__ void block_counts(uint64_t &a, uint64_t &b, uint64_t &c, uint32_t &m)
+{
+  __shared__ uint64_t s_c[kWavesPerBlock][4];
+  a = wave_sum(a);
+  b = wave_sum(b);
+  c = wave_sum(c);
+  m = wave_max(m);
+  if (lane_id() == 0) {
+    s_c[wave_in_block()][0] = a;
+    s_c[wave_in_block()][1] = b;
+    s_c[wave_in_block()][2] = c;
+    s_c[wave_in_block()][3] = m;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0)
+    for (int i = 1; i < kWavesPerBlock; i++) {
+      a += s_c[i][0];
+      b += s_c[i][1];
+      c += s_c[i][2];
+      m = max(m, (uint32_t)s_c[i][3]);
+    }
+}
+
+// A capped grid walks the word groups (the loop is wave-uniform), so the
+// blocks' counter atomics are issued by fewer blocks.  All loads of a group's
+// words are issued before any is used, and lane j stores word j's bitmap words
+// (word by word, a group was a chain of up to eight dependent round trips:
+// 11 us on 4096 words, 36 on 65536).
 template <int ALGO>  // GRD_PR, GRD_CC or GRD_SSSP
 __global__ void __launch_bounds__(kBlock) k_update(uint32_t nw, uint64_t *__restrict__ Dc, void *prop_, void *upd_,
                                                    float *__restrict__ pr, const uint32_t *__restrict__ deg,
                                                    uint64_t *__restrict__ F, uint64_t *__restrict__ Pend,
                                                    unsigned long long hi, int use_delta, Counters *cnt)
 {
+  using V = typename std::conditional<ALGO == GRD_PR, float, uint32_t>::type;
+  V *__restrict__ prop = (V *)prop_;
+  V *__restrict__ upd = (V *)upd_;
   const int l = lane_id();
   uint64_t f_cnt = 0, f_edges = 0, improved = 0;
   uint32_t f_max = 0;
-  // a capped grid walks the word groups (the loop is wave-uniform), so the
-  // block's counter atomics below are issued by fewer blocks
   for (uint32_t base = group_base(); base < nw; base += gridDim.x * kWavesPerBlock * kGroupWords) {
     const bool ok = l < (int)kGroupWords && base + l < nw;
     const uint64_t mine = ok ? Dc[base + l] : 0ull;
-    if (ok && !mine) F[base + l] = 0;  // nothing changed: empty next-frontier word
-    uint64_t todo = __ballot(mine != 0);
-    while (todo) {
-      const int j = __ffsll((unsigned long long)todo) - 1;
-      todo &= todo - 1;
-      const uint64_t d = shfl_u64(mine, j);
-      const uint32_t w = base + j, s = w * 64 + l;
-      bool f = false, pend = false, imp = false;
-      if ((d >> l) & 1ull) {
-        if constexpr (ALGO == GRD_PR) {
-          float *prop = (float *)prop_, *upd = (float *)upd_;
-          float u = upd[s];
-          if ((double)u > 1e-6) {  // pr.cpp:133-142 and :76-83 (prev is always 0 here)
-            f = true;
-            pr[s] = pr[s] + u;
-            prop[s] = (float)(0.85 * (double)u / (double)deg[s]);
-            upd[s] = 0.0f;
-          }
-        } else {
-          uint32_t *prop = (uint32_t *)prop_, *upd = (uint32_t *)upd_;
-          uint32_t u = upd[s];
-          if (prop[s] > u) {  // cc.cpp:100-106, sssp.cpp:102-108
-            prop[s] = u;
-            imp = true;
-            if (use_delta && (unsigned long long)u >= hi) pend = true;
+    uint64_t fmine = 0, pmine = 0;
+    if (use_delta && mine) pmine = Pend[base + l];
+    if (__ballot(mine != 0)) {
+      uint64_t d[kGroupWords];
+      V u[kGroupWords], o[kGroupWords];
+      uint32_t dg[kGroupWords];
+#pragma unroll
+      for (int j = 0; j < (int)kGroupWords; j++) {
+        d[j] = shfl_u64(mine, j);
+        const uint32_t s = (base + j) * 64 + l;
+        u[j] = o[j] = V(0);
+        dg[j] = 0;
+        if ((d[j] >> l) & 1ull) {
+          u[j] = upd[s];
+          o[j] = ALGO == GRD_PR ? (V)pr[s] : prop[s];
+          dg[j] = deg[s];
+        }
+      }
+#pragma unroll
+      for (int j = 0; j < (int)kGroupWords; j++) {
+        if (d[j] == 0) continue;  // uniform over the wave
+        const uint32_t s = (base + j) * 64 + l;
+        bool f = false, pend = false;
+        if ((d[j] >> l) & 1ull) {
+          if constexpr (ALGO == GRD_PR) {
+            if ((double)u[j] > 1e-6) {  // pr.cpp:133-142 and :76-83 (prev is always 0 here)
+              f = true;
+              pr[s] = o[j] + u[j];
+              prop[s] = (float)(0.85 * (double)u[j] / (double)dg[j]);
+              upd[s] = 0.0f;
+            }
+          } else if (o[j] > u[j]) {  // cc.cpp:100-106, sssp.cpp:102-108
+            prop[s] = u[j];
+            improved++;
+            if (use_delta && (unsigned long long)u[j] >= hi) pend = true;
             else f = true;
           }
         }
+        if (f) {
+          f_edges += dg[j];
+          f_max = max(f_max, dg[j]);
+        }
+        const uint64_t fm = __ballot(f);
+        if (l == j) fmine = fm;
+        if (use_delta) {
+          const uint64_t pm = __ballot(pend);
+          if (l == j) pmine = (pmine | pm) & ~fm;
+        }
       }
-      const uint64_t fm = __ballot(f);
-      if (l == 0) {
-        F[w] = fm;
-        Dc[w] = 0;
-        f_cnt += (uint64_t)__popcll(fm);
+    }
+    if (ok) {
+      F[base + l] = fmine;  // (nothing changed: an empty next-frontier word)
+      if (mine) {
+        Dc[base + l] = 0;
+        if (use_delta) Pend[base + l] = pmine;
       }
-      if (use_delta) {
-        const uint64_t pm = __ballot(pend);
-        if (l == 0 && (pm | fm)) Pend[w] = (Pend[w] | pm) & ~fm;
-      }
-      if (f) {
-        uint32_t dg = deg[s];
-        f_edges += dg;
-        f_max = dg > f_max ? dg : f_max;
-      }
-      improved += imp;
+      f_cnt += (uint64_t)__popcll(fmine);
     }
   }
-  uint64_t a = block_sum(f_cnt);
-  uint64_t b = block_sum(f_edges);
-  uint64_t c = block_sum(improved);
-  uint32_t mx = block_max(f_max);
+  block_counts(f_cnt, f_edges, improved, f_max);
   if (threadIdx.x == 0) {
-    if (a) atomicAdd(&cnt->frontier, (unsigned long long)a);
-    if (b) atomicAdd(&cnt->frontier_edges, (unsigned long long)b);
-    if (c) atomicAdd(&cnt->improved, (unsigned long long)c);
-    if (mx) atomicMax(&cnt->frontier_maxdeg, mx);
+    if (f_cnt) atomicAdd(&cnt->frontier, (unsigned long long)f_cnt);
+    if (f_edges) atomicAdd(&cnt->frontier_edges, (unsigned long long)f_edges);
+    if (improved) atomicAdd(&cnt->improved, (unsigned long long)improved);
+    if (f_max) atomicMax(&cnt->frontier_maxdeg, f_max);
   }
 }
 
@@ -486,44 +572,54 @@ __global__ void __launch_bounds__(kBlock) k_pend_min(uint32_t nw, const uint64_t
 }
 
 // delta-stepping: move pending vertices below the new bucket bound into F
+// (loads and stores of a group as in k_update)
 __global__ void __launch_bounds__(kBlock) k_select(uint32_t nw, uint64_t *__restrict__ Pend,
                                                    const uint32_t *__restrict__ prop, const uint32_t *__restrict__ deg,
                                                    unsigned long long hi, uint64_t *__restrict__ F, Counters *cnt)
 {
   const int l = lane_id();
-  uint64_t f_cnt = 0, f_edges = 0;
+  uint64_t f_cnt = 0, f_edges = 0, none = 0;
   uint32_t f_max = 0;
-  // capped grid, wave-uniform loop over the word groups
   for (uint32_t base = group_base(); base < nw; base += gridDim.x * kWavesPerBlock * kGroupWords) {
     const bool ok = l < (int)kGroupWords && base + l < nw;
     const uint64_t mine = ok ? Pend[base + l] : 0ull;
-    if (ok && !mine) F[base + l] = 0;
-    uint64_t todo = __ballot(mine != 0);
-    while (todo) {
-      const int j = __ffsll((unsigned long long)todo) - 1;
-      todo &= todo - 1;
-      const uint64_t pm = shfl_u64(mine, j);
-      const uint32_t w = base + j, s = w * 64 + l;
-      const bool f = ((pm >> l) & 1ull) && (unsigned long long)prop[s] < hi;
-      const uint64_t fm = __ballot(f);
-      if (l == 0) {
-        F[w] = fm;
-        if (fm) Pend[w] = pm & ~fm;
-        f_cnt += (uint64_t)__popcll(fm);
+    uint64_t fmine = 0;
+    if (__ballot(mine != 0)) {
+      uint64_t pm[kGroupWords];
+      uint32_t v[kGroupWords], dg[kGroupWords];
+#pragma unroll
+      for (int j = 0; j < (int)kGroupWords; j++) {
+        pm[j] = shfl_u64(mine, j);
+        const uint32_t s = (base + j) * 64 + l;
+        v[j] = 0xFFFFFFFFu;
+        dg[j] = 0;
+        if ((pm[j] >> l) & 1ull) {
+          v[j] = prop[s];
+          dg[j] = deg[s];
+        }
       }
-      if (f) {
-        uint32_t dg = deg[s];
-        f_edges += dg;
-        f_max = dg > f_max ? dg : f_max;
+#pragma unroll
+      for (int j = 0; j < (int)kGroupWords; j++) {
+        const bool f = ((pm[j] >> l) & 1ull) && (unsigned long long)v[j] < hi;
+        const uint64_t fm = __ballot(f);
+        if (l == j) fmine = fm;
+        if (f) {
+          f_edges += dg[j];
+          f_max = max(f_max, dg[j]);
+        }
       }
     }
+    if (ok) {
+      F[base + l] = fmine;
+      if (fmine) Pend[base + l] = mine & ~fmine;
+      f_cnt += (uint64_t)__popcll(fmine);
+    }
   }
-  uint64_t a = block_sum(f_cnt), b = block_sum(f_edges);
-  uint32_t mx = block_max(f_max);
+  block_counts(f_cnt, f_edges, none, f_max);
   if (threadIdx.x == 0) {
-    if (a) atomicAdd(&cnt->frontier, (unsigned long long)a);
-    if (b) atomicAdd(&cnt->frontier_edges, (unsigned long long)b);
-    if (mx) atomicMax(&cnt->frontier_maxdeg, mx);
+    if (f_cnt) atomicAdd(&cnt->frontier, (unsigned long long)f_cnt);
+    if (f_edges) atomicAdd(&cnt->frontier_edges, (unsigned long long)f_edges);
+    if (f_max) atomicMax(&cnt->frontier_maxdeg, f_max);
   }
 }
 
@@ -669,40 +765,18 @@ grd_status state_alloc(grd_state *s)
   return GRD_OK;
 }
 
-static grd_status fill_u32(hipStream_t st, void *p, uint64_t n, uint32_t v)
-{
-  hipLaunchKernelGGL(k_fill_u32, dim3((uint32_t)std::min<uint64_t>(4096, (n + kBlock - 1) / kBlock + 1)), dim3(kBlock), 0,
-                     st, (uint32_t *)p, n, v);
-  GRD_HIP(hipGetLastError());
-  return GRD_OK;
-}
-static grd_status fill_u64(hipStream_t st, void *p, uint64_t n, uint64_t v)
-{
-  hipLaunchKernelGGL(k_fill_u64, dim3((uint32_t)std::min<uint64_t>(4096, (n + kBlock - 1) / kBlock + 1)), dim3(kBlock), 0,
-                     st, (uint64_t *)p, n, v);
-  GRD_HIP(hipGetLastError());
-  return GRD_OK;
-}
-
 grd_status state_init(grd_state *s)
 {
   grd_graph *g = s->g;
   hipStream_t st = g->ctx->stream;
   const uint32_t nwS = g->S / 64, nwP = g->P / 64;
-  GRD_TRY(fill_u64(st, s->Dc, nwS, 0));
-  GRD_TRY(fill_u64(st, s->Pend, nwS, 0));
-  GRD_TRY(fill_u64(st, s->Du, nwP, 0));
-  GRD_TRY(fill_u64(st, s->bvB, nwS, 0));
-  GRD_TRY(fill_u64(st, s->bvR, nwP, 0));
   const uint32_t neutral = (s->algo == GRD_PR) ? 0u : 0xFFFFFFFFu;  // PR: 0.0f bit pattern
-  GRD_TRY(fill_u32(st, s->mprop, g->P, neutral));
-  GRD_TRY(fill_u32(st, s->mupd, g->P, neutral));
-  GRD_TRY(fill_u32(st, s->valR, g->P, neutral));
-  GRD_TRY(fill_u32(st, s->valB, g->S, neutral));
   uint32_t source_slot = 0xFFFFFFFFu;
   if (s->algo == GRD_SSSP) source_slot = g->h_gid_slot[s->prm.source];
-  hipLaunchKernelGGL(k_init_compute, dim3(wave_grid(g->ctx, nwS)), dim3(kBlock), 0, st, s->algo, nwS, g->slot_gid,
-                     g->slot_deg, s->prop, s->upd, s->pr, s->F, source_slot);
+  const InitArrays A{s->F, s->Dc, s->Pend, s->bvB, s->Du, s->bvR, (uint32_t *)s->valB,
+                     (uint32_t *)s->mprop, (uint32_t *)s->mupd, (uint32_t *)s->valR};
+  hipLaunchKernelGGL(k_init_state, dim3(wave_grid(g->ctx, std::max(nwS, nwP))), dim3(kBlock), 0, st, s->algo, nwS, nwP,
+                     g->slot_gid, g->slot_deg, s->prop, s->upd, s->pr, A, neutral, source_slot);
   GRD_HIP(hipGetLastError());
   GRD_TRY(op_zero_counters(s));
   s->hi = (s->algo == GRD_SSSP && s->prm.delta) ? (uint64_t)s->prm.delta : ~0ull;
@@ -794,7 +868,6 @@ grd_status op_broadcast(grd_state *s, int option)
   s->xb_dense = dense ? 1 : 0;
   s->xr_dense = -1;
   if (need_rank) GRD_TRY(word_ranks(st, s->F, nwS, s->blk, s->wrankB, s->totals + 0));
-  const uint32_t grid = group_grid(nwS);
   // a pull of CC / SSSP also sends the smallest value broadcast and the rows
   // that cannot improve (the pull leaves out what cannot change unless the
   // caller asked for every row); the rows-done bitmap not in the first
@@ -802,12 +875,10 @@ grd_status op_broadcast(grd_state *s, int option)
   // the frontier's smallest is done
   const bool bound = pull && s->algo != GRD_PR && !s->prm.pull_every_row;
   const bool rows_done = bound && s->iteration > 0;
-  hipLaunchKernelGGL(k_bcast_send<uint32_t>, dim3(bound ? loop_grid(g->ctx, nwS) : grid), dim3(kBlock), 0, st,
-                     nwS, s->F, (const uint32_t *)s->prop, s->wrankB, (int)dense, s->bvB, (uint32_t *)s->valB,
-                     bound ? &s->cnt->fmin : nullptr);
   const uint32_t ident = (s->algo == GRD_PR) ? 0u : 0xFFFFFFFFu;  // 0.0f or the min identity
-  hipLaunchKernelGGL(k_bcast_recv<uint32_t>, dim3(grid), dim3(kBlock), 0, st, nwS, s->bvB, (const uint32_t *)s->valB,
-                     s->wrankB, g->word_dst, (int)dense, (int)!pull, ident, (uint32_t *)s->mprop, s->AL);
+  hipLaunchKernelGGL(k_bcast<uint32_t>, dim3(bound ? loop_grid(g->ctx, nwS) : group_grid(nwS)), dim3(kBlock), 0, st,
+                     nwS, s->F, (const uint32_t *)s->prop, s->wrankB, g->word_dst, (int)dense, (int)!pull, ident,
+                     s->bvB, (uint32_t *)s->valB, (uint32_t *)s->mprop, s->AL, bound ? &s->cnt->fmin : nullptr);
   const uint32_t nwP = g->P / 64;
   uint32_t inc = 0;  // the smallest Op::edge increment over an arc
   if (bound && s->algo == GRD_SSSP) {
@@ -886,12 +957,8 @@ static grd_status reduce_t(grd_state *s, int option)
   const bool dense = option & 2;
   s->xr_dense = dense ? 1 : 0;
   if (!dense) GRD_TRY(word_ranks(st, s->Du, nwP, s->blk, s->wrankR, s->totals + 1));
-  const uint32_t grid = group_grid(nwP);
-  const uint32_t grid_send = loop_grid(g->ctx, nwP);
-  hipLaunchKernelGGL(k_reduce_send<V>, dim3(grid_send), dim3(kBlock), 0, st, nwP, s->Du, (V *)s->mupd, s->wrankR,
-                     (int)dense, (int)(s->algo == GRD_PR), s->bvR, (V *)s->valR, s->cnt);
-  hipLaunchKernelGGL((k_reduce_recv<Op>), dim3(grid), dim3(kBlock), 0, st, nwP, s->bvR, (const V *)s->valR, s->wrankR,
-                     g->proxy_slot, (int)dense, (V *)s->upd, s->Dc);
+  hipLaunchKernelGGL((k_reduce<Op>), dim3(loop_grid(g->ctx, nwP)), dim3(kBlock), 0, st, nwP, s->Du, (V *)s->mupd,
+                     s->wrankR, g->proxy_slot, (int)dense, s->bvR, (V *)s->valR, (V *)s->upd, s->Dc, s->cnt);
   GRD_HIP(hipGetLastError());
   return GRD_OK;
 }

@@ -119,21 +119,6 @@ __device__ __forceinline__ void relax_many(typename Op::V *upd, uint64_t *dirty,
     if (mark[q]) set_bit(dirty, dst[q]);
 }
 
-// relax without the dirty mark; returns whether the destination must be
-// marked (same rules as relax)
-template <class Op, bool kAlwaysMark = false>
-__device__ __forceinline__ bool relax_nomark(typename Op::V *upd, uint32_t dst, typename Op::V cand)
-{
-  if constexpr (Op::kMin) {
-    uint32_t cur = __atomic_load_n(upd + dst, __ATOMIC_RELAXED);
-    if (cand < cur) return cand < atomicMin(upd + dst, cand);
-    return false;
-  } else {
-    float old = atomicAdd(upd + dst, cand);
-    return kAlwaysMark || old == 0.0f;
-  }
-}
-
 // Sets bit i for every lane with pred.  Called by the whole wave: when all
 // marked bits fall into one 64-bit word (a wave over a word of own proxies
 // maps onto one word of slots) they are OR-ed across the wave and written by

@@ -67,3 +67,22 @@ def test_push_tile_edges(ctx, n):
     stats = S.run()
     assert np.array_equal(S.result(), ref)
     assert stats["iterations"] == int(st[0])
+
+
+@pytest.mark.parametrize("n", [524225, 524287, 524288, 524289, 600001])
+def test_rank_edges(ctx, n):
+    """Bitmaps around 8192 words, where the word ranks turn from one launch to
+    three, in sparse pushes and pulls."""
+    print("rank edges", n, flush=True)
+    v = np.arange(n, dtype=np.uint32)
+    rp = np.concatenate([[0], np.maximum(np.arange(1, n + 1) - 1, 0)]).astype(np.uint32)
+    g = O.Graph(rp, v[1:] // 2)  # v -> v / 2
+    ref, st = O.Partition(g, 1, 2).cc()
+    G = api.Graph.from_csr(ctx, g.rp, g.col, C=1, M=2)
+    for option in (api.OPT_PUSH_SPARSE, api.OPT_PULL_SPARSE, api.OPT_SHIP_EDGES):
+        S = api.State(G, api.CC)
+        S.init(sched=api.SCHED_FIXED, fixed_option=option)
+        stats = S.run()
+        assert np.array_equal(S.result(), ref)
+        assert stats["iterations"] == int(st[0])
+        S.free()
