@@ -168,7 +168,8 @@ static grd_status finish_kernel_timing(grd_state *s, uint64_t frontier_k)
 static grd_status superstep(grd_state *s, int option, bool select_next = false)
 {
   const bool ship = option == GRD_OPT_SHIP_EDGES;
-  GRD_TRY(op_zero_counters(s));
+  if (!s->cnt_clean) GRD_TRY(op_zero_counters(s));
+  s->cnt_clean = false;
   // the edge-shipping schedule broadcasts like the offloaded push
   // (GraphAlgorithm.cpp:199-343 runs for both decisions), then ships the
   // frontier's edge lists instead of generating and reducing updates
@@ -621,6 +622,7 @@ grd_status grd_broadcast(grd_state *s, int option)
   if (option < 0 || option > GRD_OPT_SHIP_EDGES) return fail(GRD_ERR_ARG, "grd_broadcast: bad option");
   if (s->algo == GRD_PR_PULL) return prp_broadcast(s);
   GRD_TRY(op_zero_counters(s));
+  s->cnt_clean = false;
   s->bcast_option = option;
   return op_broadcast(s, option == GRD_OPT_SHIP_EDGES ? GRD_OPT_PUSH_SPARSE : option);
 }
@@ -664,7 +666,7 @@ grd_status grd_update(grd_state *s, uint64_t *frontier_out)
   if (!s || !s->initialized) return fail(GRD_ERR_STATE, "grd_update: state not initialized");
   if (s->algo == GRD_PR_PULL) {
     GRD_TRY(prp_update(s));
-    GRD_TRY(op_read_counters(s));
+    GRD_TRY(op_wait_counters(s));
     GRD_TRY(finish_kernel_timing(s, 0));
     s->iteration++;
     const bool conv = s->hcnt->residual < s->prm.tolerance;
@@ -731,7 +733,6 @@ grd_status grd_run(grd_state *s, grd_run_stats *stats, grd_iter_rec *trace, uint
   GRD_HIP(hipSetDevice(ctx->device));
   grd_run_stats st{};
   const bool timing = s->prm.time_iters != 0;
-  GRD_HIP(hipStreamSynchronize(ctx->stream));
   GRD_HIP(hipEventRecord(ctx->ev[0], ctx->stream));
   bool done = false;
   while (!done) {
@@ -745,7 +746,7 @@ grd_status grd_run(grd_state *s, grd_run_stats *stats, grd_iter_rec *trace, uint
       if (timing) GRD_HIP(hipEventRecord(ctx->ev[2], ctx->stream));
       GRD_TRY(prp_iteration(s));
       if (timing) GRD_HIP(hipEventRecord(ctx->ev[3], ctx->stream));
-      GRD_TRY(op_read_counters(s));
+      GRD_TRY(op_wait_counters(s));
       GRD_TRY(finish_kernel_timing(s, 0));
       s->iteration++;
       st.residual = s->hcnt->residual;
@@ -1011,6 +1012,7 @@ grd_status grd_restore(grd_state *s)
   GRD_HIP(hipMemcpy(s->hcnt, s->cnt, sizeof(Counters), hipMemcpyDeviceToHost));
   s->sel_queued = false;
   s->bcast_option = -1;
+  s->cnt_clean = false;  // (a snapshot may have been taken within a superstep)
   return GRD_OK;
 }
 

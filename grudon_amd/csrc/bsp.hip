@@ -13,6 +13,7 @@
 //                                 termination popcount               :643-662
 //   k_popc_blocks/k_scan_blocks/k_word_rank  DynamicBitSet::getOffsets ranks
 #include <algorithm>
+#include <chrono>
 #include <cstring>
 
 #include "grd_device.hpp"
@@ -623,7 +624,9 @@ __global__ void __launch_bounds__(kBlock) k_select(uint32_t nw, uint64_t *__rest
   }
 }
 
-__global__ void k_zero_counters(Counters *cnt)
+// the counters of one superstep to their start (not the pull PageRank's
+// residual and dangling mass); one wave
+__device__ __forceinline__ void zero_counters(Counters *cnt)
 {
   if (threadIdx.x == 0) {
     cnt->frontier = 0;
@@ -644,6 +647,23 @@ __global__ void k_zero_counters(Counters *cnt)
     cnt->frontier_uncovered = 0;
   }
   for (uint32_t c = threadIdx.x; c < (uint32_t)kMaxParts; c += blockDim.x) cnt->fpart[c] = 0;
+}
+
+__global__ void __launch_bounds__(kWave) k_zero_counters(Counters *cnt) { zero_counters(cnt); }
+
+// The counters into the state's pinned copy, and to their start for the next
+// superstep.  The host waits for `seq` behind the copy (op_wait_counters): a
+// copy command and a stream synchronisation took 15 us more per superstep.
+__global__ void __launch_bounds__(kWave) k_publish(Counters *cnt, Counters *host, uint32_t *host_seq, uint32_t seq)
+{
+  static_assert(sizeof(Counters) % 8 == 0, "copied in 8-byte words");
+  const uint64_t *src = reinterpret_cast<const uint64_t *>(cnt);
+  uint64_t *dst = reinterpret_cast<uint64_t *>(host);
+  for (uint32_t i = threadIdx.x; i < sizeof(Counters) / 8; i += kWave) dst[i] = src[i];
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_store(host_seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+  zero_counters(cnt);
 }
 
 // single-element aggregate() (API compatibility path)
@@ -670,16 +690,37 @@ __global__ void __launch_bounds__(kBlock) k_gather_result(uint32_t S, const uint
 
 grd_status op_zero_counters(grd_state *s)
 {
-  hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, s->g->ctx->stream, s->cnt);
+  hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(kWave), 0, s->g->ctx->stream, s->cnt);
   GRD_HIP(hipGetLastError());
+  s->cnt_clean = true;
+  return GRD_OK;
+}
+
+// Waits for the counters published with the state's last sequence number.  A
+// superstep of a small graph is tens of microseconds, so the host looks at the
+// pinned word for a short while before it hands the wait to the runtime.
+grd_status op_wait_counters(grd_state *s)
+{
+  const uint32_t *seq = host_seq(s->hcnt);
+  const auto t0 = std::chrono::steady_clock::now();
+  for (uint32_t i = 1; __atomic_load_n(seq, __ATOMIC_ACQUIRE) != s->cnt_seq; i++) {
+    __builtin_ia32_pause();
+    if (i % 64 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(200)) {
+      GRD_HIP(hipStreamSynchronize(s->g->ctx->stream));
+      if (__atomic_load_n(seq, __ATOMIC_ACQUIRE) != s->cnt_seq)
+        return fail(GRD_ERR_HIP, "the superstep's counters did not arrive");
+    }
+  }
   return GRD_OK;
 }
 
 grd_status op_read_counters(grd_state *s)
 {
-  GRD_HIP(hipMemcpyAsync(s->hcnt, s->cnt, sizeof(Counters), hipMemcpyDeviceToHost, s->g->ctx->stream));
-  GRD_HIP(hipStreamSynchronize(s->g->ctx->stream));
-  return GRD_OK;
+  hipLaunchKernelGGL(k_publish, dim3(1), dim3(kWave), 0, s->g->ctx->stream, s->cnt, s->hcnt, host_seq(s->hcnt),
+                     ++s->cnt_seq);
+  GRD_HIP(hipGetLastError());
+  s->cnt_clean = true;
+  return op_wait_counters(s);
 }
 
 grd_status state_alloc(grd_state *s)
@@ -1021,14 +1062,12 @@ grd_status op_select_bucket(grd_state *s, bool *any_pending)
   const uint32_t nwS = g->S / 64;
   const uint32_t grid = loop_grid(g->ctx, nwS);
   *any_pending = false;
-  hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, st, s->cnt);
   hipLaunchKernelGGL(k_pend_min, dim3(grid), dim3(kBlock), 0, st, nwS, s->Pend, (const uint32_t *)s->prop, s->cnt);
   GRD_HIP(hipGetLastError());
   GRD_TRY(op_read_counters(s));
   if (s->hcnt->pending == 0) return GRD_OK;
   uint64_t mn = s->hcnt->pend_min, d = s->prm.delta;
   s->hi = (mn / d + 1) * d;
-  hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(64), 0, st, s->cnt);
   hipLaunchKernelGGL(k_select, dim3(grid), dim3(kBlock), 0, st, nwS, s->Pend, (const uint32_t *)s->prop, g->slot_deg,
                      (unsigned long long)s->hi, s->F, s->cnt);
   GRD_HIP(hipGetLastError());

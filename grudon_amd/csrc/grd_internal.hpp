@@ -115,6 +115,14 @@ struct Counters {
   unsigned long long fpart[64];       // frontier size of each compute partition (C > 1)
 };
 
+// the pinned copy of a state's counters is followed by the sequence number of
+// the last one that arrived
+constexpr uint64_t kHostCounters = ((sizeof(Counters) + 63) & ~63ull) + 64;
+inline uint32_t *host_seq(Counters *host)
+{
+  return reinterpret_cast<uint32_t *>(reinterpret_cast<char *>(host) + kHostCounters - 64);
+}
+
 // pull row block: rows [r0, r0 + nrows) with arcs [e0, e1); nrows == 0 marks
 // one segment [e0, e1) of the long row r0
 struct PullBlock {
@@ -332,7 +340,9 @@ struct grd_state {
   uint64_t last_fpart[grd::kMaxParts] = {};
   uint64_t last_uncovered = 0;
   grd::Counters *cnt = nullptr;   // device
-  grd::Counters *hcnt = nullptr;  // pinned host
+  grd::Counters *hcnt = nullptr;  // pinned host (kHostCounters bytes)
+  uint32_t cnt_seq = 0;           // sequence number of the last counters published
+  bool cnt_clean = false;         // the device counters are at their start
   // snapshot copies
   grd::DevMem snap_mem;
   std::vector<std::pair<void *, void *>> snap;  // (live, copy)
@@ -382,7 +392,9 @@ grd_status op_aggregate_one(grd_state *s, uint32_t slot, const void *value);
 grd_status op_download(grd_state *s, void *out);
 grd_status op_features(grd_state *s, float *out16);
 grd_status op_zero_counters(grd_state *s);
+// publishes the counters (and sets them to their start), waits and leaves them in hcnt
 grd_status op_read_counters(grd_state *s);
+grd_status op_wait_counters(grd_state *s);
 // copies the per-partition frontier sizes and the uncovered count of the
 // frontier just computed from the counters read back into the state
 void take_frontier_parts(grd_state *s);

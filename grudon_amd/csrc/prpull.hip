@@ -101,9 +101,10 @@ __global__ void __launch_bounds__(kBlock) k_prp_update(uint32_t nw, const uint8_
 }
 
 // Sums the update's per-workgroup (residual, dangling) pairs in a fixed order,
-// so the convergence test does not depend on scheduling.
+// so the convergence test does not depend on scheduling, and publishes the
+// residual to the host (as k_publish of bsp.hip).
 __global__ void __launch_bounds__(kBlock) k_prp_finish(const double *__restrict__ red, uint32_t nblk, int parity,
-                                                       Counters *cnt)
+                                                       Counters *cnt, Counters *host, uint32_t *host_seq, uint32_t seq)
 {
   double res = 0.0, dang = 0.0;
   for (uint32_t b = threadIdx.x; b < nblk; b += kBlock) {
@@ -115,6 +116,9 @@ __global__ void __launch_bounds__(kBlock) k_prp_finish(const double *__restrict_
   if (threadIdx.x == 0) {
     cnt->residual = res;
     cnt->dangling[parity ^ 1] = dang;
+    host->residual = res;
+    __threadfence_system();
+    __hip_atomic_store(host_seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
 
@@ -203,7 +207,8 @@ grd_status prp_traverse(grd_state *s)
   return GRD_OK;
 }
 
-// update step: aggregate the proxies of every vertex, new ranks, residual
+// update step: aggregate the proxies of every vertex, new ranks, residual (for
+// op_wait_counters)
 grd_status prp_update(grd_state *s)
 {
   grd_graph *g = s->g;
@@ -213,7 +218,7 @@ grd_status prp_update(grd_state *s)
                      g->word_dst, g->xptr, g->xlist, (const float *)s->valR, s->pr, (float *)s->mprop,
                      (float)s->prm.damping, 1.0 / (double)g->n, parity, s->cnt, s->red);
   hipLaunchKernelGGL(k_prp_finish, dim3(1), dim3(kBlock), 0, g->ctx->stream, (const double *)s->red, grid, parity,
-                     s->cnt);
+                     s->cnt, s->hcnt, host_seq(s->hcnt), ++s->cnt_seq);
   GRD_HIP(hipGetLastError());
   return GRD_OK;
 }

@@ -148,9 +148,9 @@ grd_status host_counters_take(grd_ctx *ctx, Counters **out)
     *out = (Counters *)ctx->host_counters.back();
     ctx->host_counters.pop_back();
   } else {
-    GRD_HIP(hipHostMalloc((void **)out, sizeof(Counters), hipHostMallocDefault));
+    GRD_HIP(hipHostMalloc((void **)out, kHostCounters, hipHostMallocDefault));
   }
-  memset((void *)*out, 0, sizeof(Counters));
+  memset((void *)*out, 0, kHostCounters);
   return GRD_OK;
 }
 
