@@ -181,9 +181,13 @@ static grd_status superstep(grd_state *s, int option, bool select_next = false)
     GRD_TRY(op_reduce(s, option));
   }
   GRD_TRY(op_update(s));
-  if (select_next) GRD_TRY(mlp_select_queue(s, s->last_frontier));
   s->sel_queued = select_next;
-  GRD_TRY(op_read_counters(s));
+  if (select_next) {
+    GRD_TRY(mlp_publish(s, s->last_frontier));
+    GRD_TRY(op_wait_counters(s));
+  } else {
+    GRD_TRY(op_read_counters(s));
+  }
   GRD_TRY(finish_kernel_timing(s, s->last_frontier));
   const Counters &c = *s->hcnt;
   const grd_graph *g = s->g;

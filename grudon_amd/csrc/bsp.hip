@@ -624,31 +624,6 @@ __global__ void __launch_bounds__(kBlock) k_select(uint32_t nw, uint64_t *__rest
   }
 }
 
-// the counters of one superstep to their start (not the pull PageRank's
-// residual and dangling mass); one wave
-__device__ __forceinline__ void zero_counters(Counters *cnt)
-{
-  if (threadIdx.x == 0) {
-    cnt->frontier = 0;
-    cnt->frontier_edges = 0;
-    cnt->dirty = 0;
-    cnt->pending = 0;
-    cnt->improved = 0;
-    cnt->heavy = 0;
-    cnt->heavy_edges = 0;
-    cnt->edges = 0;
-    cnt->frontier_maxdeg = 0;
-    cnt->pend_min = 0xFFFFFFFFu;
-    cnt->fmin = 0xFFFFFFFFu;
-    cnt->pull_skipped = 0;
-    cnt->pull_skipped_hot = 0;
-    cnt->pull_skipped_rows = 0;
-    cnt->pull_done_arcs = 0;
-    cnt->frontier_uncovered = 0;
-  }
-  for (uint32_t c = threadIdx.x; c < (uint32_t)kMaxParts; c += blockDim.x) cnt->fpart[c] = 0;
-}
-
 __global__ void __launch_bounds__(kWave) k_zero_counters(Counters *cnt) { zero_counters(cnt); }
 
 // The counters into the state's pinned copy, and to their start for the next

@@ -361,7 +361,7 @@ void host_counters_give(grd_ctx *ctx, Counters *p);
 // n 4-byte values from the device to the caller's array, widened to 8 bytes on
 // the way with `wide`; ordered after the context's stream, done on return
 grd_status copy_out(grd_ctx *ctx, void *dst, const void *src, uint64_t n, bool wide = false);
-// bytes to the device, ordered on the context's stream; the source is taken on return
+// bytes to the device, ordered on the context's stream; the source must stay until the stream has passed
 grd_status copy_in(grd_ctx *ctx, void *dst, const void *src, uint64_t bytes);
 // layout.cpp
 grd_status check_row_ptr(uint32_t n, const uint32_t *rp);
@@ -437,13 +437,11 @@ void make_features(const grd_state *s, float *f);
 // taken once per device; called by grd_create
 grd_status mlp_scratch_init(int device);
 grd_status mlp_select(grd_ctx *ctx, const float *feat16_host, int *option, float *margin);
-// Device-side selection for the next superstep from the counters of the one
-// just run: computes the 16 features from the counters on the device, runs
-// the MLP and queues the logits' copy to the host, so that the counters'
-// readback of the superstep also brings the next decision.  prev_frontier is
-// the frontier size before the superstep.
-grd_status mlp_select_queue(grd_state *s, uint64_t prev_frontier);
-// Reads the decision queued by mlp_select_queue from the state's counters
-// (after they were read back).
+// Publishes the counters (as op_read_counters, without the wait) together with
+// the next superstep's decision: the 16 features from the counters on the
+// device, the MLP's logits into the host copy's sel.  prev_frontier is the
+// frontier size before the superstep.
+grd_status mlp_publish(grd_state *s, uint64_t prev_frontier);
+// Reads the decision that came with the state's counters.
 void mlp_select_read(const grd_state *s, int *option, float *margin);
 }  // namespace grd

@@ -214,6 +214,31 @@ __device__ __forceinline__ uint32_t pull_bound(const Counters *cnt, uint32_t inc
   return f + inc < f ? 0xFFFFFFFFu : f + inc;
 }
 
+// the counters of one superstep to their start (not the pull PageRank's
+// residual and dangling mass); one wave
+__device__ __forceinline__ void zero_counters(Counters *cnt)
+{
+  if (threadIdx.x == 0) {
+    cnt->frontier = 0;
+    cnt->frontier_edges = 0;
+    cnt->dirty = 0;
+    cnt->pending = 0;
+    cnt->improved = 0;
+    cnt->heavy = 0;
+    cnt->heavy_edges = 0;
+    cnt->edges = 0;
+    cnt->frontier_maxdeg = 0;
+    cnt->pend_min = 0xFFFFFFFFu;
+    cnt->fmin = 0xFFFFFFFFu;
+    cnt->pull_skipped = 0;
+    cnt->pull_skipped_hot = 0;
+    cnt->pull_skipped_rows = 0;
+    cnt->pull_done_arcs = 0;
+    cnt->frontier_uncovered = 0;
+  }
+  for (uint32_t c = threadIdx.x; c < (uint32_t)kMaxParts; c += blockDim.x) cnt->fpart[c] = 0;
+}
+
 // push launchers (push.hip): the active list's arcs into the memory side's
 // updates, or (edge shipping) into the compute side's
 template <class Op>

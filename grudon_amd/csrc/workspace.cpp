@@ -281,7 +281,7 @@ grd_status copy_in(grd_ctx *ctx, void *dst, const void *src, uint64_t bytes)
 {
   if (!bytes) return GRD_OK;
   hipStream_t st = ctx->stream;
-  if (bytes < kRing) {  // the runtime has taken the source when this returns
+  if (bytes < kRing) {
     GRD_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, st));
     return GRD_OK;
   }
