@@ -140,17 +140,21 @@ static inline uint32_t wave_grid(const grd_ctx *ctx, uint64_t nwords)
   return (uint32_t)std::max<uint64_t>(1, std::min(want, cap));
 }
 
-// Word-group passes (exchange, update, bucket selection): each wave owns
-// kGroupWords consecutive bitmap words.  Lane j < kGroupWords loads word j of
-// the group (one coalesced access), the lanes finish their zero words
-// themselves, and the wave then walks only the nonzero words with one lane per
-// bit.  A sparse superstep therefore costs one pass over the bitmap, and a
-// dense one a few dependent loads per word.
-constexpr uint32_t kGroupWords = 8;
+// Word-group passes (exchange, update, bucket selection): each wave owns kG
+// consecutive bitmap words.  Lane j < kG loads word j of the group (one
+// coalesced access), the lanes finish their zero words themselves, and the wave
+// then takes the nonzero words with one lane per bit.  A sparse superstep
+// therefore costs one pass over the bitmap.  kG is 8, or 2 while groups of 2
+// still fit the waves the chip holds: a short bitmap then spreads over four
+// times the waves, each with a quarter of the words to work through in turn
+// (4096 words: the reduce 10.0 -> 5.1 us, the update 7.6 -> 4.2, the broadcast
+// 5.2 -> 3.8).
+constexpr uint32_t kGroupWide = 8, kGroupNarrow = 2;
 
+template <uint32_t kG>
 __device__ __forceinline__ uint32_t group_base()
 {
-  return (blockIdx.x * kWavesPerBlock + wave_in_block()) * kGroupWords;
+  return (blockIdx.x * kWavesPerBlock + wave_in_block()) * kG;
 }
 
 __device__ __forceinline__ uint64_t shfl_u64(uint64_t x, int src)
@@ -159,20 +163,26 @@ __device__ __forceinline__ uint64_t shfl_u64(uint64_t x, int src)
   return ((uint64_t)hi << 32) | lo;
 }
 
-static inline uint32_t group_grid(uint64_t nwords)
+static inline uint32_t group_grid(uint64_t nwords, uint32_t kg)
 {
-  const uint64_t per = (uint64_t)kGroupWords * kWavesPerBlock;
+  const uint64_t per = (uint64_t)kg * kWavesPerBlock;
   return (uint32_t)std::max<uint64_t>(1, (nwords + per - 1) / per);
 }
 
-// Passes that end in same-address counter atomics (update, reduce pack,
-// bucket selection) loop over the groups from a grid of this many
-// workgroups per CU, so that few blocks issue those atomics.
+// Passes that end in a share of the counters (update, reduce, bucket selection)
+// or an atomic (the broadcast's smallest value) loop over the groups from a grid
+// of at most this many workgroups per CU.
 constexpr uint32_t kLoopBlocksPerCU = 8;
 
-static inline uint32_t loop_grid(const grd_ctx *ctx, uint64_t nwords)
+static inline uint32_t loop_grid(const grd_ctx *ctx, uint64_t nwords, uint32_t kg = kGroupWide)
 {
-  return std::min<uint32_t>(group_grid(nwords), (uint32_t)ctx->num_cus * kLoopBlocksPerCU);
+  return std::min<uint32_t>(group_grid(nwords, kg), (uint32_t)ctx->num_cus * kLoopBlocksPerCU);
+}
+
+// groups of two words fit one round of the looping grid
+static inline bool narrow_groups(const grd_ctx *ctx, uint64_t nwords)
+{
+  return nwords <= (uint64_t)ctx->num_cus * kLoopBlocksPerCU * kWavesPerBlock * kGroupNarrow;
 }
 
 // ------------------------------------------------------------------------
@@ -268,7 +278,7 @@ __global__ void __launch_bounds__(kBlock) k_init_state(int algo, uint32_t nw, ui
 // store.  (With k_reduce, k_update, k_init_state and the one-launch ranks: CC on a thousand
 // vertices 314 -> 218 us a solve, hop SSSP by pushes on twenty thousand 727 -> 513,
 // delta-push PageRank on RMAT-18 85 -> 71 us a superstep.)
-template <typename V>
+template <typename V, uint32_t kG>
 __global__ void __launch_bounds__(kBlock) k_bcast(uint32_t nw, const uint64_t *__restrict__ F,
                                                   const V *__restrict__ prop, const uint32_t *__restrict__ wrank,
                                                   const uint32_t *__restrict__ word_dst, int dense, int want_list,
@@ -279,24 +289,24 @@ __global__ void __launch_bounds__(kBlock) k_bcast(uint32_t nw, const uint64_t *_
   const int l = lane_id();
   const bool ranks = !dense || want_list;
   uint32_t lo = 0xFFFFFFFFu;
-  for (uint32_t base = group_base(); base < nw; base += gridDim.x * kWavesPerBlock * kGroupWords) {
-    const bool ok = l < (int)kGroupWords && base + l < nw;
+  for (uint32_t base = group_base<kG>(); base < nw; base += gridDim.x * kWavesPerBlock * kG) {
+    const bool ok = l < (int)kG && base + l < nw;
     const uint64_t mine = ok ? F[base + l] : 0ull;
     const uint32_t pwl = ok ? word_dst[base + l] : 0xFFFFFFFFu;
     const uint32_t rkl = ok && ranks ? wrank[base + l] : 0u;
     if (ok) bv[base + l] = mine;
     // a sparse push walks only the words that hold a frontier vertex
     if (!dense && want_list && __ballot(mine != 0) == 0) continue;
-    V x[kGroupWords];
-    uint64_t word[kGroupWords];
+    V x[kG];
+    uint64_t word[kG];
 #pragma unroll
-    for (int j = 0; j < (int)kGroupWords; j++) {
+    for (int j = 0; j < (int)kG; j++) {
       word[j] = shfl_u64(mine, j);
       x[j] = ident;
       if (base + j < nw && (dense || ((word[j] >> l) & 1ull))) x[j] = prop[(base + j) * 64 + l];
     }
 #pragma unroll
-    for (int j = 0; j < (int)kGroupWords; j++) {
+    for (int j = 0; j < (int)kG; j++) {
       const uint32_t w = base + j, pw = __shfl(pwl, j, kWave), rank = __shfl(rkl, j, kWave);
       if (w >= nw) break;  // uniform over the wave
       const bool on = (word[j] >> l) & 1ull;
@@ -314,7 +324,8 @@ __global__ void __launch_bounds__(kBlock) k_bcast(uint32_t nw, const uint64_t *_
   }
   if (fmin) {  // uniform: a kernel argument
     lo = block_min(lo);
-    if (threadIdx.x == 0 && lo != 0xFFFFFFFFu) atomicMin(fmin, lo);
+    // (a workgroup that cannot lower it spares the atomic)
+    if (threadIdx.x == 0 && lo < __atomic_load_n(fmin, __ATOMIC_RELAXED)) atomicMin(fmin, lo);
   }
 }
 
@@ -347,20 +358,20 @@ __global__ void __launch_bounds__(kBlock) k_rows_done(uint32_t nwP, const uint32
 // into the pairs' messages (the wire) and aggregates the same values into the
 // compute side, all loads of the group (values, slots, and for min-combines the
 // current values) before the first store, all atomics before the first mark.
-// A capped grid loops over the groups (one counter atomic per workgroup).
-template <class Op>
+// A capped grid loops over the groups (one share of the counters per workgroup).
+template <class Op, uint32_t kG>
 __global__ void __launch_bounds__(kBlock) k_reduce(uint32_t nw, uint64_t *__restrict__ Du,
                                                    typename Op::V *__restrict__ mupd,
                                                    const uint32_t *__restrict__ wrank,
                                                    const uint32_t *__restrict__ proxy_slot, int dense,
                                                    uint64_t *__restrict__ bv, typename Op::V *__restrict__ val,
-                                                   typename Op::V *upd, uint64_t *Dc, Counters *cnt)
+                                                   typename Op::V *upd, uint64_t *Dc, uint32_t *__restrict__ share)
 {
   using V = typename Op::V;
   const int l = lane_id();
   uint32_t ndirty = 0;
-  for (uint32_t base = group_base(); base < nw; base += gridDim.x * kWavesPerBlock * kGroupWords) {
-    const bool ok = l < (int)kGroupWords && base + l < nw;
+  for (uint32_t base = group_base<kG>(); base < nw; base += gridDim.x * kWavesPerBlock * kG) {
+    const bool ok = l < (int)kG && base + l < nw;
     const uint64_t mine = ok ? Du[base + l] : 0ull;
     const uint32_t rkl = (ok && !dense) ? wrank[base + l] : 0u;
     if (ok) {
@@ -369,11 +380,11 @@ __global__ void __launch_bounds__(kBlock) k_reduce(uint32_t nw, uint64_t *__rest
     }
     ndirty += (uint32_t)__popcll(mine);
     if (!dense && __ballot(mine != 0) == 0) continue;
-    uint64_t word[kGroupWords];
-    uint32_t s[kGroupWords];
-    V x[kGroupWords];
+    uint64_t word[kG];
+    uint32_t s[kG];
+    V x[kG];
 #pragma unroll
-    for (int j = 0; j < (int)kGroupWords; j++) {
+    for (int j = 0; j < (int)kG; j++) {
       word[j] = shfl_u64(mine, j);
       const uint32_t p = (base + j) * 64 + l;
       const bool on = (word[j] >> l) & 1ull;
@@ -382,14 +393,14 @@ __global__ void __launch_bounds__(kBlock) k_reduce(uint32_t nw, uint64_t *__rest
       if (base + j < nw && (dense || on)) x[j] = mupd[p];
       if (on) s[j] = proxy_slot[p];
     }
-    V cur[kGroupWords];
+    V cur[kG];
     if constexpr (Op::kMin) {
 #pragma unroll
-      for (int j = 0; j < (int)kGroupWords; j++)
+      for (int j = 0; j < (int)kG; j++)
         cur[j] = s[j] != 0xFFFFFFFFu ? __atomic_load_n(upd + s[j], __ATOMIC_RELAXED) : V{};
     }
 #pragma unroll
-    for (int j = 0; j < (int)kGroupWords; j++) {
+    for (int j = 0; j < (int)kG; j++) {
       const uint32_t w = base + j, p = w * 64 + l, rank = __shfl(rkl, j, kWave);
       if (w >= nw) break;  // uniform over the wave
       const bool on = (word[j] >> l) & 1ull;
@@ -399,9 +410,9 @@ __global__ void __launch_bounds__(kBlock) k_reduce(uint32_t nw, uint64_t *__rest
       if (!Op::kMin && on) mupd[p] = V(0);
     }
     // aggregate(): minUpdate / addUpdate, then the dirty marks of the wave
-    bool mark[kGroupWords];
+    bool mark[kG];
 #pragma unroll
-    for (int j = 0; j < (int)kGroupWords; j++) {
+    for (int j = 0; j < (int)kG; j++) {
       mark[j] = false;
       if (s[j] != 0xFFFFFFFFu) {
         if constexpr (Op::kMin) {
@@ -414,43 +425,40 @@ __global__ void __launch_bounds__(kBlock) k_reduce(uint32_t nw, uint64_t *__rest
       }
     }
 #pragma unroll
-    for (int j = 0; j < (int)kGroupWords; j++) {
+    for (int j = 0; j < (int)kG; j++) {
       if (word[j] == 0) continue;  // uniform over the wave
       if constexpr (Op::kMin) mark[j] = mark[j] && x[j] < cur[j];
       mark_wave(Dc, s[j], mark[j]);
     }
   }
   uint32_t t = block_sum(ndirty);
-  if (threadIdx.x == 0 && t) atomicAdd(&cnt->dirty, (unsigned long long)t);
+  if (threadIdx.x == 0 && t) share[blockIdx.x] += t;
 }
 
 // ------------------------------------------------------------------------
 // update: update_frontier + apply_updates + frontier popcount
 // ------------------------------------------------------------------------
 
-// a workgroup's counters: sums of a, b, c and the largest m over its threads,
-// in thread 0 (one barrier)
-__device__ __forceinline__ void block_counts(uint64_t &a, uint64_t &b, uint64_t &c, uint32_t &m)
+// a workgroup's share of the next frontier (one barrier, no atomic: with three
+// atomics per workgroup the update of 65536 words took 29 us, now 7.6)
+__device__ __forceinline__ void share_frontier(uint64_t vertices, uint64_t edges, uint32_t maxdeg, BlockShare *share)
 {
-  __shared__ uint64_t s_c[kWavesPerBlock][4];
-  a = wave_sum(a);
-  b = wave_sum(b);
-  c = wave_sum(c);
-  m = wave_max(m);
+  __shared__ uint64_t s_c[kWavesPerBlock];
+  __shared__ uint32_t s_m[kWavesPerBlock];
+  uint64_t c = wave_sum((vertices << 32) + edges);
+  uint32_t m = wave_max(maxdeg);
   if (lane_id() == 0) {
-    s_c[wave_in_block()][0] = a;
-    s_c[wave_in_block()][1] = b;
-    s_c[wave_in_block()][2] = c;
-    s_c[wave_in_block()][3] = m;
+    s_c[wave_in_block()] = c;
+    s_m[wave_in_block()] = m;
   }
   __syncthreads();
-  if (threadIdx.x == 0)
+  if (threadIdx.x == 0) {
     for (int i = 1; i < kWavesPerBlock; i++) {
-      a += s_c[i][0];
-      b += s_c[i][1];
-      c += s_c[i][2];
-      m = max(m, (uint32_t)s_c[i][3]);
+      c += s_c[i];
+      m = max(m, s_m[i]);
     }
+    share[blockIdx.x] = BlockShare{c, m, 0};
+  }
 }
 
 // A capped grid walks the word groups (the loop is wave-uniform), so the
@@ -458,29 +466,30 @@ __device__ __forceinline__ void block_counts(uint64_t &a, uint64_t &b, uint64_t 
 // words are issued before any is used, and lane j stores word j's bitmap words
 // (word by word, a group was a chain of up to eight dependent round trips:
 // 11 us on 4096 words, 36 on 65536).
-template <int ALGO>  // GRD_PR, GRD_CC or GRD_SSSP
+template <int ALGO, uint32_t kG>  // GRD_PR, GRD_CC or GRD_SSSP
 __global__ void __launch_bounds__(kBlock) k_update(uint32_t nw, uint64_t *__restrict__ Dc, void *prop_, void *upd_,
                                                    float *__restrict__ pr, const uint32_t *__restrict__ deg,
                                                    uint64_t *__restrict__ F, uint64_t *__restrict__ Pend,
-                                                   unsigned long long hi, int use_delta, Counters *cnt)
+                                                   unsigned long long hi, int use_delta,
+                                                   BlockShare *__restrict__ share)
 {
   using V = typename std::conditional<ALGO == GRD_PR, float, uint32_t>::type;
   V *__restrict__ prop = (V *)prop_;
   V *__restrict__ upd = (V *)upd_;
   const int l = lane_id();
-  uint64_t f_cnt = 0, f_edges = 0, improved = 0;
+  uint64_t f_cnt = 0, f_edges = 0;
   uint32_t f_max = 0;
-  for (uint32_t base = group_base(); base < nw; base += gridDim.x * kWavesPerBlock * kGroupWords) {
-    const bool ok = l < (int)kGroupWords && base + l < nw;
+  for (uint32_t base = group_base<kG>(); base < nw; base += gridDim.x * kWavesPerBlock * kG) {
+    const bool ok = l < (int)kG && base + l < nw;
     const uint64_t mine = ok ? Dc[base + l] : 0ull;
     uint64_t fmine = 0, pmine = 0;
     if (use_delta && mine) pmine = Pend[base + l];
     if (__ballot(mine != 0)) {
-      uint64_t d[kGroupWords];
-      V u[kGroupWords], o[kGroupWords];
-      uint32_t dg[kGroupWords];
+      uint64_t d[kG];
+      V u[kG], o[kG];
+      uint32_t dg[kG];
 #pragma unroll
-      for (int j = 0; j < (int)kGroupWords; j++) {
+      for (int j = 0; j < (int)kG; j++) {
         d[j] = shfl_u64(mine, j);
         const uint32_t s = (base + j) * 64 + l;
         u[j] = o[j] = V(0);
@@ -492,7 +501,7 @@ __global__ void __launch_bounds__(kBlock) k_update(uint32_t nw, uint64_t *__rest
         }
       }
 #pragma unroll
-      for (int j = 0; j < (int)kGroupWords; j++) {
+      for (int j = 0; j < (int)kG; j++) {
         if (d[j] == 0) continue;  // uniform over the wave
         const uint32_t s = (base + j) * 64 + l;
         bool f = false, pend = false;
@@ -506,7 +515,6 @@ __global__ void __launch_bounds__(kBlock) k_update(uint32_t nw, uint64_t *__rest
             }
           } else if (o[j] > u[j]) {  // cc.cpp:100-106, sssp.cpp:102-108
             prop[s] = u[j];
-            improved++;
             if (use_delta && (unsigned long long)u[j] >= hi) pend = true;
             else f = true;
           }
@@ -532,16 +540,11 @@ __global__ void __launch_bounds__(kBlock) k_update(uint32_t nw, uint64_t *__rest
       f_cnt += (uint64_t)__popcll(fmine);
     }
   }
-  block_counts(f_cnt, f_edges, improved, f_max);
-  if (threadIdx.x == 0) {
-    if (f_cnt) atomicAdd(&cnt->frontier, (unsigned long long)f_cnt);
-    if (f_edges) atomicAdd(&cnt->frontier_edges, (unsigned long long)f_edges);
-    if (improved) atomicAdd(&cnt->improved, (unsigned long long)improved);
-    if (f_max) atomicMax(&cnt->frontier_maxdeg, f_max);
-  }
+  share_frontier(f_cnt, f_edges, f_max, share);
 }
 
 // delta-stepping: smallest pending distance and pending count
+template <uint32_t kG>
 __global__ void __launch_bounds__(kBlock) k_pend_min(uint32_t nw, const uint64_t *__restrict__ Pend,
                                                      const uint32_t *__restrict__ prop, Counters *cnt)
 {
@@ -549,8 +552,8 @@ __global__ void __launch_bounds__(kBlock) k_pend_min(uint32_t nw, const uint64_t
   uint32_t mn = 0xFFFFFFFFu;
   uint64_t c = 0;
   // capped grid, wave-uniform loop over the word groups
-  for (uint32_t base = group_base(); base < nw; base += gridDim.x * kWavesPerBlock * kGroupWords) {
-    const bool ok = l < (int)kGroupWords && base + l < nw;
+  for (uint32_t base = group_base<kG>(); base < nw; base += gridDim.x * kWavesPerBlock * kG) {
+    const bool ok = l < (int)kG && base + l < nw;
     const uint64_t mine = ok ? Pend[base + l] : 0ull;
     uint64_t todo = __ballot(mine != 0);
     while (todo) {
@@ -567,29 +570,31 @@ __global__ void __launch_bounds__(kBlock) k_pend_min(uint32_t nw, const uint64_t
   mn = block_min(mn);
   c = block_sum(c);
   if (threadIdx.x == 0 && c) {
-    atomicMin(&cnt->pend_min, mn);
+    if (mn < __atomic_load_n(&cnt->pend_min, __ATOMIC_RELAXED)) atomicMin(&cnt->pend_min, mn);
     atomicAdd(&cnt->pending, (unsigned long long)c);
   }
 }
 
 // delta-stepping: move pending vertices below the new bucket bound into F
 // (loads and stores of a group as in k_update)
+template <uint32_t kG>
 __global__ void __launch_bounds__(kBlock) k_select(uint32_t nw, uint64_t *__restrict__ Pend,
                                                    const uint32_t *__restrict__ prop, const uint32_t *__restrict__ deg,
-                                                   unsigned long long hi, uint64_t *__restrict__ F, Counters *cnt)
+                                                   unsigned long long hi, uint64_t *__restrict__ F,
+                                                   BlockShare *__restrict__ share)
 {
   const int l = lane_id();
-  uint64_t f_cnt = 0, f_edges = 0, none = 0;
+  uint64_t f_cnt = 0, f_edges = 0;
   uint32_t f_max = 0;
-  for (uint32_t base = group_base(); base < nw; base += gridDim.x * kWavesPerBlock * kGroupWords) {
-    const bool ok = l < (int)kGroupWords && base + l < nw;
+  for (uint32_t base = group_base<kG>(); base < nw; base += gridDim.x * kWavesPerBlock * kG) {
+    const bool ok = l < (int)kG && base + l < nw;
     const uint64_t mine = ok ? Pend[base + l] : 0ull;
     uint64_t fmine = 0;
     if (__ballot(mine != 0)) {
-      uint64_t pm[kGroupWords];
-      uint32_t v[kGroupWords], dg[kGroupWords];
+      uint64_t pm[kG];
+      uint32_t v[kG], dg[kG];
 #pragma unroll
-      for (int j = 0; j < (int)kGroupWords; j++) {
+      for (int j = 0; j < (int)kG; j++) {
         pm[j] = shfl_u64(mine, j);
         const uint32_t s = (base + j) * 64 + l;
         v[j] = 0xFFFFFFFFu;
@@ -600,7 +605,7 @@ __global__ void __launch_bounds__(kBlock) k_select(uint32_t nw, uint64_t *__rest
         }
       }
 #pragma unroll
-      for (int j = 0; j < (int)kGroupWords; j++) {
+      for (int j = 0; j < (int)kG; j++) {
         const bool f = ((pm[j] >> l) & 1ull) && (unsigned long long)v[j] < hi;
         const uint64_t fm = __ballot(f);
         if (l == j) fmine = fm;
@@ -616,29 +621,21 @@ __global__ void __launch_bounds__(kBlock) k_select(uint32_t nw, uint64_t *__rest
       f_cnt += (uint64_t)__popcll(fmine);
     }
   }
-  block_counts(f_cnt, f_edges, none, f_max);
-  if (threadIdx.x == 0) {
-    if (f_cnt) atomicAdd(&cnt->frontier, (unsigned long long)f_cnt);
-    if (f_edges) atomicAdd(&cnt->frontier_edges, (unsigned long long)f_edges);
-    if (f_max) atomicMax(&cnt->frontier_maxdeg, f_max);
-  }
+  share_frontier(f_cnt, f_edges, f_max, share);
 }
 
-__global__ void __launch_bounds__(kWave) k_zero_counters(Counters *cnt) { zero_counters(cnt); }
+__global__ void __launch_bounds__(kBlock) k_zero_counters(Counters *cnt, Shares sh) { zero_counters(cnt, sh); }
 
 // The counters into the state's pinned copy, and to their start for the next
 // superstep.  The host waits for `seq` behind the copy (op_wait_counters): a
 // copy command and a stream synchronisation took 15 us more per superstep.
-__global__ void __launch_bounds__(kWave) k_publish(Counters *cnt, Counters *host, uint32_t *host_seq, uint32_t seq)
+__global__ void __launch_bounds__(kBlock) k_publish(Counters *cnt, Shares sh, Counters *host, uint32_t *host_seq,
+                                                    uint32_t seq)
 {
-  static_assert(sizeof(Counters) % 8 == 0, "copied in 8-byte words");
-  const uint64_t *src = reinterpret_cast<const uint64_t *>(cnt);
-  uint64_t *dst = reinterpret_cast<uint64_t *>(host);
-  for (uint32_t i = threadIdx.x; i < sizeof(Counters) / 8; i += kWave) dst[i] = src[i];
-  __threadfence_system();
-  __syncthreads();
-  if (threadIdx.x == 0) __hip_atomic_store(host_seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-  zero_counters(cnt);
+  const FrontierCounts fc = sum_shares(sh);
+  copy_counters(cnt, host, fc);
+  publish_seq(host_seq, seq);
+  zero_counters(cnt, sh);
 }
 
 // single-element aggregate() (API compatibility path)
@@ -663,9 +660,18 @@ __global__ void __launch_bounds__(kBlock) k_gather_result(uint32_t S, const uint
 // host orchestration
 // ------------------------------------------------------------------------
 
+// most workgroups of a looping pass (the shares' arrays)
+static uint32_t loop_blocks(const grd_ctx *ctx) { return (uint32_t)ctx->num_cus * kLoopBlocksPerCU; }
+
+Shares shares(const grd_state *s)
+{
+  return Shares{s->ushare, s->n_ushare, s->rshare, s->n_rshare};
+}
+
 grd_status op_zero_counters(grd_state *s)
 {
-  hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(kWave), 0, s->g->ctx->stream, s->cnt);
+  s->n_ushare = 0;
+  hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(kBlock), 0, s->g->ctx->stream, s->cnt, shares(s));
   GRD_HIP(hipGetLastError());
   s->cnt_clean = true;
   return GRD_OK;
@@ -691,9 +697,10 @@ grd_status op_wait_counters(grd_state *s)
 
 grd_status op_read_counters(grd_state *s)
 {
-  hipLaunchKernelGGL(k_publish, dim3(1), dim3(kWave), 0, s->g->ctx->stream, s->cnt, s->hcnt, host_seq(s->hcnt),
-                     ++s->cnt_seq);
+  hipLaunchKernelGGL(k_publish, dim3(1), dim3(kBlock), 0, s->g->ctx->stream, s->cnt, shares(s), s->hcnt,
+                     host_seq(s->hcnt), ++s->cnt_seq);
   GRD_HIP(hipGetLastError());
+  s->n_ushare = 0;
   s->cnt_clean = true;
   return op_wait_counters(s);
 }
@@ -764,6 +771,9 @@ grd_status state_alloc(grd_state *s)
     if (bsp_hot_cold(s)) GRD_TRY(m.alloc_n(&s->hskip, std::max<uint32_t>(g->n_tblk, 1)));
   }
   GRD_TRY(m.alloc_n(&s->cnt, 1));
+  GRD_TRY(m.alloc_n(&s->ushare, loop_blocks(g->ctx)));
+  GRD_TRY(m.alloc_n(&s->rshare, loop_blocks(g->ctx)));
+  s->n_rshare = loop_grid(g->ctx, nwP, narrow_groups(g->ctx, nwP) ? kGroupNarrow : kGroupWide);
   GRD_TRY(host_counters_take(g->ctx, &s->hcnt));
   // snapshot list: every array whose content carries state between iterations
   s->snap = {{s->prop, nullptr}, {s->upd, nullptr}, {s->F, nullptr},     {s->Dc, nullptr},
@@ -892,9 +902,13 @@ grd_status op_broadcast(grd_state *s, int option)
   const bool bound = pull && s->algo != GRD_PR && !s->prm.pull_every_row;
   const bool rows_done = bound && s->iteration > 0;
   const uint32_t ident = (s->algo == GRD_PR) ? 0u : 0xFFFFFFFFu;  // 0.0f or the min identity
-  hipLaunchKernelGGL(k_bcast<uint32_t>, dim3(bound ? loop_grid(g->ctx, nwS) : group_grid(nwS)), dim3(kBlock), 0, st,
-                     nwS, s->F, (const uint32_t *)s->prop, s->wrankB, g->word_dst, (int)dense, (int)!pull, ident,
-                     s->bvB, (uint32_t *)s->valB, (uint32_t *)s->mprop, s->AL, bound ? &s->cnt->fmin : nullptr);
+  const auto send = [&](auto kernel, uint32_t kg) {
+    hipLaunchKernelGGL(kernel, dim3(bound ? loop_grid(g->ctx, nwS, kg) : group_grid(nwS, kg)), dim3(kBlock), 0, st, nwS,
+                       s->F, (const uint32_t *)s->prop, s->wrankB, g->word_dst, (int)dense, (int)!pull, ident, s->bvB,
+                       (uint32_t *)s->valB, (uint32_t *)s->mprop, s->AL, bound ? &s->cnt->fmin : nullptr);
+  };
+  if (narrow_groups(g->ctx, nwS)) send(k_bcast<uint32_t, kGroupNarrow>, kGroupNarrow);
+  else send(k_bcast<uint32_t, kGroupWide>, kGroupWide);
   const uint32_t nwP = g->P / 64;
   uint32_t inc = 0;  // the smallest Op::edge increment over an arc
   if (bound && s->algo == GRD_SSSP) {
@@ -973,8 +987,12 @@ static grd_status reduce_t(grd_state *s, int option)
   const bool dense = option & 2;
   s->xr_dense = dense ? 1 : 0;
   if (!dense) GRD_TRY(word_ranks(st, s->Du, nwP, s->blk, s->wrankR, s->totals + 1));
-  hipLaunchKernelGGL((k_reduce<Op>), dim3(loop_grid(g->ctx, nwP)), dim3(kBlock), 0, st, nwP, s->Du, (V *)s->mupd,
-                     s->wrankR, g->proxy_slot, (int)dense, s->bvR, (V *)s->valR, (V *)s->upd, s->Dc, s->cnt);
+  const auto send = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(s->n_rshare), dim3(kBlock), 0, st, nwP, s->Du, (V *)s->mupd,
+                       s->wrankR, g->proxy_slot, (int)dense, s->bvR, (V *)s->valR, (V *)s->upd, s->Dc, s->rshare);
+  };
+  if (narrow_groups(g->ctx, nwP)) send(k_reduce<Op, kGroupNarrow>);
+  else send(k_reduce<Op, kGroupWide>);
   GRD_HIP(hipGetLastError());
   return GRD_OK;
 }
@@ -989,26 +1007,27 @@ grd_status op_reduce(grd_state *s, int option)
   }
 }
 
+template <int ALGO>
+static void launch_update(grd_state *s, int use_delta)
+{
+  grd_graph *g = s->g;
+  const uint32_t nwS = g->S / 64;
+  const auto go = [&](auto kernel, uint32_t kg) {
+    hipLaunchKernelGGL(kernel, dim3(loop_grid(g->ctx, nwS, kg)), dim3(kBlock), 0, g->ctx->stream, nwS, s->Dc, s->prop,
+                       s->upd, s->pr, g->slot_deg, s->F, s->Pend, (unsigned long long)s->hi, use_delta, s->ushare);
+    s->n_ushare = loop_grid(g->ctx, nwS, kg);
+  };
+  if (narrow_groups(g->ctx, nwS)) go(k_update<ALGO, kGroupNarrow>, kGroupNarrow);
+  else go(k_update<ALGO, kGroupWide>, kGroupWide);
+}
+
 grd_status op_update(grd_state *s)
 {
   grd_graph *g = s->g;
-  hipStream_t st = g->ctx->stream;
-  const uint32_t nwS = g->S / 64;
-  const uint32_t grid = loop_grid(g->ctx, nwS);
-  const int use_delta = (s->algo == GRD_SSSP && s->prm.delta) ? 1 : 0;
   switch (s->algo) {
-  case GRD_PR:
-    hipLaunchKernelGGL(k_update<GRD_PR>, dim3(grid), dim3(kBlock), 0, st, nwS, s->Dc, s->prop, s->upd, s->pr,
-                       g->slot_deg, s->F, s->Pend, (unsigned long long)s->hi, 0, s->cnt);
-    break;
-  case GRD_CC:
-    hipLaunchKernelGGL(k_update<GRD_CC>, dim3(grid), dim3(kBlock), 0, st, nwS, s->Dc, s->prop, s->upd, s->pr,
-                       g->slot_deg, s->F, s->Pend, (unsigned long long)s->hi, 0, s->cnt);
-    break;
-  case GRD_SSSP:
-    hipLaunchKernelGGL(k_update<GRD_SSSP>, dim3(grid), dim3(kBlock), 0, st, nwS, s->Dc, s->prop, s->upd, s->pr,
-                       g->slot_deg, s->F, s->Pend, (unsigned long long)s->hi, use_delta, s->cnt);
-    break;
+  case GRD_PR: launch_update<GRD_PR>(s, 0); break;
+  case GRD_CC: launch_update<GRD_CC>(s, 0); break;
+  case GRD_SSSP: launch_update<GRD_SSSP>(s, s->prm.delta ? 1 : 0); break;
   default: return fail(GRD_ERR_STATE, "update: algorithm has no BSP update");
   }
   GRD_HIP(hipGetLastError());
@@ -1037,14 +1056,15 @@ grd_status op_select_bucket(grd_state *s, bool *any_pending)
   const uint32_t nwS = g->S / 64;
   const uint32_t grid = loop_grid(g->ctx, nwS);
   *any_pending = false;
-  hipLaunchKernelGGL(k_pend_min, dim3(grid), dim3(kBlock), 0, st, nwS, s->Pend, (const uint32_t *)s->prop, s->cnt);
+  hipLaunchKernelGGL(k_pend_min<kGroupWide>, dim3(grid), dim3(kBlock), 0, st, nwS, s->Pend, (const uint32_t *)s->prop, s->cnt);
   GRD_HIP(hipGetLastError());
   GRD_TRY(op_read_counters(s));
   if (s->hcnt->pending == 0) return GRD_OK;
   uint64_t mn = s->hcnt->pend_min, d = s->prm.delta;
   s->hi = (mn / d + 1) * d;
-  hipLaunchKernelGGL(k_select, dim3(grid), dim3(kBlock), 0, st, nwS, s->Pend, (const uint32_t *)s->prop, g->slot_deg,
-                     (unsigned long long)s->hi, s->F, s->cnt);
+  hipLaunchKernelGGL(k_select<kGroupWide>, dim3(grid), dim3(kBlock), 0, st, nwS, s->Pend, (const uint32_t *)s->prop, g->slot_deg,
+                     (unsigned long long)s->hi, s->F, s->ushare);
+  s->n_ushare = grid;
   GRD_HIP(hipGetLastError());
   if (g->C > 1) GRD_TRY(op_frontier_parts(s));
   GRD_TRY(op_read_counters(s));

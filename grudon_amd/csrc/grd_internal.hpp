@@ -92,21 +92,21 @@ struct DevMem {
 
 // Counters written by device kernels and read back once per iteration.
 struct Counters {
+  // the host's copy only (kHostOnly words), summed from the blocks' shares
   unsigned long long frontier;        // popcount of the new frontier
   unsigned long long frontier_edges;  // out-degree sum of the new frontier
   unsigned long long dirty;           // dirty memory proxies at reduce
+  unsigned int frontier_maxdeg, pad0;
+  // added up on the device
   unsigned long long pending;         // SSSP delta-stepping: pending vertices
-  unsigned long long improved;        // compute vertices improved by update
   unsigned long long heavy;           // push: heavy-vertex chunks appended this iteration
   unsigned long long edges;           // edges examined by the traversal
-  unsigned int frontier_maxdeg;
   unsigned int pend_min;
+  unsigned int fmin;                  // CC / SSSP pull: smallest value broadcast this superstep
   double residual;                    // PR pull: L1 change
   double dangling[2];                 // PR pull: FP64 dangling mass (ping-pong)
   unsigned long long heavy_edges;     // push: edges of heavy vertices (k_push_heavy)
   unsigned long long frontier_uncovered;  // frontier vertices with an out-neighbour of another master
-  unsigned int fmin;                  // CC / SSSP pull: smallest value broadcast this superstep
-  unsigned int pad32;
   unsigned long long pull_skipped;    // CC / SSSP pull: arcs of the cold row blocks left out (not read)
   unsigned long long pull_skipped_hot;   // and of the hot wave blocks left out
   unsigned long long pull_skipped_rows;  // rows of the cold row blocks left out
@@ -117,6 +117,15 @@ struct Counters {
 
 // the pinned copy of a state's counters is followed by the sequence number of
 // the last one that arrived
+constexpr uint32_t kHostOnly = 4;  // leading 8-byte words that only the host's copy holds
+// a workgroup's share of the next frontier (update, bucket selection) and of
+// the dirty proxies (reduce): stored per workgroup and summed by the wave that
+// publishes the counters, since atomics of thousands of workgroups on one cache
+// line come one after another, 9 ns each
+struct BlockShare {
+  unsigned long long front;  // vertices << 32 | out-degrees, both below 2^32
+  unsigned int maxdeg, pad;
+};
 constexpr uint64_t kHostCounters = ((sizeof(Counters) + 63) & ~63ull) + 64;
 inline uint32_t *host_seq(Counters *host)
 {
@@ -340,6 +349,9 @@ struct grd_state {
   uint64_t last_fpart[grd::kMaxParts] = {};
   uint64_t last_uncovered = 0;
   grd::Counters *cnt = nullptr;   // device
+  grd::BlockShare *ushare = nullptr;  // [loop_blocks] of the last update / selection
+  uint32_t *rshare = nullptr;         // [loop_blocks] dirty proxies, zero after each publishing
+  uint32_t n_ushare = 0, n_rshare = 0;
   grd::Counters *hcnt = nullptr;  // pinned host (kHostCounters bytes)
   uint32_t cnt_seq = 0;           // sequence number of the last counters published
   bool cnt_clean = false;         // the device counters are at their start

@@ -130,7 +130,9 @@ __device__ __forceinline__ void mark_wave(uint64_t *bits, uint32_t i, bool pred)
   const int leader = __ffsll((unsigned long long)m) - 1;
   const uint32_t wl = __shfl(i >> 6, leader, kWave);
   const bool same = !pred || (i >> 6) == wl;
-  if (__ballot(!same) == 0) {
+  if (__ballot(pred && i != wl * 64 + lane_id()) == 0) {  // every lane's bit is its own: the ballot is the word
+    if (lane_id() == leader) atomicOr((unsigned long long *)(bits + wl), (unsigned long long)m);
+  } else if (__ballot(!same) == 0) {
     uint32_t lo = 0, hi = 0;
     if (pred) {
       if ((i & 63) < 32) lo = 1u << (i & 31);
@@ -214,20 +216,26 @@ __device__ __forceinline__ uint32_t pull_bound(const Counters *cnt, uint32_t inc
   return f + inc < f ? 0xFFFFFFFFu : f + inc;
 }
 
+// Publishing the counters (k_publish of bsp.hip, k_mlp_publish of mlp.hip): a
+// workgroup of kBlock threads.
+struct Shares {
+  const BlockShare *u;
+  uint32_t nu;
+  uint32_t *r;
+  uint32_t nr;
+};
+
+Shares shares(const grd_state *s);
+
 // the counters of one superstep to their start (not the pull PageRank's
-// residual and dangling mass); one wave
-__device__ __forceinline__ void zero_counters(Counters *cnt)
+// residual and dangling mass)
+__device__ __forceinline__ void zero_counters(Counters *cnt, const Shares &sh)
 {
   if (threadIdx.x == 0) {
-    cnt->frontier = 0;
-    cnt->frontier_edges = 0;
-    cnt->dirty = 0;
     cnt->pending = 0;
-    cnt->improved = 0;
     cnt->heavy = 0;
     cnt->heavy_edges = 0;
     cnt->edges = 0;
-    cnt->frontier_maxdeg = 0;
     cnt->pend_min = 0xFFFFFFFFu;
     cnt->fmin = 0xFFFFFFFFu;
     cnt->pull_skipped = 0;
@@ -236,7 +244,70 @@ __device__ __forceinline__ void zero_counters(Counters *cnt)
     cnt->pull_done_arcs = 0;
     cnt->frontier_uncovered = 0;
   }
-  for (uint32_t c = threadIdx.x; c < (uint32_t)kMaxParts; c += blockDim.x) cnt->fpart[c] = 0;
+  for (uint32_t c = threadIdx.x; c < (uint32_t)kMaxParts; c += kBlock) cnt->fpart[c] = 0;
+  for (uint32_t b = threadIdx.x; b < sh.nr; b += kBlock) sh.r[b] = 0;
+}
+
+// the sums of the blocks' shares, in every thread
+struct FrontierCounts {
+  unsigned long long frontier, edges, dirty;
+  uint32_t maxdeg;
+};
+__device__ __forceinline__ FrontierCounts sum_shares(const Shares &sh)
+{
+  __shared__ unsigned long long s_f[kWavesPerBlock], s_d[kWavesPerBlock];
+  __shared__ uint32_t s_m[kWavesPerBlock];
+  unsigned long long f = 0, d = 0;
+  uint32_t m = 0;
+#pragma unroll 8
+  for (uint32_t b = threadIdx.x; b < sh.nu; b += kBlock) {
+    f += sh.u[b].front;
+    m = max(m, sh.u[b].maxdeg);
+  }
+#pragma unroll 8
+  for (uint32_t b = threadIdx.x; b < sh.nr; b += kBlock) d += sh.r[b];
+  f = wave_sum(f);
+  d = wave_sum(d);
+  m = wave_max(m);
+  if (lane_id() == 0) {
+    s_f[wave_in_block()] = f;
+    s_d[wave_in_block()] = d;
+    s_m[wave_in_block()] = m;
+  }
+  __syncthreads();
+  f = d = 0;
+  m = 0;
+#pragma unroll
+  for (int i = 0; i < kWavesPerBlock; i++) {
+    f += s_f[i];
+    d += s_d[i];
+    m = max(m, s_m[i]);
+  }
+  return FrontierCounts{f >> 32, f & 0xFFFFFFFFull, d, m};
+}
+
+// the counters into the host's copy, except the words [skip0, skip1)
+__device__ __forceinline__ void copy_counters(const Counters *cnt, Counters *host, const FrontierCounts &fc,
+                                              uint32_t skip0 = 0, uint32_t skip1 = 0)
+{
+  static_assert(sizeof(Counters) % 8 == 0, "copied in 8-byte words");
+  for (uint32_t i = threadIdx.x; i < sizeof(Counters) / 8; i += kBlock)
+    if (i >= kHostOnly && (i < skip0 || i >= skip1))
+      reinterpret_cast<uint64_t *>(host)[i] = reinterpret_cast<const uint64_t *>(cnt)[i];
+  if (threadIdx.x == 0) {
+    host->frontier = fc.frontier;
+    host->frontier_edges = fc.edges;
+    host->dirty = fc.dirty;
+    host->frontier_maxdeg = fc.maxdeg;
+  }
+}
+
+// everything stored to the host's copy is there before its sequence number
+__device__ __forceinline__ void publish_seq(uint32_t *host_seq, uint32_t seq)
+{
+  __threadfence_system();
+  __syncthreads();
+  if (threadIdx.x == 0) __hip_atomic_store(host_seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // push launchers (push.hip): the active list's arcs into the memory side's

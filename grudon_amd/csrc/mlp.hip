@@ -370,12 +370,12 @@ struct SelInputs {
 };
 
 // The counters of a superstep to the host (as k_publish of bsp.hip) together
-// with the next decision, 4 logits and the argmax in sel, in one wave.  All
+// with the next decision, 4 logits and the argmax in sel.  All
 // weights are in flight before the counters are looked at, and each lane
 // computes one feature, so that the doubles' divisions and logarithms run side
 // by side (one thread after another, and a launch of its own, took 5 us more).
-__global__ void __launch_bounds__(kWave) k_mlp_publish(const uint16_t *__restrict__ wb, Counters *cnt, SelInputs in,
-                                                       Counters *host, uint32_t *host_seq, uint32_t seq)
+__global__ void __launch_bounds__(kBlock) k_mlp_publish(const uint16_t *__restrict__ wb, Counters *cnt, Shares sh,
+                                                        SelInputs in, Counters *host, uint32_t *host_seq, uint32_t seq)
 {
   __shared__ float s_x[kIn];
   __shared__ __align__(16) float s_h1[kH];
@@ -405,16 +405,17 @@ __global__ void __launch_bounds__(kWave) k_mlp_publish(const uint16_t *__restric
   // the counters' copy; sel follows below
   constexpr uint32_t kSel0 = offsetof(Counters, sel) / 8, kSel1 = kSel0 + sizeof(Counters::sel) / 8;
   static_assert(offsetof(Counters, sel) % 8 == 0 && sizeof(Counters::sel) % 8 == 0, "sel is whole words");
-  for (uint32_t i = j; i < sizeof(Counters) / 8; i += kWave)
-    if (i < kSel0 || i >= kSel1) reinterpret_cast<uint64_t *>(host)[i] = reinterpret_cast<const uint64_t *>(cnt)[i];
+  const FrontierCounts fc = sum_shares(sh);
+  copy_counters(cnt, host, fc, kSel0, kSel1);
+  // every wave computes the same decision (their LDS rows hold equal values)
   {
-    const double fr = (double)cnt->frontier, fe = (double)cnt->frontier_edges;
+    const double fr = (double)fc.frontier, fe = (double)fc.edges;
     const double m = in.m > 1.0 ? in.m : 1.0;
     double num = 0.0, den = 1.0, den2 = 1.0;
     if (j == 1) num = fr, den = in.n;
     if (j == 2) num = fe, den = m;
-    if (j == 4) num = (double)cnt->dirty, den = in.P;
-    if (j == 5) num = (double)cnt->frontier_maxdeg, den = fe + 1.0;
+    if (j == 4) num = (double)fc.dirty, den = in.P;
+    if (j == 5) num = (double)fc.maxdeg, den = fe + 1.0;
     if (j == 6 && fr > 0) num = fe, den = fr, den2 = fmax(1e-9, in.avg_deg * 4.0);
     if (j == 12) num = in.prev_frontier > 0 ? fr : 1.0, den = in.prev_frontier > 0 ? in.prev_frontier : 1.0;
     double q = num / den / den2;
@@ -426,12 +427,12 @@ __global__ void __launch_bounds__(kWave) k_mlp_publish(const uint16_t *__restric
     const bool counted = j <= 6 || j == 12;
     if (j < kIn) s_x[j] = counted ? (float)q : in.x[j];
   }
-  wave_lds_order();
+  __syncthreads();
   float a = b1;
 #pragma unroll
   for (int i = 0; i < kIn; i++) a += bf16_to_f32(w1.h[i]) * s_x[i];
   s_h1[j] = a > 0.0f ? a : 0.0f;
-  wave_lds_order();
+  __syncthreads();
   float b = b2;
 #pragma unroll
   for (int k = 0; k < kH; k++) b += bf16_to_f32(w2.h[k]) * s_h1[k];
@@ -439,7 +440,7 @@ __global__ void __launch_bounds__(kWave) k_mlp_publish(const uint16_t *__restric
   float lg[kOut];
 #pragma unroll
   for (int o = 0; o < kOut; o++) lg[o] = wave_sum(w3[o] * h2) + b3[o];
-  if (j == 0) {
+  if (threadIdx.x == 0) {
     int best = 0;
 #pragma unroll
     for (int o = 1; o < kOut; o++)
@@ -448,10 +449,8 @@ __global__ void __launch_bounds__(kWave) k_mlp_publish(const uint16_t *__restric
     for (int o = 0; o < kOut; o++) host->sel[o] = lg[o];
     host->sel[4] = (float)best;
   }
-  __threadfence_system();
-  __syncthreads();
-  if (j == 0) __hip_atomic_store(host_seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
-  zero_counters(cnt);
+  publish_seq(host_seq, seq);
+  zero_counters(cnt, sh);
 }
 
 // ------------------------------------------------------------------------
@@ -481,9 +480,10 @@ grd_status mlp_publish(grd_state *s, uint64_t prev_frontier)
   grd_ctx *ctx = g->ctx;
   SelInputs in{(double)g->n, (double)g->m, (double)g->P, g->avg_degree, (double)prev_frontier, {}};
   make_features(s, in.x);  // (those of the counters are computed on the device)
-  hipLaunchKernelGGL(k_mlp_publish, dim3(1), dim3(kWave), 0, ctx->stream, ctx->sel_w, s->cnt, in, s->hcnt,
+  hipLaunchKernelGGL(k_mlp_publish, dim3(1), dim3(kBlock), 0, ctx->stream, ctx->sel_w, s->cnt, shares(s), in, s->hcnt,
                      host_seq(s->hcnt), ++s->cnt_seq);
   GRD_HIP(hipGetLastError());
+  s->n_ushare = 0;
   s->cnt_clean = true;
   return GRD_OK;
 }
