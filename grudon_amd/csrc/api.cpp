@@ -156,7 +156,7 @@ static grd_status finish_kernel_timing(grd_state *s, uint64_t frontier_k)
   GRD_HIP(hipEventElapsedTime(&ms, s->kev[0], s->kev[1]));
   s->kern_ms += ms;
   s->kern_launches++;
-  if (s->kern_pending == 2) s->kern_bytes += 12 * (s->hcnt->edges + s->hcnt->heavy_edges) + 16 * frontier_k;
+  if (s->kern_pending == 2) s->kern_bytes += 12 * s->last_frontier_edges + 16 * frontier_k;
   else s->kern_bytes += s->kern_pending_bytes;
   s->kern_pending = 0;
   return GRD_OK;
@@ -198,7 +198,6 @@ static grd_status superstep(grd_state *s, int option, bool select_next = false)
     uint64_t vals = (option & 2) ? (uint64_t)g->n + g->X : c.dirty;
     s->bytes += bitvector_bytes(g) + vals * s->vbytes;
   }
-  s->edges += c.edges + c.heavy_edges;
   s->prev_frontier = s->last_frontier;
   s->last_dirty = c.dirty;
   s->last_frontier = c.frontier;
@@ -685,7 +684,6 @@ grd_status grd_update(grd_state *s, uint64_t *frontier_out)
     uint64_t vals = (s->last_option & 2) ? (uint64_t)s->g->n + s->g->X : c.dirty;
     s->bytes += bitvector_bytes(s->g) + vals * s->vbytes;
   }
-  s->edges += c.edges + c.heavy_edges;
   s->prev_frontier = s->last_frontier;
   s->last_dirty = c.dirty;
   s->last_frontier = c.frontier;

@@ -632,8 +632,9 @@ __global__ void __launch_bounds__(kBlock) k_zero_counters(Counters *cnt, Shares 
 __global__ void __launch_bounds__(kBlock) k_publish(Counters *cnt, Shares sh, Counters *host, uint32_t *host_seq,
                                                     uint32_t seq)
 {
+  const uint64_t word = counter_word(cnt);
   const FrontierCounts fc = sum_shares(sh);
-  copy_counters(cnt, host, fc);
+  copy_counters(word, host, fc);
   publish_seq(host_seq, seq);
   zero_counters(cnt, sh);
 }
@@ -661,16 +662,16 @@ __global__ void __launch_bounds__(kBlock) k_gather_result(uint32_t S, const uint
 // ------------------------------------------------------------------------
 
 // most workgroups of a looping pass (the shares' arrays)
-static uint32_t loop_blocks(const grd_ctx *ctx) { return (uint32_t)ctx->num_cus * kLoopBlocksPerCU; }
+uint32_t loop_blocks(const grd_ctx *ctx) { return (uint32_t)ctx->num_cus * kLoopBlocksPerCU; }
 
 Shares shares(const grd_state *s)
 {
-  return Shares{s->ushare, s->n_ushare, s->rshare, s->n_rshare};
+  return Shares{s->ushare, s->n_ushare, s->rshare, s->n_rshare, s->sshare, s->n_sshare};
 }
 
 grd_status op_zero_counters(grd_state *s)
 {
-  s->n_ushare = 0;
+  s->n_ushare = s->n_sshare = 0;
   hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(kBlock), 0, s->g->ctx->stream, s->cnt, shares(s));
   GRD_HIP(hipGetLastError());
   s->cnt_clean = true;
@@ -700,7 +701,7 @@ grd_status op_read_counters(grd_state *s)
   hipLaunchKernelGGL(k_publish, dim3(1), dim3(kBlock), 0, s->g->ctx->stream, s->cnt, shares(s), s->hcnt,
                      host_seq(s->hcnt), ++s->cnt_seq);
   GRD_HIP(hipGetLastError());
-  s->n_ushare = 0;
+  s->n_ushare = s->n_sshare = 0;
   s->cnt_clean = true;
   return op_wait_counters(s);
 }
@@ -773,6 +774,7 @@ grd_status state_alloc(grd_state *s)
   GRD_TRY(m.alloc_n(&s->cnt, 1));
   GRD_TRY(m.alloc_n(&s->ushare, loop_blocks(g->ctx)));
   GRD_TRY(m.alloc_n(&s->rshare, loop_blocks(g->ctx)));
+  GRD_TRY(m.alloc_n(&s->sshare, 2 * loop_blocks(g->ctx)));
   s->n_rshare = loop_grid(g->ctx, nwP, narrow_groups(g->ctx, nwP) ? kGroupNarrow : kGroupWide);
   GRD_TRY(host_counters_take(g->ctx, &s->hcnt));
   // snapshot list: every array whose content carries state between iterations

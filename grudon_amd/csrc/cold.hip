@@ -272,7 +272,8 @@ __global__ void __launch_bounds__(T, 8) k_bsp_pull_cold(const PullBlock *__restr
 __global__ void __launch_bounds__(kBlock) k_cold_blocks_done(uint32_t nblk, const PullBlock *__restrict__ blocks,
                                                              const uint64_t *__restrict__ done,
                                                              const uint64_t *__restrict__ hasarc,
-                                                             uint8_t *__restrict__ bskip, Counters *cnt)
+                                                             uint8_t *__restrict__ bskip,
+                                                             SkipShare *__restrict__ share)
 {
   unsigned long long arcs = 0, rows = 0;
   const uint32_t lane = lane_id();
@@ -299,10 +300,7 @@ __global__ void __launch_bounds__(kBlock) k_cold_blocks_done(uint32_t nblk, cons
   }
   arcs = block_sum(arcs);
   rows = block_sum(rows);
-  if (threadIdx.x == 0) {
-    if (arcs) atomicAdd(&cnt->pull_skipped, arcs);
-    if (rows) atomicAdd(&cnt->pull_skipped_rows, rows);
-  }
+  if (threadIdx.x == 0) share[blockIdx.x] = SkipShare{arcs, 0, rows};
 }
 
 // Sorts each block's arcs by source in place (once per graph): the columns
@@ -444,12 +442,12 @@ grd_status cold_blocks_done(grd_state *s)
 {
   grd_graph *g = s->g;
   const ColdSet &c = *s->cold;
-  if (c.nblk)
-    hipLaunchKernelGGL(k_cold_blocks_done,
-                       dim3(std::min<uint32_t>((c.nblk + kWavesPerBlock - 1) / kWavesPerBlock,
-                                               (uint32_t)g->ctx->num_cus * 8)),
-                       dim3(kBlock), 0, g->ctx->stream, c.nblk, c.blk, (const uint64_t *)s->Rdone,
-                       (const uint64_t *)g->rarc, s->bskip, s->cnt);
+  if (c.nblk) {
+    const uint32_t grid = std::min<uint32_t>((c.nblk + kWavesPerBlock - 1) / kWavesPerBlock, loop_blocks(g->ctx));
+    hipLaunchKernelGGL(k_cold_blocks_done, dim3(grid), dim3(kBlock), 0, g->ctx->stream, c.nblk, c.blk,
+                       (const uint64_t *)s->Rdone, (const uint64_t *)g->rarc, s->bskip, s->sshare + s->n_sshare);
+    s->n_sshare += grid;
+  }
   GRD_HIP(hipGetLastError());
   return GRD_OK;
 }

@@ -97,19 +97,17 @@ struct Counters {
   unsigned long long frontier_edges;  // out-degree sum of the new frontier
   unsigned long long dirty;           // dirty memory proxies at reduce
   unsigned int frontier_maxdeg, pad0;
+  unsigned long long pull_skipped;       // CC / SSSP pull: arcs of the cold row blocks left out (not read)
+  unsigned long long pull_skipped_hot;   // and of the hot wave blocks left out
+  unsigned long long pull_skipped_rows;  // rows of the (cold) row blocks left out
   // added up on the device
   unsigned long long pending;         // SSSP delta-stepping: pending vertices
   unsigned long long heavy;           // push: heavy-vertex chunks appended this iteration
-  unsigned long long edges;           // edges examined by the traversal
   unsigned int pend_min;
   unsigned int fmin;                  // CC / SSSP pull: smallest value broadcast this superstep
   double residual;                    // PR pull: L1 change
   double dangling[2];                 // PR pull: FP64 dangling mass (ping-pong)
-  unsigned long long heavy_edges;     // push: edges of heavy vertices (k_push_heavy)
   unsigned long long frontier_uncovered;  // frontier vertices with an out-neighbour of another master
-  unsigned long long pull_skipped;    // CC / SSSP pull: arcs of the cold row blocks left out (not read)
-  unsigned long long pull_skipped_hot;   // and of the hot wave blocks left out
-  unsigned long long pull_skipped_rows;  // rows of the cold row blocks left out
   unsigned long long pull_done_arcs;     // cold arcs of rows that gathered none (measured with time_kernel)
   float sel[8];                       // learned selector: the next superstep's 4 logits and argmax
   unsigned long long fpart[64];       // frontier size of each compute partition (C > 1)
@@ -117,7 +115,7 @@ struct Counters {
 
 // the pinned copy of a state's counters is followed by the sequence number of
 // the last one that arrived
-constexpr uint32_t kHostOnly = 4;  // leading 8-byte words that only the host's copy holds
+constexpr uint32_t kHostOnly = 7;  // leading 8-byte words that only the host's copy holds
 // a workgroup's share of the next frontier (update, bucket selection) and of
 // the dirty proxies (reduce): stored per workgroup and summed by the wave that
 // publishes the counters, since atomics of thousands of workgroups on one cache
@@ -125,6 +123,10 @@ constexpr uint32_t kHostOnly = 4;  // leading 8-byte words that only the host's 
 struct BlockShare {
   unsigned long long front;  // vertices << 32 | out-degrees, both below 2^32
   unsigned int maxdeg, pad;
+};
+// and of what a CC / SSSP pull leaves out
+struct SkipShare {
+  unsigned long long arcs, hot_arcs, rows;
 };
 constexpr uint64_t kHostCounters = ((sizeof(Counters) + 63) & ~63ull) + 64;
 inline uint32_t *host_seq(Counters *host)
@@ -351,7 +353,8 @@ struct grd_state {
   grd::Counters *cnt = nullptr;   // device
   grd::BlockShare *ushare = nullptr;  // [loop_blocks] of the last update / selection
   uint32_t *rshare = nullptr;         // [loop_blocks] dirty proxies, zero after each publishing
-  uint32_t n_ushare = 0, n_rshare = 0;
+  grd::SkipShare *sshare = nullptr;   // [2 * loop_blocks] row blocks left out by the last pull: cold, then hot
+  uint32_t n_ushare = 0, n_rshare = 0, n_sshare = 0;
   grd::Counters *hcnt = nullptr;  // pinned host (kHostCounters bytes)
   uint32_t cnt_seq = 0;           // sequence number of the last counters published
   bool cnt_clean = false;         // the device counters are at their start

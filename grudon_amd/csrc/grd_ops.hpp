@@ -223,9 +223,12 @@ struct Shares {
   uint32_t nu;
   uint32_t *r;
   uint32_t nr;
+  const SkipShare *s;
+  uint32_t ns;
 };
 
 Shares shares(const grd_state *s);
+uint32_t loop_blocks(const grd_ctx *ctx);  // most workgroups of a pass that leaves shares
 
 // the counters of one superstep to their start (not the pull PageRank's
 // residual and dangling mass)
@@ -234,13 +237,8 @@ __device__ __forceinline__ void zero_counters(Counters *cnt, const Shares &sh)
   if (threadIdx.x == 0) {
     cnt->pending = 0;
     cnt->heavy = 0;
-    cnt->heavy_edges = 0;
-    cnt->edges = 0;
     cnt->pend_min = 0xFFFFFFFFu;
     cnt->fmin = 0xFFFFFFFFu;
-    cnt->pull_skipped = 0;
-    cnt->pull_skipped_hot = 0;
-    cnt->pull_skipped_rows = 0;
     cnt->pull_done_arcs = 0;
     cnt->frontier_uncovered = 0;
   }
@@ -250,55 +248,70 @@ __device__ __forceinline__ void zero_counters(Counters *cnt, const Shares &sh)
 
 // the sums of the blocks' shares, in every thread
 struct FrontierCounts {
-  unsigned long long frontier, edges, dirty;
+  unsigned long long frontier, edges, dirty, skipped, skipped_hot, skipped_rows;
   uint32_t maxdeg;
 };
 __device__ __forceinline__ FrontierCounts sum_shares(const Shares &sh)
 {
-  __shared__ unsigned long long s_f[kWavesPerBlock], s_d[kWavesPerBlock];
+  __shared__ unsigned long long s_c[kWavesPerBlock][5];
   __shared__ uint32_t s_m[kWavesPerBlock];
-  unsigned long long f = 0, d = 0;
+  unsigned long long c[5] = {0, 0, 0, 0, 0};
   uint32_t m = 0;
 #pragma unroll 8
   for (uint32_t b = threadIdx.x; b < sh.nu; b += kBlock) {
-    f += sh.u[b].front;
+    c[0] += sh.u[b].front;
     m = max(m, sh.u[b].maxdeg);
   }
 #pragma unroll 8
-  for (uint32_t b = threadIdx.x; b < sh.nr; b += kBlock) d += sh.r[b];
-  f = wave_sum(f);
-  d = wave_sum(d);
+  for (uint32_t b = threadIdx.x; b < sh.nr; b += kBlock) c[1] += sh.r[b];
+#pragma unroll 4
+  for (uint32_t b = threadIdx.x; b < sh.ns; b += kBlock) {
+    c[2] += sh.s[b].arcs;
+    c[3] += sh.s[b].hot_arcs;
+    c[4] += sh.s[b].rows;
+  }
+#pragma unroll
+  for (int q = 0; q < 5; q++) c[q] = wave_sum(c[q]);
   m = wave_max(m);
   if (lane_id() == 0) {
-    s_f[wave_in_block()] = f;
-    s_d[wave_in_block()] = d;
+#pragma unroll
+    for (int q = 0; q < 5; q++) s_c[wave_in_block()][q] = c[q];
     s_m[wave_in_block()] = m;
   }
   __syncthreads();
-  f = d = 0;
   m = 0;
 #pragma unroll
+  for (int q = 0; q < 5; q++) c[q] = 0;
+#pragma unroll
   for (int i = 0; i < kWavesPerBlock; i++) {
-    f += s_f[i];
-    d += s_d[i];
+#pragma unroll
+    for (int q = 0; q < 5; q++) c[q] += s_c[i][q];
     m = max(m, s_m[i]);
   }
-  return FrontierCounts{f >> 32, f & 0xFFFFFFFFull, d, m};
+  return FrontierCounts{c[0] >> 32, c[0] & 0xFFFFFFFFull, c[1], c[2], c[3], c[4], m};
 }
 
-// the counters into the host's copy, except the words [skip0, skip1)
-__device__ __forceinline__ void copy_counters(const Counters *cnt, Counters *host, const FrontierCounts &fc,
+// the counters into the host's copy, except the words [skip0, skip1); `word` is
+// the thread's own (counter_word, loaded before the shares are waited for)
+__device__ __forceinline__ uint64_t counter_word(const Counters *cnt)
+{
+  static_assert(sizeof(Counters) % 8 == 0 && sizeof(Counters) / 8 <= kBlock, "a word per thread");
+  return threadIdx.x < sizeof(Counters) / 8 ? reinterpret_cast<const uint64_t *>(cnt)[threadIdx.x] : 0ull;
+}
+__device__ __forceinline__ void copy_counters(uint64_t word, Counters *host, const FrontierCounts &fc,
                                               uint32_t skip0 = 0, uint32_t skip1 = 0)
 {
-  static_assert(sizeof(Counters) % 8 == 0, "copied in 8-byte words");
-  for (uint32_t i = threadIdx.x; i < sizeof(Counters) / 8; i += kBlock)
-    if (i >= kHostOnly && (i < skip0 || i >= skip1))
-      reinterpret_cast<uint64_t *>(host)[i] = reinterpret_cast<const uint64_t *>(cnt)[i];
+  const uint32_t i = threadIdx.x;
+  if (i >= kHostOnly && i < sizeof(Counters) / 8 && (i < skip0 || i >= skip1))
+    reinterpret_cast<uint64_t *>(host)[i] = word;
   if (threadIdx.x == 0) {
     host->frontier = fc.frontier;
     host->frontier_edges = fc.edges;
     host->dirty = fc.dirty;
     host->frontier_maxdeg = fc.maxdeg;
+    host->pull_skipped = fc.skipped;
+    host->pull_skipped_hot = fc.skipped_hot;
+    host->pull_skipped_rows = fc.skipped_rows;
   }
 }
 

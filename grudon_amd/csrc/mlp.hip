@@ -405,8 +405,9 @@ __global__ void __launch_bounds__(kBlock) k_mlp_publish(const uint16_t *__restri
   // the counters' copy; sel follows below
   constexpr uint32_t kSel0 = offsetof(Counters, sel) / 8, kSel1 = kSel0 + sizeof(Counters::sel) / 8;
   static_assert(offsetof(Counters, sel) % 8 == 0 && sizeof(Counters::sel) % 8 == 0, "sel is whole words");
+  const uint64_t word = counter_word(cnt);
   const FrontierCounts fc = sum_shares(sh);
-  copy_counters(cnt, host, fc, kSel0, kSel1);
+  copy_counters(word, host, fc, kSel0, kSel1);
   // every wave computes the same decision (their LDS rows hold equal values)
   {
     const double fr = (double)fc.frontier, fe = (double)fc.edges;
@@ -483,7 +484,7 @@ grd_status mlp_publish(grd_state *s, uint64_t prev_frontier)
   hipLaunchKernelGGL(k_mlp_publish, dim3(1), dim3(kBlock), 0, ctx->stream, ctx->sel_w, s->cnt, shares(s), in, s->hcnt,
                      host_seq(s->hcnt), ++s->cnt_seq);
   GRD_HIP(hipGetLastError());
-  s->n_ushare = 0;
+  s->n_ushare = s->n_sshare = 0;
   s->cnt_clean = true;
   return GRD_OK;
 }

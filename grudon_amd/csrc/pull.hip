@@ -179,12 +179,13 @@ __global__ void __launch_bounds__(kBlock) k_prp_pull_fixup(const PullLong *__res
 // bitmap, k_rows_done): a row block whose rows with arcs are all done is left
 // out whole (flag 1); one with some done rows (flag 2) gathers only the arcs
 // of its other rows.  This pass sets the flags and counts the arcs and rows of
-// the blocks left out (one atomic per workgroup), so that the pull reads one
+// the blocks left out (a share per workgroup), so that the pull reads one
 // flag per block.
 __global__ void __launch_bounds__(kBlock) k_blocks_done(uint32_t nblk, const PullBlock *__restrict__ blocks,
                                                         const uint64_t *__restrict__ done,
                                                         const uint64_t *__restrict__ hasarc,
-                                                        uint8_t *__restrict__ bskip, Counters *cnt, int hot)
+                                                        uint8_t *__restrict__ bskip,
+                                                        SkipShare *__restrict__ share, int hot)
 {
   unsigned long long arcs = 0, rows = 0;
   for (uint32_t b = blockIdx.x * kBlock + threadIdx.x; b < nblk; b += gridDim.x * kBlock) {
@@ -211,10 +212,8 @@ __global__ void __launch_bounds__(kBlock) k_blocks_done(uint32_t nblk, const Pul
   }
   arcs = block_sum(arcs);
   rows = block_sum(rows);
-  if (threadIdx.x == 0) {
-    if (arcs) atomicAdd(hot ? &cnt->pull_skipped_hot : &cnt->pull_skipped, arcs);
-    if (rows && !hot) atomicAdd(&cnt->pull_skipped_rows, rows);
-  }
+  // (the hot blocks' rows are counted with the cold ones)
+  if (threadIdx.x == 0) share[blockIdx.x] = hot ? SkipShare{0, arcs, 0} : SkipShare{arcs, 0, rows};
 }
 
 // Measurement only (time_kernel): the arcs, in the row-block pull's CSC (rp:
@@ -439,6 +438,7 @@ static grd_status blocks_done(grd_state *s, bool cold, const uint8_t **flags)
 {
   *flags = nullptr;
   s->hskip_on = false;
+  s->n_sshare = 0;
   if (!Op::kMin || !s->bound_sent) return GRD_OK;
   s->skip_pending = true;  // the rows that gathered nothing come off with the counters
   if (!s->rdone_sent) return GRD_OK;
@@ -454,19 +454,18 @@ static grd_status blocks_done(grd_state *s, bool cold, const uint8_t **flags)
                                                                    (uint32_t)g->ctx->num_cus * 8)),
                          dim3(kBlock), 0, st, nwP, g->crp, g->rarc);
   }
-  const uint32_t cap = (uint32_t)g->ctx->num_cus * 8;
-  if (cold) {
-    GRD_TRY(cold_blocks_done(s));
-  } else if (g->n_pblk) {
-    hipLaunchKernelGGL(k_blocks_done, dim3(std::min<uint32_t>((g->n_pblk + kBlock - 1) / kBlock, cap)), dim3(kBlock), 0,
-                       st, g->n_pblk, g->pblk, (const uint64_t *)s->Rdone, (const uint64_t *)g->rarc, s->bskip, s->cnt,
-                       0);
-  }
-  // the hot pass's wave blocks (their rows are counted once, with the cold pass's)
+  // thread-per-block passes; their shares lie behind one another
+  const auto flag = [&](uint32_t nblk, const PullBlock *blocks, uint8_t *out, int hot) {
+    const uint32_t grid = std::min<uint32_t>((nblk + kBlock - 1) / kBlock, loop_blocks(g->ctx));
+    hipLaunchKernelGGL(k_blocks_done, dim3(grid), dim3(kBlock), 0, st, nblk, blocks, (const uint64_t *)s->Rdone,
+                       (const uint64_t *)g->rarc, out, s->sshare + s->n_sshare, hot);
+    s->n_sshare += grid;
+  };
+  if (cold) GRD_TRY(cold_blocks_done(s));
+  else if (g->n_pblk) flag(g->n_pblk, g->pblk, s->bskip, 0);
+  // the hot pass's wave blocks
   if (cold && g->n_tblk && s->hskip) {
-    hipLaunchKernelGGL(k_blocks_done, dim3(std::min<uint32_t>((g->n_tblk + kBlock - 1) / kBlock, cap)), dim3(kBlock), 0,
-                       st, g->n_tblk, g->tblk, (const uint64_t *)s->Rdone, (const uint64_t *)g->rarc, s->hskip,
-                       s->cnt, 1);
+    flag(g->n_tblk, g->tblk, s->hskip, 1);
     s->hskip_on = true;
   }
   GRD_HIP(hipGetLastError());

@@ -57,7 +57,6 @@ __global__ void __launch_bounds__(kBlock) k_push(const uint32_t *__restrict__ AL
   __shared__ V s_val[kBlock];
   __shared__ unsigned long long s_slot;
   const uint32_t k = *nact;
-  uint64_t my_edges = 0;
   for (uint32_t t0 = blockIdx.x * tile; t0 < k; t0 += gridDim.x * tile) {
     const uint32_t i = t0 + threadIdx.x;
     uint32_t deg = 0, beg = 0, p = 0, nch = 0;
@@ -70,13 +69,9 @@ __global__ void __launch_bounds__(kBlock) k_push(const uint32_t *__restrict__ AL
       if (deg >= kHeavyDeg) nch = (deg + kHeavyChunk - 1) / kHeavyChunk;
     }
     if (__syncthreads_or(nch != 0)) {
-      uint32_t hch, hdeg;
+      uint32_t hch;
       const uint32_t at = block_excl_scan(nch, &hch);
-      (void)block_excl_scan(nch ? deg : 0u, &hdeg);
-      if (threadIdx.x == 0) {
-        s_slot = atomicAdd(&cnt->heavy, (unsigned long long)hch);
-        atomicAdd(&cnt->heavy_edges, (unsigned long long)hdeg);
-      }
+      if (threadIdx.x == 0) s_slot = atomicAdd(&cnt->heavy, (unsigned long long)hch);
       __syncthreads();
       for (uint32_t c = 0; c < nch; c++) heavy[s_slot + at + c] = make_uint2(p, c * kHeavyChunk);
       if (nch) deg = 0;
@@ -107,10 +102,8 @@ __global__ void __launch_bounds__(kBlock) k_push(const uint32_t *__restrict__ AL
       for (int q = 0; q < kIlp; q++) x[q] = Op::edge(x[q], w[q]);
       relax_many<Op, kIlp, kShip>(upd, dirty, c, x, (total - j0 + kBlock - 1) / kBlock);
     }
-    if (threadIdx.x == 0) my_edges += total;
     __syncthreads();
   }
-  if (threadIdx.x == 0 && my_edges) atomicAdd(&cnt->edges, (unsigned long long)my_edges);
 }
 
 template <class Op, bool kShip, class W>
@@ -166,6 +159,7 @@ static grd_status launch(grd_state *s, const uint32_t *col, const W *wt, typenam
     hipLaunchKernelGGL((k_push_heavy<Op, kShip, W>), dim3((uint32_t)slots), dim3(kBlock), 0, st, s->heavy, s->cnt,
                        g->rp, col, wt, (const V *)s->mprop, upd, dirty);
   GRD_HIP(hipGetLastError());
+  s->edges += s->last_frontier_edges;  // every out-arc of the active list
   return GRD_OK;
 }
 
