@@ -13,7 +13,6 @@
 //                                 termination popcount               :643-662
 //   k_popc_blocks/k_scan_blocks/k_word_rank  DynamicBitSet::getOffsets ranks
 #include <algorithm>
-#include <chrono>
 #include <cstring>
 
 #include "grd_device.hpp"
@@ -678,23 +677,7 @@ grd_status op_zero_counters(grd_state *s)
   return GRD_OK;
 }
 
-// Waits for the counters published with the state's last sequence number.  A
-// superstep of a small graph is tens of microseconds, so the host looks at the
-// pinned word for a short while before it hands the wait to the runtime.
-grd_status op_wait_counters(grd_state *s)
-{
-  const uint32_t *seq = host_seq(s->hcnt);
-  const auto t0 = std::chrono::steady_clock::now();
-  for (uint32_t i = 1; __atomic_load_n(seq, __ATOMIC_ACQUIRE) != s->cnt_seq; i++) {
-    __builtin_ia32_pause();
-    if (i % 64 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(200)) {
-      GRD_HIP(hipStreamSynchronize(s->g->ctx->stream));
-      if (__atomic_load_n(seq, __ATOMIC_ACQUIRE) != s->cnt_seq)
-        return fail(GRD_ERR_HIP, "the superstep's counters did not arrive");
-    }
-  }
-  return GRD_OK;
-}
+grd_status op_wait_counters(grd_state *s) { return wait_pinned(s->g->ctx, host_seq(s->hcnt), s->cnt_seq); }
 
 grd_status op_read_counters(grd_state *s)
 {

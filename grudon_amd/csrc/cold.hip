@@ -20,75 +20,16 @@
 // is left is the L2's misses (84 M lines, 6.4 TB/s from the fabric): every XCD
 // draws the partition's 33 MB of values through its own 4 MB.  Loads that go
 // past the L1 measured the same, nontemporal ones 1.7 times slower.
-#include <rocprim/block/block_radix_sort.hpp>
-
 #include <algorithm>
 
 #include "grd_device.hpp"
 #include "grd_internal.hpp"
 #include "grd_ops.hpp"
+#include "grd_rows.hpp"
 
 namespace grd {
 
 namespace {
-
-// arcs in flight per thread
-constexpr int kBatch = 8;
-
-// lanes per row of a block of nrows rows for a workgroup of T threads
-template <int T>
-__device__ __forceinline__ uint32_t cold_group(uint32_t nrows)
-{
-  uint32_t g = kWave;
-  while (g > 1 && g * nrows > (uint32_t)T) g >>= 1;
-  return g;
-}
-
-// The row sums of one round: groups of G lanes over [b, e) of the staged
-// values; the sum is valid in the group's first lane.  A row much longer than
-// its group is left to the whole wave (blocks mix rows of one arc with rows of
-// thousands; a lane alone takes about 30 ns per compensated add).  Called by
-// the whole wave.
-constexpr uint32_t kWideRow = 24;  // arcs per lane beyond which the wave takes the row
-template <class Pol>
-__device__ __forceinline__ typename Pol::Acc cold_row(const typename Pol::V *s_v, uint32_t b, uint32_t e, uint32_t G)
-{
-  const uint32_t lane = lane_id(), sub = lane % G;
-  const bool wide = G < (uint32_t)kWave && e - b > kWideRow * G;
-  auto a = Pol::zero();
-  if (!wide)
-    for (uint32_t x = b + sub; x < e; x += G) Pol::add(a, s_v[x]);
-  Pol::merge_lanes(a, (int)G);
-  uint64_t m = __ballot(wide && sub == 0);
-  while (m) {
-    const int src = __ffsll((unsigned long long)m) - 1;
-    m &= m - 1;
-    const uint32_t wb = __shfl(b, src, kWave), we = __shfl(e, src, kWave);
-    auto t = Pol::zero();
-    for (uint32_t x = wb + lane; x < we; x += kWave) Pol::add(t, s_v[x]);
-    Pol::merge_lanes(t, kWave);
-    if ((int)lane == src) a = t;
-  }
-  return a;
-}
-
-// one segment of a long row: every thread over its staged values in order, the
-// waves merged in wave order by the first thread, which gets the sum
-template <class Pol, int T>
-__device__ __forceinline__ typename Pol::Acc cold_segment(const typename Pol::V *s_v, uint32_t ne)
-{
-  using Acc = typename Pol::Acc;
-  __shared__ uint64_t s_w[T / kWave];
-  static_assert(sizeof(Acc) <= 8, "an accumulator fits its slot");
-  auto a = Pol::zero();
-  for (uint32_t x = threadIdx.x; x < ne; x += T) Pol::add(a, s_v[x]);
-  Pol::merge_lanes(a, kWave);
-  if (lane_id() == 0) *reinterpret_cast<Acc *>(&s_w[wave_in_block()]) = a;
-  __syncthreads();
-  if (threadIdx.x == 0)
-    for (int j = 1; j < T / kWave; j++) Pol::merge(a, *reinterpret_cast<const Acc *>(&s_w[j]));
-  return a;
-}
 
 template <int T, int N>
 __global__ void __launch_bounds__(T, 8) k_prp_pull_cold(const PullBlock *__restrict__ blocks,
@@ -101,7 +42,7 @@ __global__ void __launch_bounds__(T, 8) k_prp_pull_cold(const PullBlock *__restr
   __shared__ float s_v[N];
   const PullBlock d = blocks[blockIdx.x];
   const uint32_t ne = d.e1 - d.e0;
-  const uint32_t G = cold_group<T>(d.nrows), ngroups = T / G;
+  const uint32_t G = row_group<T>(d.nrows), ngroups = T / G;
   const uint32_t rounds = (d.nrows + ngroups - 1) / ngroups, r1 = d.r0 + d.nrows;
   // the first round's rows are loaded with the columns
   uint32_t r = d.r0 + threadIdx.x / G, b = 0, e = 0;
@@ -132,7 +73,7 @@ __global__ void __launch_bounds__(T, 8) k_prp_pull_cold(const PullBlock *__restr
   }
   __syncthreads();
   if (d.nrows == 0) {
-    const Kahan t = cold_segment<HotPR, T>(s_v, ne);
+    const Kahan t = segment_sum<HotPR, T>(s_v, ne);
     if (threadIdx.x == 0) partial[blockIdx.x] = make_float2(t.s, t.c);
     return;
   }
@@ -141,7 +82,7 @@ __global__ void __launch_bounds__(T, 8) k_prp_pull_cold(const PullBlock *__restr
     const float hn = hot;
     r += ngroups;
     row();  // the next round's rows are in flight during this one's sums
-    const Kahan acc = cold_row<HotPR>(s_v, bn, en, G);
+    const Kahan acc = row_sum<HotPR>(s_v, bn, en, G);
     if (threadIdx.x % G == 0 && rn < r1) {
       Kahan t;
       t.s = hn;  // the row's hot partial comes first
@@ -182,7 +123,7 @@ __global__ void __launch_bounds__(T, 8) k_bsp_pull_cold(const PullBlock *__restr
     if (threadIdx.x == 0) partial[blockIdx.x] = op_identity<Op>();
     return;
   }
-  const uint32_t G = cold_group<T>(d.nrows), ngroups = T / G, sub = threadIdx.x % G;
+  const uint32_t G = row_group<T>(d.nrows), ngroups = T / G, sub = threadIdx.x % G;
   const uint32_t rounds = (d.nrows + ngroups - 1) / ngroups, r1 = d.r0 + d.nrows;
   const uint32_t w0 = d.r0 >> 6;
   for (uint32_t i = threadIdx.x; i < d.nrows / 64 + 2; i += T) s_dirty[i] = 0ull;
@@ -234,7 +175,7 @@ __global__ void __launch_bounds__(T, 8) k_bsp_pull_cold(const PullBlock *__restr
   }
   __syncthreads();
   if (d.nrows == 0) {
-    const V t = cold_segment<Pol, T>(s_v, ne);
+    const V t = segment_sum<Pol, T>(s_v, ne);
     if (threadIdx.x == 0) partial[blockIdx.x] = t;
     return;
   }
@@ -257,7 +198,7 @@ __global__ void __launch_bounds__(T, 8) k_bsp_pull_cold(const PullBlock *__restr
     const V hn = hot;
     r += ngroups;
     row();
-    const V acc = op_combine<Op>(hn, cold_row<Pol>(s_v, bn, en, G));  // the row's hot partial first
+    const V acc = op_combine<Op>(hn, row_sum<Pol>(s_v, bn, en, G));  // the row's hot partial first
     if (sub == 0 && ln && pull_apply<Op>(upd, rn, acc)) atomicOr(&s_dirty[(rn >> 6) - w0], 1ull << (rn & 63));
   }
   __syncthreads();
@@ -303,44 +244,6 @@ __global__ void __launch_bounds__(kBlock) k_cold_blocks_done(uint32_t nblk, cons
   if (threadIdx.x == 0) share[blockIdx.x] = SkipShare{arcs, 0, rows};
 }
 
-// Sorts each block's arcs by source in place (once per graph): the columns
-// come in row order, leave in source order with their row-order places in pos,
-// the weights with them.  Sources below 2^bits; padding keys sort last.
-template <class W, int T, int N>
-__global__ void __launch_bounds__(T) k_cold_sort(const PullBlock *__restrict__ blocks, uint32_t *__restrict__ col,
-                                                 W *__restrict__ cw, uint16_t *__restrict__ pos, int bits)
-{
-  constexpr int kPer = N / T;
-  using Sort = rocprim::block_radix_sort<uint32_t, T, kPer, uint16_t>;
-  __shared__ typename Sort::storage_type s_sort;
-  const PullBlock d = blocks[blockIdx.x];
-  const uint32_t ne = d.e1 - d.e0;
-  uint32_t key[kPer];
-  uint16_t at[kPer];
-#pragma unroll
-  for (int k = 0; k < kPer; k++) {
-    const uint32_t i = threadIdx.x + k * T;
-    key[k] = i < ne ? col[d.e0 + i] : 1u << bits;
-    at[k] = (uint16_t)i;
-  }
-  Sort().sort_to_striped(key, at, s_sort, 0, bits + 1);
-  W w[kPer];
-  if (cw) {
-#pragma unroll
-    for (int k = 0; k < kPer; k++) w[k] = threadIdx.x + k * T < ne ? cw[d.e0 + at[k]] : W(0);
-  }
-  __syncthreads();  // every weight is read before one is written
-#pragma unroll
-  for (int k = 0; k < kPer; k++) {
-    const uint32_t i = threadIdx.x + k * T;
-    if (i < ne) {
-      col[d.e0 + i] = key[k];
-      pos[d.e0 + i] = at[k];
-      if (cw) cw[d.e0 + i] = w[k];
-    }
-  }
-}
-
 }  // namespace
 
 // Cold set 0 serves the sums (pull and reference PageRank), 1 the min-combines
@@ -380,9 +283,9 @@ grd_status cold_sort(grd_graph *g, const ColdSet &c)
   while (bits < 31 && (g->P >> bits)) bits++;
 #define F(T, N)                                                                                                     \
   if (c.w8)                                                                                                         \
-    hipLaunchKernelGGL((k_cold_sort<uint8_t, T, N>), dim3(c.nblk), dim3(T), 0, st, c.blk, c.col, c.w8, c.pos, bits); \
+    hipLaunchKernelGGL((k_block_sort<PullBlock, uint8_t, T, N>), dim3(c.nblk), dim3(T), 0, st, c.blk, c.col, c.w8, c.pos, bits); \
   else                                                                                                              \
-    hipLaunchKernelGGL((k_cold_sort<uint32_t, T, N>), dim3(c.nblk), dim3(T), 0, st, c.blk, c.col, c.w, c.pos, bits)
+    hipLaunchKernelGGL((k_block_sort<PullBlock, uint32_t, T, N>), dim3(c.nblk), dim3(T), 0, st, c.blk, c.col, c.w, c.pos, bits)
   COLD_SHAPES(c.nnz, F)
 #undef F
   GRD_HIP(hipGetLastError());

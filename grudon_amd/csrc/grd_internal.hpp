@@ -371,6 +371,8 @@ struct grd_state {
 namespace grd {
 // workspace.cpp
 void workspace_release(grd_ctx *ctx);
+// until a kernel has stored `want` to a pinned word
+grd_status wait_pinned(grd_ctx *ctx, const uint32_t *word, uint32_t want);
 grd_status host_counters_take(grd_ctx *ctx, Counters **out);
 void host_counters_give(grd_ctx *ctx, Counters *p);
 // n 4-byte values from the device to the caller's array, widened to 8 bytes on

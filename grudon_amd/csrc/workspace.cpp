@@ -10,6 +10,7 @@
 // more than the solve.
 #include <algorithm>
 #include <atomic>
+#include <chrono>
 #include <cstring>
 #include <thread>
 #include <vector>
@@ -159,6 +160,22 @@ void host_counters_give(grd_ctx *ctx, Counters *p)
   if (!p) return;
   if (ctx->host_counters.size() < 8) ctx->host_counters.push_back(p);
   else (void)hipHostFree(p);
+}
+
+// A superstep of a small graph is tens of microseconds, so the host looks at the
+// pinned word for a short while before it hands the wait to the runtime.
+grd_status wait_pinned(grd_ctx *ctx, const uint32_t *word, uint32_t want)
+{
+  const auto t0 = std::chrono::steady_clock::now();
+  for (uint32_t i = 1; __atomic_load_n(word, __ATOMIC_ACQUIRE) != want; i++) {
+    __builtin_ia32_pause();
+    if (i % 64 == 0 && std::chrono::steady_clock::now() - t0 > std::chrono::microseconds(200)) {
+      GRD_HIP(hipStreamSynchronize(ctx->stream));
+      if (__atomic_load_n(word, __ATOMIC_ACQUIRE) != want)
+        return fail(GRD_ERR_HIP, "a device pass did not report its end");
+    }
+  }
+  return GRD_OK;
 }
 
 // Helper threads of one transfer: thread t of T copies part t of every chunk

@@ -348,9 +348,9 @@ typedef struct grd_batch grd_batch;
 grd_status grd_batch_create(grd_ctx *ctx, uint32_t count, const uint32_t *n, const uint64_t *m,
                             const uint32_t *const *row_ptr, const uint32_t *const *col, grd_batch **out);
 grd_status grd_batch_free(grd_batch *b);
-/* Tunables (0 = keep): tile = arcs per row block and long-row threshold
- * (1024, 2048 or 4096), grid_per_cu = persistent workgroups per CU (<= 64),
- * K = iterations per captured hipGraph (<= 64). */
+/* Tunables (0 = keep): tile = arcs of the smallest row block (1024, 2048 or
+ * 4096; larger batches use larger blocks), grid_per_cu = persistent workgroups
+ * per CU (<= 64), K = iterations per captured hipGraph (<= 64). */
 grd_status grd_batch_tune(grd_batch *b, uint32_t tile, uint32_t grid_per_cu, uint32_t K);
 /* Autotune the tunables by timing candidate settings on this batch
  * (tile x grid_per_cu x K); chosen3 (may be NULL) receives the winner. */
