@@ -296,6 +296,7 @@ grd_status grd_destroy(grd_ctx *c)
   if (c->sel_w) (void)hipFree(c->sel_w);
   if (c->sel_out) (void)hipFree(c->sel_out);
   if (c->sel_out_host) (void)hipHostFree(c->sel_out_host);
+  if (c->sel_stage) (void)hipHostFree(c->sel_stage);
   workspace_release(c);
   (void)hipStreamDestroy(c->stream);
   delete c;

@@ -194,6 +194,8 @@ struct grd_ctx {
   float sel_margin = 0.0f;
   float *sel_out = nullptr;       // device: 4 logits + chosen option
   float *sel_out_host = nullptr;  // pinned
+  float *sel_stage = nullptr;     // pinned: an inference's features, logits and flags (mlp.hip)
+  uint32_t sel_seq = 0;           // inferences so far
   // kept between calls (workspace.cpp)
   grd::BlockCache cache;
   char *stage = nullptr;        // pinned, kStageSlots slots

@@ -8,8 +8,7 @@
 // network is trained as a classifier of the fastest option with a
 // cost-weighted softmax cross-entropy: sample weight = clamp((t_max -
 // t_min) / t_min, 0.1, 10), so iterations where the choice matters weigh
-// more.  One wave evaluates one sample, lane j owning hidden unit j; the
-// forward pass of training reads BF16-rounded weights so that training and
+// more.  The forward pass of training reads BF16-rounded weights so that training and
 // inference see the same network.  The selector only picks the schedule of
 // an iteration: every option computes the same result.
 #include <algorithm>
@@ -318,29 +317,102 @@ __global__ void __launch_bounds__(kWave) k_mlp_adam(float *__restrict__ w, float
   wb[i] = f32_to_bf16(w[i]);
 }
 
-// inference: one wave per sample, BF16 weights; logits[n*4]
-__global__ void __launch_bounds__(kBlock) k_mlp_infer(const uint16_t *__restrict__ wb, const float *__restrict__ feat,
-                                                      uint32_t n, float *__restrict__ logits)
+// Inference with the BF16 weights, logits[n*4]: a workgroup takes 16 samples,
+// wave u the hidden units 16u to 16u + 15 of both layers, as FP32 matrix
+// products (16x16x4) of unit rows by sample columns.  The order of the inputs
+// within a product is free as long as both operands agree on it, so lane group
+// q takes the inputs 4q.. (layer 1) and 16q.. (layer 2): each lane's weights and
+// values are whole 16-byte loads, and the lane that computes a unit's four
+// results stores them as one.  The last layer's four outputs are summed in the
+// lanes that hold the units, then over the lane groups and the waves.
+//
+// features and logits may lie in pinned host memory (one coalesced read and one
+// coalesced write per workgroup); with flags, workgroup b then reports its end
+// there.  2000 samples: a wave per sample, weights through the caches for each,
+// took 6 us and each of the two copies around it as long again; a call took 43
+// us.  Now 19 us a call, of which the kernel is
+// about 6: a PCIe read, the tile, a PCIe write (1 sample 11 us, 4096 28 us).
+typedef float Vec4 __attribute__((ext_vector_type(4)));
+constexpr int kTileS = 16;
+
+__device__ __forceinline__ Vec4 bf16x4(const uint16_t *__restrict__ p)
 {
-  __shared__ float s_h1[kWavesPerBlock][kH];
-  const uint32_t nwaves = gridDim.x * kWavesPerBlock;
-  const uint32_t iters = (n + nwaves - 1) / nwaves;
-  for (uint32_t it = 0; it < iters; it++) {
-    uint32_t t = it * nwaves + blockIdx.x * kWavesPerBlock + wave_in_block();
-    bool active = t < n;
-    float x[kIn];
+  const uint2 q = *reinterpret_cast<const uint2 *>(p);
+  return Vec4{__uint_as_float(q.x << 16), __uint_as_float(q.x & 0xFFFF0000u), __uint_as_float(q.y << 16),
+              __uint_as_float(q.y & 0xFFFF0000u)};
+}
+
+__global__ void __launch_bounds__(kBlock) k_mlp_infer(const uint16_t *__restrict__ wb, const float *__restrict__ feat,
+                                                      uint32_t n, float *__restrict__ logits, uint32_t *flags,
+                                                      uint32_t seq)
+{
+  static_assert(kBlock == kTileS * kIn && kWavesPerBlock * 16 == kH && kIn == 16 && kOut == 4, "tile shapes");
+  static_assert(oB1 % 4 == 0 && oW2 % 4 == 0 && oB2 % 4 == 0 && oW3 % 4 == 0, "weights are loaded four at a time");
+  __shared__ __align__(16) float s_x[kTileS * kIn];
+  __shared__ __align__(16) float s_h[kTileS][kH + 4];  // (rows four banks apart)
+  __shared__ __align__(16) float s_o[kWavesPerBlock][kTileS][kOut];
+  const int l = lane_id(), i = l % 16, q = l / 16, u = wave_in_block() * 16, t = threadIdx.x;
+  const Vec4 w1 = bf16x4(wb + oW1 + (u + i) * kIn + 4 * q);
+  Vec4 w2[4], w3[kOut];
 #pragma unroll
-    for (int i = 0; i < kIn; i++) x[i] = active ? feat[(uint64_t)t * kIn + i] : 0.0f;
-    Fwd r = forward_wave<true>(nullptr, wb, x, s_h1[wave_in_block()]);
-    if (active && lane_id() < kOut) {
-      float v = r.logit[0];
+  for (int k = 0; k < 4; k++) w2[k] = bf16x4(wb + oW2 + (u + i) * kH + 16 * q + 4 * k);
 #pragma unroll
-      for (int o = 1; o < kOut; o++)
-        if (lane_id() == o) v = r.logit[o];
-      logits[(uint64_t)t * kOut + lane_id()] = v;
-    }
+  for (int o = 0; o < kOut; o++) w3[o] = bf16x4(wb + oW3 + o * kH + u + 4 * q);
+  const Vec4 b1 = bf16x4(wb + oB1 + u + 4 * q), b2 = bf16x4(wb + oB2 + u + 4 * q);
+  const float b3 = bf16_to_f32(wb[oB3 + t % kOut]);
+  const uint32_t tiles = (uint32_t)(((uint64_t)n + kTileS - 1) / kTileS);
+  for (uint32_t tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
+    const uint64_t x0 = (uint64_t)tile * kTileS * kIn;
+    s_x[t] = x0 + t < (uint64_t)n * kIn ? feat[x0 + t] : 0.0f;
     __syncthreads();
+    const Vec4 x = *reinterpret_cast<const Vec4 *>(&s_x[i * kIn + 4 * q]);
+    // units u + 4q + (0..3) of sample i, in two sums (four in the second layer):
+    // shorter chains, and a smaller rounding error than one chain's
+    const Vec4 zero{};
+    Vec4 a = __builtin_amdgcn_mfma_f32_16x16x4f32(w1[0], x[0], b1, 0, 0, 0);
+    Vec4 c = __builtin_amdgcn_mfma_f32_16x16x4f32(w1[1], x[1], zero, 0, 0, 0);
+    a = __builtin_amdgcn_mfma_f32_16x16x4f32(w1[2], x[2], a, 0, 0, 0);
+    c = __builtin_amdgcn_mfma_f32_16x16x4f32(w1[3], x[3], c, 0, 0, 0);
+    a += c;
+#pragma unroll
+    for (int k = 0; k < 4; k++) a[k] = a[k] > 0.0f ? a[k] : 0.0f;
+    *reinterpret_cast<Vec4 *>(&s_h[i][u + 4 * q]) = a;
+    __syncthreads();
+    Vec4 s[4] = {b2, zero, zero, zero};
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const Vec4 h = *reinterpret_cast<const Vec4 *>(&s_h[i][16 * q + 4 * j]);
+#pragma unroll
+      for (int k = 0; k < 4; k++) s[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(w2[j][k], h[k], s[j], 0, 0, 0);
+    }
+    a = (s[0] + s[1]) + (s[2] + s[3]);
+    Vec4 o4;
+#pragma unroll
+    for (int o = 0; o < kOut; o++) {
+      float v = 0.0f;
+#pragma unroll
+      for (int k = 0; k < 4; k++) v += w3[o][k] * (a[k] > 0.0f ? a[k] : 0.0f);
+      v += __shfl_xor(v, 16, kWave);
+      v += __shfl_xor(v, 32, kWave);
+      o4[o] = v;
+    }
+    if (q == 0) *reinterpret_cast<Vec4 *>(s_o[wave_in_block()][i]) = o4;
+    __syncthreads();
+    if (t < kTileS * kOut) {  // (the first wave)
+      float v = b3;
+#pragma unroll
+      for (int w = 0; w < kWavesPerBlock; w++) v += s_o[w][t / kOut][t % kOut];
+      const uint64_t at = (uint64_t)tile * kTileS * kOut + t;
+      if (at < (uint64_t)n * kOut) logits[at] = v;
+    }
   }
+  if (flags && t == 0) __hip_atomic_store(flags + blockIdx.x, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// workgroups of k_mlp_infer: one per tile up to four per CU
+static uint32_t infer_blocks(const grd_ctx *ctx, uint64_t n)
+{
+  return (uint32_t)std::min<uint64_t>((n + kTileS - 1) / kTileS, 4ull * (uint64_t)std::max(1, ctx->num_cus));
 }
 
 // per-iteration selection: one wave; writes 4 logits + argmax to out[0..4]
@@ -465,6 +537,19 @@ static grd_status sel_buffers(grd_ctx *ctx)
   return GRD_OK;
 }
 
+// pinned: features and logits of kInferMax samples, and a flag per workgroup
+// (allocated with the weights, 20 us)
+static grd_status infer_stage(grd_ctx *ctx)
+{
+  constexpr size_t kFlags = kInferMax / kTileS;
+  if (!ctx->sel_stage) {
+    const size_t bytes = ((size_t)kInferMax * (kIn + kOut) + kFlags) * 4;
+    GRD_HIP(hipHostMalloc((void **)&ctx->sel_stage, bytes, hipHostMallocDefault));
+    memset(ctx->sel_stage, 0, bytes);
+  }
+  return GRD_OK;
+}
+
 static void decode_logits(const float *o, int *option, float *margin)
 {
   int best = (int)o[4];
@@ -519,6 +604,7 @@ grd_status grd_selector_load(grd_ctx *ctx, const uint16_t *w, uint64_t count, fl
   GRD_HIP(hipSetDevice(ctx->device));
   if (!ctx->sel_w) GRD_HIP(hipMalloc((void **)&ctx->sel_w, kParams * sizeof(uint16_t)));
   GRD_HIP(hipMemcpy(ctx->sel_w, w, kParams * sizeof(uint16_t), hipMemcpyHostToDevice));
+  GRD_TRY(infer_stage(ctx));
   ctx->sel_loaded = true;
   ctx->sel_margin = min_margin;
   return GRD_OK;
@@ -625,17 +711,29 @@ grd_status grd_selector_infer(grd_ctx *ctx, const float *feat, uint64_t n, float
   if (!ctx || !feat || !logits || n == 0) return fail(GRD_ERR_ARG, "grd_selector_infer: bad argument");
   if (!ctx->sel_loaded) return fail(GRD_ERR_STATE, "grd_selector_infer: no weights loaded");
   GRD_HIP(hipSetDevice(ctx->device));
+  if (n <= kInferMax) {
+    // the kernel reads the features from, and writes the logits to, pinned memory
+    float *x = ctx->sel_stage;
+    float *out = x + (size_t)kInferMax * kIn;
+    uint32_t *flags = reinterpret_cast<uint32_t *>(out + (size_t)kInferMax * kOut);
+    memcpy(x, feat, n * kIn * 4);
+    const uint32_t grid = infer_blocks(ctx, n), seq = ++ctx->sel_seq;
+    hipLaunchKernelGGL(k_mlp_infer, dim3(grid), dim3(kBlock), 0, ctx->stream, ctx->sel_w, x, (uint32_t)n, out, flags,
+                       seq);
+    GRD_HIP(hipGetLastError());
+    for (uint32_t b = 0; b < grid; b++) GRD_TRY(wait_pinned(ctx, flags + b, seq));
+    memcpy(logits, out, n * kOut * 4);
+    return GRD_OK;
+  }
   DevMem mem(ctx);
   float *df, *dl;
   GRD_TRY(mem.alloc_n(&df, n * kIn));
   GRD_TRY(mem.alloc_n(&dl, n * kOut));
-  GRD_HIP(hipMemcpy(df, feat, n * kIn * 4, hipMemcpyHostToDevice));
-  uint32_t grid = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(1024, (n + 3) / 4));
-  hipLaunchKernelGGL(k_mlp_infer, dim3(grid), dim3(kBlock), 0, ctx->stream, ctx->sel_w, df, (uint32_t)n, dl);
+  GRD_TRY(copy_in(ctx, df, feat, n * kIn * 4));
+  hipLaunchKernelGGL(k_mlp_infer, dim3(infer_blocks(ctx, n)), dim3(kBlock), 0, ctx->stream, ctx->sel_w, df, (uint32_t)n,
+                     dl, (uint32_t *)nullptr, 0u);
   GRD_HIP(hipGetLastError());
-  GRD_HIP(hipMemcpyAsync(logits, dl, n * kOut * 4, hipMemcpyDeviceToHost, ctx->stream));
-  GRD_HIP(hipStreamSynchronize(ctx->stream));
-  return GRD_OK;
+  return copy_out(ctx, logits, dl, n * kOut);
 }
 
 grd_status grd_selector_infer_noalloc(grd_ctx *ctx, const float *feat, uint64_t n, float *logits)
@@ -652,8 +750,8 @@ grd_status grd_selector_infer_noalloc(grd_ctx *ctx, const float *feat, uint64_t 
   float *df = g_scratch_ptr[ctx->device];
   float *dl = df + (size_t)kInferMax * kIn;
   GRD_HIP(hipMemcpyAsync(df, feat, n * kIn * 4, hipMemcpyHostToDevice, ctx->stream));
-  uint32_t grid = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>(1024, (n + 3) / 4));
-  hipLaunchKernelGGL(k_mlp_infer, dim3(grid), dim3(kBlock), 0, ctx->stream, ctx->sel_w, df, (uint32_t)n, dl);
+  hipLaunchKernelGGL(k_mlp_infer, dim3(infer_blocks(ctx, n)), dim3(kBlock), 0, ctx->stream, ctx->sel_w, df, (uint32_t)n,
+                     dl, (uint32_t *)nullptr, 0u);
   GRD_HIP(hipGetLastError());
   GRD_HIP(hipMemcpyAsync(logits, dl, n * kOut * 4, hipMemcpyDeviceToHost, ctx->stream));
   GRD_HIP(hipStreamSynchronize(ctx->stream));
