@@ -371,7 +371,6 @@ __global__ void __launch_bounds__(kWave) k_balive(uint32_t *alive, uint32_t *seq
     *alive = 0;
     const uint32_t n = *seq + 1;
     *seq = n;
-    __threadfence_system();
     __hip_atomic_store(host + 1, n, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }

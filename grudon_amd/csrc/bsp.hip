@@ -631,9 +631,9 @@ __global__ void __launch_bounds__(kBlock) k_zero_counters(Counters *cnt, Shares 
 __global__ void __launch_bounds__(kBlock) k_publish(Counters *cnt, Shares sh, Counters *host, uint32_t *host_seq,
                                                     uint32_t seq)
 {
-  const uint64_t word = counter_word(cnt);
+  const CounterWords words = counter_words(cnt);
   const FrontierCounts fc = sum_shares(sh);
-  copy_counters(word, host, fc);
+  copy_counters(words, host, fc);
   publish_seq(host_seq, seq);
   zero_counters(cnt, sh);
 }

@@ -117,7 +117,6 @@ __global__ void __launch_bounds__(kBlock) k_prp_finish(const double *__restrict_
     cnt->residual = res;
     cnt->dangling[parity ^ 1] = dang;
     host->residual = res;
-    __threadfence_system();
     __hip_atomic_store(host_seq, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
   }
 }
