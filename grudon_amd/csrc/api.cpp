@@ -536,6 +536,33 @@ grd_status grd_graph_coverage(const grd_graph *g, uint8_t *covered, uint64_t *n_
 
 grd_status grd_state_create(grd_graph *g, int algo, grd_state **out) { return grd_state_create_typed(g, algo, 4, out); }
 
+// Whether the default pull of a graph is the row-block pull and not the hot /
+// cold split.  The split takes two passes and their fix-ups where the row-block
+// pull takes one (12 us a superstep more on graphs of up to 65536 vertices), and
+// 40 % of the state's creation; what it saves grows with the arcs.  Pull
+// PageRank's update waits for one pass at a time, so its line is by the arcs of
+// a partition; delta-push PageRank's and the min-combines' are by all of them.
+// us a superstep, every superstep a pull, row-block / split, RMAT with 16 arcs
+// a vertex:
+//   pull PageRank     262 K vertices, M = 1: 33 / 38   1 M, M = 4: 71 / 77
+//                     524 K, M = 1: 51 / 53            2 M, M = 4: 126 / 122
+//   delta PageRank    262 K, M = 1: 45 / 48            524 K, M = 1: 66 / 63
+//   CC (symmetrized)  262 K, M = 1: 51 / 66            1 M, heuristic: 104 / 102
+//   weighted SSSP     524 K, heuristic: 84 / 85        1 M, heuristic: 107 / 100
+static bool small_graph_pull(const grd_graph *g, int algo)
+{
+  const grd_ctx *ctx = g->ctx;
+  if (ctx->pull_mode != 3 || ctx->tier_bits != 0) return false;
+  // (a graph keeps a regrouping that was asked for)
+  if (g->tiers_built && (g->tier_mode != 3 || g->tier_bits != kTierBitsMax)) return false;
+  constexpr uint64_t kSums = 6ull << 20, kMost = 16ull << 20;
+  switch (algo) {
+  case GRD_PR: return g->m <= kSums;
+  case GRD_PR_PULL: return g->m <= std::min<uint64_t>(kSums * (uint64_t)g->M, kMost);
+  default: return g->m <= kMost;
+  }
+}
+
 grd_status grd_state_create_typed(grd_graph *g, int algo, uint32_t value_bytes, grd_state **out)
 {
   if (!g || !out) return fail(GRD_ERR_ARG, "grd_state_create: NULL argument");
@@ -556,8 +583,9 @@ grd_status grd_state_create_typed(grd_graph *g, int algo, uint32_t value_bytes, 
   s->wide = value_bytes == 8;
   grd_status st = GRD_OK;
   // the pull modes: modes 1-2 serve pull PageRank only, the hot / cold split
-  // (mode 3) every pull (the BSP pull of CC, SSSP and reference PageRank too)
-  const int pm = g->ctx->pull_mode;
+  // (mode 3) every pull (the BSP pull of CC, SSSP and reference PageRank too);
+  // with the default window, small graphs keep the row-block pull
+  const int pm = small_graph_pull(g, algo) ? 0 : g->ctx->pull_mode;
   if ((algo == GRD_PR_PULL && pm != 0) || pm == 3) {
     try {
       st = build_tiers(g);

@@ -140,12 +140,15 @@ __global__ void __launch_bounds__(T, 8) k_bsp_pull_cold(const PullBlock *__restr
     // gathers nothing, 0 where the arc's value is wanted
     for (uint32_t k = 0; k < rounds; k++) {
       const uint32_t q = d.r0 + k * ngroups + threadIdx.x / G;
+      bool gat = false;
+      uint32_t b = 0, e = 0;
       if (q < r1) {
-        bool gat = live_row(q);
+        gat = live_row(q);
         if (gat && bcnt) gat = pre[q] > bnd;
-        const uint32_t b = rptr[q] - d.e0, e = rptr[q + 1] - d.e0;
-        for (uint32_t x = b + sub; x < e; x += G) s_v[x] = gat ? V(0) : op_identity<Op>();
+        b = rptr[q] - d.e0;
+        e = rptr[q + 1] - d.e0;
       }
+      row_fill(s_v, b, e, G, gat ? V(0) : op_identity<Op>());
     }
     __syncthreads();
   }
@@ -207,10 +210,11 @@ __global__ void __launch_bounds__(T, 8) k_bsp_pull_cold(const PullBlock *__restr
     if (s_dirty[i]) atomicOr((unsigned long long *)(dirty + w0 + i), s_dirty[i]);
 }
 
-// Flags of the cold blocks (k_blocks_done of pull.hip, with a wave per block:
-// a block spans up to kColdRows rows): 1 = every row with arcs is done, 2 =
-// some are; counts the arcs and rows left out.
-__global__ void __launch_bounds__(kBlock) k_cold_blocks_done(uint32_t nblk, const PullBlock *__restrict__ blocks,
+// Flags of the row blocks of a CC / SSSP pull (the cold blocks, or those of the
+// whole CSC): 1 = every row with arcs is done, 2 = some are; counts the arcs and
+// rows left out.  A wave per block: a block spans up to kColdRows rows, 129 words
+// of each bitmap, which a thread alone would walk one after another.
+__global__ void __launch_bounds__(kBlock) k_row_blocks_done(uint32_t nblk, const PullBlock *__restrict__ blocks,
                                                              const uint64_t *__restrict__ done,
                                                              const uint64_t *__restrict__ hasarc,
                                                              uint8_t *__restrict__ bskip,
@@ -341,13 +345,12 @@ template grd_status bsp_pull_cold<OpHop>(grd_state *, const uint8_t *, const Cou
 template grd_status bsp_pull_cold<OpWeighted>(grd_state *, const uint8_t *, const Counters *);
 template grd_status bsp_pull_cold<OpPR>(grd_state *, const uint8_t *, const Counters *);
 
-grd_status cold_blocks_done(grd_state *s)
+grd_status row_blocks_done(grd_state *s, uint32_t nblk, const PullBlock *blocks)
 {
   grd_graph *g = s->g;
-  const ColdSet &c = *s->cold;
-  if (c.nblk) {
-    const uint32_t grid = std::min<uint32_t>((c.nblk + kWavesPerBlock - 1) / kWavesPerBlock, loop_blocks(g->ctx));
-    hipLaunchKernelGGL(k_cold_blocks_done, dim3(grid), dim3(kBlock), 0, g->ctx->stream, c.nblk, c.blk,
+  if (nblk) {
+    const uint32_t grid = std::min<uint32_t>((nblk + kWavesPerBlock - 1) / kWavesPerBlock, loop_blocks(g->ctx));
+    hipLaunchKernelGGL(k_row_blocks_done, dim3(grid), dim3(kBlock), 0, g->ctx->stream, nblk, blocks,
                        (const uint64_t *)s->Rdone, (const uint64_t *)g->rarc, s->bskip, s->sshare + s->n_sshare);
     s->n_sshare += grid;
   }

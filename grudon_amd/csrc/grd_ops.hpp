@@ -354,7 +354,7 @@ grd_status pull_done_arcs(grd_state *s);
 // the hot pass of the hot / cold split for the BSP pull (tiers.hip)
 template <class Op>
 grd_status bsp_pull_hot(grd_state *s);
-// its cold pass (cold.hip); skip: a flag per cold block (k_cold_blocks_done),
+// its cold pass (cold.hip); skip: a flag per cold block (k_row_blocks_done),
 // bcnt: the superstep's bound (either may be null)
 template <class Op>
 grd_status bsp_pull_cold(grd_state *s, const uint8_t *skip, const Counters *bcnt);

@@ -21,6 +21,7 @@
 #include "grd_device.hpp"
 #include "grd_internal.hpp"
 #include "grd_ops.hpp"
+#include "grd_rows.hpp"
 
 namespace grd {
 
@@ -31,13 +32,6 @@ constexpr int kDirtyWords = kPullMaxRows / 64 + 2;
 static inline uint32_t fixup_grid(uint32_t nlong)
 {
   return std::max<uint32_t>(1, std::min<uint32_t>(65535, (nlong + kWavesPerBlock - 1) / kWavesPerBlock));
-}
-
-__device__ __forceinline__ int group_size(uint32_t nrows)
-{
-  int g = 64;
-  while (g > 1 && (uint32_t)g * nrows > (uint32_t)kBlock) g >>= 1;
-  return g;
 }
 
 // ---- PageRank pull: Kahan FP32 ----
@@ -126,22 +120,21 @@ __global__ void __launch_bounds__(kBlock) k_prp_pull_rb(const PullBlock *__restr
     }
   }
   __syncthreads();
-  const int G = group_size(d.nrows);
-  const int sub = threadIdx.x % G;
-  const uint32_t ngroups = kBlock / G;
   // every group runs the same number of rounds so that the group shuffles
-  // stay in step
+  // stay in step; a row far longer than the others is the whole wave's (row_sum:
+  // pull PageRank over RMAT-16 in four partitions, 92 us an iteration with the
+  // longest rows on a lane each, now 27)
+  const uint32_t G = row_group<kBlock>(d.nrows), ngroups = kBlock / G;
   const uint32_t rounds = (d.nrows + ngroups - 1) / ngroups;
   for (uint32_t k = 0; k < rounds; k++) {
-    uint32_t rl = k * ngroups + threadIdx.x / G;
-    Kahan acc;
-    uint32_t r = d.r0 + rl;
+    const uint32_t rl = k * ngroups + threadIdx.x / G, r = d.r0 + rl;
+    uint32_t b = 0, e = 0;
     if (rl < d.nrows) {
-      uint32_t b = crp[r] - d.e0, e = crp[r + 1] - d.e0;
-      for (uint32_t x = b + sub; x < e; x += G) acc.add(s_v[x]);
+      b = crp[r] - d.e0;
+      e = crp[r + 1] - d.e0;
     }
-    kahan_wave_merge(acc, G);
-    if (sub == 0 && rl < d.nrows) out[r] = acc.value();
+    const Kahan acc = row_sum<HotPR>(s_v, b, e, G);
+    if (threadIdx.x % G == 0 && rl < d.nrows) out[r] = acc.value();
   }
 }
 
@@ -178,16 +171,18 @@ __global__ void __launch_bounds__(kBlock) k_prp_pull_fixup(const PullLong *__res
 // Rows of a CC / SSSP pull that cannot improve (the broadcast's rows-done
 // bitmap, k_rows_done): a row block whose rows with arcs are all done is left
 // out whole (flag 1); one with some done rows (flag 2) gathers only the arcs
-// of its other rows.  This pass sets the flags and counts the arcs and rows of
-// the blocks left out (a share per workgroup), so that the pull reads one
-// flag per block.
-__global__ void __launch_bounds__(kBlock) k_blocks_done(uint32_t nblk, const PullBlock *__restrict__ blocks,
-                                                        const uint64_t *__restrict__ done,
-                                                        const uint64_t *__restrict__ hasarc,
-                                                        uint8_t *__restrict__ bskip,
-                                                        SkipShare *__restrict__ share, int hot)
+// of its other rows.  A pass before the pull sets the flags and counts the arcs
+// and rows of the blocks left out (a share per workgroup), so that the pull
+// reads one flag per block: for the row blocks k_row_blocks_done (cold.hip),
+// for the hot pass's wave blocks this one, a thread per block (at most 256 rows,
+// five words of the bitmaps).
+__global__ void __launch_bounds__(kBlock) k_hot_blocks_done(uint32_t nblk, const PullBlock *__restrict__ blocks,
+                                                            const uint64_t *__restrict__ done,
+                                                            const uint64_t *__restrict__ hasarc,
+                                                            uint8_t *__restrict__ bskip,
+                                                            SkipShare *__restrict__ share)
 {
-  unsigned long long arcs = 0, rows = 0;
+  unsigned long long arcs = 0;
   for (uint32_t b = blockIdx.x * kBlock + threadIdx.x; b < nblk; b += gridDim.x * kBlock) {
     const PullBlock d = blocks[b];
     bool all, any = false;
@@ -205,15 +200,10 @@ __global__ void __launch_bounds__(kBlock) k_blocks_done(uint32_t nblk, const Pul
       }
     }
     bskip[b] = all ? 1 : any ? 2 : 0;
-    if (all) {
-      arcs += d.e1 - d.e0;
-      rows += d.nrows;
-    }
+    if (all) arcs += d.e1 - d.e0;
   }
   arcs = block_sum(arcs);
-  rows = block_sum(rows);
-  // (the hot blocks' rows are counted with the cold ones)
-  if (threadIdx.x == 0) share[blockIdx.x] = hot ? SkipShare{0, arcs, 0} : SkipShare{arcs, 0, rows};
+  if (threadIdx.x == 0) share[blockIdx.x] = SkipShare{0, arcs, 0};  // (its rows are counted with the cold ones)
 }
 
 // Measurement only (time_kernel): the arcs, in the row-block pull's CSC (rp:
@@ -263,10 +253,9 @@ __global__ void __launch_bounds__(kBlock) k_bsp_pull_rb(const PullBlock *__restr
   __shared__ V s_v[kPullNnz];
   __shared__ V s_hot[kPullHot];
   __shared__ unsigned long long s_dirty[kDirtyWords];
-  __shared__ uint8_t s_live[kPullNnz];  // a partially done block: 1 = the arc's row may improve
   const uint32_t bid = blockIdx.x;
   const PullBlock d = blocks[bid];
-  const uint32_t flag = bskip ? bskip[bid] : 0u;  // k_blocks_done: 1 = left out, 2 = some rows done
+  const uint32_t flag = bskip ? bskip[bid] : 0u;  // k_row_blocks_done: 1 = left out, 2 = some rows done
   if (flag == 1) return;
   if (d.nrows == 0) {  // segment (<= kPullNnz arcs) of a long row
     // column ids (and weights), then the gathers (hot sources from LDS),
@@ -298,9 +287,7 @@ __global__ void __launch_bounds__(kBlock) k_bsp_pull_rb(const PullBlock *__restr
   }
   for (int i = threadIdx.x; i < kDirtyWords; i += kBlock) s_dirty[i] = 0ull;
   const uint32_t ne = d.e1 - d.e0;
-  const int G = group_size(d.nrows);
-  const int sub = threadIdx.x % G;
-  const uint32_t ngroups = kBlock / G;
+  const uint32_t G = row_group<kBlock>(d.nrows), ngroups = kBlock / G, sub = threadIdx.x % G;
   const uint32_t rounds = (d.nrows + ngroups - 1) / ngroups;
   const uint32_t w0 = d.r0 >> 6;
   {
@@ -317,8 +304,9 @@ __global__ void __launch_bounds__(kBlock) k_bsp_pull_rb(const PullBlock *__restr
     }
     const bool marked = flag == 2;  // uniform over the block
     if (marked) {
-      // each row's group marks the row's arcs to gather or not (every arc of
-      // the block belongs to one of its rows): not for a done row
+      // each row's group marks the row's places (every arc of the block belongs
+      // to one of its rows): the identity for a done row, 0 where the arc's
+      // value is wanted
       for (uint32_t k = 0; k < rounds; k++) {
         const uint32_t rl = k * ngroups + threadIdx.x / G, r = d.r0 + rl;
         bool gat = false;
@@ -329,7 +317,7 @@ __global__ void __launch_bounds__(kBlock) k_bsp_pull_rb(const PullBlock *__restr
           b = crp[r] - d.e0;
           e = crp[r + 1] - d.e0;
         }
-        for (uint32_t x = b + sub; x < e; x += G) s_live[x] = gat ? 1 : 0;
+        row_fill(s_v, b, e, G, gat ? V(0) : op_identity<Op>());
       }
     }
     const uint32_t hb = hot_base[bid];
@@ -340,7 +328,7 @@ __global__ void __launch_bounds__(kBlock) k_bsp_pull_rb(const PullBlock *__restr
     for (int k = 0; k < kPer; k++) {
       uint32_t i = threadIdx.x + k * kBlock;
       const uint32_t h = src[k] - hb;
-      const bool on = i < ne && (!marked || s_live[i]);
+      const bool on = i < ne && (!marked || s_v[i] == V(0));
       v[k] = on ? Op::edge(h < hn ? s_hot[h] : mprop[src[k]], wt[k]) : op_identity<Op>();
     }
 #pragma unroll
@@ -351,19 +339,18 @@ __global__ void __launch_bounds__(kBlock) k_bsp_pull_rb(const PullBlock *__restr
   }
   __syncthreads();
   for (uint32_t k = 0; k < rounds; k++) {
-    uint32_t rl = k * ngroups + threadIdx.x / G;
-    V acc = op_identity<Op>();
-    uint32_t r = d.r0 + rl;
+    const uint32_t rl = k * ngroups + threadIdx.x / G, r = d.r0 + rl;
     bool live = rl < d.nrows;
     if (done && live) {
       const uint64_t bit = 1ull << (r & 63);
       live = !(done[r >> 6] & bit) && (hasarc[r >> 6] & bit);
     }
+    uint32_t b = 0, e = 0;
     if (live) {
-      uint32_t b = crp[r] - d.e0, e = crp[r + 1] - d.e0;
-      for (uint32_t x = b + sub; x < e; x += G) acc = op_combine<Op>(acc, s_v[x]);
+      b = crp[r] - d.e0;
+      e = crp[r + 1] - d.e0;
     }
-    for (int o = G / 2; o > 0; o >>= 1) acc = op_combine<Op>(acc, __shfl_xor(acc, o, kWave));
+    const V acc = row_sum<HotBsp<Op>>(s_v, b, e, G);
     if (sub == 0 && live && pull_apply<Op>(upd, r, acc))
       atomicOr(&s_dirty[(r >> 6) - w0], 1ull << (r & 63));
   }
@@ -381,7 +368,7 @@ __global__ void __launch_bounds__(kBlock) k_bsp_pull_fixup(const PullLong *__res
                                                            const uint64_t *__restrict__ done)
 {
   // a wave per long row, as k_prp_pull_fixup; a done row's segments were
-  // left out (k_blocks_done flags every segment of it)
+  // left out (k_row_blocks_done flags every segment of it)
   const uint32_t lane = lane_id();
   for (uint32_t i = blockIdx.x * kWavesPerBlock + wave_in_block(); i < nlong; i += gridDim.x * kWavesPerBlock) {
     const PullLong L = longs[i];
@@ -454,18 +441,12 @@ static grd_status blocks_done(grd_state *s, bool cold, const uint8_t **flags)
                                                                    (uint32_t)g->ctx->num_cus * 8)),
                          dim3(kBlock), 0, st, nwP, g->crp, g->rarc);
   }
-  // thread-per-block passes; their shares lie behind one another
-  const auto flag = [&](uint32_t nblk, const PullBlock *blocks, uint8_t *out, int hot) {
-    const uint32_t grid = std::min<uint32_t>((nblk + kBlock - 1) / kBlock, loop_blocks(g->ctx));
-    hipLaunchKernelGGL(k_blocks_done, dim3(grid), dim3(kBlock), 0, st, nblk, blocks, (const uint64_t *)s->Rdone,
-                       (const uint64_t *)g->rarc, out, s->sshare + s->n_sshare, hot);
-    s->n_sshare += grid;
-  };
-  if (cold) GRD_TRY(cold_blocks_done(s));
-  else if (g->n_pblk) flag(g->n_pblk, g->pblk, s->bskip, 0);
-  // the hot pass's wave blocks
+  GRD_TRY(cold ? row_blocks_done(s, s->cold->nblk, s->cold->blk) : row_blocks_done(s, g->n_pblk, g->pblk));
   if (cold && g->n_tblk && s->hskip) {
-    flag(g->n_tblk, g->tblk, s->hskip, 1);
+    const uint32_t grid = std::min<uint32_t>((g->n_tblk + kBlock - 1) / kBlock, loop_blocks(g->ctx));
+    hipLaunchKernelGGL(k_hot_blocks_done, dim3(grid), dim3(kBlock), 0, st, g->n_tblk, g->tblk,
+                       (const uint64_t *)s->Rdone, (const uint64_t *)g->rarc, s->hskip, s->sshare + s->n_sshare);
+    s->n_sshare += grid;
     s->hskip_on = true;
   }
   GRD_HIP(hipGetLastError());
@@ -488,7 +469,8 @@ grd_status bsp_pull_launch(grd_state *s, const uint32_t *cw)
     GRD_TRY(bsp_pull_cold<Op>(s, skip, bcnt));
   } else {
     GRD_TRY(blocks_done<Op>(s, false, &skip));
-    hipLaunchKernelGGL(k_bsp_pull_rb<Op>, dim3(g->n_pblk), dim3(kBlock), 0, g->ctx->stream, g->pblk,
+    if (g->n_pblk)
+      hipLaunchKernelGGL(k_bsp_pull_rb<Op>, dim3(g->n_pblk), dim3(kBlock), 0, g->ctx->stream, g->pblk,
                        g->pblk_hot, g->crp, g->ccol, cw, (const V *)s->mprop, g->P, (V *)s->mupd, s->Du,
                        (V *)s->partial, skip, skip ? (const uint64_t *)s->Rdone : nullptr,
                        skip ? (const uint64_t *)g->rarc : nullptr);

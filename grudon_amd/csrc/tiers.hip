@@ -603,7 +603,7 @@ __device__ __forceinline__ uint32_t hot_group(uint32_t n)
 }
 
 // kSkip (CC / SSSP): skip[b] = 1 marks a wave block whose rows are all done
-// or without arcs (k_blocks_done; 2, some rows done, runs in full); it is
+// or without arcs (k_row_blocks_done; 2, some rows done, runs in full); it is
 // taken as an empty segment (no loads, the identity written to its hseg slot)
 // and its rows' partials are not written, which the cold pass never reads for
 // such rows.
