@@ -718,7 +718,7 @@ grd_status state_alloc(grd_state *s)
   GRD_TRY(m.alloc_n(&s->AL, S));
   // heavy chunks: a vertex's last chunk may be short, and at most m / kHeavyDeg
   // vertices are heavy
-  GRD_TRY(m.alloc_n(&s->heavy, g->m / kHeavyChunk + g->m / kHeavyDeg + 64));
+  if (s->algo != GRD_PR_PULL) GRD_TRY(m.alloc_n(&s->heavy, g->m / kHeavyChunk + g->m / kHeavyDeg + 64));
   GRD_TRY(m.alloc(&s->partial, (uint64_t)std::max<uint32_t>(1, g->n_pblk) * 8));
   if (s->algo == GRD_PR_PULL) {
     GRD_TRY(m.alloc_n(&s->red, 2ull * prp_grid(g)));

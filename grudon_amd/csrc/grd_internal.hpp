@@ -165,8 +165,8 @@ constexpr uint32_t kPullNnz = 2048;     // arcs per block (8 per thread)
 constexpr uint32_t kPullMaxRows = 1024;  // rows per block
 constexpr uint32_t kPullHot = 2048;      // PR pull: hottest sources of a partition kept in LDS
 constexpr uint32_t kColdRows = 8192;     // hot / cold pull: most rows per cold block
-constexpr uint32_t kHeavyDeg = 256;      // push: out-degree handled by k_push_heavy,
-constexpr uint32_t kHeavyChunk = 1024;   // in chunks of this many arcs (a workgroup each)
+constexpr uint32_t kHeavyDeg = 64;       // push: out-degree handled by k_push_heavy,
+constexpr uint32_t kHeavyChunk = 256;    // in chunks of this many arcs (a wave each)
 constexpr int kMaxParts = 64;            // largest C and M
 constexpr uint32_t kTierBitsMax = 15;    // tiled pull: largest tier, 2^15 sources (128 KB of LDS)
 constexpr uint32_t kTierTileArcs = 65536;  // tiled pull: default arcs per tile

@@ -32,13 +32,16 @@ __device__ __forceinline__ uint32_t push_owner(const uint32_t *s_off, uint32_t j
 // source by binary search in the LDS prefix array, four arcs in flight per
 // thread.  Vertices with degree >= kHeavyDeg are appended to the heavy list as
 // chunks of kHeavyChunk arcs (one counter atomic per tile) and handled by
-// k_push_heavy, one workgroup per chunk.
+// k_push_heavy, a wave per chunk.
 //
 // The active list is in degree order, so the vertices just below the threshold
-// share tiles: the threshold bounds a tile's work.  With 4096 (and chunks of
+// share tiles: the threshold bounds a tile's work, and a round of 1024 arcs takes
+// about 4.5 us in a full chip whatever they find.  With 4096 (and chunks of
 // 4096) the first tiles held a million arcs each and ran alone: CC by pushes
-// over RMAT-20 symmetrized (31 M arcs) 16.7 ms a solve, with 256 and chunks of
-// 1024 3.4 ms.
+// over RMAT-20 symmetrized (31 M arcs) 16.7 ms a solve; with 256 and a workgroup
+// per chunk of 1024 3.3, of which 1.8 in the longest tiles; with 64 and a wave
+// per chunk of 256 2.5 (32 to 96 and chunks of 128 to 512 within 2 %; two arcs in
+// flight a lane in the heavy pass, four measured the same).
 //
 // kShip: the edge-shipping superstep (ship.hip).  The columns are the
 // out-neighbours' compute slots and the updates go to the compute side, where
@@ -114,29 +117,30 @@ __global__ void __launch_bounds__(kBlock) k_push_heavy(const uint2 *__restrict__
                                                        uint64_t *dirty)
 {
   using V = typename Op::V;
-  constexpr int kIlp = kHeavyChunk / kBlock;
-  const uint32_t nch = (uint32_t)cnt->heavy;
-  for (uint32_t h = blockIdx.x; h < nch; h += gridDim.x) {
+  constexpr int kIlp = 2;
+  const uint32_t nch = (uint32_t)cnt->heavy, l = lane_id();
+  for (uint32_t h = blockIdx.x * kWavesPerBlock + wave_in_block(); h < nch; h += gridDim.x * kWavesPerBlock) {
     const uint2 ch = heavy[h];
     const uint32_t end = rp[ch.x + 1];
-    const uint32_t b = rp[ch.x] + ch.y, e = min(end, b + kHeavyChunk);
+    const uint32_t b = rp[ch.x] + ch.y, ne = min(end - b, kHeavyChunk);
     const V v = mprop[ch.x];
-    if (b + threadIdx.x >= e) continue;
-    uint32_t c[kIlp], w[kIlp];
-    V x[kIlp];
+    for (uint32_t j0 = l; j0 < ne; j0 += kIlp * kWave) {
+      uint32_t c[kIlp], w[kIlp];
+      V x[kIlp];
 #pragma unroll
-    for (int q = 0; q < kIlp; q++) {
-      const uint32_t at = b + threadIdx.x + q * kBlock;
-      c[q] = 0;
-      w[q] = 1u;
-      if (at < e) {
-        c[q] = col[at];
-        if constexpr (std::is_same<Op, OpWeighted>::value) w[q] = wt[at];
+      for (int q = 0; q < kIlp; q++) {
+        const uint32_t j = j0 + q * kWave;
+        c[q] = 0;
+        w[q] = 1u;
+        if (j < ne) {
+          c[q] = col[b + j];
+          if constexpr (std::is_same<Op, OpWeighted>::value) w[q] = wt[b + j];
+        }
       }
-    }
 #pragma unroll
-    for (int q = 0; q < kIlp; q++) x[q] = Op::edge(v, w[q]);
-    relax_many<Op, kIlp, kShip>(upd, dirty, c, x, (e - b - threadIdx.x + kBlock - 1) / kBlock);
+      for (int q = 0; q < kIlp; q++) x[q] = Op::edge(v, w[q]);
+      relax_many<Op, kIlp, kShip>(upd, dirty, c, x, (ne - j0 + kWave - 1) / kWave);
+    }
   }
 }
 
@@ -149,7 +153,7 @@ static grd_status launch(grd_state *s, const uint32_t *col, const W *wt, typenam
   using V = typename Op::V;
   // tiles of 64 active vertices until those fill every workgroup slot
   const uint64_t slots = (uint64_t)ctx->num_cus * 8;
-  const uint32_t tile = s->last_frontier <= 64 * slots ? 64u : (uint32_t)kBlock;
+    const uint32_t tile = s->last_frontier <= 64 * slots ? 64u : (uint32_t)kBlock;
   const uint32_t grid = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((s->last_frontier + tile - 1) / tile, slots));
   hipLaunchKernelGGL((k_push<Op, kShip, W>), dim3(grid), dim3(kBlock), 0, st, s->AL, s->totals + 0, g->rp, col, wt,
                      (const V *)s->mprop, upd, dirty, s->heavy, s->cnt, tile);

@@ -1,5 +1,5 @@
 """The push's split of the frontier against the oracle: out-degrees at the
-edges of the heavy threshold (256) and of the heavy chunks (1024 arcs), tiles
+edges of the heavy threshold (64) and of the heavy chunks (256 arcs), tiles
 of 64 and of 256 active vertices, ragged last tiles.  CC and SSSP bit-exact
 with equal iteration counts."""
 import numpy as np
