@@ -210,6 +210,8 @@ struct grd_graph {
   uint64_t m = 0;
   int C = 1, M = 1;
   bool weighted = false;
+  uint32_t wmax = 0;  // largest arc weight (weight_max)
+  bool wmax_known = false;
   uint32_t S = 0;       // compute slots (padded)
   uint32_t P = 0;       // memory proxies (padded)
   uint64_t X = 0;       // cross mirrors
@@ -380,6 +382,7 @@ void host_counters_give(grd_ctx *ctx, Counters *p);
 // n 4-byte values from the device to the caller's array, widened to 8 bytes on
 // the way with `wide`; ordered after the context's stream, done on return
 grd_status copy_out(grd_ctx *ctx, void *dst, const void *src, uint64_t n, bool wide = false);
+grd_status weight_max(grd_graph *g, uint32_t *out);
 // bytes to the device, ordered on the context's stream; the source must stay until the stream has passed
 grd_status copy_in(grd_ctx *ctx, void *dst, const void *src, uint64_t bytes);
 // layout.cpp

@@ -78,14 +78,6 @@ __device__ __forceinline__ uint32_t part_of(const uint32_t *__restrict__ pb, uin
 }
 
 __global__ void k_t_fill(uint32_t *p, uint64_t n, uint32_t v) { TIER_LOOP(i, n) p[i] = v; }
-__global__ void k_w_max(uint64_t n, const uint32_t *__restrict__ w, uint32_t *__restrict__ out)
-{
-  uint32_t mx = 0;
-  TIER_LOOP(i, n) mx = max(mx, w[i]);
-  for (int o = kWave / 2; o > 0; o >>= 1) mx = max(mx, (uint32_t)__shfl_xor(mx, o, kWave));
-  if (lane_id() == 0 && mx) atomicMax(out, mx);
-}
-
 // head[crp[r]] = r for every row with arcs (positions are distinct)
 __global__ void k_t_heads(uint32_t P, const uint32_t *__restrict__ crp, uint32_t *__restrict__ head)
 {
@@ -830,12 +822,8 @@ static grd_status build_hotcold(grd_graph *g)
   // arc weights follow their arcs (the BSP pull of weighted SSSP), one byte
   // each when every weight is below 256
   if (g->cw) {
-    uint32_t *d_wmax = nullptr, wmax = 0;
-    GRD_TRY(tmp.alloc_n(&d_wmax, 1));
-    hipLaunchKernelGGL(k_t_fill, dim3(1), dim3(kBlock), 0, st, d_wmax, 1, 0u);
-    hipLaunchKernelGGL(k_w_max, dim3(tgrid(g->m)), dim3(kBlock), 0, st, g->m, g->cw, d_wmax);
-    GRD_HIP(hipMemcpyAsync(&wmax, d_wmax, 4, hipMemcpyDeviceToHost, st));
-    GRD_HIP(hipStreamSynchronize(st));
+    uint32_t wmax = 0;
+    GRD_TRY(weight_max(g, &wmax));
     g->w8_fits = wmax < 256;
     if (g->w8_fits) GRD_TRY(gm.alloc_n(&g->hw8, (uint64_t)hrp[P] + kWave));
     else GRD_TRY(gm.alloc_n(&g->hw, (uint64_t)hrp[P] + kWave));
