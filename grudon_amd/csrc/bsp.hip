@@ -656,6 +656,42 @@ __global__ void __launch_bounds__(kBlock) k_gather_result(uint32_t S, const uint
   }
 }
 
+// Up to kSmallOut values into pinned memory: a workgroup per kOutPart of them,
+// each wave reporting its end in a flag of its own.  Slots are in degree order,
+// so a workgroup looks at all slots and puts the values of its vertices
+// in order in LDS first (a 4-byte store across the bus costs as much as a whole
+// line).
+constexpr uint32_t kOutPart = 4096;
+constexpr int kOutBlock = 1024;
+__global__ void __launch_bounds__(kOutBlock) k_small_out(const uint32_t *__restrict__ src,
+                                                         const uint32_t *__restrict__ gid, uint32_t S, uint32_t n,
+                                                         uint32_t *__restrict__ host, uint32_t *flags, uint32_t seq)
+{
+  __shared__ uint32_t s_o[kOutPart];
+  const uint32_t g0 = blockIdx.x * kOutPart, cnt = min(n - g0, kOutPart);
+#pragma unroll 8
+  for (uint32_t s = threadIdx.x; s < S; s += kOutBlock) {
+    const uint32_t g = gid[s], v = src[s];
+    if (g != kNone && g - g0 < cnt) s_o[g - g0] = v;
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < cnt; i += kOutBlock) host[g0 + i] = s_o[i];
+  if (lane_id() == 0)
+    __hip_atomic_store(flags + blockIdx.x * (kOutBlock / kWave) + threadIdx.x / kWave, seq, __ATOMIC_RELEASE,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+grd_status small_out(grd_ctx *ctx, const uint32_t *src, const uint32_t *gid, uint32_t S, uint32_t n, uint32_t *host,
+                     uint32_t *flags, uint32_t seq, uint32_t *nflags)
+{
+  static_assert((kSmallOut + kOutPart - 1) / kOutPart * (kOutBlock / kWave) <= kSmallFlags, "a flag per wave");
+  const uint32_t grid = (n + kOutPart - 1) / kOutPart;
+  *nflags = grid * (kOutBlock / kWave);
+  hipLaunchKernelGGL(k_small_out, dim3(grid), dim3(kOutBlock), 0, ctx->stream, src, gid, S, n, host, flags, seq);
+  GRD_HIP(hipGetLastError());
+  return GRD_OK;
+}
+
 // ------------------------------------------------------------------------
 // host orchestration
 // ------------------------------------------------------------------------
@@ -1077,15 +1113,16 @@ grd_status op_download(grd_state *s, void *out)
 {
   grd_graph *g = s->g;
   hipStream_t st = g->ctx->stream;
+  const uint32_t *src = (s->algo == GRD_PR || s->algo == GRD_PR_PULL) ? (const uint32_t *)s->pr : (const uint32_t *)s->prop;
+  // 8-byte properties are widened on the way, the unreached 2^32 - 1 to 2^64 - 1
+  // (numeric_limits<uint64_t>::max)
+  if (g->n <= kSmallOut) return copy_out_slots(g->ctx, out, src, g->slot_gid, g->S, g->n, s->wide);
   DevMem tmp(g->ctx);
   uint32_t *dout = nullptr;
   GRD_TRY(tmp.alloc_n(&dout, g->n));
-  const void *src = (s->algo == GRD_PR || s->algo == GRD_PR_PULL) ? (const void *)s->pr : s->prop;
   hipLaunchKernelGGL(k_gather_result<uint32_t>, dim3(std::min<uint32_t>(4096, g->S / kBlock + 1)), dim3(kBlock), 0, st,
-                     g->S, g->slot_gid, (const uint32_t *)src, dout);
+                     g->S, g->slot_gid, src, dout);
   GRD_HIP(hipGetLastError());
-  // 8-byte properties are widened on the way, the unreached 2^32 - 1 to 2^64 - 1
-  // (numeric_limits<uint64_t>::max)
   return copy_out(g->ctx, out, dout, g->n, s->wide);
 }
 

