@@ -280,7 +280,7 @@ struct grd_graph {
   uint32_t n_twide = 0;
   // mode 3, the hot / cold split: a row's arcs from its partition's kHotWin
   // hottest sources (a prefix of the row) are summed from an LDS window into
-  // a per-row partial; its other arcs are pulled by the row-block kernel,
+  // a per-row partial; its other arcs are pulled by the cold pass,
   // which merges that partial.  Hot arcs reuse tcol (16-bit window offsets),
   // tblk / tlong (their wave blocks and long rows) and ttile (each hot
   // workgroup's range of blocks, all of one partition); n_pairs = P (one

@@ -415,7 +415,7 @@ grd_status prp_pull_rows_fixup(hipStream_t st, const PullLong *longs, uint32_t n
 }
 
 // A state over a graph split by the hot / cold pull (mode 3) runs the hot
-// pass first and then the row-block kernel over the cold arcs, which combines
+// pass first and then the cold pass, which combines
 // each row's hot partial with its own; otherwise the row-block kernel over
 // the whole CSC.
 // CC / SSSP after a broadcast that sent the rows-done bitmap: flag the row

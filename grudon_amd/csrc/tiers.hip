@@ -7,13 +7,13 @@
 // Infinity Cache / HBM at worst.  Three reorganisations of the CSC, built
 // once per graph when its first state is created (grd_set_pull_tiling):
 //
-// mode 3, the hot / cold split (the default, for every pull): a row's arcs
+// mode 3, the hot / cold split (the default of large graphs, for every pull): a row's arcs
 // from its partition's 2^b hottest sources (b <= 15) are a prefix of the row,
 // because rows keep their sources ascending.  The hot prefixes, with 16-bit
 // offsets into the partition's window, are reduced from a 128 KB LDS window
 // into one 4-byte partial per row (k_pull_hot, under an accumulation policy:
 // FP32 Kahan for pull PageRank, the BSP operator for CC / SSSP / reference
-// PageRank); the cold rest goes through the row-block kernel of pull.hip,
+// PageRank); the cold rest goes through the cold pass (cold.hip),
 // which merges the row's partial first.  Arc weights (weighted SSSP) follow
 // their arcs, one byte each when every weight is below 256.
 //
@@ -493,8 +493,8 @@ __global__ void __launch_bounds__(kBlock) k_prp_tier_merge_wide(const uint32_t *
 // the row, since rows keep their sources ascending.  1024-thread workgroups,
 // each with one partition's window of those sources in LDS, sum the
 // prefixes into one Kahan partial per row, written in row order.  The rest
-// of each row goes to the row-block kernel over a CSC of the remaining arcs,
-// which merges the row's partial first.
+// of each row goes to the cold pass over a CSC of the remaining arcs
+// (cold.hip), which merges the row's partial first.
 
 // hot and cold arc counts of every row: the first source at or beyond the
 // partition's window end, by binary search over the sorted row

@@ -158,8 +158,8 @@ grd_status grd_set_layout(grd_ctx *ctx, int on_device);
  *     blocks run) and the row-block pull's kernel over them;
  *   mode 3: hot / cold split -- each row's arcs from its partition's
  *     2^tier_bits hottest sources (4..15, 0 = 15) summed from an LDS window
- *     into a per-row partial, the rest of the row pulled by the row-block
- *     kernel, which merges that partial first (tile_arcs must be 0); the
+ *     into a per-row partial, the rest of the row summed in blocks of arcs in
+ *     source order, that partial first (tile_arcs must be 0); the
  *     default, and the fastest measured on large graphs; with tier_bits 0
  *     small ones (up to some millions of arcs) are pulled as by mode 0, which
  *     is the faster there.  Mode 3 also serves the pull
