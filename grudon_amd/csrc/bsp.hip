@@ -786,6 +786,7 @@ Shares shares(const grd_state *s)
 grd_status op_zero_counters(grd_state *s)
 {
   s->n_ushare = s->n_sshare = 0;
+  s->heavy_listed = false;
   hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(kBlock), 0, s->g->ctx->stream, s->cnt, shares(s));
   GRD_HIP(hipGetLastError());
   s->cnt_clean = true;
@@ -800,6 +801,7 @@ grd_status op_read_counters(grd_state *s)
                      host_seq(s->hcnt), ++s->cnt_seq);
   GRD_HIP(hipGetLastError());
   s->n_ushare = s->n_sshare = 0;
+  s->heavy_listed = false;
   s->cnt_clean = true;
   return op_wait_counters(s);
 }

@@ -342,6 +342,7 @@ struct grd_state {
   uint32_t *blk = nullptr, *wrankB = nullptr, *wrankR = nullptr, *totals = nullptr;
   uint32_t *AL = nullptr;
   uint2 *heavy = nullptr;  // push: (proxy, first arc offset) of each heavy-vertex chunk
+  bool heavy_listed = false;  // a push has listed chunks since the counters were last at their start
   void *partial = nullptr;  // pull: one 8-byte partial per row block (long-row segments)
   bool tiled = false;       // PR_PULL: the tiled pull runs (else the plain row-block pull)
   const grd::ColdSet *cold = nullptr;  // hot / cold pull: the cold blocks this state pulls over

@@ -581,6 +581,7 @@ grd_status mlp_publish(grd_state *s, uint64_t prev_frontier)
                      host_seq(s->hcnt), ++s->cnt_seq);
   GRD_HIP(hipGetLastError());
   s->n_ushare = s->n_sshare = 0;
+  s->heavy_listed = false;
   s->cnt_clean = true;
   return GRD_OK;
 }

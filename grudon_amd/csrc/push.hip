@@ -144,6 +144,11 @@ __global__ void __launch_bounds__(kBlock) k_push_heavy(const uint2 *__restrict__
   }
 }
 
+__global__ void k_heavy_restart(Counters *cnt)
+{
+  if (threadIdx.x == 0) cnt->heavy = 0;
+}
+
 template <class Op, bool kShip, class W>
 static grd_status launch(grd_state *s, const uint32_t *col, const W *wt, typename Op::V *upd, uint64_t *dirty)
 {
@@ -153,8 +158,12 @@ static grd_status launch(grd_state *s, const uint32_t *col, const W *wt, typenam
   using V = typename Op::V;
   // tiles of 64 active vertices until those fill every workgroup slot
   const uint64_t slots = (uint64_t)ctx->num_cus * 8;
-    const uint32_t tile = s->last_frontier <= 64 * slots ? 64u : (uint32_t)kBlock;
+  const uint32_t tile = s->last_frontier <= 64 * slots ? 64u : (uint32_t)kBlock;
   const uint32_t grid = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((s->last_frontier + tile - 1) / tile, slots));
+  // the heavy list holds one pass over the active list: another push of the same
+  // broadcast lists its chunks anew
+  if (s->heavy_listed) hipLaunchKernelGGL(k_heavy_restart, dim3(1), dim3(kWave), 0, st, s->cnt);
+  s->heavy_listed = true;
   hipLaunchKernelGGL((k_push<Op, kShip, W>), dim3(grid), dim3(kBlock), 0, st, s->AL, s->totals + 0, g->rp, col, wt,
                      (const V *)s->mprop, upd, dirty, s->heavy, s->cnt, tile);
   // a vertex's out-arcs all hang off its own proxy, so the frontier's largest

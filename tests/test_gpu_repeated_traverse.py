@@ -1,0 +1,66 @@
+"""The superstep's entry points called more than once, or later than usual,
+after one broadcast (the operator API's gen_updates is such a call): results
+against the oracle on graphs of which every vertex has enough out-arcs for the
+push's heavy list."""
+import numpy as np
+import pytest
+
+import oracle_lib as O
+from grudon_amd import api
+
+pytestmark = pytest.mark.gpu
+
+DEGREES = [64, 20, 65, 257, 64]
+
+
+def _graph(n):
+    """Vertex v points at the DEGREES[v % 5] vertices after it, 7 apart."""
+    deg = np.array(DEGREES)[np.arange(n) % len(DEGREES)]
+    src = np.repeat(np.arange(n), deg)
+    k = np.arange(len(src)) - np.repeat(np.cumsum(deg) - deg, deg)
+    keys = np.unique(src.astype(np.int64) * n + (src + 1 + 7 * k) % n)
+    rp = np.concatenate([[0], np.cumsum(np.bincount(keys // n, minlength=n))])
+    return O.Graph(rp.astype(np.uint32), (keys % n).astype(np.uint32))
+
+
+def _call(name, S, *args):
+    api._check(getattr(api.lib(), name)(S.h, *args), name)
+
+
+@pytest.mark.parametrize("M", [1, 3])
+@pytest.mark.parametrize("option", [api.OPT_PUSH_SPARSE, api.OPT_PUSH_DENSE, api.OPT_SHIP_EDGES])
+def test_push_traversal_repeated(ctx, M, option):
+    """Two and three traversals of one broadcast: the min-combine's labels are
+    those of one, the sums count every arc as often as it was traversed."""
+    print("push traversal repeated", M, option, flush=True)
+    g = _graph(3001)
+    ref, st = O.Partition(g, 1, M).cc()
+    G = api.Graph.from_csr(ctx, g.rp, g.col, C=1, M=M)
+    S = api.State(G, api.CC)
+    S.init()
+    steps, left = 0, 1
+    while left:
+        _call("grd_broadcast", S, option)
+        for _ in range(3):
+            _call("grd_traverse", S, option)
+        _call("grd_reduce", S, option)
+        left = S.step_update()
+        steps += 1
+    assert np.array_equal(S.result(), ref) and steps == int(st[0])
+    S.free()
+    S = api.State(G, api.PR)
+    S.init()
+    _call("grd_broadcast", S, option)
+    for _ in range(2):
+        _call("grd_traverse", S, option)
+    _call("grd_reduce", S, option)
+    S.step_update()
+    deg = np.diff(g.rp.astype(np.int64))
+    src = np.repeat(np.arange(g.n), deg)
+    upd = 2 * np.bincount(g.col, weights=0.85 * 0.15 / deg[src], minlength=g.n)
+    want = 0.15 + upd
+    terms = 2 * np.bincount(g.col, minlength=g.n)
+    # FP32 addends of two roundings each, summed in any order, and the last sum
+    assert (np.abs(S.result() - want) <= (terms + 4) * 2.0 ** -24 * want).all()
+    S.free()
+    G.free()
