@@ -169,7 +169,6 @@ static grd_status superstep(grd_state *s, int option, bool select_next = false)
 {
   const bool ship = option == GRD_OPT_SHIP_EDGES;
   if (!s->cnt_clean) GRD_TRY(op_zero_counters(s));
-  s->cnt_clean = false;
   // the edge-shipping schedule broadcasts like the offloaded push
   // (GraphAlgorithm.cpp:199-343 runs for both decisions), then ships the
   // frontier's edge lists instead of generating and reducing updates
@@ -654,7 +653,6 @@ grd_status grd_broadcast(grd_state *s, int option)
   if (option < 0 || option > GRD_OPT_SHIP_EDGES) return fail(GRD_ERR_ARG, "grd_broadcast: bad option");
   if (s->algo == GRD_PR_PULL) return prp_broadcast(s);
   GRD_TRY(op_zero_counters(s));
-  s->cnt_clean = false;
   s->bcast_option = option;
   return op_broadcast(s, option == GRD_OPT_SHIP_EDGES ? GRD_OPT_PUSH_SPARSE : option);
 }

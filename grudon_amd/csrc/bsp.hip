@@ -993,6 +993,7 @@ grd_status op_broadcast(grd_state *s, int option)
   const uint32_t nwS = g->S / 64;
   const bool pull = option & 1, dense = option & 2;
   const bool need_rank = !dense || !pull;
+  s->cnt_clean = false;
   s->xb_dense = dense ? 1 : 0;
   s->xr_dense = -1;
   if (need_rank) GRD_TRY(word_ranks(st, s->F, nwS, s->blk, s->wrankB, s->totals + 0));
@@ -1071,6 +1072,7 @@ static grd_status traverse_t(grd_state *s, int option)
 
 grd_status op_traverse(grd_state *s, int option)
 {
+  s->cnt_clean = false;
   switch (s->algo) {
   case GRD_PR: return traverse_t<OpPR>(s, option);
   case GRD_CC: return traverse_t<OpCC>(s, option);
@@ -1105,6 +1107,7 @@ static grd_status reduce_t(grd_state *s, int option)
 
 grd_status op_reduce(grd_state *s, int option)
 {
+  s->cnt_clean = false;
   switch (s->algo) {
   case GRD_PR: return reduce_t<OpPR>(s, option);
   case GRD_CC: return reduce_t<OpCC>(s, option);
@@ -1130,6 +1133,7 @@ static void launch_update(grd_state *s, int use_delta)
 grd_status op_update(grd_state *s)
 {
   grd_graph *g = s->g;
+  s->cnt_clean = false;
   switch (s->algo) {
   case GRD_PR: launch_update<GRD_PR>(s, 0); break;
   case GRD_CC: launch_update<GRD_CC>(s, 0); break;

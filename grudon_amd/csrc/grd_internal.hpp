@@ -363,7 +363,8 @@ struct grd_state {
   uint32_t n_ushare = 0, n_rshare = 0, n_sshare = 0;
   grd::Counters *hcnt = nullptr;  // pinned host (kHostCounters bytes)
   uint32_t cnt_seq = 0;           // sequence number of the last counters published
-  bool cnt_clean = false;         // the device counters are at their start
+  bool cnt_clean = false;         // the device counters and shares are at their start: set by what puts them
+                                  // there, cleared by every pass that writes one
   // snapshot copies
   grd::DevMem snap_mem;
   std::vector<std::pair<void *, void *>> snap;  // (live, copy)

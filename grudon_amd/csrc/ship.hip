@@ -230,6 +230,7 @@ static grd_status ship_t(grd_state *s)
 
 grd_status op_ship(grd_state *s)
 {
+  s->cnt_clean = false;
   switch (s->algo) {
   case GRD_PR: return ship_t<OpPR>(s);
   case GRD_CC: return ship_t<OpCC>(s);

@@ -64,3 +64,24 @@ def test_push_traversal_repeated(ctx, M, option):
     assert (np.abs(S.result() - want) <= (terms + 4) * 2.0 ** -24 * want).all()
     S.free()
     G.free()
+
+
+def test_reduce_after_the_update(ctx):
+    """A reduce that follows its superstep's update belongs to no superstep of
+    the run after it: the run's first one (an empty frontier) has sent nothing,
+    and the run ends with the oracle's labels."""
+    print("reduce after the update", flush=True)
+    g = O.rmat(10, 8, seed=5, symmetrize=True)
+    ref, _ = O.Partition(g, 1, 2).cc()
+    G = api.Graph.from_csr(ctx, g.rp, g.col, C=1, M=2)
+    S = api.State(G, api.CC)
+    S.init(sched=api.SCHED_FIXED, fixed_option=api.OPT_PUSH_SPARSE)
+    _call("grd_broadcast", S, api.OPT_PUSH_SPARSE)
+    _call("grd_traverse", S, api.OPT_PUSH_SPARSE)
+    assert S.step_update() == 0  # nothing has been reduced
+    _call("grd_reduce", S, api.OPT_PUSH_SPARSE)
+    _, trace = S.run(trace_cap=50)
+    assert trace[1].frontier == 0 and trace[1].dirty == 0
+    assert np.array_equal(S.result(), ref)
+    S.free()
+    G.free()
