@@ -133,8 +133,8 @@ static uint64_t bitvector_bytes(const grd_graph *g)
 }
 
 // after the iteration's counters are read: accumulate the dominant kernel's
-// event time and algorithmic bytes (frontier_k = vertices pushed)
-static grd_status finish_kernel_timing(grd_state *s, uint64_t frontier_k)
+// event time and algorithmic bytes
+static grd_status finish_kernel_timing(grd_state *s)
 {
   if (s->skip_pending) {
     // a CC / SSSP pull left out the blocks whose rows could not improve (their
@@ -156,7 +156,7 @@ static grd_status finish_kernel_timing(grd_state *s, uint64_t frontier_k)
   GRD_HIP(hipEventElapsedTime(&ms, s->kev[0], s->kev[1]));
   s->kern_ms += ms;
   s->kern_launches++;
-  if (s->kern_pending == 2) s->kern_bytes += 12 * s->last_frontier_edges + 16 * frontier_k;
+  if (s->kern_pending == 2) s->kern_bytes += 12 * s->al_edges + 16 * s->al_vertices;
   else s->kern_bytes += s->kern_pending_bytes;
   s->kern_pending = 0;
   return GRD_OK;
@@ -187,7 +187,7 @@ static grd_status superstep(grd_state *s, int option, bool select_next = false)
   } else {
     GRD_TRY(op_read_counters(s));
   }
-  GRD_TRY(finish_kernel_timing(s, s->last_frontier));
+  GRD_TRY(finish_kernel_timing(s));
   const Counters &c = *s->hcnt;
   const grd_graph *g = s->g;
   // reduce bytes (GraphAlgorithm.cpp:409-423): bitvector + dirty values
@@ -697,7 +697,7 @@ grd_status grd_update(grd_state *s, uint64_t *frontier_out)
   if (s->algo == GRD_PR_PULL) {
     GRD_TRY(prp_update(s));
     GRD_TRY(op_wait_counters(s));
-    GRD_TRY(finish_kernel_timing(s, 0));
+    GRD_TRY(finish_kernel_timing(s));
     s->iteration++;
     const bool conv = s->hcnt->residual < s->prm.tolerance;
     if (frontier_out) *frontier_out = conv ? 0 : s->g->n;
@@ -705,7 +705,7 @@ grd_status grd_update(grd_state *s, uint64_t *frontier_out)
   }
   GRD_TRY(op_update(s));
   GRD_TRY(op_read_counters(s));
-  GRD_TRY(finish_kernel_timing(s, s->last_frontier));
+  GRD_TRY(finish_kernel_timing(s));
   const Counters &c = *s->hcnt;
   if (s->last_option != GRD_OPT_SHIP_EDGES) {
     uint64_t vals = (s->last_option & 2) ? (uint64_t)s->g->n + s->g->X : c.dirty;
@@ -776,7 +776,7 @@ grd_status grd_run(grd_state *s, grd_run_stats *stats, grd_iter_rec *trace, uint
       GRD_TRY(prp_iteration(s));
       if (timing) GRD_HIP(hipEventRecord(ctx->ev[3], ctx->stream));
       GRD_TRY(op_wait_counters(s));
-      GRD_TRY(finish_kernel_timing(s, 0));
+      GRD_TRY(finish_kernel_timing(s));
       s->iteration++;
       st.residual = s->hcnt->residual;
       rec.option = GRD_OPT_PULL_DENSE;

@@ -994,6 +994,11 @@ grd_status op_broadcast(grd_state *s, int option)
   const bool pull = option & 1, dense = option & 2;
   const bool need_rank = !dense || !pull;
   s->cnt_clean = false;
+  if (!pull) {
+    s->al_vertices = s->last_frontier;
+    s->al_edges = s->last_frontier_edges;
+    s->al_maxdeg = s->last_maxdeg;
+  }
   s->xb_dense = dense ? 1 : 0;
   s->xr_dense = -1;
   if (need_rank) GRD_TRY(word_ranks(st, s->F, nwS, s->blk, s->wrankB, s->totals + 0));

@@ -341,6 +341,11 @@ struct grd_state {
   // scan scratch
   uint32_t *blk = nullptr, *wrankB = nullptr, *wrankR = nullptr, *totals = nullptr;
   uint32_t *AL = nullptr;
+  // the active list's vertices, their out-arcs and largest out-degree (the
+  // frontier's at the push broadcast that wrote it; an update moves the last_*
+  // ones on, and a traversal may still follow)
+  uint64_t al_vertices = 0, al_edges = 0;
+  uint32_t al_maxdeg = 0;
   uint2 *heavy = nullptr;  // push: (proxy, first arc offset) of each heavy-vertex chunk
   bool heavy_listed = false;  // a push has listed chunks since the counters were last at their start
   void *partial = nullptr;  // pull: one 8-byte partial per row block (long-row segments)

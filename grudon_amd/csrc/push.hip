@@ -158,21 +158,21 @@ static grd_status launch(grd_state *s, const uint32_t *col, const W *wt, typenam
   using V = typename Op::V;
   // tiles of 64 active vertices until those fill every workgroup slot
   const uint64_t slots = (uint64_t)ctx->num_cus * 8;
-  const uint32_t tile = s->last_frontier <= 64 * slots ? 64u : (uint32_t)kBlock;
-  const uint32_t grid = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((s->last_frontier + tile - 1) / tile, slots));
+  const uint32_t tile = s->al_vertices <= 64 * slots ? 64u : (uint32_t)kBlock;
+  const uint32_t grid = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((s->al_vertices + tile - 1) / tile, slots));
   // the heavy list holds one pass over the active list: another push of the same
   // broadcast lists its chunks anew
   if (s->heavy_listed) hipLaunchKernelGGL(k_heavy_restart, dim3(1), dim3(kWave), 0, st, s->cnt);
   s->heavy_listed = true;
   hipLaunchKernelGGL((k_push<Op, kShip, W>), dim3(grid), dim3(kBlock), 0, st, s->AL, s->totals + 0, g->rp, col, wt,
                      (const V *)s->mprop, upd, dirty, s->heavy, s->cnt, tile);
-  // a vertex's out-arcs all hang off its own proxy, so the frontier's largest
+  // a vertex's out-arcs all hang off its own proxy, so the list's largest
   // out-degree tells whether any chunk was appended
-  if (s->last_maxdeg >= kHeavyDeg)
+  if (s->al_maxdeg >= kHeavyDeg)
     hipLaunchKernelGGL((k_push_heavy<Op, kShip, W>), dim3((uint32_t)slots), dim3(kBlock), 0, st, s->heavy, s->cnt,
                        g->rp, col, wt, (const V *)s->mprop, upd, dirty);
   GRD_HIP(hipGetLastError());
-  s->edges += s->last_frontier_edges;  // every out-arc of the active list
+  s->edges += s->al_edges;  // every out-arc of the active list
   return GRD_OK;
 }
 

@@ -85,3 +85,26 @@ def test_reduce_after_the_update(ctx):
     assert np.array_equal(S.result(), ref)
     S.free()
     G.free()
+
+
+@pytest.mark.parametrize("M", [1, 3])
+@pytest.mark.parametrize("option", [api.OPT_PUSH_SPARSE, api.OPT_PUSH_DENSE])
+def test_push_traversal_after_the_update(ctx, M, option):
+    """A push traversal pushes the frontier that was broadcast, heavy vertices
+    included, also when an update has come between (and found nothing)."""
+    print("push traversal after the update", M, option, flush=True)
+    g = _graph(3001)
+    ref, st = O.Partition(g, 1, M).cc()
+    G = api.Graph.from_csr(ctx, g.rp, g.col, C=1, M=M)
+    S = api.State(G, api.CC)
+    S.init(sched=api.SCHED_FIXED, fixed_option=option)
+    _call("grd_broadcast", S, option)
+    assert S.step_update() == 0
+    _call("grd_traverse", S, option)
+    _call("grd_reduce", S, option)
+    S.step_update()
+    stats = S.run()
+    assert np.array_equal(S.result(), ref)
+    assert stats["iterations"] == int(st[0]) + 1 and stats["edges_examined"] == int(st[2])
+    S.free()
+    G.free()
