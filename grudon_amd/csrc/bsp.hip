@@ -785,11 +785,9 @@ Shares shares(const grd_state *s)
 
 grd_status op_zero_counters(grd_state *s)
 {
-  s->n_ushare = s->n_sshare = 0;
-  s->heavy_listed = false;
   hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(kBlock), 0, s->g->ctx->stream, s->cnt, shares(s));
   GRD_HIP(hipGetLastError());
-  s->cnt_clean = true;
+  counters_at_start(s);
   return GRD_OK;
 }
 
@@ -800,9 +798,7 @@ grd_status op_read_counters(grd_state *s)
   hipLaunchKernelGGL(k_publish, dim3(1), dim3(kBlock), 0, s->g->ctx->stream, s->cnt, shares(s), s->hcnt,
                      host_seq(s->hcnt), ++s->cnt_seq);
   GRD_HIP(hipGetLastError());
-  s->n_ushare = s->n_sshare = 0;
-  s->heavy_listed = false;
-  s->cnt_clean = true;
+  counters_at_start(s);
   return op_wait_counters(s);
 }
 

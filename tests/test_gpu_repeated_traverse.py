@@ -108,3 +108,37 @@ def test_push_traversal_after_the_update(ctx, M, option):
     assert stats["iterations"] == int(st[0]) + 1 and stats["edges_examined"] == int(st[2])
     S.free()
     G.free()
+
+
+@pytest.mark.parametrize("mode,tb", [(0, 0), (3, 4), (3, 8)])
+@pytest.mark.parametrize("option", [api.OPT_PULL_SPARSE, api.OPT_PULL_DENSE])
+@pytest.mark.parametrize("algo", ["cc", "hop", "weighted"])
+def test_pull_traversal_after_the_update(ctx, mode, tb, option, algo):
+    """A pull traversal pulls what was broadcast also when an update has come
+    between (and found nothing): in the first superstep and in the second,
+    which leaves out rows that cannot improve."""
+    print("pull traversal after the update", mode, tb, option, algo, flush=True)
+    g = O.rmat(12, 16, seed=5, symmetrize=True).with_weights(11)
+    P = O.Partition(g, 1, 2)
+    kw = {"cc": {}, "hop": {"source": 3}, "weighted": {"source": 3, "weighted": True}}[algo]
+    ref, st = P.cc() if algo == "cc" else P.sssp(3, weighted=algo == "weighted")
+    ctx.set_pull_tiling(mode, tb, 0)
+    try:
+        G = api.Graph.from_csr(ctx, g.rp, g.col, g.w, C=1, M=2)
+        for before in (0, 1):
+            S = api.State(G, api.CC if algo == "cc" else api.SSSP)
+            S.init(sched=api.SCHED_FIXED, fixed_option=option, **kw)
+            for _ in range(before):
+                S.step(option)
+            _call("grd_broadcast", S, option)
+            assert S.step_update() == 0
+            _call("grd_traverse", S, option)
+            _call("grd_reduce", S, option)
+            S.step_update()
+            stats = S.run()
+            assert np.array_equal(S.result(), ref)
+            assert stats["iterations"] == int(st[0]) + 1
+            S.free()
+        G.free()
+    finally:
+        ctx.set_pull_tiling(3, 0, 0)  # the default
