@@ -163,10 +163,29 @@ class Context:
         self.h = h
         self.device = device
         self._deps = []  # weak references to the graphs, states and batches made on it
+        # The handles not freed yet, oldest first: (free function, handle, the
+        # owner's entry).  The weak references find the Python objects; when
+        # those go with their owner in one reference cycle, the references are
+        # cleared before anything is finalized, in any order, and an owner that
+        # goes first frees by this list (the others then find theirs gone).
+        self._live = {}
+        self._entries = 0
         _LIVE_CONTEXTS.add(self)
 
-    def _track(self, obj):
+    def _track(self, obj, free, owner=None):
         self._deps.append(weakref.ref(obj))
+        self._entries += 1
+        self._live[self._entries] = (free, obj.h, owner)
+        return self._entries
+
+    def _release(self, entry):
+        free, h, _ = self._live.pop(entry, (None, None, None))
+        if free:
+            getattr(lib(), free)(h)
+
+    def _release_owned(self, owner):
+        for entry in [e for e, (_, _, o) in self._live.items() if o == owner]:
+            self._release(entry)
 
     def close(self):
         """Frees what is still alive on the context (newest first: states
@@ -177,6 +196,8 @@ class Context:
                 if obj is not None:
                     obj.free()
             self._deps = []
+            for entry in sorted(self._live, reverse=True):
+                self._release(entry)
             lib().grd_destroy(self.h)
             self.h = None
 
@@ -268,7 +289,7 @@ class Graph:
         self.ctx = ctx
         self.h = h
         self._states = []  # weak references: a graph frees its states first
-        ctx._track(self)
+        self._entry = ctx._track(self, "grd_graph_free")
         info = np.zeros(16, dtype=np.uint64)
         _check(lib().grd_graph_info(self.h, _ptr(info)), "grd_graph_info")
         self.n, self.m, self.C, self.M = int(info[0]), int(info[1]), int(info[2]), int(info[3])
@@ -345,7 +366,8 @@ class Graph:
                 if st is not None:
                     st.free()
             self._states = []
-            lib().grd_graph_free(self.h)
+            self.ctx._release_owned(self._entry)
+            self.ctx._release(self._entry)
             self.h = None
 
     def __del__(self):
@@ -366,7 +388,7 @@ class State:
         _check(lib().grd_state_create_typed(graph.h, algo, value_bytes, ct.byref(h)), "grd_state_create")
         self.h = h
         graph._states.append(weakref.ref(self))
-        graph.ctx._track(self)
+        self._entry = graph.ctx._track(self, "grd_state_free", graph._entry)
 
     def _vdtype(self):
         if self.algo in (PR, PR_PULL):
@@ -439,7 +461,7 @@ class State:
 
     def free(self):
         if self.h:
-            lib().grd_state_free(self.h)
+            self.graph.ctx._release(self._entry)
             self.h = None
 
     def __del__(self):
@@ -467,7 +489,7 @@ class Batch:
         _check(lib().grd_batch_create(ctx.h, cnt, _ptr(self.n), _ptr(self.m), rps, cols, ct.byref(h)),
                "grd_batch_create")
         self.h = h
-        ctx._track(self)
+        self._entry = ctx._track(self, "grd_batch_free")
         self.count = cnt
 
     def tune(self, tile=0, grid_per_cu=0, K=0):
@@ -498,7 +520,7 @@ class Batch:
 
     def free(self):
         if self.h:
-            lib().grd_batch_free(self.h)
+            self.ctx._release(self._entry)
             self.h = None
 
     def __del__(self):
