@@ -194,6 +194,10 @@ static grd_status ship_t(grd_state *s)
   hipStream_t st = g->ctx->stream;
   const uint64_t k = s->last_frontier, E = s->last_frontier_edges;
   if (k == 0) return GRD_OK;
+  // (an update since the broadcast: what was checked for coverage and is sized
+  // here is not what the list holds)
+  if (s->al_vertices != k || s->al_edges != E)
+    return fail(GRD_ERR_STATE, "edge shipping: the active list differs from the frontier");
   const uint64_t total = k + E;
   // the records' entries (a source each, and its out-neighbours) are counted in 32 bits
   if (total > 0xFFFFFFFFull - 1024) return fail(GRD_ERR_ARG, "edge shipping: the wire would exceed 2^32 entries");

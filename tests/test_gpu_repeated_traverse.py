@@ -142,3 +142,28 @@ def test_pull_traversal_after_the_update(ctx, mode, tb, option, algo):
         G.free()
     finally:
         ctx.set_pull_tiling(3, 0, 0)  # the default
+
+
+@pytest.mark.parametrize("C", [1, 2])
+def test_shipping_a_stale_list_is_refused(ctx, C):
+    """Edge shipping after an update, whose frontier is another one than the
+    list that was broadcast, is refused, and the state goes on as if it had not
+    been called."""
+    print("stale shipping", C, flush=True)
+    # even and odd vertices apart, so that two compute partitions cover theirs
+    v = np.arange(2000)
+    g = O.from_edges(2000, [(int(a), int(b)) for a in v for b in ((a + 2) % 2000, a // 4 * 2 + a % 2) if a != b])
+    ref, st = O.Partition(g, C, 2).cc()
+    G = api.Graph.from_csr(ctx, g.rp, g.col, C=C, M=2)
+    assert G.coverage()[1] == 0
+    S = api.State(G, api.CC)
+    S.init(sched=api.SCHED_FIXED, fixed_option=api.OPT_SHIP_EDGES)
+    left = S.step(api.OPT_SHIP_EDGES)
+    assert 0 < left < 2000
+    with pytest.raises(api.GrdError):
+        _call("grd_traverse", S, api.OPT_SHIP_EDGES)
+        S.step_update()
+    stats = S.run()
+    assert np.array_equal(S.result(), ref) and stats["iterations"] == int(st[0])
+    S.free()
+    G.free()
