@@ -1010,7 +1010,7 @@ grd_status grd_snapshot(grd_state *s)
   s->snap_iteration = s->iteration;
   s->snap_hi = s->hi;
   s->snap_host = {s->last_frontier, s->prev_frontier, s->last_frontier_edges, s->last_dirty, s->last_maxdeg,
-                  s->last_uncovered, s->bytes, s->edges};
+                  s->last_uncovered, s->bytes, s->edges, s->n_sshare, s->skip_pending};
   memcpy(s->snap_fpart, s->last_fpart, sizeof(s->snap_fpart));
   return GRD_OK;
 }
@@ -1035,6 +1035,8 @@ grd_status grd_restore(grd_state *s)
   s->last_uncovered = s->snap_host[5];
   s->bytes = s->snap_host[6];
   s->edges = s->snap_host[7];
+  s->n_sshare = (uint32_t)s->snap_host[8];
+  s->skip_pending = s->snap_host[9] != 0;
   memcpy(s->last_fpart, s->snap_fpart, sizeof(s->snap_fpart));
   // the counters restored with the device arrays (the pull PageRank's FP64
   // dangling mass and residual live there) are the host's copy too

@@ -867,10 +867,15 @@ grd_status state_alloc(grd_state *s)
     GRD_TRY(m.alloc_n(&s->bskip, std::max<uint32_t>(nblk, 1)));
     if (bsp_hot_cold(s)) GRD_TRY(m.alloc_n(&s->hskip, std::max<uint32_t>(g->n_tblk, 1)));
   }
-  GRD_TRY(m.alloc_n(&s->cnt, 1));
-  GRD_TRY(m.alloc_n(&s->ushare, loop_blocks(g->ctx)));
-  GRD_TRY(m.alloc_n(&s->rshare, loop_blocks(g->ctx)));
-  GRD_TRY(m.alloc_n(&s->sshare, 2 * loop_blocks(g->ctx)));
+  // the counters and the shares that wait for the next publishing are one
+  // piece, so that a snapshot within a superstep holds both in one copy
+  const uint64_t lb = loop_blocks(g->ctx);
+  const uint64_t cnt_bytes = sizeof(Counters) + 2 * lb * sizeof(SkipShare) + lb * sizeof(uint32_t);
+  static_assert(sizeof(Counters) % 8 == 0 && sizeof(SkipShare) % 8 == 0, "the shares are aligned");
+  GRD_TRY(m.alloc(reinterpret_cast<void **>(&s->cnt), cnt_bytes));
+  s->sshare = reinterpret_cast<SkipShare *>(s->cnt + 1);
+  s->rshare = reinterpret_cast<uint32_t *>(s->sshare + 2 * lb);
+  GRD_TRY(m.alloc_n(&s->ushare, lb));
   s->n_rshare = loop_grid(g->ctx, nwP, narrow_groups(g->ctx, nwP) ? kGroupNarrow : kGroupWide);
   GRD_TRY(host_counters_take(g->ctx, &s->hcnt));
   // snapshot list: every array whose content carries state between iterations
@@ -885,7 +890,7 @@ grd_status state_alloc(grd_state *s)
   // the counters carry the pull PageRank's FP64 dangling mass of the next
   // update (ping-pong by iteration parity) and the last residual
   s->snap.push_back({s->cnt, nullptr});
-  s->snap_bytes.push_back(sizeof(Counters));
+  s->snap_bytes.push_back(cnt_bytes);
   return GRD_OK;
 }
 

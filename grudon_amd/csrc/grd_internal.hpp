@@ -361,7 +361,7 @@ struct grd_state {
   // partition and frontier vertices not covered
   uint64_t last_fpart[grd::kMaxParts] = {};
   uint64_t last_uncovered = 0;
-  grd::Counters *cnt = nullptr;   // device
+  grd::Counters *cnt = nullptr;   // device, with sshare and rshare behind it
   grd::BlockShare *ushare = nullptr;  // [loop_blocks] of the last update / selection
   uint32_t *rshare = nullptr;         // [loop_blocks] dirty proxies, zero after each publishing
   grd::SkipShare *sshare = nullptr;   // [2 * loop_blocks] row blocks left out by the last pull: cold, then hot
@@ -376,7 +376,7 @@ struct grd_state {
   std::vector<uint64_t> snap_bytes;
   uint32_t snap_iteration = 0;
   uint64_t snap_hi = 0;
-  std::array<uint64_t, 8> snap_host{};  // frontier statistics, bytes and edges at the snapshot
+  std::array<uint64_t, 10> snap_host{};  // frontier statistics, bytes, edges and the pull's shares at the snapshot
   uint64_t snap_fpart[grd::kMaxParts] = {};
 };
 

@@ -1,0 +1,53 @@
+"""Counts of a superstep taken apart: what a snapshot within a superstep, a
+repeated pull traversal and an earlier state on the same context leave in the
+statistics (edges, exchanged bytes, features, residual)."""
+import ctypes as ct
+
+import numpy as np
+import pytest
+
+import oracle_lib as O
+from grudon_amd import api
+
+pytestmark = pytest.mark.gpu
+
+
+def _call(name, S, *args):
+    api._check(getattr(api.lib(), name)(S.h, *args), name)
+
+
+def _stats(S):
+    st = api.RunStats()
+    _call("grd_state_stats", S, ct.byref(st))
+    return st.as_dict()
+
+
+def _graph():
+    return O.rmat(12, 16, seed=5, symmetrize=True)
+
+
+@pytest.mark.parametrize("option", [api.OPT_PUSH_SPARSE, api.OPT_PULL_SPARSE])
+def test_snapshot_between_reduce_and_update(ctx, option):
+    """An update after the restore counts what the first one counted: the dirty
+    proxies (a feature, and the bytes of a sparse reduce) and the arcs left out."""
+    print("snapshot between reduce and update", option, flush=True)
+    g = _graph()
+    G = api.Graph.from_csr(ctx, g.rp, g.col, C=1, M=2)
+    S = api.State(G, api.CC)
+    S.init()
+    S.step(option)
+    for name in ("grd_broadcast", "grd_traverse", "grd_reduce"):
+        _call(name, S, option)
+    S.snapshot()
+    left = S.step_update()
+    want, feat = _stats(S), S.features()
+    assert feat[4] > 0  # dirty proxies
+    for _ in range(2):
+        S.restore()
+        assert S.step_update() == left
+        got = _stats(S)
+        assert [got[k] for k in ("bytes_exchanged", "edges_examined")] == \
+               [want[k] for k in ("bytes_exchanged", "edges_examined")]
+        assert np.array_equal(S.features(), feat)
+    S.free()
+    G.free()
