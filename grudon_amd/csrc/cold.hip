@@ -218,7 +218,7 @@ __global__ void __launch_bounds__(kBlock) k_row_blocks_done(uint32_t nblk, const
                                                              const uint64_t *__restrict__ done,
                                                              const uint64_t *__restrict__ hasarc,
                                                              uint8_t *__restrict__ bskip,
-                                                             SkipShare *__restrict__ share)
+                                                             SkipShare *__restrict__ share, bool again)
 {
   unsigned long long arcs = 0, rows = 0;
   const uint32_t lane = lane_id();
@@ -245,7 +245,7 @@ __global__ void __launch_bounds__(kBlock) k_row_blocks_done(uint32_t nblk, const
   }
   arcs = block_sum(arcs);
   rows = block_sum(rows);
-  if (threadIdx.x == 0) share[blockIdx.x] = SkipShare{arcs, 0, rows};
+  if (threadIdx.x == 0) add_share(share + blockIdx.x, SkipShare{arcs, 0, rows}, again);
 }
 
 }  // namespace
@@ -345,13 +345,13 @@ template grd_status bsp_pull_cold<OpHop>(grd_state *, const uint8_t *, const Cou
 template grd_status bsp_pull_cold<OpWeighted>(grd_state *, const uint8_t *, const Counters *);
 template grd_status bsp_pull_cold<OpPR>(grd_state *, const uint8_t *, const Counters *);
 
-grd_status row_blocks_done(grd_state *s, uint32_t nblk, const PullBlock *blocks)
+grd_status row_blocks_done(grd_state *s, uint32_t nblk, const PullBlock *blocks, bool again)
 {
   grd_graph *g = s->g;
   if (nblk) {
     const uint32_t grid = std::min<uint32_t>((nblk + kWavesPerBlock - 1) / kWavesPerBlock, loop_blocks(g->ctx));
     hipLaunchKernelGGL(k_row_blocks_done, dim3(grid), dim3(kBlock), 0, g->ctx->stream, nblk, blocks,
-                       (const uint64_t *)s->Rdone, (const uint64_t *)g->rarc, s->bskip, s->sshare + s->n_sshare);
+                       (const uint64_t *)s->Rdone, (const uint64_t *)g->rarc, s->bskip, s->sshare + s->n_sshare, again);
     s->n_sshare += grid;
   }
   GRD_HIP(hipGetLastError());

@@ -456,7 +456,8 @@ grd_status prp_pull_rows_fixup(hipStream_t st, const PullLong *longs, uint32_t n
 uint32_t cold_set(const grd_graph *g, int algo, uint32_t *nnz);  // which cold set an algorithm pulls over
 grd_status cold_sort(grd_graph *g, const ColdSet &c);  // the cold blocks' arcs into source order
 grd_status prp_pull_cold(grd_state *s, float *out, const float *pre);
-grd_status row_blocks_done(grd_state *s, uint32_t nblk, const PullBlock *blocks);  // flags of the row blocks
+// flags of the row blocks and the arcs and rows left out (again: added to the shares that are there)
+grd_status row_blocks_done(grd_state *s, uint32_t nblk, const PullBlock *blocks, bool again);
 // tiers.hip
 grd_status build_tiers(grd_graph *g);
 grd_status build_cold(grd_graph *g, int algo, const ColdSet **out);  // mode 3: the algorithm's cold set

@@ -257,6 +257,17 @@ __device__ __forceinline__ void zero_counters(Counters *cnt, const Shares &sh)
   for (uint32_t b = threadIdx.x; b < sh.nr; b += kBlock) sh.r[b] = 0;
 }
 
+// a workgroup's share of what a pull leaves out
+__device__ __forceinline__ void add_share(SkipShare *p, SkipShare x, bool again)
+{
+  if (again) {
+    x.arcs += p->arcs;
+    x.hot_arcs += p->hot_arcs;
+    x.rows += p->rows;
+  }
+  *p = x;
+}
+
 // the sums of the blocks' shares, in every thread
 struct FrontierCounts {
   unsigned long long frontier, edges, dirty, skipped, skipped_hot, skipped_rows;

@@ -180,7 +180,7 @@ __global__ void __launch_bounds__(kBlock) k_hot_blocks_done(uint32_t nblk, const
                                                             const uint64_t *__restrict__ done,
                                                             const uint64_t *__restrict__ hasarc,
                                                             uint8_t *__restrict__ bskip,
-                                                            SkipShare *__restrict__ share)
+                                                            SkipShare *__restrict__ share, bool again)
 {
   unsigned long long arcs = 0;
   for (uint32_t b = blockIdx.x * kBlock + threadIdx.x; b < nblk; b += gridDim.x * kBlock) {
@@ -203,7 +203,8 @@ __global__ void __launch_bounds__(kBlock) k_hot_blocks_done(uint32_t nblk, const
     if (all) arcs += d.e1 - d.e0;
   }
   arcs = block_sum(arcs);
-  if (threadIdx.x == 0) share[blockIdx.x] = SkipShare{0, arcs, 0};  // (its rows are counted with the cold ones)
+  // (its rows are counted with the cold ones)
+  if (threadIdx.x == 0) add_share(share + blockIdx.x, SkipShare{0, arcs, 0}, again);
 }
 
 // Measurement only (time_kernel): the arcs, in the row-block pull's CSC (rp:
@@ -425,6 +426,9 @@ static grd_status blocks_done(grd_state *s, bool cold, const uint8_t **flags)
 {
   *flags = nullptr;
   s->hskip_on = false;
+  // another pull of the same broadcast runs the same grids: it adds to the
+  // shares of the one before
+  const bool again = s->n_sshare != 0;
   s->n_sshare = 0;
   if (!Op::kMin || !s->bound_sent) return GRD_OK;
   s->skip_pending = true;  // the rows that gathered nothing come off with the counters
@@ -441,11 +445,12 @@ static grd_status blocks_done(grd_state *s, bool cold, const uint8_t **flags)
                                                                    (uint32_t)g->ctx->num_cus * 8)),
                          dim3(kBlock), 0, st, nwP, g->crp, g->rarc);
   }
-  GRD_TRY(cold ? row_blocks_done(s, s->cold->nblk, s->cold->blk) : row_blocks_done(s, g->n_pblk, g->pblk));
+  GRD_TRY(cold ? row_blocks_done(s, s->cold->nblk, s->cold->blk, again)
+               : row_blocks_done(s, g->n_pblk, g->pblk, again));
   if (cold && g->n_tblk && s->hskip) {
     const uint32_t grid = std::min<uint32_t>((g->n_tblk + kBlock - 1) / kBlock, loop_blocks(g->ctx));
     hipLaunchKernelGGL(k_hot_blocks_done, dim3(grid), dim3(kBlock), 0, st, g->n_tblk, g->tblk,
-                       (const uint64_t *)s->Rdone, (const uint64_t *)g->rarc, s->hskip, s->sshare + s->n_sshare);
+                       (const uint64_t *)s->Rdone, (const uint64_t *)g->rarc, s->hskip, s->sshare + s->n_sshare, again);
     s->n_sshare += grid;
     s->hskip_on = true;
   }

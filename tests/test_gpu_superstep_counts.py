@@ -51,3 +51,32 @@ def test_snapshot_between_reduce_and_update(ctx, option):
         assert np.array_equal(S.features(), feat)
     S.free()
     G.free()
+
+
+@pytest.mark.parametrize("mode,tb", [(0, 0), (3, 4)])
+def test_repeated_pull_counts_twice(ctx, mode, tb):
+    """Two pull traversals of one broadcast examine twice the arcs of one, less
+    twice those that were left out."""
+    print("repeated pull", mode, tb, flush=True)
+    g = _graph()
+    ctx.set_pull_tiling(mode, tb, 0)
+    try:
+        G = api.Graph.from_csr(ctx, g.rp, g.col, C=1, M=2)
+        S = api.State(G, api.CC)
+        edges = []
+        for times in (1, 2, 3):
+            S.init()
+            S.step(api.OPT_PULL_DENSE)
+            before = _stats(S)["edges_examined"]
+            _call("grd_broadcast", S, api.OPT_PULL_DENSE)
+            for _ in range(times):
+                _call("grd_traverse", S, api.OPT_PULL_DENSE)
+            _call("grd_reduce", S, api.OPT_PULL_DENSE)
+            S.step_update()
+            edges.append(_stats(S)["edges_examined"] - before)
+        assert 0 < edges[0] < g.m  # some arcs were left out
+        assert edges[1:] == [2 * edges[0], 3 * edges[0]]
+        S.free()
+        G.free()
+    finally:
+        ctx.set_pull_tiling(3, 0, 0)  # the default
