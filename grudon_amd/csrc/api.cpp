@@ -894,7 +894,8 @@ grd_status grd_state_stats(const grd_state *s, grd_run_stats *out)
   out->iterations = s->iteration;
   out->bytes_exchanged = s->bytes;
   out->edges_examined = s->edges;
-  out->residual = s->hcnt ? s->hcnt->residual : 0.0;
+  // (the other algorithms never write it)
+  out->residual = s->algo == GRD_PR_PULL && s->hcnt ? s->hcnt->residual : 0.0;
   out->kernel_ms = s->kern_ms;
   out->kernel_launches = s->kern_launches;
   out->kernel_bytes = s->kern_bytes;

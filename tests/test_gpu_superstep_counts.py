@@ -80,3 +80,23 @@ def test_repeated_pull_counts_twice(ctx, mode, tb):
         G.free()
     finally:
         ctx.set_pull_tiling(3, 0, 0)  # the default
+
+
+def test_residual_is_pull_pageranks(ctx):
+    """The residual of another state, whose memory a new one got, is not the new
+    one's: an algorithm without a residual reports none."""
+    print("residual", flush=True)
+    g = _graph()
+    G = api.Graph.from_csr(ctx, g.rp, g.col, C=1, M=2)
+    for algo in (api.CC, api.PR, api.SSSP):
+        S = api.State(G, api.PR_PULL)
+        S.init(max_iter=2)
+        S.run()
+        assert _stats(S)["residual"] > 0
+        S.free()
+        S = api.State(G, algo)
+        S.init(max_iter=2)
+        S.run()
+        assert _stats(S)["residual"] == 0
+        S.free()
+    G.free()
