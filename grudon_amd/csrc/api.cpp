@@ -553,7 +553,7 @@ static bool small_graph_pull(const grd_graph *g, int algo)
   const grd_ctx *ctx = g->ctx;
   if (ctx->pull_mode != 3 || ctx->tier_bits != 0) return false;
   // (a graph keeps a regrouping that was asked for)
-  if (g->tiers_built && (g->tier_mode != 3 || g->tier_bits != kTierBitsMax)) return false;
+  if (g->tiers_built && (g->tier_mode != 3 || g->tier_asked)) return false;
   constexpr uint64_t kSums = 6ull << 20, kMost = 16ull << 20;
   switch (algo) {
   case GRD_PR: return g->m <= kSums;

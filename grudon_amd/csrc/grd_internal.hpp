@@ -262,6 +262,7 @@ struct grd_graph {
   bool tiers_built = false;
   int tier_mode = 0;               // 1 LDS-tiled (16-bit offsets, tiles), 2 L2-segmented (32-bit sources)
   uint32_t tier_bits = 0;          // a tier is 2^tier_bits consecutive proxies of a partition
+  bool tier_asked = false;         // mode 3: the window was given, not the default
   uint32_t tile_arcs = 0;
   uint64_t n_pairs = 0;
   uint16_t *tcol = nullptr;        // [m] mode 1: source offset within the pair's tier window

@@ -917,6 +917,7 @@ static grd_status build_hotcold(grd_graph *g)
   g->n_pairs = P;
   g->tier_mode = 3;
   g->tier_bits = tb;
+  g->tier_asked = ctx->tier_bits != 0;
   g->tile_arcs = 0;
   g->tiers_built = true;
   return GRD_OK;

@@ -162,7 +162,8 @@ grd_status grd_set_layout(grd_ctx *ctx, int on_device);
  *     source order, that partial first (tile_arcs must be 0); the
  *     default, and the fastest measured on large graphs; with tier_bits 0
  *     small ones (up to some millions of arcs) are pulled as by mode 0, which
- *     is the faster there.  Mode 3 also serves the pull
+ *     is the faster there, unless the graph was split with a window that was
+ *     given.  Mode 3 also serves the pull
  *     supersteps of CC, SSSP and reference PageRank (states of any algorithm
  *     created afterwards); modes 1 and 2 serve GRD_PR_PULL only.
  * Modes 1-3 regroup a graph when its first pull-PageRank state is created,
