@@ -24,7 +24,7 @@ SELECTOR_MARGIN = 1.0  # GRD_SELECTOR_MARGIN of include/grudon_hip.h: the packag
 
 # every extern "C" symbol declared in include/grudon_hip.h
 EXPORTS = [
-    "grd_last_error", "grd_create", "grd_destroy", "grd_set_host_threads", "grd_set_layout", "grd_set_pull_tiling", "grd_graph_digest",
+    "grd_last_error", "grd_create", "grd_destroy", "grd_trim", "grd_set_host_threads", "grd_set_layout", "grd_set_pull_tiling", "grd_graph_digest",
     "grd_generate_rmat", "grd_generate_er", "grd_edge_weights", "grd_graph_from_csr", "grd_graph_rmat",
     "grd_graph_er", "grd_graph_load", "grd_graph_read", "grd_graph_write_gr", "grd_graph_free", "grd_graph_info",
     "grd_graph_table", "grd_graph_out_degree", "grd_graph_coverage",
@@ -83,7 +83,8 @@ def lib():
         vp = ct.c_void_p
         pp = ct.POINTER(ct.c_void_p)
         sigs = {
-            "grd_create": [ct.c_int, pp], "grd_destroy": [vp], "grd_set_host_threads": [vp, ct.c_int],
+            "grd_create": [ct.c_int, pp], "grd_destroy": [vp], "grd_trim": [vp],
+            "grd_set_host_threads": [vp, ct.c_int],
             "grd_set_layout": [vp, ct.c_int], "grd_graph_digest": [vp, vp],
             "grd_set_pull_tiling": [vp, ct.c_int, ct.c_uint32, ct.c_uint32],
             "grd_generate_rmat": [vp, ct.c_int, ct.c_int, ct.c_double, ct.c_double, ct.c_double, ct.c_uint64,
@@ -209,6 +210,10 @@ class Context:
 
     def set_host_threads(self, n):
         _check(lib().grd_set_host_threads(self.h, n), "grd_set_host_threads")
+
+    def trim(self):
+        """Gives back the device memory kept from freed graphs and states."""
+        _check(lib().grd_trim(self.h), "grd_trim")
 
     def set_pull_tiling(self, mode=3, tier_bits=0, tile_arcs=0):
         """How states created afterwards pull: 0 the row-block pull, 1 LDS

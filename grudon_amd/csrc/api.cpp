@@ -274,6 +274,7 @@ grd_status grd_create(int device, grd_ctx **out)
     c->num_cus = cus;
   // the allocation-free selector entry point's scratch on this device
   grd_status sst = mlp_scratch_init(device);
+  if (sst == GRD_OK) sst = workspace_open(c);
   if (sst != GRD_OK) {
     for (auto &ev : c->ev)
       if (ev) (void)hipEventDestroy(ev);
@@ -299,6 +300,14 @@ grd_status grd_destroy(grd_ctx *c)
   workspace_release(c);
   (void)hipStreamDestroy(c->stream);
   delete c;
+  return GRD_OK;
+}
+
+grd_status grd_trim(grd_ctx *c)
+{
+  if (!c) return fail(GRD_ERR_ARG, "grd_trim: NULL context");
+  GRD_HIP(hipSetDevice(c->device));
+  c->cache.trim();
   return GRD_OK;
 }
 

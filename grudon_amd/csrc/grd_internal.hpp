@@ -60,8 +60,8 @@ constexpr uint32_t kNone = 0xFFFFFFFFu;
 inline uint64_t pad64(uint64_t x) { return (x + 63) & ~uint64_t(63); }
 
 // Freed device blocks a context keeps for its next allocations (workspace.cpp):
-// at most kMaxHeld bytes, given back when the context goes or when an
-// allocation would fail.
+// at most kMaxHeld bytes, given back by grd_trim, when the context goes, or
+// when an allocation on its device would fail.
 struct BlockCache {
   static constexpr uint64_t kMaxHeld = 4ull << 30, kMaxBlock = 1ull << 30;
   std::mutex mu;
@@ -73,7 +73,7 @@ struct BlockCache {
 };
 
 // Device allocation list owned by a graph or a state, from its context's
-// cache.  A block's users are ordered on the context's stream; release() waits
+// cache (ctx is set before the first allocation).  A block's users are ordered on the context's stream; release() waits
 // for that stream before the blocks can be taken again.
 struct DevMem {
   grd_ctx *ctx = nullptr;
@@ -383,7 +383,10 @@ struct grd_state {
 
 namespace grd {
 // workspace.cpp
+grd_status workspace_open(grd_ctx *ctx);
 void workspace_release(grd_ctx *ctx);
+// hipMalloc on the current device, `device`, after what the contexts keep there if need be
+grd_status device_malloc(int device, void **p, uint64_t bytes);
 // until a kernel has stored `want` to a pinned word
 grd_status wait_pinned(grd_ctx *ctx, const uint32_t *word, uint32_t want);
 grd_status host_counters_take(grd_ctx *ctx, Counters **out);

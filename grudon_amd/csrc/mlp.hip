@@ -542,7 +542,7 @@ __global__ void __launch_bounds__(kBlock) k_mlp_publish(const uint16_t *__restri
 static grd_status sel_buffers(grd_ctx *ctx)
 {
   if (!ctx->sel_out) {
-    GRD_HIP(hipMalloc((void **)&ctx->sel_out, 32 * sizeof(float)));
+    GRD_TRY(device_malloc(ctx->device, (void **)&ctx->sel_out, 32 * sizeof(float)));
     GRD_HIP(hipHostMalloc((void **)&ctx->sel_out_host, 32 * sizeof(float), hipHostMallocDefault));
   }
   return GRD_OK;
@@ -612,7 +612,7 @@ grd_status grd_selector_load(grd_ctx *ctx, const uint16_t *w, uint64_t count, fl
   if (count != (uint64_t)kParams)
     return fail(GRD_ERR_ARG, "grd_selector_load: expected " + std::to_string(kParams) + " BF16 weights");
   GRD_HIP(hipSetDevice(ctx->device));
-  if (!ctx->sel_w) GRD_HIP(hipMalloc((void **)&ctx->sel_w, kParams * sizeof(uint16_t)));
+  if (!ctx->sel_w) GRD_TRY(device_malloc(ctx->device, (void **)&ctx->sel_w, kParams * sizeof(uint16_t)));
   GRD_HIP(hipMemcpy(ctx->sel_w, w, kParams * sizeof(uint16_t), hipMemcpyHostToDevice));
   GRD_TRY(infer_stage(ctx));
   ctx->sel_loaded = true;

@@ -12,6 +12,8 @@
 #include <atomic>
 #include <chrono>
 #include <cstring>
+#include <mutex>
+#include <new>
 #include <thread>
 #include <vector>
 
@@ -63,29 +65,53 @@ void BlockCache::trim()
   held = 0;
 }
 
+// The process's contexts: what they keep goes back before an allocation on
+// their device may fail (the blocks kept are idle, and a cache has its lock).
+static std::mutex g_contexts_mu;
+static std::vector<grd_ctx *> &contexts()
+{
+  static std::vector<grd_ctx *> *v = new std::vector<grd_ctx *>();  // (outlives every context)
+  return *v;
+}
+
+grd_status workspace_open(grd_ctx *ctx)
+{
+  std::lock_guard<std::mutex> lock(g_contexts_mu);
+  try {
+    contexts().push_back(ctx);
+  } catch (const std::bad_alloc &) {
+    return fail(GRD_ERR_OOM, "grd_create: host allocation failed");
+  }
+  return GRD_OK;
+}
+
+grd_status device_malloc(int device, void **p, uint64_t bytes)
+{
+  hipError_t e = hipMalloc(p, bytes);
+  if (e != hipSuccess) {
+    (void)hipGetLastError();
+    {
+      std::lock_guard<std::mutex> lock(g_contexts_mu);
+      for (grd_ctx *c : contexts())
+        if (c->device == device) c->cache.trim();
+    }
+    e = hipMalloc(p, bytes);
+  }
+  if (e != hipSuccess) {
+    *p = nullptr;
+    (void)hipGetLastError();
+    return fail(GRD_ERR_OOM, "hipMalloc(" + std::to_string(bytes) + " bytes) failed: " + hipGetErrorString(e));
+  }
+  return GRD_OK;
+}
+
 grd_status DevMem::alloc(void **p, uint64_t nbytes)
 {
   *p = nullptr;
   const uint64_t b = nbytes ? nbytes : 64;
-  uint64_t size = b;
-  if (ctx) {
-    size = block_size(b);
-    *p = ctx->cache.take(size, &size);
-  }
-  if (!*p) {
-    hipError_t e = hipMalloc(p, size);
-    if (e != hipSuccess && ctx) {
-      // the cache gives everything back before an allocation may fail
-      (void)hipGetLastError();
-      ctx->cache.trim();
-      e = hipMalloc(p, size);
-    }
-    if (e != hipSuccess) {
-      *p = nullptr;
-      (void)hipGetLastError();
-      return fail(GRD_ERR_OOM, "hipMalloc(" + std::to_string(size) + " bytes) failed: " + hipGetErrorString(e));
-    }
-  }
+  uint64_t size = block_size(b);
+  *p = ctx->cache.take(size, &size);
+  if (!*p) GRD_TRY(device_malloc(ctx->device, p, size));
   ptrs.emplace_back(*p, size);
   bytes += b;
   return GRD_OK;
@@ -94,9 +120,9 @@ grd_status DevMem::alloc(void **p, uint64_t nbytes)
 void DevMem::release()
 {
   // as hipFree does, wait for what may still use the blocks
-  if (ctx && !ptrs.empty()) (void)hipStreamSynchronize(ctx->stream);
+  if (!ptrs.empty()) (void)hipStreamSynchronize(ctx->stream);
   for (auto &b : ptrs)
-    if (!ctx || !ctx->cache.give(b.first, b.second)) (void)hipFree(b.first);
+    if (!ctx->cache.give(b.first, b.second)) (void)hipFree(b.first);
   ptrs.clear();
   bytes = 0;
 }
@@ -133,6 +159,11 @@ static grd_status stage_ring(grd_ctx *ctx)
 
 void workspace_release(grd_ctx *ctx)
 {
+  {
+    std::lock_guard<std::mutex> lock(g_contexts_mu);
+    auto &v = contexts();
+    v.erase(std::remove(v.begin(), v.end(), ctx), v.end());
+  }
   ctx->cache.trim();
   if (ctx->stage) (void)hipHostFree(ctx->stage);
   if (ctx->stage_small) (void)hipHostFree(ctx->stage_small);

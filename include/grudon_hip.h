@@ -139,6 +139,12 @@ typedef struct {
 const char *grd_last_error(void);
 grd_status grd_create(int device, grd_ctx **out);
 grd_status grd_destroy(grd_ctx *ctx);
+/* A context keeps device memory that its graphs, states and batches have freed
+ * for its next allocations: blocks of up to 1 GiB, 4 GiB in all.  They go back
+ * to the device with grd_destroy, when an allocation of this library on the
+ * same device would otherwise fail, or with this call (for another library in
+ * the process that needs the memory). */
+grd_status grd_trim(grd_ctx *ctx);
 /* Host threads used for graph construction (reference -t, src/main.cpp:25). */
 grd_status grd_set_host_threads(grd_ctx *ctx, int nthreads);
 /* Where the partitioned layout (DistributedGraph ctor,

@@ -1,0 +1,124 @@
+"""What the library's host code does with device memory, on a HIP runtime that
+has none (fake_hip.cpp, built with g++): each script runs in a process of its
+own, with the fake loaded first (no GPU)."""
+import os
+import shutil
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
+
+PRELUDE = r"""
+import ctypes as ct, os, sys
+fake = ct.CDLL(sys.argv[1], mode=os.RTLD_NOW | ct.RTLD_GLOBAL)
+fake.fake_live.restype = fake.fake_launches.restype = fake.fake_bad_frees.restype = ct.c_uint64
+fake.fake_limit.argtypes = [ct.c_uint64]
+sys.path[:0] = [sys.argv[2], os.path.join(sys.argv[2], "tests")]
+import numpy as np
+from grudon_amd import api
+live, limit, UNLIMITED = fake.fake_live, fake.fake_limit, 2 ** 64 - 1
+
+
+def ring(n, k=8):
+    rp = np.arange(n + 1) * k
+    col = (np.repeat(np.arange(n), k) + np.tile(np.arange(1, k + 1), n)) % n
+    return rp.astype(np.uint32), col.astype(np.uint32)
+
+
+def context():
+    ctx = api.Context(0)
+    ctx.set_layout(False)  # (kernels do nothing here)
+    return ctx
+
+
+def refused(f, what):
+    try:
+        f()
+    except api.GrdError as e:
+        assert what in str(e), e
+        return True
+    return False
+"""
+
+
+@pytest.fixture(scope="module")
+def fake(tmp_path_factory):
+    gxx = shutil.which("g++")
+    if gxx is None or not os.path.exists(os.path.join(ROCM, "include", "hip", "hip_runtime.h")):
+        pytest.skip("no g++ or HIP headers on this machine")
+    out = str(tmp_path_factory.mktemp("fake") / "libfake_hip.so")
+    subprocess.run([gxx, "-std=c++17", "-O1", "-fPIC", "-shared", "-w", "-D__HIP_PLATFORM_AMD__", "-I",
+                    os.path.join(ROCM, "include"), os.path.join(ROOT, "tests", "fake_hip.cpp"), "-o", out], check=True)
+    return out
+
+
+def _run(fake, body):
+    p = subprocess.run([sys.executable, "-c", PRELUDE + body, fake, ROOT], capture_output=True, text=True, timeout=120)
+    assert p.returncode == 0 and p.stdout.split()[-1:] == ["done"], (p.returncode, p.stdout, p.stderr)
+
+
+def test_freed_memory_is_given_back(fake):
+    """What a context keeps goes back when it is asked to trim, and when it ends."""
+    _run(fake, r"""
+ctx = context()
+base = live()
+G = api.Graph.from_csr(ctx, *ring(5000))
+S = api.State(G, api.CC)
+assert live() > base
+S.free()
+G.free()
+assert live() > base  # kept for the next allocations
+ctx.trim()
+assert live() == base
+G = api.Graph.from_csr(ctx, *ring(5000))
+G.free()
+ctx.close()
+assert live() == 0 and fake.fake_bad_frees() == 0
+print("done")
+""")
+
+
+@pytest.mark.parametrize("call", ["graph", "weights"])
+def test_kept_memory_serves_every_context(fake, call):
+    """No allocation fails while another context of the device only keeps blocks:
+    neither one through a context's own blocks nor a plain one."""
+    _run(fake, r"""
+A, B = context(), context()
+G = api.Graph.from_csr(A, *ring(5000))
+used = live()
+G.free()
+assert live() == used  # A keeps all of it
+limit(used)
+if "%s" == "graph":
+    G = api.Graph.from_csr(B, *ring(5000))
+    G.free()
+else:
+    B.selector_load(np.zeros(api.MLP_PARAMS, dtype=np.uint16))
+limit(UNLIMITED)
+A.close()
+G = api.Graph.from_csr(B, *ring(5000))  # (a context that is gone is not asked)
+G.free()
+B.close()
+assert live() == 0 and fake.fake_bad_frees() == 0
+print("done")
+""" % call)
+
+
+def test_device_of_another_context_is_left_alone(fake):
+    """A context on another device keeps its blocks."""
+    _run(fake, r"""
+A, B = context(), api.Context(1)
+G = api.Graph.from_csr(A, *ring(5000))
+used = live()
+G.free()
+limit(used)
+assert refused(lambda: B.selector_load(np.zeros(api.MLP_PARAMS, dtype=np.uint16)), "failed")
+assert live() == used
+limit(UNLIMITED)
+A.close()
+B.close()
+print("done")
+""")
