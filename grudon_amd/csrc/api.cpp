@@ -594,18 +594,18 @@ grd_status grd_state_create_typed(grd_graph *g, int algo, uint32_t value_bytes, 
   // (mode 3) every pull (the BSP pull of CC, SSSP and reference PageRank too);
   // with the default window, small graphs keep the row-block pull
   const int pm = small_graph_pull(g, algo) ? 0 : g->ctx->pull_mode;
-  if ((algo == GRD_PR_PULL && pm != 0) || pm == 3) {
-    try {
+  try {
+    if ((algo == GRD_PR_PULL && pm != 0) || pm == 3) {
       st = build_tiers(g);
       if (st == GRD_OK && g->tier_mode == 3) st = build_cold(g, algo, &s->cold);
-    } catch (const std::bad_alloc &) {
-      st = fail(GRD_ERR_OOM, "tiled pull: host allocation failed");
+      // a graph keeps the regrouping it was given first; the BSP pull uses
+      // only the hot / cold one
+      s->tiled = st == GRD_OK && (algo == GRD_PR_PULL || g->tier_mode == 3);
     }
-    // a graph keeps the regrouping it was given first; the BSP pull uses
-    // only the hot / cold one
-    s->tiled = st == GRD_OK && (algo == GRD_PR_PULL || g->tier_mode == 3);
+    if (st == GRD_OK) st = state_alloc(s);
+  } catch (const std::bad_alloc &) {
+    st = fail(GRD_ERR_OOM, "grd_state_create: host allocation failed");
   }
-  if (st == GRD_OK) st = state_alloc(s);
   if (st == GRD_OK && (hipEventCreate(&s->kev[0]) != hipSuccess || hipEventCreate(&s->kev[1]) != hipSuccess))
     st = fail(GRD_ERR_HIP, "grd_state_create: hipEventCreate failed");
   if (st != GRD_OK) {

@@ -52,7 +52,11 @@ bool BlockCache::give(void *p, uint64_t size)
 {
   std::lock_guard<std::mutex> lock(mu);
   if (size > kMaxBlock || held + size > kMaxHeld) return false;
-  blocks.emplace(size, p);
+  try {
+    blocks.emplace(size, p);
+  } catch (const std::bad_alloc &) {
+    return false;  // (objects are freed without memory to note it: the block goes back)
+  }
   held += size;
   return true;
 }
@@ -67,6 +71,7 @@ void BlockCache::trim()
 
 // The process's contexts: what they keep goes back before an allocation on
 // their device may fail (the blocks kept are idle, and a cache has its lock).
+constexpr size_t kHostCountersKept = 8;
 static std::mutex g_contexts_mu;
 static std::vector<grd_ctx *> &contexts()
 {
@@ -78,6 +83,7 @@ grd_status workspace_open(grd_ctx *ctx)
 {
   std::lock_guard<std::mutex> lock(g_contexts_mu);
   try {
+    ctx->host_counters.reserve(kHostCountersKept);  // (giving one back never allocates)
     contexts().push_back(ctx);
   } catch (const std::bad_alloc &) {
     return fail(GRD_ERR_OOM, "grd_create: host allocation failed");
@@ -110,9 +116,20 @@ grd_status DevMem::alloc(void **p, uint64_t nbytes)
   *p = nullptr;
   const uint64_t b = nbytes ? nbytes : 64;
   uint64_t size = block_size(b);
+  try {
+    ptrs.emplace_back(nullptr, 0);  // room first: a block is never left without a note of it
+  } catch (const std::bad_alloc &) {
+    return fail(GRD_ERR_OOM, "host allocation failed");
+  }
   *p = ctx->cache.take(size, &size);
-  if (!*p) GRD_TRY(device_malloc(ctx->device, p, size));
-  ptrs.emplace_back(*p, size);
+  if (!*p) {
+    const grd_status st = device_malloc(ctx->device, p, size);
+    if (st != GRD_OK) {
+      ptrs.pop_back();
+      return st;
+    }
+  }
+  ptrs.back() = {*p, size};
   bytes += b;
   return GRD_OK;
 }
@@ -187,7 +204,7 @@ grd_status host_counters_take(grd_ctx *ctx, Counters **out)
 void host_counters_give(grd_ctx *ctx, Counters *p)
 {
   if (!p) return;
-  if (ctx->host_counters.size() < 8) ctx->host_counters.push_back(p);
+  if (ctx->host_counters.size() < kHostCountersKept) ctx->host_counters.push_back(p);
   else (void)hipHostFree(p);
 }
 

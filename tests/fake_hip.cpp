@@ -27,6 +27,8 @@ struct Plain {  // (its own bookkeeping never fails)
 std::map<void *, size_t, std::less<void *>, Plain<std::pair<void *const, size_t>>> blocks;
 uint64_t live = 0, limit = ~0ull, launches = 0, bad_frees = 0;
 bool new_fails = false;
+long new_fails_in = 0;  // the how many-th from now fails, once (0: none)
+bool new_ok() { return !new_fails && (new_fails_in == 0 || --new_fails_in != 0); }
 struct Call {
   dim3 grid, block;
   size_t shared;
@@ -36,11 +38,11 @@ struct Call {
 
 void *operator new(size_t n)
 {
-  void *p = new_fails ? nullptr : malloc(n ? n : 1);
+  void *p = new_ok() ? malloc(n ? n : 1) : nullptr;
   if (!p) throw std::bad_alloc();
   return p;
 }
-void *operator new(size_t n, const std::nothrow_t &) noexcept { return new_fails ? nullptr : malloc(n ? n : 1); }
+void *operator new(size_t n, const std::nothrow_t &) noexcept { return new_ok() ? malloc(n ? n : 1) : nullptr; }
 void operator delete(void *p) noexcept { free(p); }
 void operator delete(void *p, size_t) noexcept { free(p); }
 
@@ -50,6 +52,8 @@ uint64_t fake_launches() { return launches; }
 uint64_t fake_bad_frees() { return bad_frees; }
 void fake_limit(uint64_t bytes) { limit = bytes; }
 void fake_new_fails(int on) { new_fails = on != 0; }
+void fake_new_fails_in(long n) { new_fails_in = n; }
+long fake_new_left() { return new_fails_in; }
 
 hipError_t hipMalloc(void **p, size_t n)
 {

@@ -122,3 +122,63 @@ A.close()
 B.close()
 print("done")
 """)
+
+
+def test_freeing_needs_no_memory(fake):
+    """Objects can be freed while the host has no memory left: the blocks that
+    cannot be noted for later use go back to the device."""
+    _run(fake, r"""
+ctx = context()
+base = live()
+L = api.lib()
+G = api.Graph.from_csr(ctx, *ring(5000))
+states = [api.State(G, api.CC) for _ in range(3)]
+B = api.Batch(ctx, [ring(100)])
+calls = [(L.grd_batch_free, B.h)] + [(L.grd_state_free, S.h) for S in states] + [(L.grd_graph_free, G.h)]
+ctx._live.clear()
+B.h = G.h = None
+for S in states:
+    S.h = None
+fake.fake_new_fails(1)
+rc = 0
+for f, h in calls:
+    rc |= f(h)
+fake.fake_new_fails(0)
+assert rc == 0 and live() == base and fake.fake_bad_frees() == 0
+ctx.close()
+assert live() == 0
+print("done")
+""")
+
+
+def test_state_creation_without_host_memory_fails_cleanly(fake):
+    """Whichever host allocation of a state's creation fails, the call returns an
+    error (no exception through the C interface) and no device block is lost."""
+    _run(fake, r"""
+fake.fake_new_fails_in.argtypes, fake.fake_new_left.restype = [ct.c_long], ct.c_long
+ctx = context()
+ctx.set_pull_tiling(3, 4)
+G = api.Graph.from_csr(ctx, *ring(5000))
+L = api.lib()
+base = live()
+failures = 0
+for algo in (api.CC, api.PR_PULL):
+    for k in range(1, 10000):
+        h = ct.c_void_p()
+        fake.fake_new_fails_in(k)
+        rc = L.grd_state_create(G.h, algo, ct.byref(h))
+        left = fake.fake_new_left()
+        fake.fake_new_fails_in(0)
+        if rc == 0:
+            assert L.grd_state_free(h) == 0
+        if left:
+            break
+        failures += rc != 0
+        assert rc in (0, 3)  # (the state is created all the same, or GRD_ERR_OOM)
+    assert rc == 0
+assert failures > 20
+G.free()
+ctx.close()
+assert live() == 0 and fake.fake_bad_frees() == 0
+print("done")
+""")
