@@ -292,7 +292,7 @@ struct grd_graph {
   uint8_t *hw8 = nullptr;           // the same as bytes, in their place when every weight is below 256
   bool w8_fits = false;             // every weight is below 256 (hw8 / the cold sets' w8)
   grd::ColdSet cold[2];             // the cold arcs as the sums / as the min-combines block them (cold_set)
-  grd::DevMem tmem;
+  grd::DevMem tmem, cold_mem[2];
 };
 
 struct grd_state {

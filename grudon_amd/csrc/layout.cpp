@@ -125,7 +125,7 @@ static grd_status build_impl(grd_ctx *ctx, uint32_t n, const uint32_t *rp, const
   const uint32_t NW = (n + 63) / 64;
 
   grd_graph *g = new grd_graph();
-  g->ctx = g->mem.ctx = g->tmem.ctx = ctx;
+  g->ctx = g->mem.ctx = g->tmem.ctx = g->cold_mem[0].ctx = g->cold_mem[1].ctx = ctx;
   g->n = n;
   g->m = m;
   g->C = C;

@@ -592,7 +592,7 @@ grd_status build_graph_device(grd_ctx *ctx, uint32_t n, const uint32_t *rp, cons
   GRD_TRY(check_row_ptr(n, rp));  // the device passes index by row_ptr
   grd_graph *g = new (std::nothrow) grd_graph();
   if (!g) return fail(GRD_ERR_OOM, "graph: host allocation failed");
-  g->ctx = g->mem.ctx = g->tmem.ctx = ctx;
+  g->ctx = g->mem.ctx = g->tmem.ctx = g->cold_mem[0].ctx = g->cold_mem[1].ctx = ctx;
   g->n = n;
   g->m = rp[n];
   g->C = C;

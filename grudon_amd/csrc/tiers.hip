@@ -923,13 +923,9 @@ static grd_status build_hotcold(grd_graph *g)
   return GRD_OK;
 }
 
-// mode 3: the cold arcs blocked for one algorithm, once per graph and set
-grd_status build_cold(grd_graph *g, int algo, const ColdSet **out)
+// the cold arcs in row blocks of at most N arcs, into t
+static grd_status cut_cold(grd_graph *g, uint32_t N, DevMem &gm, ColdSet &t)
 {
-  uint32_t N = 0;
-  ColdSet &c = g->cold[cold_set(g, algo, &N)];
-  *out = &c;
-  if (c.nnz) return GRD_OK;
   hipStream_t st = g->ctx->stream;
   const uint32_t P = g->P;
   std::vector<uint32_t> corp((size_t)P + 1);
@@ -952,8 +948,6 @@ grd_status build_cold(grd_graph *g, int algo, const ColdSet **out)
     blk.push_back(PullBlock{r0, r - r0, e0, corp[r]});
   }
   if (blk.size() >= 0x7FFFFFFFull) return fail(GRD_ERR_ARG, "hot / cold pull: too many row blocks");
-  DevMem &gm = g->tmem;
-  ColdSet t;
   const uint64_t arcs = std::max<uint64_t>(corp[P], 1);
   GRD_TRY(gm.alloc_n(&t.col, arcs));
   GRD_TRY(gm.alloc_n(&t.pos, arcs));
@@ -975,16 +969,35 @@ grd_status build_cold(grd_graph *g, int algo, const ColdSet **out)
   t.nnz = N;
   GRD_TRY(cold_sort(g, t));
   GRD_HIP(hipStreamSynchronize(st));  // the host vectors go out of scope
-  c = t;
   return GRD_OK;
+}
+
+// mode 3: the cold arcs blocked for one algorithm, once per graph and set (6
+// bytes a cold arc, with weights 7 or 10; a graph that both kinds of algorithms
+// pull over holds both sets).  A set that cannot be built leaves nothing behind.
+grd_status build_cold(grd_graph *g, int algo, const ColdSet **out)
+{
+  uint32_t N = 0;
+  const uint32_t set = cold_set(g, algo, &N);
+  ColdSet &c = g->cold[set];
+  *out = &c;
+  if (c.nnz) return GRD_OK;
+  ColdSet t;
+  grd_status st;
+  try {
+    st = cut_cold(g, N, g->cold_mem[set], t);
+  } catch (const std::bad_alloc &) {
+    st = fail(GRD_ERR_OOM, "hot / cold pull: host allocation failed");
+  }
+  if (st == GRD_OK) c = t;
+  else g->cold_mem[set].release();
+  return st;
 }
 
 // Regroups the CSC by (partition, tier, row) on the device; the cut into row
 // blocks and tiles, a sequential pass over the pair lengths, runs on the host.
-grd_status build_tiers(grd_graph *g)
+static grd_status build_pairs(grd_graph *g)
 {
-  if (g->tiers_built) return GRD_OK;
-  if (g->ctx->pull_mode == 3) return build_hotcold(g);
   grd_ctx *ctx = g->ctx;
   hipStream_t st = ctx->stream;
   const uint32_t P = g->P, M = (uint32_t)g->M, C = (uint32_t)g->C;
@@ -1148,6 +1161,26 @@ grd_status build_tiers(grd_graph *g)
   g->tile_arcs = tile_arcs;
   g->tiers_built = true;
   return GRD_OK;
+}
+
+// once per graph; a regrouping that cannot be built leaves nothing behind
+grd_status build_tiers(grd_graph *g)
+{
+  if (g->tiers_built) return GRD_OK;
+  grd_status st;
+  try {
+    st = g->ctx->pull_mode == 3 ? build_hotcold(g) : build_pairs(g);
+  } catch (const std::bad_alloc &) {
+    st = fail(GRD_ERR_OOM, "tiled pull: host allocation failed");
+  }
+  if (st != GRD_OK) {
+    g->tmem.release();
+    g->n_tblk = g->n_tlong = g->n_ttile = g->n_twide = 0;
+    g->tcol = nullptr;
+    g->hw = nullptr;
+    g->hw8 = nullptr;
+  }
+  return st;
 }
 
 grd_status prp_pull_tiled(grd_state *s)

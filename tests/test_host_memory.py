@@ -182,3 +182,50 @@ ctx.close()
 assert live() == 0 and fake.fake_bad_frees() == 0
 print("done")
 """)
+
+
+@pytest.mark.parametrize("algo,weighted", [("CC", False), ("SSSP", True), ("PR_PULL", False)])
+@pytest.mark.parametrize("mode", [1, 2, 3])
+def test_a_failed_state_leaves_its_graph_as_it_was(fake, algo, weighted, mode):
+    """With too little device memory for a state and the regrouping it asks for,
+    however far it gets, nothing half made stays behind: after all the failures
+    the graph and its state hold what they hold without one."""
+    _run(fake, r"""
+algo, weighted, mode = api.%s, %s, %d
+ctx = context()
+rp, col = ring(5000)
+w = np.arange(len(col), dtype=np.uint32) if weighted else None
+
+
+def graph():
+    ctx.set_pull_tiling(0)
+    G = api.Graph.from_csr(ctx, rp, col, w)
+    for a in (api.CC, api.PR_PULL):  # (what a graph computes once for every state)
+        api.State(G, a).free()
+    ctx.set_pull_tiling(mode, 4)
+    ctx.trim()
+    return G, live()
+
+
+G, base = graph()
+S = api.State(G, algo)
+ctx.trim()
+want = live() - base
+S.free()
+G.free()
+G, base = graph()
+failures, made = 0, []
+for extra in range(0, 1 << 22, 5000):
+    limit(base + extra)
+    if not refused(lambda: made.append(api.State(G, algo)), "failed"):
+        break
+    failures += 1
+ctx.trim()
+assert failures > 3 and live() - base == want, (failures, live() - base, want)
+made.pop().free()
+G.free()
+limit(UNLIMITED)
+ctx.close()
+assert live() == 0 and fake.fake_bad_frees() == 0
+print("done")
+""" % (algo, weighted, mode))
