@@ -27,6 +27,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <array>
 #include <functional>
@@ -71,6 +72,16 @@ struct BlockCache {
   bool give(void *p, uint64_t size);
   void trim();
 };
+
+// The segments of at most n arcs of a long row [e0, e1), in order; returns their
+// number.  In 64 bits: e1 may lie within n arcs of 2^32.
+template <class F>
+inline uint32_t cut_long_row(uint32_t e0, uint32_t e1, uint32_t n, F segment)
+{
+  uint32_t k = 0;
+  for (uint64_t e = e0; e < e1; e += n, k++) segment((uint32_t)e, (uint32_t)std::min<uint64_t>(e1, e + n));
+  return k;
+}
 
 // Device allocation list owned by a graph or a state, from its context's
 // cache (ctx is set before the first allocation).  A block's users are ordered on the context's stream; release() waits

@@ -81,10 +81,8 @@ grd_status build_row_blocks(grd_graph *g, const std::vector<uint32_t> &crp)
     uint32_t deg = crp[r + 1] - crp[r];
     if (deg > kPullNnz) {
       PullLong L{r, (uint32_t)blks.size(), 0, 0};
-      for (uint32_t e = crp[r]; e < crp[r + 1]; e += kPullNnz) {
-        blks.push_back(PullBlock{r, 0, e, std::min(crp[r + 1], e + kPullNnz)});
-        L.nseg++;
-      }
+      L.nseg = cut_long_row(crp[r], crp[r + 1], kPullNnz,
+                            [&](uint32_t a, uint32_t b) { blks.push_back(PullBlock{r, 0, a, b}); });
       longs.push_back(L);
       r++;
       continue;

@@ -852,10 +852,8 @@ static grd_status build_hotcold(grd_graph *g)
       const uint32_t len = hrp[r + 1] - hrp[r];
       if (len > kWNnz) {
         PullLong L{r, (uint32_t)hblk.size(), 0, 0};
-        for (uint32_t e = hrp[r]; e < hrp[r + 1]; e += kWNnz) {
-          hblk.push_back(PullBlock{r, 0, e, std::min(hrp[r + 1], e + kWNnz)});
-          L.nseg++;
-        }
+        L.nseg = cut_long_row(hrp[r], hrp[r + 1], kWNnz,
+                              [&](uint32_t a, uint32_t b) { hblk.push_back(PullBlock{r, 0, a, b}); });
         hlong.push_back(L);
         r++;
         continue;
@@ -935,10 +933,8 @@ static grd_status cut_cold(grd_graph *g, uint32_t N, DevMem &gm, ColdSet &t)
   for (uint32_t r = 0; r < P;) {
     if (corp[r + 1] - corp[r] > N) {
       PullLong L{r, (uint32_t)blk.size(), 0, 0};
-      for (uint32_t e = corp[r]; e < corp[r + 1]; e += N) {
-        blk.push_back(PullBlock{r, 0, e, std::min(corp[r + 1], e + N)});
-        L.nseg++;
-      }
+      L.nseg = cut_long_row(corp[r], corp[r + 1], N,
+                            [&](uint32_t a, uint32_t b) { blk.push_back(PullBlock{r, 0, a, b}); });
       lng.push_back(L);
       r++;
       continue;
@@ -1116,10 +1112,8 @@ static grd_status build_pairs(grd_graph *g)
       const size_t before = blks.size();
       if (len > blk_nnz) {
         PullLong L{(uint32_t)q, (uint32_t)blks.size(), 0, 0};
-        for (uint32_t e = tptr[q]; e < tptr[q + 1]; e += blk_nnz) {
-          blks.push_back(PullBlock{(uint32_t)q, 0, e, std::min(tptr[q + 1], e + blk_nnz)});
-          L.nseg++;
-        }
+        L.nseg = cut_long_row(tptr[q], tptr[q + 1], blk_nnz,
+                              [&](uint32_t a, uint32_t b) { blks.push_back(PullBlock{(uint32_t)q, 0, a, b}); });
         longs.push_back(L);
         add_arcs = len;
         q++;
