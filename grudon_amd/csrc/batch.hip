@@ -416,13 +416,18 @@ static void drop_captured(grd_batch *b)
 // LDS stores 33, the gathers 89, the row sums and updates 39.  The whole
 // PageRank took 4.36 ms with the arcs in row order, a separate update pass and
 // blocks of 1024, and takes 2.72; CC took 1.70 and takes 1.41.
-static grd_status batch_build_blocks(grd_batch *b)
+static uint32_t block_arcs(const grd_batch *b, uint32_t tile)
+{
+  while (tile < 16384 && b->E / (2 * tile) >= 2ull * (uint64_t)b->ctx->num_cus) tile *= 2;
+  return tile;
+}
+
+static grd_status cut_blocks(grd_batch *b)
 {
   std::vector<BatchBlock> blks;
   std::vector<BatchLong> longs;
   std::vector<uint32_t> gblk(b->count + 1, 0), glong(b->count + 1, 0);
-  uint32_t T = b->tile;
-  while (T < 16384 && b->E / (2 * T) >= 2ull * (uint64_t)b->ctx->num_cus) T *= 2;
+  const uint32_t T = block_arcs(b, b->tile);
   const uint32_t rows = std::min<uint32_t>(T, 8192);
   for (uint32_t g = 0; g < b->count; g++) {
     gblk[g] = (uint32_t)blks.size();
@@ -479,6 +484,24 @@ static grd_status batch_build_blocks(grd_batch *b)
   GRD_HIP(hipGetLastError());
   GRD_HIP(hipStreamSynchronize(st));  // the host vectors go out of scope
   return GRD_OK;
+}
+
+// the blocks for the present tile; without memory for them the batch has none
+// (nnz 0) until a later tuning or run gets them
+static grd_status batch_build_blocks(grd_batch *b)
+{
+  grd_status st;
+  try {
+    st = cut_blocks(b);
+  } catch (const std::bad_alloc &) {
+    st = fail(GRD_ERR_OOM, "batch: host allocation failed");
+  }
+  if (st != GRD_OK) {
+    drop_captured(b);
+    b->blk_mem.release();
+    b->nnz = 0;
+  }
+  return st;
 }
 
 static uint32_t persistent_grid(const grd_batch *b) { return (uint32_t)b->ctx->num_cus * b->grid_per_cu; }
@@ -567,6 +590,7 @@ static grd_status capture(grd_batch *b, int algo, double damping, double tol, ui
 static grd_status batch_run(grd_batch *b, int algo, double damping, double tol, uint32_t max_iter, uint32_t *iters_out,
                             double *ms_out)
 {
+  if (!b->nnz) GRD_TRY(batch_build_blocks(b));
   hipStream_t st = b->ctx->stream;
   const uint32_t cnt = b->count;
   // per-graph state (fill kernels: nothing memset-like inside the graph)
@@ -736,10 +760,8 @@ grd_status grd_batch_tune(grd_batch *b, uint32_t tile, uint32_t grid_per_cu, uin
   if (grid_per_cu > 64 || K > 64) return fail(GRD_ERR_ARG, "grd_batch_tune: grid_per_cu and K must be <= 64");
   if (grid_per_cu) b->grid_per_cu = grid_per_cu;
   if (K) b->K = K;
-  if (tile && tile != b->tile) {
-    b->tile = tile;
-    GRD_TRY(batch_build_blocks(b));
-  }
+  if (tile) b->tile = tile;
+  if (block_arcs(b, b->tile) != b->nnz) GRD_TRY(batch_build_blocks(b));
   return GRD_OK;
 }
 
@@ -748,8 +770,12 @@ grd_status grd_batch_autotune(grd_batch *b, uint32_t *chosen3)
   if (!b) return fail(GRD_ERR_ARG, "grd_batch_autotune: NULL batch");
   const uint32_t tiles[] = {1024, 2048, 4096}, grids[] = {4, 8, 16}, Ks[] = {2, 4, 8};
   double best = 1e30;
-  uint32_t bt = b->tile, bg = b->grid_per_cu, bk = b->K;
-  for (uint32_t t : tiles)
+  uint32_t bt = b->tile, bg = b->grid_per_cu, bk = b->K, last = 0;
+  for (uint32_t t : tiles) {
+    // tiles that give the same blocks are one candidate (from 8192 arcs
+    // per CU on all of them do)
+    if (block_arcs(b, t) == last) continue;
+    last = block_arcs(b, t);
     for (uint32_t gpc : grids)
       for (uint32_t k : Ks) {
         GRD_TRY(grd_batch_tune(b, t, gpc, k));
@@ -763,6 +789,7 @@ grd_status grd_batch_autotune(grd_batch *b, uint32_t *chosen3)
           bk = k;
         }
       }
+  }
   GRD_TRY(grd_batch_tune(b, bt, bg, bk));
   if (chosen3) {
     chosen3[0] = bt;

@@ -358,11 +358,13 @@ grd_status grd_batch_create(grd_ctx *ctx, uint32_t count, const uint32_t *n, con
                             const uint32_t *const *row_ptr, const uint32_t *const *col, grd_batch **out);
 grd_status grd_batch_free(grd_batch *b);
 /* Tunables (0 = keep): tile = arcs of the smallest row block (1024, 2048 or
- * 4096; larger batches use larger blocks), grid_per_cu = persistent workgroups
+ * 4096; larger batches use larger blocks, and from 8192 arcs per CU on the
+ * tile makes no difference), grid_per_cu = persistent workgroups
  * per CU (<= 64), K = iterations per captured hipGraph (<= 64). */
 grd_status grd_batch_tune(grd_batch *b, uint32_t tile, uint32_t grid_per_cu, uint32_t K);
 /* Autotune the tunables by timing candidate settings on this batch
- * (tile x grid_per_cu x K); chosen3 (may be NULL) receives the winner. */
+ * (tile x grid_per_cu x K, of the tiles that give the same blocks the smallest);
+ * chosen3 (may be NULL) receives the winner. */
 grd_status grd_batch_autotune(grd_batch *b, uint32_t *chosen3);
 /* PageRank pull (Kahan FP32, FP64 dangling/residual) on every graph, with
  * iterations captured in a hipGraph; iters_out[count], ms_out may be NULL. */

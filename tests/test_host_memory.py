@@ -229,3 +229,37 @@ ctx.close()
 assert live() == 0 and fake.fake_bad_frees() == 0
 print("done")
 """ % (algo, weighted, mode))
+
+
+def test_batch_blocks_are_cut_when_they_change(fake):
+    """Tiles that give a batch the same blocks cost nothing; without memory for
+    other blocks the tuning fails and the batch has none to run over until there
+    is memory again."""
+    _run(fake, r"""
+ctx = context()
+launches = fake.fake_launches
+large = api.Batch(ctx, [ring(300000)])  # 2.4 M arcs: blocks of 4096 for every tile
+small = api.Batch(ctx, [ring(3000)])
+for tile in (1024, 2048, 4096):
+    at = launches()
+    large.tune(tile=tile)
+    assert launches() == at
+    small.tune(tile=tile)
+    assert launches() > at
+small.tune(tile=1024)
+ctx.trim()
+limit(0)
+assert refused(lambda: small.tune(tile=4096), "failed")
+at = launches()
+assert refused(lambda: small.pagerank(), "failed") and launches() == at
+assert refused(lambda: small.autotune(), "failed")
+limit(UNLIMITED)
+at = launches()
+small.tune(tile=4096)
+assert launches() > at
+small.free()
+large.free()
+ctx.close()
+assert live() == 0 and fake.fake_bad_frees() == 0
+print("done")
+""")
