@@ -85,7 +85,8 @@ __global__ void __launch_bounds__(kBlock) k_push(const uint32_t *__restrict__ AL
     s_beg[threadIdx.x] = beg;
     s_val[threadIdx.x] = v;
     __syncthreads();
-    for (uint32_t j0 = threadIdx.x; j0 < total; j0 += kIlp * kBlock) {
+    const uint32_t l = lane_id();
+    for (uint32_t j0 = threadIdx.x; j0 - l < total; j0 += kIlp * kBlock) {  // the same rounds for every lane of a wave
       uint32_t c[kIlp], w[kIlp];
       V x[kIlp];
 #pragma unroll
@@ -103,7 +104,7 @@ __global__ void __launch_bounds__(kBlock) k_push(const uint32_t *__restrict__ AL
       }
 #pragma unroll
       for (int q = 0; q < kIlp; q++) x[q] = Op::edge(x[q], w[q]);
-      relax_many<Op, kIlp, kShip>(upd, dirty, c, x, (total - j0 + kBlock - 1) / kBlock);
+      relax_many<Op, kIlp, kShip>(upd, dirty, c, x, j0 < total ? (total - j0 + kBlock - 1) / kBlock : 0u);
     }
     __syncthreads();
   }
@@ -124,7 +125,7 @@ __global__ void __launch_bounds__(kBlock) k_push_heavy(const uint2 *__restrict__
     const uint32_t end = rp[ch.x + 1];
     const uint32_t b = rp[ch.x] + ch.y, ne = min(end - b, kHeavyChunk);
     const V v = mprop[ch.x];
-    for (uint32_t j0 = l; j0 < ne; j0 += kIlp * kWave) {
+    for (uint32_t j0 = l; j0 - l < ne; j0 += kIlp * kWave) {
       uint32_t c[kIlp], w[kIlp];
       V x[kIlp];
 #pragma unroll
@@ -139,7 +140,7 @@ __global__ void __launch_bounds__(kBlock) k_push_heavy(const uint2 *__restrict__
       }
 #pragma unroll
       for (int q = 0; q < kIlp; q++) x[q] = Op::edge(v, w[q]);
-      relax_many<Op, kIlp, kShip>(upd, dirty, c, x, (ne - j0 + kWave - 1) / kWave);
+      relax_many<Op, kIlp, kShip>(upd, dirty, c, x, j0 < ne ? (ne - j0 + kWave - 1) / kWave : 0u);
     }
   }
 }
