@@ -119,12 +119,15 @@ grd_status DevMem::alloc(void **p, uint64_t nbytes)
   try {
     ptrs.emplace_back(nullptr, 0);  // room first: a block is never left without a note of it
   } catch (const std::bad_alloc &) {
+    (void)hipStreamSynchronize(ctx->stream);
     return fail(GRD_ERR_OOM, "host allocation failed");
   }
   *p = ctx->cache.take(size, &size);
   if (!*p) {
     const grd_status st = device_malloc(ctx->device, p, size);
     if (st != GRD_OK) {
+      // the caller gives up: what it has queued still reads its host arrays
+      (void)hipStreamSynchronize(ctx->stream);
       ptrs.pop_back();
       return st;
     }

@@ -1,12 +1,17 @@
 // A HIP runtime without a device, for tests of what the library's host code does
 // with memory: device memory is host memory within a limit, copies are copies,
 // kernels do nothing.  Loaded before the library, its functions are taken.
-// It also takes operator new, which can be told to fail.
+// It also takes operator new, which can be told to fail, and asynchronous copies
+// can be told to wait for the next synchronisation, so that a host array that goes
+// before its copy is noticed.
 #include <cstdint>
 #include <cstdlib>
 #include <cstring>
 #include <map>
 #include <new>
+#include <vector>
+
+#include <malloc.h>
 
 #include <hip/hip_runtime.h>
 
@@ -29,6 +34,35 @@ uint64_t live = 0, limit = ~0ull, launches = 0, bad_frees = 0;
 bool new_fails = false;
 long new_fails_in = 0;  // the how many-th from now fails, once (0: none)
 bool new_ok() { return !new_fails && (new_fails_in == 0 || --new_fails_in != 0); }
+uint64_t mallocs_left = ~0ull;
+bool defer = false;
+uint64_t lost = 0;  // host arrays that went before their copy
+struct Copy {
+  void *d;
+  const void *s;
+  size_t n;
+};
+std::vector<Copy, Plain<Copy>> pending;
+void run_pending()
+{
+  for (const Copy &c : pending) memcpy(c.d, c.s, c.n);
+  pending.clear();
+}
+void drop(void *p)
+{
+  if (!p) return;
+  const char *a = static_cast<char *>(p), *b = a + malloc_usable_size(p);
+  for (size_t i = 0; i < pending.size();) {
+    const char *s = static_cast<const char *>(pending[i].s), *d = static_cast<const char *>(pending[i].d);
+    if ((s >= a && s < b) || (d >= a && d < b)) {
+      lost++;
+      pending.erase(pending.begin() + i);
+    } else {
+      i++;
+    }
+  }
+  free(p);
+}
 struct Call {
   dim3 grid, block;
   size_t shared;
@@ -43,13 +77,16 @@ void *operator new(size_t n)
   return p;
 }
 void *operator new(size_t n, const std::nothrow_t &) noexcept { return new_ok() ? malloc(n ? n : 1) : nullptr; }
-void operator delete(void *p) noexcept { free(p); }
-void operator delete(void *p, size_t) noexcept { free(p); }
+void operator delete(void *p) noexcept { drop(p); }
+void operator delete(void *p, size_t) noexcept { drop(p); }
 
 extern "C" {
 uint64_t fake_live() { return live; }
 uint64_t fake_launches() { return launches; }
 uint64_t fake_bad_frees() { return bad_frees; }
+void fake_mallocs_left(uint64_t n) { mallocs_left = n; }
+void fake_defer(int on) { defer = on != 0; }
+uint64_t fake_lost() { return lost; }
 void fake_limit(uint64_t bytes) { limit = bytes; }
 void fake_new_fails(int on) { new_fails = on != 0; }
 void fake_new_fails_in(long n) { new_fails_in = n; }
@@ -58,7 +95,9 @@ long fake_new_left() { return new_fails_in; }
 hipError_t hipMalloc(void **p, size_t n)
 {
   *p = nullptr;
+  if (mallocs_left == 0) return hipErrorOutOfMemory;
   if (n > limit || live > limit - n) return hipErrorOutOfMemory;
+  mallocs_left--;
   *p = calloc(n ? n : 1, 1);
   blocks[*p] = n;
   live += n;
@@ -66,6 +105,7 @@ hipError_t hipMalloc(void **p, size_t n)
 }
 hipError_t hipFree(void *p)
 {
+  run_pending();
   if (!p) return hipSuccess;
   auto it = blocks.find(p);
   if (it == blocks.end()) {
@@ -84,17 +124,25 @@ hipError_t hipHostMalloc(void **p, size_t n, unsigned int)
 }
 hipError_t hipHostFree(void *p)
 {
+  run_pending();
   free(p);
   return hipSuccess;
 }
 hipError_t hipMemcpy(void *d, const void *s, size_t n, hipMemcpyKind)
 {
+  run_pending();
   if (n) memcpy(d, s, n);
   return hipSuccess;
 }
-hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t) { return hipMemcpy(d, s, n, k); }
+hipError_t hipMemcpyAsync(void *d, const void *s, size_t n, hipMemcpyKind k, hipStream_t)
+{
+  if (!defer) return hipMemcpy(d, s, n, k);
+  if (n) pending.push_back(Copy{d, s, n});
+  return hipSuccess;
+}
 hipError_t hipMemsetAsync(void *d, int v, size_t n, hipStream_t)
 {
+  run_pending();
   if (n) memset(d, v, n);
   return hipSuccess;
 }
@@ -135,7 +183,11 @@ hipError_t hipStreamCreateWithFlags(hipStream_t *s, unsigned int)
   return hipSuccess;
 }
 hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
-hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t)
+{
+  run_pending();
+  return hipSuccess;
+}
 int hipGetStreamDeviceId(hipStream_t) { return 0; }
 hipError_t hipEventCreate(hipEvent_t *e)
 {
@@ -145,7 +197,7 @@ hipError_t hipEventCreate(hipEvent_t *e)
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return hipEventCreate(e); }
 hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
 hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
-hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipStreamSynchronize(nullptr); }
 hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t)
 {
   *ms = 0.0f;

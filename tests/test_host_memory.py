@@ -14,7 +14,7 @@ ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 PRELUDE = r"""
 import ctypes as ct, os, sys
 fake = ct.CDLL(sys.argv[1], mode=os.RTLD_NOW | ct.RTLD_GLOBAL)
-fake.fake_live.restype = fake.fake_launches.restype = fake.fake_bad_frees.restype = ct.c_uint64
+fake.fake_live.restype = fake.fake_launches.restype = fake.fake_bad_frees.restype = fake.fake_lost.restype = ct.c_uint64
 fake.fake_limit.argtypes = [ct.c_uint64]
 sys.path[:0] = [sys.argv[2], os.path.join(sys.argv[2], "tests")]
 import numpy as np
@@ -263,3 +263,45 @@ ctx.close()
 assert live() == 0 and fake.fake_bad_frees() == 0
 print("done")
 """)
+
+
+@pytest.mark.parametrize("what", ["graph", "mode 1", "mode 2", "mode 3", "batch"])
+def test_host_arrays_outlive_their_copies(fake, what):
+    """Copies run at the next synchronisation at the latest, and device memory
+    runs out at every allocation in turn: whatever a failing call copies from is
+    there until the copy has run."""
+    _run(fake, r"""
+what = "%s"
+fake.fake_defer(1)
+ctx = context()
+rp, col = ring(5000)
+w = np.arange(len(col), dtype=np.uint32)
+G = api.Graph.from_csr(ctx, rp, col, w)
+for a in (api.CC, api.PR_PULL):
+    api.State(G, a).free()
+if what.startswith("mode"):
+    ctx.set_pull_tiling(int(what[-1]), 4)
+
+
+def make():
+    if what == "graph":
+        return api.Graph.from_csr(ctx, rp, col, w)
+    if what == "batch":
+        return api.Batch(ctx, [(rp, col)])
+    return api.State(api.Graph.from_csr(ctx, rp, col, w), api.PR_PULL)
+
+
+failures, made = 0, []
+fake.fake_mallocs_left.argtypes = [ct.c_uint64]
+for n in range(1000):
+    ctx.trim()
+    fake.fake_mallocs_left(n)
+    if not refused(lambda: made.append(make()), "failed"):
+        break
+    failures += 1
+fake.fake_mallocs_left(UNLIMITED)
+assert failures > 10 and fake.fake_lost() == 0, (failures, fake.fake_lost())
+ctx.close()
+assert live() == 0 and fake.fake_bad_frees() == 0
+print("done")
+""" % what)
