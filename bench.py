@@ -207,6 +207,13 @@ def line(args, value, unit, ms_per_step, dtype, config, roofline, cpu, extra=Non
     return out
 
 
+def pull_run(args, G):
+    """The pull mode that the first pull PageRank state of a graph runs: with
+    the default window the hot / cold split leaves small graphs to the row-block
+    pull, and the graph then holds no regrouping."""
+    return args.pull if any(G.info()[11:15]) else "plain"
+
+
 def layout_desc(args, scale, sym):
     return ("RMAT-%d EF%d seed 1%s, %d compute + %d memory partitions resident in HBM, "
             "on-device bitvector master/mirror sync" % (scale, args.ef, " symmetrized" if sym else "",
@@ -367,8 +374,8 @@ def run_pagerank(api, ctx, args):
     gteps = G.m * iters / secs / 1e9
     log("timed %d steps: %.3f s, %d iterations, %.2f ms/step, %.1f GTEPS"
         % (args.steps, secs, iters, secs * 1e3 / args.steps, gteps))
-    kname = PULL_KERNELS[args.pull] if pull else "k_bsp_traverse"
-    traffic = traffic_from_profiles("k_prp_pull_%s_rmat%d" % (args.pull, args.scale)) if pull else None
+    kname = PULL_KERNELS[pull_run(args, G)] if pull else "k_bsp_traverse"
+    traffic = traffic_from_profiles("k_prp_pull_%s_rmat%d" % (pull_run(args, G), args.scale)) if pull else None
     roof = roofline_of(kms, kl, kb, kname, traffic)
     # edges the traversals examined (a pull examines every arc) per second
     extra = {"work_gteps": round(last["timed_edges_examined"] / secs / 1e9, 3)}
@@ -617,8 +624,8 @@ def run_headline(api, ctx, args):
         api, S, args, {"max_iter": 1000, "tolerance": 1e-6}, G.m, per_iteration=True)
     pr_iters = last["iterations"]
     log("PR pull: %d steps, %.2f ms/step, %d iterations, %.1f GTEPS" % (args.steps, ms_step, pr_iters, gteps))
-    roof = roofline_of(kms, kl, kb, PULL_KERNELS[args.pull],
-                       traffic_from_profiles("k_prp_pull_%s_rmat%d" % (args.pull, scale)))
+    mode = pull_run(args, G)
+    roof = roofline_of(kms, kl, kb, PULL_KERNELS[mode], traffic_from_profiles("k_prp_pull_%s_rmat%d" % (mode, scale)))
     extra = {"work_gteps": round(last["timed_edges_examined"] / secs / 1e9, 3)}
     if kl:
         extra["gather_ceiling"] = gather_ceiling(api, ctx, G.n, G.m, args.parts, kms, kl)
