@@ -434,10 +434,6 @@ __global__ void __launch_bounds__(kBlock) k_reduce(uint32_t nw, uint64_t *__rest
   if (threadIdx.x == 0 && t) share[blockIdx.x] += t;
 }
 
-// ------------------------------------------------------------------------
-// update: update_frontier + apply_updates + frontier popcount
-// ------------------------------------------------------------------------
-
 // The dense reduce of a min-combine from the compute side: a proxy's update only
 // falls and the vertex has seen every earlier one, so the smallest of a vertex's
 // proxies (its own, at the same place of its pair, and its cross mirrors, which
@@ -517,6 +513,10 @@ __global__ void __launch_bounds__(kBlock) k_reduce_min(uint32_t nwP, uint64_t *_
   if (threadIdx.x == 0 && t) share[blockIdx.x] += t;
 }
 
+// ------------------------------------------------------------------------
+// update: update_frontier + apply_updates + frontier popcount
+// ------------------------------------------------------------------------
+
 // a workgroup's share of the next frontier (one barrier, no atomic: with three
 // atomics per workgroup the update of 65536 words took 29 us, now 7.6)
 __device__ __forceinline__ void share_frontier(uint64_t vertices, uint64_t edges, uint32_t maxdeg, BlockShare *share)
@@ -539,8 +539,8 @@ __device__ __forceinline__ void share_frontier(uint64_t vertices, uint64_t edges
   }
 }
 
-// A capped grid walks the word groups (the loop is wave-uniform), so the
-// blocks' counter atomics are issued by fewer blocks.  All loads of a group's
+// A capped grid walks the word groups (the loop is wave-uniform), so that few
+// blocks leave a share of the counters.  All loads of a group's
 // words are issued before any is used, and lane j stores word j's bitmap words
 // (word by word, a group was a chain of up to eight dependent round trips:
 // 11 us on 4096 words, 36 on 65536).
@@ -1069,7 +1069,7 @@ static grd_status traverse_t(grd_state *s, int option)
     GRD_TRY(push_launch<Op>(s));
     if (timed) {
       GRD_HIP(hipEventRecord(s->kev[1], st));
-      s->kern_pending = 2;  // bytes from the edge counters after the iteration
+      s->kern_pending = 2;  // bytes from the active list's vertices and arcs
     }
   }
   GRD_HIP(hipGetLastError());

@@ -224,7 +224,7 @@ static grd_status ship_t(grd_state *s)
   GRD_TRY(ship_launch<Op>(s));
   if (timed) {
     GRD_HIP(hipEventRecord(s->kev[1], st));
-    s->kern_pending = 2;  // bytes from the edge counters after the iteration
+    s->kern_pending = 2;  // bytes from the active list's vertices and arcs
   }
   // wire bytes (MPI.hpp:44 counts count * sizeof(GNode) per send): one id
   // per record header and per arc, plus the weights of a weighted SSSP

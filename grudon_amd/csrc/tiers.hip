@@ -872,8 +872,10 @@ static grd_status build_hotcold(grd_graph *g)
   }
   std::vector<TierTile> ranges;
   // Up to sixteen ranges per CU, in turn, for dynamic balance; but staging the
-  // window costs a workgroup about 3 us, so a range is given at least
-  // kRangeCost of work (about 10 us), and never fewer blocks than it has waves.
+  // window costs a workgroup about 3 us, so beyond one range per CU there is one
+  // more per CU for every kRangeCost of work that each CU has (about 10 us), and
+  // a partition gets one range for each sixteen blocks it has or begins (a
+  // block per wave).
   // With sixteen per CU at every size the staging alone moved 0.5 GB: the hot
   // pass of RMAT-18 took 53 us for 4 M arcs, a million vertices 73 us (pull
   // PageRank 3.2 -> 2.5 ms a solve with this rule); 32 K to 512 K of work per
@@ -887,7 +889,7 @@ static grd_status build_hotcold(grd_graph *g)
     const uint32_t wbase = pb[mp], wlen = std::min<uint32_t>(win, pb[mp + 1] - pb[mp]);
     uint64_t cm = 0;
     for (uint32_t i = b0; i < b1; i++) cm += bcost[i];
-    // a range keeps at least every wave of its workgroup busy
+    // about a block for each wave of a range's workgroup
     const uint64_t most = (b1 - b0 + kTierBlock / kWave - 1) / (kTierBlock / kWave);
     const uint64_t k = std::max<uint64_t>(1, std::min<uint64_t>(most, cm * nwg / std::max<uint64_t>(total, 1)));
     uint64_t acc = 0;

@@ -222,7 +222,8 @@ grd_status grd_graph_read(const char *path, uint32_t *n, uint64_t *m, uint32_t *
 grd_status grd_graph_write_gr(const char *path, uint32_t n, const uint32_t *row_ptr, const uint32_t *col,
                               const uint32_t *weights);
 /* info[0] n, [1] m, [2] C, [3] M, [4] compute slots, [5] memory proxies,
- * [6] cross mirrors, [7] weighted, [8] device bytes held by the graph,
+ * [6] cross mirrors, [7] weighted, [8] device bytes held by the graph (without
+ * a pull mode's reorganisation),
  * [9] pull row blocks, [10] long rows; [11]-[14] describe the pull mode's
  * reorganisation (0 until a state of the graph built it): modes 1 and 2
  * [11] (row, tier) pairs, [12] tiles, [13] row blocks, [14] long pairs;
