@@ -33,7 +33,12 @@ std::map<void *, size_t, std::less<void *>, Plain<std::pair<void *const, size_t>
 uint64_t live = 0, limit = ~0ull, launches = 0, bad_frees = 0;
 bool new_fails = false;
 long new_fails_in = 0;  // the how many-th from now fails, once (0: none)
-bool new_ok() { return !new_fails && (new_fails_in == 0 || --new_fails_in != 0); }
+uint64_t news = 0;
+bool new_ok()
+{
+  news++;
+  return !new_fails && (new_fails_in == 0 || --new_fails_in != 0);
+}
 uint64_t mallocs_left = ~0ull;
 bool defer = false;
 uint64_t lost = 0;  // host arrays that went before their copy
@@ -90,6 +95,7 @@ uint64_t fake_lost() { return lost; }
 void fake_limit(uint64_t bytes) { limit = bytes; }
 void fake_new_fails(int on) { new_fails = on != 0; }
 void fake_new_fails_in(long n) { new_fails_in = n; }
+uint64_t fake_news() { return news; }
 long fake_new_left() { return new_fails_in; }
 
 hipError_t hipMalloc(void **p, size_t n)
