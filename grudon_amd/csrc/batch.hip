@@ -438,7 +438,7 @@ static grd_status cut_blocks(grd_batch *b)
       uint32_t deg = b->h_crp[r + 1] - b->h_crp[r];
       if (deg > T) {
         BatchLong L{(uint32_t)r, (uint32_t)blks.size(), 0, g};
-        L.nseg = cut_long_row(b->h_crp[r], b->h_crp[r + 1], T, [&](uint32_t x, uint32_t y) {
+        L.nseg = cut_long_row(b->h_crp[r], b->h_crp[r + 1], T, [&blks, r, g](uint32_t x, uint32_t y) {
           blks.push_back(BatchBlock{(uint32_t)r, 0, x, y, g, 0, 0, 0});
         });
         longs.push_back(L);

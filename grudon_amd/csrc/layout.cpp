@@ -82,7 +82,7 @@ grd_status build_row_blocks(grd_graph *g, const std::vector<uint32_t> &crp)
     if (deg > kPullNnz) {
       PullLong L{r, (uint32_t)blks.size(), 0, 0};
       L.nseg = cut_long_row(crp[r], crp[r + 1], kPullNnz,
-                            [&](uint32_t a, uint32_t b) { blks.push_back(PullBlock{r, 0, a, b}); });
+                            [&blks, r](uint32_t a, uint32_t b) { blks.push_back(PullBlock{r, 0, a, b}); });
       longs.push_back(L);
       r++;
       continue;

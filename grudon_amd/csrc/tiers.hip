@@ -853,7 +853,7 @@ static grd_status build_hotcold(grd_graph *g)
       if (len > kWNnz) {
         PullLong L{r, (uint32_t)hblk.size(), 0, 0};
         L.nseg = cut_long_row(hrp[r], hrp[r + 1], kWNnz,
-                              [&](uint32_t a, uint32_t b) { hblk.push_back(PullBlock{r, 0, a, b}); });
+                              [&hblk, r](uint32_t a, uint32_t b) { hblk.push_back(PullBlock{r, 0, a, b}); });
         hlong.push_back(L);
         r++;
         continue;
@@ -936,7 +936,7 @@ static grd_status cut_cold(grd_graph *g, uint32_t N, DevMem &gm, ColdSet &t)
     if (corp[r + 1] - corp[r] > N) {
       PullLong L{r, (uint32_t)blk.size(), 0, 0};
       L.nseg = cut_long_row(corp[r], corp[r + 1], N,
-                            [&](uint32_t a, uint32_t b) { blk.push_back(PullBlock{r, 0, a, b}); });
+                            [&blk, r](uint32_t a, uint32_t b) { blk.push_back(PullBlock{r, 0, a, b}); });
       lng.push_back(L);
       r++;
       continue;
@@ -1115,7 +1115,7 @@ static grd_status build_pairs(grd_graph *g)
       if (len > blk_nnz) {
         PullLong L{(uint32_t)q, (uint32_t)blks.size(), 0, 0};
         L.nseg = cut_long_row(tptr[q], tptr[q + 1], blk_nnz,
-                              [&](uint32_t a, uint32_t b) { blks.push_back(PullBlock{(uint32_t)q, 0, a, b}); });
+                              [&blks, q](uint32_t a, uint32_t b) { blks.push_back(PullBlock{(uint32_t)q, 0, a, b}); });
         longs.push_back(L);
         add_arcs = len;
         q++;
