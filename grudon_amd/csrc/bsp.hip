@@ -787,18 +787,26 @@ grd_status op_zero_counters(grd_state *s)
 {
   hipLaunchKernelGGL(k_zero_counters, dim3(1), dim3(kBlock), 0, s->g->ctx->stream, s->cnt, shares(s));
   GRD_HIP(hipGetLastError());
-  counters_at_start(s);
+  counters_at_start(s, false);
   return GRD_OK;
 }
 
-grd_status op_wait_counters(grd_state *s) { return wait_pinned(s->g->ctx, host_seq(s->hcnt), s->cnt_seq); }
+grd_status op_wait_counters(grd_state *s)
+{
+  GRD_TRY(wait_pinned(s->g->ctx, host_seq(s->hcnt), s->cnt_seq));
+  if (s->bound_at == grd_state::kBoundPublished) {
+    s->bound_value = s->hcnt->fmin;
+    s->bound_at = grd_state::kBoundOnHost;
+  }
+  return GRD_OK;
+}
 
 grd_status op_read_counters(grd_state *s)
 {
   hipLaunchKernelGGL(k_publish, dim3(1), dim3(kBlock), 0, s->g->ctx->stream, s->cnt, shares(s), s->hcnt,
                      host_seq(s->hcnt), ++s->cnt_seq);
   GRD_HIP(hipGetLastError());
-  counters_at_start(s);
+  counters_at_start(s, true);
   return op_wait_counters(s);
 }
 
@@ -1030,6 +1038,7 @@ grd_status op_broadcast(grd_state *s, int option)
   GRD_HIP(hipGetLastError());
   s->rdone_sent = rows_done;
   s->bound_sent = bound;
+  s->bound_at = grd_state::kBoundOnDevice;
   s->bound_inc = inc;
   // exchange bytes (GraphAlgorithm.cpp:251-265): bitvector of every pair +
   // packed values (sparse) or the pair's full own slice (dense), and the

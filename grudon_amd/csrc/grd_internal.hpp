@@ -340,7 +340,11 @@ struct grd_state {
   // superstep's smallest broadcast value (sent with a pull broadcast)
   uint64_t *Rdone = nullptr;
   bool rdone_sent = false;   // the last broadcast sent Rdone (a pull of CC / SSSP)
-  bool bound_sent = false;   // the counters hold the smallest value it sent (fmin)
+  bool bound_sent = false;   // it sent the smallest broadcast value (counters: fmin)
+  // where that value is: publishing puts the device's back to its start, and the
+  // host keeps it for a pull that follows the update
+  enum { kBoundOnDevice, kBoundPublished, kBoundOnHost } bound_at = kBoundOnDevice;
+  uint32_t bound_value = 0;
   uint32_t bound_inc = 0;    // the smallest Op::edge increment over an arc
   bool skip_pending = false; // the last pull's skipped arcs are still to be taken from the counters
   uint64_t skip_arc_bytes = 0;  // algorithmic bytes per arc of that pull
@@ -446,12 +450,13 @@ grd_status op_download(grd_state *s, void *out);
 grd_status op_features(grd_state *s, float *out16);
 grd_status op_zero_counters(grd_state *s);
 // what the host notes once the counters and shares are at their start: no
-// shares, no chunks listed, and the smallest broadcast value is gone with them
-// (a pull after that gathers every row's arcs)
-inline void counters_at_start(grd_state *s)
+// shares, no chunks listed, and the smallest broadcast value no longer there
+inline void counters_at_start(grd_state *s, bool published)
 {
   s->n_ushare = s->n_sshare = 0;
-  s->heavy_listed = s->bound_sent = false;
+  s->heavy_listed = false;
+  if (!published) s->bound_sent = false;
+  else if (s->bound_sent && s->bound_at == grd_state::kBoundOnDevice) s->bound_at = grd_state::kBoundPublished;
   s->cnt_clean = true;
 }
 // publishes the counters (and sets them to their start), waits and leaves them in hcnt

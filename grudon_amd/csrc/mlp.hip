@@ -580,7 +580,7 @@ grd_status mlp_publish(grd_state *s, uint64_t prev_frontier)
   hipLaunchKernelGGL(k_mlp_publish, dim3(1), dim3(kBlock), 0, ctx->stream, ctx->sel_w, s->cnt, shares(s), in, s->hcnt,
                      host_seq(s->hcnt), ++s->cnt_seq);
   GRD_HIP(hipGetLastError());
-  counters_at_start(s);
+  counters_at_start(s, true);
   return GRD_OK;
 }
 

@@ -421,6 +421,11 @@ grd_status prp_pull_rows_fixup(hipStream_t st, const PullLong *longs, uint32_t n
 // the whole CSC.
 // CC / SSSP after a broadcast that sent the rows-done bitmap: flag the row
 // blocks (of the cold CSC, or of the whole CSC) that the pull leaves out
+__global__ void k_bound_back(Counters *cnt, uint32_t fmin)
+{
+  if (threadIdx.x == 0) cnt->fmin = fmin;
+}
+
 template <class Op>
 static grd_status blocks_done(grd_state *s, bool cold, const uint8_t **flags)
 {
@@ -431,6 +436,10 @@ static grd_status blocks_done(grd_state *s, bool cold, const uint8_t **flags)
   const bool again = s->n_sshare != 0;
   s->n_sshare = 0;
   if (!Op::kMin || !s->bound_sent) return GRD_OK;
+  if (s->bound_at != grd_state::kBoundOnDevice) {  // an update has come between
+    hipLaunchKernelGGL(k_bound_back, dim3(1), dim3(kWave), 0, s->g->ctx->stream, s->cnt, s->bound_value);
+    s->bound_at = grd_state::kBoundOnDevice;
+  }
   s->skip_pending = true;  // the rows that gathered nothing come off with the counters
   if (!s->rdone_sent) return GRD_OK;
   grd_graph *g = s->g;

@@ -100,3 +100,32 @@ def test_residual_is_pull_pageranks(ctx):
         assert _stats(S)["residual"] == 0
         S.free()
     G.free()
+
+
+@pytest.mark.parametrize("mode,tb", [(0, 0), (3, 4), (3, 8)])
+@pytest.mark.parametrize("algo", ["cc", "weighted"])
+def test_pull_after_the_update_marks_nothing(ctx, mode, tb, algo):
+    """A pull traversal that repeats the superstep's own after its update leaves
+    out the same rows, finds the same values and so marks no proxy for the next
+    reduce."""
+    print("pull after the update", mode, tb, algo, flush=True)
+    g = _graph().with_weights(11)
+    ctx.set_pull_tiling(mode, tb, 0)
+    try:
+        G = api.Graph.from_csr(ctx, g.rp, g.col, g.w, C=1, M=2)
+        seen = []
+        for extra in (0, 1, 2):
+            S = api.State(G, api.CC if algo == "cc" else api.SSSP)
+            S.init(source=3, weighted=algo != "cc")
+            steps = []
+            for _ in range(3):
+                S.step(api.OPT_PULL_SPARSE)
+                for _ in range(extra):
+                    _call("grd_traverse", S, api.OPT_PULL_SPARSE)
+                steps.append((_stats(S)["bytes_exchanged"], S.features().tolist()))
+            seen.append(steps)
+            S.free()
+        assert seen[1] == seen[0] and seen[2] == seen[0]
+        G.free()
+    finally:
+        ctx.set_pull_tiling(3, 0, 0)  # the default
