@@ -1002,7 +1002,7 @@ grd_status op_broadcast(grd_state *s, int option)
   const uint32_t nwS = g->S / 64;
   const bool pull = option & 1, dense = option & 2;
   const bool need_rank = !dense || !pull;
-  s->cnt_clean = false;
+  s->cnt_clean = s->bcast_stale = false;
   if (!pull) {
     s->al_vertices = s->last_frontier;
     s->al_edges = s->last_frontier_edges;
@@ -1149,6 +1149,7 @@ grd_status op_update(grd_state *s)
 {
   grd_graph *g = s->g;
   s->cnt_clean = false;
+  s->bcast_stale = true;
   switch (s->algo) {
   case GRD_PR: launch_update<GRD_PR>(s, 0); break;
   case GRD_CC: launch_update<GRD_CC>(s, 0); break;

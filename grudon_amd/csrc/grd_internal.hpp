@@ -357,6 +357,7 @@ struct grd_state {
   // scan scratch
   uint32_t *blk = nullptr, *wrankB = nullptr, *wrankR = nullptr, *totals = nullptr;
   uint32_t *AL = nullptr;
+  bool bcast_stale = false;  // an update has moved the properties since the broadcast
   // the active list's vertices, their out-arcs and largest out-degree (the
   // frontier's at the push broadcast that wrote it; an update moves the last_*
   // ones on, and a traversal may still follow)

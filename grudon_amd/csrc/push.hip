@@ -45,13 +45,14 @@ __device__ __forceinline__ uint32_t push_owner(const uint32_t *s_off, uint32_t j
 //
 // kShip: the edge-shipping superstep (ship.hip).  The columns are the
 // out-neighbours' compute slots and the updates go to the compute side, where
-// every add marks (addUpdate, relax).  W: the weights' storage.
+// every add marks (addUpdate, relax).  W: the weights' storage.  The values pushed
+// are val by proxy, or by compute slot with the proxies' slots in slot.
 template <class Op, bool kShip, class W>
 __global__ void __launch_bounds__(kBlock) k_push(const uint32_t *__restrict__ AL, const uint32_t *__restrict__ nact,
                                                  const uint32_t *__restrict__ rp, const uint32_t *__restrict__ col,
-                                                 const W *__restrict__ wt, const typename Op::V *__restrict__ mprop,
-                                                 typename Op::V *upd, uint64_t *dirty, uint2 *heavy, Counters *cnt,
-                                                 uint32_t tile)
+                                                 const W *__restrict__ wt, const typename Op::V *__restrict__ val,
+                                                 const uint32_t *__restrict__ slot, typename Op::V *upd,
+                                                 uint64_t *dirty, uint2 *heavy, Counters *cnt, uint32_t tile)
 {
   using V = typename Op::V;
   constexpr int kIlp = 4;
@@ -68,7 +69,7 @@ __global__ void __launch_bounds__(kBlock) k_push(const uint32_t *__restrict__ AL
       p = AL[i];
       beg = rp[p];
       deg = rp[p + 1] - beg;
-      v = mprop[p];
+      v = val[slot ? slot[p] : p];
       if (deg >= kHeavyDeg) nch = (deg + kHeavyChunk - 1) / kHeavyChunk;
     }
     if (__syncthreads_or(nch != 0)) {
@@ -114,7 +115,8 @@ template <class Op, bool kShip, class W>
 __global__ void __launch_bounds__(kBlock) k_push_heavy(const uint2 *__restrict__ heavy, const Counters *cnt,
                                                        const uint32_t *__restrict__ rp, const uint32_t *__restrict__ col,
                                                        const W *__restrict__ wt,
-                                                       const typename Op::V *__restrict__ mprop, typename Op::V *upd,
+                                                       const typename Op::V *__restrict__ val,
+                                                       const uint32_t *__restrict__ slot, typename Op::V *upd,
                                                        uint64_t *dirty)
 {
   using V = typename Op::V;
@@ -124,7 +126,7 @@ __global__ void __launch_bounds__(kBlock) k_push_heavy(const uint2 *__restrict__
     const uint2 ch = heavy[h];
     const uint32_t end = rp[ch.x + 1];
     const uint32_t b = rp[ch.x] + ch.y, ne = min(end - b, kHeavyChunk);
-    const V v = mprop[ch.x];
+    const V v = val[slot ? slot[ch.x] : ch.x];
     for (uint32_t j0 = l; j0 - l < ne; j0 += kIlp * kWave) {
       uint32_t c[kIlp], w[kIlp];
       V x[kIlp];
@@ -157,6 +159,12 @@ static grd_status launch(grd_state *s, const uint32_t *col, const W *wt, typenam
   grd_ctx *ctx = g->ctx;
   hipStream_t st = ctx->stream;
   using V = typename Op::V;
+  // The memory side's proxies hold what was broadcast.  Edge shipping aggregates
+  // the source's property on the compute side: the same value, until an update
+  // has come between.
+  const bool moved = kShip && s->bcast_stale;
+  const V *val = moved ? (const V *)s->prop : (const V *)s->mprop;
+  const uint32_t *slot = moved ? g->proxy_slot : nullptr;
   // tiles of 64 active vertices until those fill every workgroup slot
   const uint64_t slots = (uint64_t)ctx->num_cus * 8;
   const uint32_t tile = s->al_vertices <= 64 * slots ? 64u : (uint32_t)kBlock;
@@ -166,12 +174,12 @@ static grd_status launch(grd_state *s, const uint32_t *col, const W *wt, typenam
   if (s->heavy_listed) hipLaunchKernelGGL(k_heavy_restart, dim3(1), dim3(kWave), 0, st, s->cnt);
   s->heavy_listed = true;
   hipLaunchKernelGGL((k_push<Op, kShip, W>), dim3(grid), dim3(kBlock), 0, st, s->AL, s->totals + 0, g->rp, col, wt,
-                     (const V *)s->mprop, upd, dirty, s->heavy, s->cnt, tile);
+                     val, slot, upd, dirty, s->heavy, s->cnt, tile);
   // a vertex's out-arcs all hang off its own proxy, so the list's largest
   // out-degree tells whether any chunk was appended
   if (s->al_maxdeg >= kHeavyDeg)
     hipLaunchKernelGGL((k_push_heavy<Op, kShip, W>), dim3((uint32_t)slots), dim3(kBlock), 0, st, s->heavy, s->cnt,
-                       g->rp, col, wt, (const V *)s->mprop, upd, dirty);
+                       g->rp, col, wt, val, slot, upd, dirty);
   GRD_HIP(hipGetLastError());
   s->edges += s->al_edges;  // every out-arc of the active list
   return GRD_OK;

@@ -167,3 +167,27 @@ def test_shipping_a_stale_list_is_refused(ctx, C):
     assert np.array_equal(S.result(), ref) and stats["iterations"] == int(st[0])
     S.free()
     G.free()
+
+
+@pytest.mark.parametrize("degree", [8, 70])
+def test_shipping_after_the_update_ships_the_present_values(ctx, degree):
+    """Edge shipping aggregates what the compute side holds: after an update whose
+    frontier is again every vertex, the values of that update and not those that
+    were broadcast (light and heavy vertices)."""
+    print("shipping after the update", degree, flush=True)
+    n = 500
+    src = np.repeat(np.arange(n), degree)
+    dst = (src + np.tile(np.arange(1, degree + 1), n)) % n
+    col = dst.reshape(n, degree)
+    col.sort(axis=1)
+    G = api.Graph.from_csr(ctx, (np.arange(n + 1) * degree).astype(np.uint32), col.ravel().astype(np.uint32), C=1, M=2)
+    S = api.State(G, api.PR)
+    S.init()
+    assert S.step(api.OPT_SHIP_EDGES) == n
+    _call("grd_traverse", S, api.OPT_SHIP_EDGES)
+    assert S.step_update() == n
+    # every vertex gets its in-neighbours' 0.85 u / degree, `degree` of them
+    want = 0.15 * (1 + 0.85 + 0.85 ** 2)
+    assert (np.abs(S.result() - want) <= (3 * degree + 8) * 2.0 ** -24 * want).all()
+    S.free()
+    G.free()
